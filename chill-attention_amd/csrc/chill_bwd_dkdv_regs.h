@@ -42,7 +42,7 @@ constexpr bool dkdv_has_generated_loop() {
 }
 
 template <typename E, int D, int MASK, int CB, int NS>
-__global__ __launch_bounds__(256) void dkdv_regs_kernel(BwdParams p, int n_k_tiles, int total_items,
+__global__ __launch_bounds__(256) void dkdv_regs_kernel(BwdParams p, int n_k_tiles,
                                                        int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     static_assert(Elem<E>::k16, "16-bit element types");
@@ -62,12 +62,10 @@ __global__ __launch_bounds__(256) void dkdv_regs_kernel(BwdParams p, int n_k_til
     static_assert(NS >= 2 && NS <= 4, "ring stages");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int item = xcd_contiguous_item(blockIdx.x, total_items);
-    if (item < 0) return;
-    const int bh = item / n_k_tiles;
     // key tiles first-to-last: for causal-like masks the longest run first
-    const int ktile = item % n_k_tiles;
-    const int b = bh / p.H_kv;
+    int bh, ktile;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, p.work_block, 1, 1, &bh, &ktile)) return;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 
     const int tid = threadIdx.x;

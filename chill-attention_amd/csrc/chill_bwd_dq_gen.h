@@ -62,7 +62,7 @@ CHILL_MFMA16_RB(f16_t, "v_mfma_f32_32x32x16_f16")
 #undef CHILL_MFMA16_RB
 
 template <typename E, int D, int MASK, int NS>
-__global__ __launch_bounds__(256) void dq_regs2_kernel(BwdParams p, int n_q_tiles, int total_items,
+__global__ __launch_bounds__(256) void dq_regs2_kernel(BwdParams p, int n_q_tiles,
                                                       int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     static_assert(Elem<E>::k16 && D == 128 && NS == 4, "16-bit inputs, head dim 128, four ring stages");
@@ -78,11 +78,10 @@ __global__ __launch_bounds__(256) void dq_regs2_kernel(BwdParams p, int n_q_tile
     constexpr int LA = NS - 2;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int item = xcd_contiguous_item(blockIdx.x, total_items);
-    if (item < 0) return;
-    const int bh = item / n_q_tiles;
-    const int qt = n_q_tiles - 1 - item % n_q_tiles;
-    const int b = bh / p.H;
+    int bh, qt;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.work_block, p.group, 1, &bh, &qt)) return;
+    qt = n_q_tiles - 1 - qt;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int hkv = hd / p.group;
 

@@ -22,7 +22,7 @@
 namespace chill {
 
 template <typename E, int D, int MASK, int TK, int NS>
-__global__ __launch_bounds__(256) void dq_regs_kernel(BwdParams p, int n_q_tiles, int total_items,
+__global__ __launch_bounds__(256) void dq_regs_kernel(BwdParams p, int n_q_tiles,
                                                      int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     static_assert(Elem<E>::k16, "16-bit element types");
@@ -38,11 +38,10 @@ __global__ __launch_bounds__(256) void dq_regs_kernel(BwdParams p, int n_q_tiles
     static_assert(NS == 2 || NS == 3, "two or three LDS stages");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int item = xcd_contiguous_item(blockIdx.x, total_items);
-    if (item < 0) return;
-    const int bh = item / n_q_tiles;
-    const int qt = n_q_tiles - 1 - item % n_q_tiles;
-    const int b = bh / p.H;
+    int bh, qt;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.work_block, p.group, 1, &bh, &qt)) return;
+    qt = n_q_tiles - 1 - qt;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int hkv = hd / p.group;
 

@@ -120,7 +120,7 @@ constexpr int dq_waves_per_simd() {
 
 template <typename E, int D, int MASK, int NW, int TK, int NS>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_waves_per_simd<E, D, NW, TK, NS>())))
-void dq_kernel(BwdParams p, int n_q_tiles, int total_items,
+void dq_kernel(BwdParams p, int n_q_tiles,
                                                      int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     constexpr int TQ = NW * 32;
@@ -134,11 +134,10 @@ void dq_kernel(BwdParams p, int n_q_tiles, int total_items,
     static_assert(NS == 2 || NS == 3, "two or three LDS stages");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int item = xcd_contiguous_item(blockIdx.x, total_items, dq_waves_per_simd<E, D, NW, TK, NS>());
-    if (item < 0) return;
-    const int bh = item / n_q_tiles;
-    const int qt = n_q_tiles - 1 - item % n_q_tiles;
-    const int b = bh / p.H;
+    int bh, qt;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.work_block, p.group, dq_waves_per_simd<E, D, NW, TK, NS>(), &bh, &qt)) return;
+    qt = n_q_tiles - 1 - qt;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int hkv = hd / p.group;
 
@@ -368,7 +367,7 @@ void dq_kernel(BwdParams p, int n_q_tiles, int total_items,
 // One (mask, tile shape): SHORT selects the table row for short sequences.
 // (defined below, next to the kernel it is modelled on)
 template <typename E, int D, int MASK, int NW, int NS>
-__global__ void dq_split_kernel(BwdParams p, int n_q_tiles, int total_items, int wave_has_full_blocks);
+__global__ void dq_split_kernel(BwdParams p, int n_q_tiles, int wave_has_full_blocks);
 
 template <typename E, int D, int MASK_ID, bool SHORT>
 int launch_dq_shape(const BwdParams& p, hipStream_t stream) {
@@ -381,7 +380,7 @@ int launch_dq_shape(const BwdParams& p, hipStream_t stream) {
     if (total64 > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
     const int total = (int)total64;
     dim3 grid(cdiv(total, 8) * 8), block(cfg.waves * 64);
-    void (*kern)(BwdParams, int, int, int);
+    void (*kern)(BwdParams, int, int);
     if constexpr (dq_regs_keys(D, Elem<E>::kDType) > 0)
         kern = dq_regs_kernel<E, D, MASK_ID, cfg.streamed, NS>;
     else if constexpr (dq_is_split(D, Elem<E>::kDType))
@@ -394,7 +393,7 @@ int launch_dq_shape(const BwdParams& p, hipStream_t stream) {
                                 cfg.lds_bytes) != hipSuccess)
             return CHILL_ERR_HIP;
     }
-    hipLaunchKernelGGL(kern, grid, block, cfg.lds_bytes, stream, p, n_q_tiles, total, hfb ? 1 : 0);
+    hipLaunchKernelGGL(kern, grid, block, cfg.lds_bytes, stream, p, n_q_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -406,12 +405,12 @@ int launch_dq_regs2(const BwdParams& p, hipStream_t stream) {
     const int64_t total64 = (int64_t)p.B * p.H * n_q_tiles;
     if (total64 > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
     const int total = (int)total64;
-    void (*kern)(BwdParams, int, int, int) = dq_regs2_kernel<E, D, MASK_ID, 4>;
+    void (*kern)(BwdParams, int, int) = dq_regs2_kernel<E, D, MASK_ID, 4>;
     const bool hfb = Mask<MASK_ID>::has_full_blocks(64, cfg.streamed, p.T, p.margs);
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, cfg.lds_bytes) !=
         hipSuccess)
         return CHILL_ERR_HIP;
-    hipLaunchKernelGGL(kern, dim3(cdiv(total, 8) * 8), dim3(cfg.waves * 64), cfg.lds_bytes, stream, p, n_q_tiles, total, hfb ? 1 : 0);
+    hipLaunchKernelGGL(kern, dim3(cdiv(total, 8) * 8), dim3(cfg.waves * 64), cfg.lds_bytes, stream, p, n_q_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -449,7 +448,9 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
 }
 
 template <typename E, int D>
-int launch_dq(const BwdParams& p, int mask_id, hipStream_t stream) {
+int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
+    BwdParams p = args;
+    p.work_block = work_block(mask_id, p.lens != nullptr, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes);
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
     int status = CHILL_ERR_BAD_MASK;
@@ -484,7 +485,7 @@ int launch_dq(const BwdParams& p, int mask_id, hipStream_t stream) {
 // the two products meet in LDS, both waves compute P and dS, and each accumulates half of the head-dim
 // blocks of dQ^T += K^T dS^T.  No MFMA is issued twice and both waves issue the same number.
 template <typename E, int D, int MASK, int NW, int NS>
-__global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_tiles, int total_items,
+__global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_tiles,
                                                       int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     typedef LdsTile<E, D> L;
@@ -502,11 +503,10 @@ __global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_
     static_assert(NS == 2, "two ring stages");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int item = xcd_contiguous_item(blockIdx.x, total_items);
-    if (item < 0) return;
-    const int bh = item / n_q_tiles;
-    const int qt = n_q_tiles - 1 - item % n_q_tiles;
-    const int b = bh / p.H;
+    int bh, qt;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.work_block, p.group, 1, &bh, &qt)) return;
+    qt = n_q_tiles - 1 - qt;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int hkv = hd / p.group;
 
@@ -690,7 +690,7 @@ __global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_
 // and one wave's vector work hides behind the other's MFMAs, with no redundant MFMA work.
 // Four-wave workgroups are compiled for two per CU, those of head dims <= 64 (50 KiB of LDS) for three: 168 registers.
 template <typename E, int D, int MASK, int NW, int NS>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4 ? (D <= 64 ? 3 : 2) : 1))) void dkdv_kernel(BwdParams p, int n_k_tiles, int total_items,
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4 ? (D <= 64 ? 3 : 2) : 1))) void dkdv_kernel(BwdParams p, int n_k_tiles,
                                                        int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     typedef LdsTile<E, D> L;
@@ -711,12 +711,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     // (the 64-row workgroups of head dims up to 64 run three to a CU)
-    const int item = xcd_contiguous_item(blockIdx.x, total_items, (NW == 4 && D <= 64) ? 3 : 1);
-    if (item < 0) return;
-    const int bh = item / n_k_tiles;
     // key tiles first-to-last: for causal-like masks the longest run first
-    const int ktile = item % n_k_tiles;
-    const int b = bh / p.H_kv;
+    int bh, ktile;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, p.work_block, 1, (NW == 4 && D <= 64) ? 3 : 1, &bh, &ktile)) return;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 
     const int tid = threadIdx.x;
@@ -1107,7 +1105,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
 // Q and dO tiles of 32 query rows, for every query head of the GQA group in turn
 // (chill_bwd_dkdv.py:156), with the LSE2 / delta of those rows.
 template <typename E, int D, int MASK, int NW, int SPLIT, int NS>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void dkdv_split_kernel(BwdParams p, int n_k_tiles, int total_items,
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void dkdv_split_kernel(BwdParams p, int n_k_tiles,
                                                         int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     typedef LdsTile<E, D> L;
@@ -1128,12 +1126,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D >= 25
     static_assert(SPLIT % 2 == 0 && DB % SPLIT == 0 && NW % SPLIT == 0, "whole shares");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    const int item = xcd_contiguous_item(blockIdx.x, total_items);
-    if (item < 0) return;
-    const int bh = item / n_k_tiles;
     // key tiles first-to-last: for causal-like masks the longest run first
-    const int ktile = item % n_k_tiles;
-    const int b = bh / p.H_kv;
+    int bh, ktile;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, p.work_block, 1, 1, &bh, &ktile)) return;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 
     const int tid = threadIdx.x;
@@ -1377,7 +1373,7 @@ int launch_dkdv_shape(const BwdParams& p, hipStream_t stream) {
     const int total = (int)total64;
     dim3 grid(cdiv(total, 8) * 8), block(cfg.waves * 64);
     static_assert(!paired || cfg.lds_bytes >= dkdv_paired_exchange_bytes(D) * cfg.waves / 8, "LDS for the pair exchange");
-    void (*kern)(BwdParams, int, int, int);
+    void (*kern)(BwdParams, int, int);
     if constexpr (CB > 0)
         kern = dkdv_regs_kernel<E, D, MASK_ID, CB, dkdv_regs_stages(D)>;
     else if constexpr (paired)
@@ -1391,12 +1387,14 @@ int launch_dkdv_shape(const BwdParams& p, hipStream_t stream) {
                                 cfg.lds_bytes) != hipSuccess)
             return CHILL_ERR_HIP;
     }
-    hipLaunchKernelGGL(kern, grid, block, cfg.lds_bytes, stream, p, n_k_tiles, total, hfb ? 1 : 0);
+    hipLaunchKernelGGL(kern, grid, block, cfg.lds_bytes, stream, p, n_k_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
 template <typename E, int D>
-int launch_dkdv(const BwdParams& p, int mask_id, hipStream_t stream) {
+int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
+    BwdParams p = args;
+    p.work_block = work_block(mask_id, p.lens != nullptr, 1, 2ll * p.group * p.T * D * Elem<E>::kBytes, kWorkBlockBytes);
     int64_t max_stride = p.sq.t > p.sdo.t ? p.sq.t : p.sdo.t;
     if (p.sk.t > max_stride) max_stride = p.sk.t;
     if (p.sv.t > max_stride) max_stride = p.sv.t;

@@ -821,6 +821,21 @@ __device__ __forceinline__ void zero_rows(typename Elem<E>::type* base, int64_t 
     }
 }
 
-// (work-item order: xcd_contiguous_item, chill_tiles.h)
+// (work-item order: work_item, chill_tiles.h)
+
+// The batch element of place `rank` when the elements are ordered by their lengths, longest first (ties by index).
+// The kernels take the heads of a padded batch in this order, so that the short elements end the launch; every
+// workgroup finds it by itself (lane l holds the length of element l: up to 64 elements, others stay in place).
+__device__ __forceinline__ int batch_by_length(const int32_t* lens, int64_t lens_stride, int B, int T, int rank) {
+    if (lens == nullptr || B > 64) return rank;
+    const int lane = threadIdx.x & 63;
+    const int mine = lane < B ? imin(lens[lane * lens_stride], T) : 0;
+    int place = 0;
+    for (int j = 0; j < B; j++) {
+        const int other = __builtin_amdgcn_readlane(mine, j);
+        place += (other > mine || (other == mine && j < lane)) ? 1 : 0;
+    }
+    return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < B && place == rank));
+}
 
 }  // namespace chill

@@ -432,18 +432,16 @@ constexpr int fwd_waves_per_simd() {
 // pair add up to the same amount for every workgroup and the grid finishes without a tail.
 template <typename E, int D, int MASK, int NW, int TK, int NS>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd<E, D, NW, TK, NS>())))
-void fwd_kernel(FwdParams p, int n_q_tiles, int total_items,
+void fwd_kernel(FwdParams p, int n_q_tiles,
                                                       int wave_has_full_blocks, int paired) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // (unpaired q-tiles differ in length: the order for a grid that is resident at once)
-    const int item = xcd_contiguous_item(blockIdx.x, total_items, paired ? 1 : fwd_waves_per_simd<E, D, NW, TK, NS>());
-    if (item < 0) return;
     // paired: a workgroup takes q-tile j from the end and q-tile j from the start (equal work under
     // causal-like masks); unpaired: one q-tile per workgroup, last tiles first
     const int per_head = paired ? (n_q_tiles + 1) / 2 : n_q_tiles;
-    const int bh = item / per_head;
-    const int j = item % per_head;
-    const int b = bh / p.H;
+    int bh, j;
+    if (!work_item(blockIdx.x, p.B * p.H, per_head, p.work_block, p.group, paired ? 1 : fwd_waves_per_simd<E, D, NW, TK, NS>(), &bh, &j)) return;
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int qt_hi = n_q_tiles - 1 - j;
     if constexpr (fwd_is_fast<E, D, TK, NS>()) {
@@ -463,6 +461,16 @@ void fwd_kernel(FwdParams p, int n_q_tiles, int total_items,
 // fewer paired workgroups than an MI355X has CUs: launch one q-tile per workgroup (measured on causal
 // shapes: 16-35 % faster below the threshold, 7-16 % slower at two to four times it)
 constexpr int kPairedMinWorkgroups = 256;
+// Pairs are all of the same length, so a launch of few of them ends with a round that leaves CUs idle; single q-tiles,
+// longest first (work_block), fill it.  Taken where more than a fifth of the last round's share is lost (`slots` =
+// workgroups the chip holds at once: 1.5 rounds of pairs, prefix-LM D128 B4 H16 T3000, 171 -> 159 us; 2.5 rounds, causal
+// B4 H32/8 T2085, 172 / 174; whole rounds 3-4 % slower), and on padded batches, where a pair has no fixed length
+// (causal D128 B8 H16 T1000 48 -> 41 us, T8192 1004 -> 951).
+inline bool fwd_takes_pairs(int64_t pairs, int slots, bool padded) {
+    if (pairs < kPairedMinWorkgroups || padded) return false;
+    const int64_t rounds = (pairs + slots - 1) / slots;
+    return 5 * pairs >= 4 * rounds * slots || pairs < slots;
+}
 
 // One (mask, tile shape): SHORT selects the table row for short sequences.
 template <typename E, int D, int MASK_ID, bool SHORT>
@@ -476,12 +484,14 @@ int launch_fwd_shape(const FwdParams& p, hipStream_t stream) {
     const int n_q_tiles = cdiv(p.T, cfg.rows);
     // pairing q-tiles balances long causal runs; with few workgroups it only halves the number of
     // CUs that get work
-    const bool paired = (int64_t)p.B * p.H * ((n_q_tiles + 1) / 2) >= kPairedMinWorkgroups;
+    const int64_t pairs = (int64_t)p.B * p.H * ((n_q_tiles + 1) / 2);
+    constexpr int kSlots = kComputeUnits * (fwd_uses_regs(D, Elem<E>::kDType) ? 1 : fwd_waves_per_simd<E, D, cfg.waves, cfg.streamed, NS>());
+    const bool paired = fwd_takes_pairs(pairs, kSlots, p.lens != nullptr);
     const int64_t total64 = (int64_t)p.B * p.H * (paired ? (n_q_tiles + 1) / 2 : n_q_tiles);
     if (total64 > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
     const int total = (int)total64;
     dim3 grid(cdiv(total, 8) * 8), block(cfg.waves * 64);
-    void (*kern)(FwdParams, int, int, int, int);
+    void (*kern)(FwdParams, int, int, int);
     if constexpr (fwd_uses_regs(D, Elem<E>::kDType))
         kern = fwd_regs_kernel<E, D, MASK_ID, cfg.streamed, NS>;
     else
@@ -492,7 +502,7 @@ int launch_fwd_shape(const FwdParams& p, hipStream_t stream) {
                                 kLdsBytes) != hipSuccess)
             return CHILL_ERR_HIP;
     }
-    hipLaunchKernelGGL(kern, grid, block, kLdsBytes, stream, p, n_q_tiles, total, hfb ? 1 : 0, paired ? 1 : 0);
+    hipLaunchKernelGGL(kern, grid, block, kLdsBytes, stream, p, n_q_tiles, hfb ? 1 : 0, paired ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -522,7 +532,9 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
 }
 
 template <typename E, int D>
-int launch_fwd(const FwdParams& p, int mask_id, hipStream_t stream) {
+int launch_fwd(const FwdParams& args, int mask_id, hipStream_t stream) {
+    FwdParams p = args;
+    p.work_block = work_block(mask_id, p.lens != nullptr, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes / 2);
     // the async loader keeps per-lane global offsets in 32 bits
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;

@@ -287,16 +287,14 @@ __device__ __forceinline__ void fwd_q_tile_regs(const FwdParams& p, char* smem, 
 
 // The workgroup-to-q-tile mapping of fwd_kernel (pairs of q-tiles, or one each).
 template <typename E, int D, int MASK, int TK, int NS>
-__global__ __launch_bounds__(256) void fwd_regs_kernel(FwdParams p, int n_q_tiles, int total_items,
+__global__ __launch_bounds__(256) void fwd_regs_kernel(FwdParams p, int n_q_tiles,
                                                       int wave_has_full_blocks, int paired) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int item = xcd_contiguous_item(blockIdx.x, total_items);
-    if (item < 0) return;
-    agpr_reserve();
     const int per_head = paired ? (n_q_tiles + 1) / 2 : n_q_tiles;
-    const int bh = item / per_head;
-    const int j = item % per_head;
-    const int b = bh / p.H;
+    int bh, j;
+    if (!work_item(blockIdx.x, p.B * p.H, per_head, p.work_block, p.group, 1, &bh, &j)) return;
+    agpr_reserve();
+    const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int qt_hi = n_q_tiles - 1 - j;
     fwd_q_tile_regs<E, D, MASK, TK, NS>(p, smem, b, hd, qt_hi, wave_has_full_blocks);

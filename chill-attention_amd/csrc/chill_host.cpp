@@ -155,6 +155,15 @@ int chill_work_item(int32_t workgroup, int32_t total, int32_t resident) {
     return xcd_contiguous_item(workgroup, total, resident);
 }
 
+int chill_launch_item(int32_t workgroup, int32_t heads, int32_t per_head, int32_t block, int32_t streams,
+                      int32_t resident, int32_t out[2]) {
+    if (out == nullptr) return CHILL_ERR_NULL_POINTER;
+    if (workgroup < 0 || heads < 1 || per_head < 1 || block < 0 || streams < 1 || heads % streams != 0 || resident < 1 ||
+        (int64_t)heads * per_head > (1 << 30))
+        return CHILL_ERR_BAD_ARGUMENT;
+    return work_item(workgroup, heads, per_head, block, streams, resident, &out[0], &out[1]) ? 1 : 0;
+}
+
 const char* chill_status_string(int32_t status) {
     switch (status) {
         case CHILL_OK: return "ok";

@@ -23,6 +23,7 @@ struct FwdParams {
     int64_t lens_stride;
     int32_t B, H, H_kv, T;
     int32_t group;         // H / H_kv
+    int32_t work_block;    // order of the workgroups (work_block, chill_tiles.h)
     float scale_log2;      // sm_scale * log2(e)
     MaskArgs margs;
 };
@@ -57,6 +58,7 @@ struct BwdParams {
     int64_t lens_stride;
     int32_t B, H, H_kv, T;
     int32_t group;
+    int32_t work_block;  // order of the workgroups (work_block, chill_tiles.h)
     float sm_scale;
     float scale_log2;
     MaskArgs margs;

@@ -484,4 +484,71 @@ CHILL_HD int xcd_contiguous_item(int wg, int total, int resident = 1) {
     return (local < per && item < total) ? item : -1;
 }
 
+// The order in which a launch's workgroups take their (head, tile) items, as the number of heads of a BLOCK: the blocks
+// follow each other, inside one the workgroups take tile 0 of every head, then tile 1 of every head, and so on, and head
+// u of a block belongs to XCD u % 8 (work_item).  The kernels number a head's tiles from the heavy end of a causal-like
+// mask, so a block, the last one above all, ends with its short tiles; a whole launch as one block is longest first, but
+// streams the K and V (in dK/dV the Q and dO) of all its heads at once through an XCD's L2 (4 MiB) and the last-level
+// cache (256 MiB).  So a block holds as many heads per XCD as stream about 16 MiB, two at the least.
+// 0: every XCD takes a contiguous run of heads, one after the other (xcd_contiguous_item).
+// Measured, forward / dQ / dK/dV in us, contiguous runs -> blocks of this size (bf16):
+//   causal D128 B4 H32/8 T2085    205 / 233 / 354 -> 172 / 214 / 288      causal D64 B4 H16 T4096  144 / 222 / 327 -> 143 / 191 / 284
+//   causal D128 B8 H16 T4096  488 / 755 / 1060 -> 488 / 717 / 988         causal D128 B8 H16 T8192 1741 / 2560 / 3435 -> 1735 / 2506 / 3350
+//   (D128 B8 H16 as one block: T4096 501 / 747 / 998, T8192 1878 / 2660 / 3518)
+//   causal D256 B4 H8 T2048 87 / 158 / 227 -> 86 / 113 / 155; full mask fp16 D64 B8 H12 T4042 469 / 579 / 724 -> 433 / 576 / 725
+// The forward, whose pairs of q-tiles are all of the same length, has nothing to balance and takes half of that (causal
+// D128 B8 H16 T8192: 1735 with two heads per XCD, 1748 with four).  Banded masks, whose tiles are all alike and share
+// their keys with the next tile, keep the contiguous runs (within 2 % either way).
+// A padded batch: the work of a head depends on its batch element, and contiguous runs gave the long elements to some
+// XCDs and the short ones to others.  Two heads per XCD, the elements longest first (batch_by_length): the order that
+// was never far from the best over blocks of 1, 2, 4, 8 and all heads, lengths of T/4 .. T, unsorted or sorted: causal
+// D128 B4 H32/8 T2085 197 / 219 / 340 -> 116 / 139 / 210, B8 H16 T8192 1456 / 2199 / 2935 -> 969 / 1368 / 1830,
+// full mask B8 H16 T2085 303 / 348 / 446 -> 172 / 229 / 290, sliding window 128 + 128 B8 H16 T4042 154 / 183 / 271 ->
+// 127 / 158 / 217.
+// `streams` = heads that share what they stream (H / H_kv in the forward and dQ, 1 in dK/dV); `bytes` = what is streamed
+// for one such set of heads.
+constexpr long long kWorkBlockBytes = 16ll << 20;
+constexpr int work_block(int mask_id, bool padded, int streams, long long bytes, long long budget) {
+    if (padded) budget = 0;
+    else if (mask_is_banded(mask_id)) return 0;
+    const long long heads = (budget / bytes < 2 ? 2 : budget / bytes) * 8 * streams;
+    return heads < (1ll << 30) ? (int)heads : 1 << 30;
+}
+
+// Workgroup `wg` of a launch of `heads` heads (query heads, or key / value heads in dK/dV; `streams` of them share what
+// they stream) of `per_head` tiles each, in the order `block`: its head and tile, or false if it has nothing to do.
+// `resident` as in xcd_contiguous_item.
+CHILL_HD bool work_item(int wg, int heads, int per_head, int block, int streams, int resident, int* head, int* tile) {
+    constexpr int kXcds = 8, kCusPerXcd = 32;
+    const int total = heads * per_head;
+    if (block == 0) {
+        const int item = xcd_contiguous_item(wg, total, resident);
+        if (item < 0) return false;
+        *head = item / per_head;
+        *tile = item - *head * per_head;
+        return true;
+    }
+    if (wg >= total) return false;
+    if (resident > 1 && total > kXcds * kCusPerXcd && total <= resident * kXcds * kCusPerXcd) {
+        const int xcd = wg % kXcds, local = wg / kXcds, pass = local / kCusPerXcd;
+        const int mine = (total - xcd + kXcds - 1) / kXcds;  // items of this XCD
+        if (pass & 1) {
+            const int len = mine - pass * kCusPerXcd < kCusPerXcd ? mine - pass * kCusPerXcd : kCusPerXcd;
+            wg = (pass * kCusPerXcd + len - 1 - (local - pass * kCusPerXcd)) * kXcds + xcd;
+        }
+    }
+    const int first = block < heads ? wg / (block * per_head) * block : 0;  // first head of the block
+    const int size = heads - first < block ? heads - first : block;
+    const int i = wg - first * per_head;
+    *tile = i / size;
+    int u = i - *tile * size;
+    // in whole rounds of sets the heads of a set stay on one XCD
+    if (streams > 1 && size % (kXcds * streams) == 0) {
+        const int xcd = u % kXcds, k = u / kXcds;
+        u = (xcd + kXcds * (k / streams)) * streams + k % streams;
+    }
+    *head = first + u;
+    return true;
+}
+
 }  // namespace chill

@@ -210,6 +210,13 @@ int chill_mask_limits(const ChillMaskDesc* mask, int32_t which, int32_t n, int32
  * the reference's kernels (chill_fwd.py:58-61, chill_bwd.py:71-84). */
 int chill_work_item(int32_t workgroup, int32_t total, int32_t resident);
 
+/* The head and the tile (out[0], out[1]) that workgroup `workgroup` of a launch of `heads` heads of `per_head` tiles
+ * each takes, and 1; 0 when it has none.  `block` = heads taken together, tile by tile (0: head by head, in the order of
+ * chill_work_item); `streams` = neighbouring heads that share what they stream.  Over the workgroups of a grid the
+ * (head, tile) pairs are a permutation of all of them. */
+int chill_launch_item(int32_t workgroup, int32_t heads, int32_t per_head, int32_t block, int32_t streams,
+                      int32_t resident, int32_t out[2]);
+
 /* Host twin of chill_tile_ranges_device (same functors compiled for the host). */
 int chill_tile_ranges(const ChillMaskDesc* mask, int32_t pass, int32_t T, int32_t seq_len,
                       int32_t tile_in, int32_t tile_out, int32_t* out);

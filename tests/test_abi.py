@@ -290,6 +290,31 @@ def test_work_items_are_a_permutation_and_resident_grids_balance():
             assert len(plain) > 1
 
 
+@pytest.mark.parametrize("resident", [1, 2, 3])
+@pytest.mark.parametrize("streams", [1, 4])
+def test_launch_items_are_a_permutation(streams, resident):
+    """Every (head, tile) of a launch is taken by exactly one workgroup, whatever the block: sizes that divide the heads or
+    leave a remainder, one head, more than all heads, grids either side of what the chip holds at once."""
+    out = (ctypes.c_int32 * 2)()
+    f = _lib.lib.chill_launch_item
+    for sets in (1, 3, 8, 13, 16, 24):
+        heads = sets * streams
+        for per_head in (1, 5, 17):
+            for block in (0, 1, 8 * streams, 16 * streams, 40, heads, 1 << 30):
+                grid = -(-heads * per_head // 8) * 8
+                got = []
+                for w in range(grid):
+                    if f(w, heads, per_head, block, streams, resident, out):
+                        got.append((out[0], out[1]))
+                want = [(u, t) for u in range(heads) for t in range(per_head)]
+                assert sorted(got) == want, (heads, per_head, block, streams, resident)
+    # a head stays on one XCD where the block is made of whole rounds, and with it the heads that share what they stream
+    for w in range(64 * streams * 5):
+        assert f(w, 64 * streams, 5, 16 * streams, streams, 1, out) == 1
+        assert out[0] // streams % 8 == w % 8
+    assert f(-1, 8, 1, 0, 1, 1, out) == -8 and f(0, 6, 1, 0, 4, 1, out) == -8 and f(0, 8, 1, 0, 1, 1, None) == -1
+
+
 def test_cpu_tensors_are_refused():
     import torch
 

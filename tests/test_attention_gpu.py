@@ -1012,3 +1012,37 @@ def test_device_functors_equal_host():
                     ctypes.byref(desc), pass_id, T, seq_len, tin, tout, ctypes.c_void_p(out.data_ptr()),
                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
                 assert torch.equal(out.cpu(), mask._calc_tile_ranges(T, tin, tout, pass_id, seq_len))
+
+
+@pytest.mark.parametrize("D,dtype,B,H,Hkv,T", [(128, torch.bfloat16, 5, 8, 2, 1100), (64, torch.float16, 9, 3, 3, 1030),
+                                               (256, torch.bfloat16, 3, 4, 4, 700), (64, torch.float32, 70, 2, 1, 1056)])
+@pytest.mark.parametrize("m", [("CausalChillMask", ()), ("SlidingWindowChillMask", (60, 20)), ("FullChillMask", ())], ids=mask_id)
+def test_padded_batches_in_order_of_length(m, D, dtype, B, H, Hkv, T):
+    """The heads of a padded batch run in the order of their lengths (up to 64 elements; 70 stay in place), equal lengths
+    and empty elements among them, on grids that the ordinary kernels serve; tolerances as in the matrix."""
+    mask = make_mask(m)
+    rng = np.random.default_rng(stable_seed(m, D, B, "order"))
+    vals = rng.integers(1, T + 1, B)
+    vals[0], vals[1], vals[2] = T, 0, T + 5
+    lens = torch.tensor(vals, dtype=torch.int32, device=DEV)
+    print(f"padded order {mask} {dtype} D={D} B={B} H={H}/{Hkv} T={T} lens={vals.tolist()}", flush=True)
+    q = make_qkv((B, H, T, D), dtype, False).requires_grad_()
+    k = make_qkv((B, Hkv, T, D), dtype, False).requires_grad_()
+    v = make_qkv((B, Hkv, T, D), dtype, False).requires_grad_()
+    dout = make_qkv((B, H, T, D), torch.float32, False)
+    in_len = torch.arange(T, device=DEV)[None, None, :, None] < lens[:, None, None, None]
+    dout = (dout * in_len).to(dtype)
+    out = ca.chill_attention(q, k, v, mask=mask, lens=lens)
+    out.backward(dout)
+    for b in range(B):
+        n = min(int(vals[b]), T)
+        for x in (out, q.grad, k.grad, v.grad):
+            assert (x[b, :, n:] == 0).all(), f"element {b}: rows beyond its length"
+        if n == 0:
+            continue
+        qf, kf, vf = (x.detach()[b : b + 1, :, :n].float().clone().requires_grad_() for x in (q, k, v))
+        ref, _ = orc.reference_naive(m[0], m[1], qf, kf, vf, None)
+        ref.backward(dout[b : b + 1, :, :n].float())
+        check_close(out.detach()[b : b + 1, :, :n], ref.detach(), dtype, OUT_TOL[dtype], D, f"O[{b}]")
+        for name, got, want in (("dq", q.grad, qf.grad), ("dk", k.grad, kf.grad), ("dv", v.grad, vf.grad)):
+            check_close(got[b : b + 1, :, :n], want, dtype, GRAD_TOL[dtype], D, f"{name}[{b}]")
