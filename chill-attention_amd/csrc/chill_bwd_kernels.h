@@ -450,7 +450,7 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
 template <typename E, int D>
 int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
-    p.work_block = work_block(mask_id, p.lens != nullptr, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes);
+    p.work_block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes);
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
     int status = CHILL_ERR_BAD_MASK;
@@ -1394,7 +1394,7 @@ int launch_dkdv_shape(const BwdParams& p, hipStream_t stream) {
 template <typename E, int D>
 int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
-    p.work_block = work_block(mask_id, p.lens != nullptr, 1, 2ll * p.group * p.T * D * Elem<E>::kBytes, kWorkBlockBytes);
+    p.work_block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H_kv, 1, 2ll * p.group * p.T * D * Elem<E>::kBytes, kWorkBlockBytes);
     int64_t max_stride = p.sq.t > p.sdo.t ? p.sq.t : p.sdo.t;
     if (p.sk.t > max_stride) max_stride = p.sk.t;
     if (p.sv.t > max_stride) max_stride = p.sv.t;

@@ -534,7 +534,7 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
 template <typename E, int D>
 int launch_fwd(const FwdParams& args, int mask_id, hipStream_t stream) {
     FwdParams p = args;
-    p.work_block = work_block(mask_id, p.lens != nullptr, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes / 2);
+    p.work_block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes / 2);
     // the async loader keeps per-lane global offsets in 32 bits
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;

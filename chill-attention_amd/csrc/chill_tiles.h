@@ -505,14 +505,17 @@ CHILL_HD int xcd_contiguous_item(int wg, int total, int resident = 1) {
 // D128 B4 H32/8 T2085 197 / 219 / 340 -> 116 / 139 / 210, B8 H16 T8192 1456 / 2199 / 2935 -> 969 / 1368 / 1830,
 // full mask B8 H16 T2085 303 / 348 / 446 -> 172 / 229 / 290, sliding window 128 + 128 B8 H16 T4042 154 / 183 / 271 ->
 // 127 / 158 / 217.
-// `streams` = heads that share what they stream (H / H_kv in the forward and dQ, 1 in dK/dV); `bytes` = what is streamed
+// `heads` = heads of the launch; `streams` = heads that share what they stream (H / H_kv in the forward and dQ, 1 in dK/dV); `bytes` = what is streamed
 // for one such set of heads.
 constexpr long long kWorkBlockBytes = 16ll << 20;
-constexpr int work_block(int mask_id, bool padded, int streams, long long bytes, long long budget) {
-    if (padded) budget = 0;
-    else if (mask_is_banded(mask_id)) return 0;
-    const long long heads = (budget / bytes < 2 ? 2 : budget / bytes) * 8 * streams;
-    return heads < (1ll << 30) ? (int)heads : 1 << 30;
+// Blocks of one size: a last block of fewer heads would end the launch on a part of the XCDs' CUs (causal D128 B4 H32/8
+// T2085 dK/dV, four heads per XCD: 290 us as one block of four, 373 as three and one).
+constexpr int work_block(int mask_id, bool padded, long long heads, int streams, long long bytes, long long budget) {
+    if (!padded && mask_is_banded(mask_id)) return 0;
+    const long long rounds = (heads + 8 * streams - 1) / (8 * streams);  // sets per XCD
+    const long long most = padded || budget / bytes < 2 ? 2 : budget / bytes;
+    const long long blocks = rounds / most < 1 ? 1 : rounds / most;
+    return (int)((rounds + blocks - 1) / blocks * 8 * streams);
 }
 
 // Workgroup `wg` of a launch of `heads` heads (query heads, or key / value heads in dK/dV; `streams` of them share what
