@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void dq_regs_kernel(BwdParams p, int n_q_tiles
     const Range vis = visible_range<MASK, true>(q_pos, seq_len, p.margs);  // the keys this lane's row sees
 
     TileRange wr = {wg.start, wg.start, wg.start, wg.start};
-    if (qw < seq_len) wr = tile_range<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
+    if (qw < seq_len) wr = tile_range_rows_discarded<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
     const int ta = wr.start - wg.start, tb = wr.end - wg.start;
     const int fa = wr.full_start - wg.start, fb = wr.full_end - wg.start;
 

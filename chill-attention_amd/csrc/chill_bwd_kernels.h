@@ -202,7 +202,7 @@ void dq_kernel(BwdParams p, int n_q_tiles,
     const Range vis = visible_range<MASK, true>(q_pos, seq_len, p.margs);  // the keys this lane's row sees
 
     TileRange wr = {wg.start, wg.start, wg.start, wg.start};
-    if (qw < seq_len) wr = tile_range<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
+    if (qw < seq_len) wr = tile_range_rows_discarded<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
     const int ta = wr.start - wg.start, tb = wr.end - wg.start;
     const int fa = wr.full_start - wg.start, fb = wr.full_end - wg.start;
 
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_
     }
 
     TileRange wr = {wg.start, wg.start, wg.start, wg.start};
-    if (qw < seq_len) wr = tile_range<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
+    if (qw < seq_len) wr = tile_range_rows_discarded<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
     const int ta = wr.start - wg.start, tb = wr.end - wg.start;
     const int fa = wr.full_start - wg.start, fb = wr.full_end - wg.start;
 
@@ -822,7 +822,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
     ofs.init(lane);
 
     TileRange wr = {wg.start, wg.start, wg.start, wg.start};
-    if (kw < seq_len) wr = tile_range<MASK, false>(kw, 32, TQS, seq_len, wave_has_full_blocks != 0, p.margs);
+    if (kw < seq_len) wr = tile_range_rows_discarded<MASK, false>(kw, 32, TQS, seq_len, wave_has_full_blocks != 0, p.margs);
     const int ta = wr.start - wg.start, tb = wr.end - wg.start;
     const int fa = wr.full_start - wg.start, fb = wr.full_end - wg.start;
 
@@ -1210,7 +1210,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D >= 25
     }
 
     TileRange wr = {wg.start, wg.start, wg.start, wg.start};
-    if (kw < seq_len) wr = tile_range<MASK, false>(kw, 32, TQS, seq_len, wave_has_full_blocks != 0, p.margs);
+    if (kw < seq_len) wr = tile_range_rows_discarded<MASK, false>(kw, 32, TQS, seq_len, wave_has_full_blocks != 0, p.margs);
     const int ta = wr.start - wg.start, tb = wr.end - wg.start;
     const int fa = wr.full_start - wg.start, fb = wr.full_end - wg.start;
 

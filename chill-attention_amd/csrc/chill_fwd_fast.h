@@ -203,7 +203,7 @@ __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem,
         int g0 = 0, g1 = 0, f0 = 0, f1 = 0;
         if (qw < seq_len) {
             const TileRange wr =
-                tile_range<MASK, true>(qw, 32, 32, seq_len, M::has_full_blocks(32, 32, p.T, p.margs), p.margs);
+                tile_range_rows_discarded<MASK, true>(qw, 32, 32, seq_len, M::has_full_blocks(32, 32, p.T, p.margs), p.margs);
             const int base = wg.start * KB;
             g0 = imax(wr.start - base, 0);
             g1 = imin(wr.end - base, n_tiles * KB);

@@ -113,7 +113,7 @@ __device__ __forceinline__ void fwd_q_tile(const FwdParams& p, char* smem, int b
     load_resident<E, D>(qf, qptr + (int64_t)qw * p.sq.t, p.sq.t, p.T - qw, lane);
 
     TileRange wr = {wg.start, wg.start, wg.start, wg.start};
-    if (qw < seq_len) wr = tile_range<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
+    if (qw < seq_len) wr = tile_range_rows_discarded<MASK, true>(qw, 32, TK, seq_len, wave_has_full_blocks != 0, p.margs);
     // this wave's tiles, as offsets into the workgroup's ring
     const int ta = wr.start - wg.start, tb = wr.end - wg.start;
     const int fa = wr.full_start - wg.start, fb = wr.full_end - wg.start;
