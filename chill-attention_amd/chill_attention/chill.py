@@ -120,14 +120,19 @@ def register_chill_mask(mask: ChillMask):
             LSE = torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
         lens_ptr, lens_stride = _lens_args(lens)
         tq, tk, tv, to = _lib.tensor4(qv), _lib.tensor4(kv), _lib.tensor4(vv), _lib.tensor4(O)
+        workspace_bytes = mask_lib.chill_fwd_workspace_bytes(
+            batch, heads, T, head_dim, _DTYPES[q.dtype], ctypes.byref(desc), lens is not None
+        )
+        workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device) if workspace_bytes > 0 else None
         with torch.cuda.device(q.device):
-            status = mask_lib.chill_fwd(
+            status = mask_lib.chill_fwd_workspace(
                 ctypes.byref(tq), ctypes.byref(tk), ctypes.byref(tv), ctypes.byref(to),
                 ctypes.c_void_p(LSE.data_ptr()) if LSE is not None else None,
                 _lib.strides3(LSE) if LSE is not None else None,
                 lens_ptr, lens_stride,
                 batch, heads, k.shape[1], T, head_dim, _DTYPES[q.dtype], float(sm_scale),
-                ctypes.byref(desc), ctypes.c_void_p(_stream_ptr(q)),
+                ctypes.byref(desc), ctypes.c_void_p(workspace.data_ptr()) if workspace is not None else None,
+                max(workspace_bytes, 0), ctypes.c_void_p(_stream_ptr(q)),
             )
         _lib.check("chill_fwd", status)
         if LSE is None:

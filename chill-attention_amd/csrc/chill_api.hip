@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "chill_mask.h"
+#include "chill_fwd_split.h"
 #include "chill_params.h"
 
 namespace chill {
@@ -16,14 +17,14 @@ namespace chill {
     X(bf16, 16) X(bf16, 32) X(bf16, 64) X(bf16, 128) X(bf16, 256)
 
 #define CHILL_DECLARE(name, d)                                                              \
-    int launch_fwd_##name##_##d(const FwdParams&, int, hipStream_t);                        \
+    int launch_fwd_##name##_##d(const FwdParams&, int, const FwdSplit*, hipStream_t);                        \
     int launch_delta_##name##_##d(const DeltaParams&, hipStream_t);                         \
     int launch_dq_##name##_##d(const BwdParams&, int, hipStream_t);                         \
     int launch_dkdv_##name##_##d(const BwdParams&, int, hipStream_t);
 CHILL_FOR_EACH_INST(CHILL_DECLARE)
 #undef CHILL_DECLARE
 
-typedef int (*FwdLauncher)(const FwdParams&, int, hipStream_t);
+typedef int (*FwdLauncher)(const FwdParams&, int, const FwdSplit*, hipStream_t);
 typedef int (*DeltaLauncher)(const DeltaParams&, hipStream_t);
 typedef int (*BwdLauncher)(const BwdParams&, int, hipStream_t);
 
@@ -113,6 +114,47 @@ int chill_fwd(const ChillTensor4* q, const ChillTensor4* k, const ChillTensor4* 
               const int32_t* lens, int64_t lens_stride,
               int32_t B, int32_t H, int32_t H_kv, int32_t T, int32_t D,
               int32_t dtype, float sm_scale, const ChillMaskDesc* mask, void* stream) {
+    return chill_fwd_workspace(q, k, v, o, lse, lse_stride, lens, lens_stride, B, H, H_kv, T, D, dtype, sm_scale, mask, nullptr,
+                               0, stream);
+}
+
+int64_t chill_fwd_workspace_bytes(int32_t B, int32_t H, int32_t T, int32_t D, int32_t dtype, const ChillMaskDesc* mask,
+                                  int32_t has_lens) {
+    int es = 0;
+    MaskArgs margs;
+    FwdSplit split;
+    CHILL_TRY(check_dtype_dim(dtype, D, &es));
+    CHILL_TRY(check_shape(B, H, H, T));
+    CHILL_TRY(lower_mask(mask, &margs));
+    return has_lens ? 0 : plan_fwd_split(mask->id, margs, (int64_t)B * H, T, D, dtype, nullptr, &split);
+}
+
+int chill_fwd_split_items(int32_t B, int32_t H, int32_t T, int32_t D, int32_t dtype, const ChillMaskDesc* mask,
+                          int32_t items[CHILL_FWD_SPLIT_MAX_ITEMS][4]) {
+    int es = 0;
+    MaskArgs margs;
+    FwdSplit split;
+    if (items == nullptr) return CHILL_ERR_NULL_POINTER;
+    CHILL_TRY(check_dtype_dim(dtype, D, &es));
+    CHILL_TRY(check_shape(B, H, H, T));
+    CHILL_TRY(lower_mask(mask, &margs));
+    if (plan_fwd_split(mask->id, margs, (int64_t)B * H, T, D, dtype, nullptr, &split) == 0) return 0;
+    for (int i = 0; i < split.n_items; i++) {
+        const uint32_t item = split.item[i];
+        items[i][0] = item & 1023;
+        items[i][1] = (item >> 10) & 31;
+        items[i][2] = (item >> 15) & 31;
+        items[i][3] = item >> 20;
+    }
+    return split.n_items;
+}
+
+int chill_fwd_workspace(const ChillTensor4* q, const ChillTensor4* k, const ChillTensor4* v,
+                        const ChillTensor4* o, float* lse, const int64_t lse_stride[3],
+                        const int32_t* lens, int64_t lens_stride,
+                        int32_t B, int32_t H, int32_t H_kv, int32_t T, int32_t D,
+                        int32_t dtype, float sm_scale, const ChillMaskDesc* mask, void* workspace,
+                        int64_t workspace_bytes, void* stream) {
     int es = 0;
     FwdParams p = {};
     CHILL_TRY(check_dtype_dim(dtype, D, &es));
@@ -137,7 +179,15 @@ int chill_fwd(const ChillTensor4* q, const ChillTensor4* k, const ChillTensor4* 
     p.T = T;
     p.group = H / H_kv;
     CHILL_TRY(lower_scale(sm_scale, &p.scale_log2));
-    return kFwd[dtype][dim_index(D)](p, mask->id, static_cast<hipStream_t>(stream));
+    FwdSplit split;
+    bool use_split = false;
+    if (workspace != nullptr && lens == nullptr) {
+        if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return CHILL_ERR_BAD_STRIDE;
+        const int64_t bytes = plan_fwd_split(mask->id, p.margs, (int64_t)B * H, T, D, dtype, workspace, &split);
+        if (bytes > workspace_bytes) return CHILL_ERR_BAD_ARGUMENT;
+        use_split = bytes > 0;
+    }
+    return kFwd[dtype][dim_index(D)](p, mask->id, use_split ? &split : nullptr, static_cast<hipStream_t>(stream));
 }
 
 int chill_bwd_delta(const ChillTensor4* o, const ChillTensor4* d_o, float* delta,

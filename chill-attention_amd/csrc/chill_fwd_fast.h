@@ -81,13 +81,35 @@ __device__ __forceinline__ bool workgroup_any(bool mine, char* flags) {
     return __builtin_amdgcn_readfirstlane(any) != 0;  // (the same in every lane: say so to the compiler)
 }
 
-// The q-tiles qt_a and then qt_b (-1: none) of one head, start to finish.  While the rows of one q-tile
+// One part of a q-tile's keys (FwdSplit): which of how many, and where its partial result goes: O^T as the accumulators
+// hold it, then the row's reference m0 and sum l of every lane.  l = NaN: a row left the range the reference-free softmax
+// is exact in.  A q-tile of one part leaves its result, and in `again` whether such a row makes it wrong.
+struct FwdPart {
+    int index, count, tiles;
+    float* partial;
+    uint32_t* again;
+};
+template <int D, int NW>
+__device__ __forceinline__ void store_partial(float* to, const f32x16 (&o)[D / 32], float m0, float l) {
+    constexpr int DB = D / 32, NT = NW * 64;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *reinterpret_cast<f32x4*>(to + ((db * 4 + g) * NT + tid) * 4) =
+                f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+    to[DB * 16 * NT + tid] = m0;
+    to[DB * 16 * NT + NT + tid] = l;
+}
+
+// The q-tiles qt_a and then qt_b (-1: none) of one head, start to finish, or (SPLIT) one part of q-tile qt_a's keys.  While the rows of one q-tile
 // are normalised and stored, the first K/V tiles and the Q rows of the next one are already on their
 // way.  A q-tile in which a row left the range the reference-free softmax is exact in is computed
 // again by fwd_q_tile.
-template <typename E, int D, int MASK, int NW, int TK, int NS>
+template <typename E, int D, int MASK, int NW, int TK, int NS, bool SPLIT = false>
 __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem, int b, int hd, int qt_a, int qt_b,
-                                                 int wave_has_full_blocks) {
+                                                 int wave_has_full_blocks, FwdPart part = FwdPart{0, 1, 0, nullptr, nullptr}) {
     using ET = typename Elem<E>::type;
     using M = Mask<MASK>;
     typedef FwdLds<E, D, TK> Lds;
@@ -172,6 +194,12 @@ __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem,
         wg_pre = TileRange{0, 0, 0, 0};
         if (qb >= seq_len) return;
         wg_pre = tile_range<MASK, true>(qb, TQ, TK, seq_len, false, p.margs);
+        if constexpr (SPLIT) {
+            if (part.count > 1) {
+                wg_pre.start += part.index * part.tiles;
+                if (part.index + 1 < part.count) wg_pre.end = wg_pre.start + part.tiles;
+            }
+        }
 #pragma unroll
         for (int i = 0; i <= 1 + FL; i++)
             if (wg_pre.start + i < wg_pre.end) issue_tile(wg_pre.start + i, i);
@@ -428,6 +456,14 @@ __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem,
 
         // epilogue: O = acc / l, LSE2 = m0 + log2(l) (chill_fwd.py:288-289, 327-328)
         const float l_tot = sum_across_halves(l_run);
+        if constexpr (SPLIT) {
+            if (part.count > 1) {
+                const bool sees = imax(vis.lo, wg.start * TK) <= imin(vis.hi, wg.end * TK - 1);
+                const bool out_of_range = sees && !(l_tot >= Lim::kLo && l_tot <= Lim::kHi);
+                store_partial<D, NW>(part.partial, o, m0, out_of_range ? __builtin_nanf("") : l_tot);
+                return;
+            }
+        }
         const float l_safe = (l_tot == 0.f) ? 1.f : l_tot;
         const float inv = 1.f / l_safe;
         const bool valid = q_pos < seq_len;
@@ -441,6 +477,11 @@ __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem,
         // a row that sees keys must end with a sum inside the range (a NaN fails the comparison too)
         const bool bad = (vis.lo <= vis.hi) && !(l_tot >= Lim::kLo && l_tot <= Lim::kHi);
         const bool again = __builtin_amdgcn_ballot_w64(bad) != 0;
+        if constexpr (SPLIT) {
+            const bool any = workgroup_any<NW>(again, smem + NS * Lds::STAGE_BYTES);
+            if (tid == 0) *part.again = any ? 1 : 0;
+            return;
+        }
         if (workgroup_any<NW>(again, smem + NS * Lds::STAGE_BYTES)) {
             // rare: give the ring to the kernel whose softmax follows the running max, then start over on
             // the next q-tile
@@ -451,6 +492,53 @@ __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem,
             if (qt_next >= 0) prefetch(qt_next);
         }
     }
+}
+
+// The result of q-tile qt from the partial results of its `count` parts, added up in the order of the keys.
+template <typename E, int D, int MASK, int NW, int TK, int NS>
+__device__ __forceinline__ void fwd_merge_q_tile(const FwdParams& p, char* smem, int b, int hd, int qt, const float* partials,
+                                                 int count, int wave_has_full_blocks) {
+    using ET = typename Elem<E>::type;
+    typedef FastSoftmaxLimits<E> Lim;
+    constexpr int DB = D / 32, NT = NW * 64, ROW = DB * 16 * NT, SIZE = ROW + 2 * NT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, q_pos = qt * NW * 32 + 32 * wave + (lane & 31);
+    float top = -INFINITY;
+    for (int i = 0; i < count; i++)
+        if (partials[i * SIZE + ROW + NT + tid] != 0.f) top = fmaxf(top, partials[i * SIZE + ROW + tid]);
+    if (top == -INFINITY) top = 0.f;  // no key in any part
+    float l = 0.f;
+    f32x16 o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[db][r] = 0.f;
+#pragma nounroll
+    for (int i = 0; i < count; i++) {
+        const float* from = partials + i * SIZE;
+        const float l_i = from[ROW + NT + tid];
+        const float w = l_i != 0.f ? fast_exp2(from[ROW + tid] - top) : 0.f;
+        l += l_i * w;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(from + ((db * 4 + g) * NT + tid) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[db][4 * g + e] += x[e] * w;
+            }
+    }
+    // (no lens here: every row below T is one of the sequence's)
+    const bool in_t = q_pos < p.T;
+    const bool bad = in_t && !(l == 0.f || (l >= Lim::kLo && l <= Lim::kHi));
+    if (workgroup_any<NW>(__builtin_amdgcn_ballot_w64(bad) != 0, smem + NS * FwdLds<E, D, TK>::STAGE_BYTES)) {
+        fwd_q_tile<E, D, MASK, NW, TK, 3>(p, smem, b, hd, qt, wave_has_full_blocks);
+        return;
+    }
+    if (!in_t) return;
+    const float inv = 1.f / (l == 0.f ? 1.f : l);
+    store_row_transposed<E, D>(reinterpret_cast<ET*>(p.o) + b * p.so.b + hd * p.so.h + (int64_t)q_pos * p.so.t, o, inv, true, h);
+    if (p.lse != nullptr && h == 0) p.lse[b * p.lse_b + hd * p.lse_h + q_pos] = l == 0.f ? -INFINITY : top + __log2f(l);
 }
 
 }  // namespace chill

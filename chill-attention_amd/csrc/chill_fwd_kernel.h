@@ -406,6 +406,7 @@ __device__ __forceinline__ void fwd_q_tile(const FwdParams& p, char* smem, int b
 #include "chill_fwd_regs.h"
 #include "chill_fwd_fast.h"
 #include "chill_fwd_small.h"
+#include "chill_fwd_split.h"
 namespace chill {
 
 // Shapes served by fwd_q_tile_fast (16-bit inputs, head dim 64 or 128, 64-key tiles with one resident
@@ -454,6 +455,40 @@ void fwd_kernel(FwdParams p, int n_q_tiles,
             fwd_q_tile<E, D, MASK, NW, TK, NS>(p, smem, b, hd, j, wave_has_full_blocks);
         }
     }
+}
+
+// The same for a launch whose long q-tiles are split along their keys: one workgroup per (batch, head, item of `split`),
+// the items of all heads longest first.
+template <typename E, int D, int MASK, int NW, int TK, int NS>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd<E, D, NW, TK, NS>())))
+void fwd_split_kernel(FwdParams p, FwdSplit split, int wave_has_full_blocks) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int heads = p.B * p.H;
+    const int i = blockIdx.x / heads, bh = blockIdx.x - i * heads;
+    const unsigned item = split.item[i];
+    const int qt = item & 1023;
+    FwdPart part;
+    part.index = (item >> 10) & 31;
+    part.count = (item >> 15) & 31;
+    part.tiles = split.part_tiles;
+    part.partial = split.partials + ((int64_t)bh * split.partials_per_head + (item >> 20) + part.index) * split.partial_floats;
+    part.again = split.again + bh * split.n_q_tiles + qt;
+    fwd_fast_q_tiles<E, D, MASK, NW, TK, NS, true>(p, smem, bh / p.H, bh % p.H, qt, -1, wave_has_full_blocks, part);
+}
+// ... and the split q-tiles' results from the partial ones, one workgroup per (batch, head, q-tile).
+template <typename E, int D, int MASK, int NW, int TK, int NS>
+__global__ __launch_bounds__(NW * 64) void fwd_merge_kernel(FwdParams p, FwdSplit split, int wave_has_full_blocks) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int heads = p.B * p.H;
+    const int i = blockIdx.x / heads, bh = blockIdx.x - i * heads;
+    const unsigned item = split.merge[i];
+    if (((item >> 15) & 31) == 1) {
+        if (split.again[bh * split.n_q_tiles + i] != 0)
+            fwd_q_tile<E, D, MASK, NW, TK, 3>(p, smem, bh / p.H, bh % p.H, i, wave_has_full_blocks);
+        return;
+    }
+    const float* partials = split.partials + ((int64_t)bh * split.partials_per_head + (item >> 20)) * split.partial_floats;
+    fwd_merge_q_tile<E, D, MASK, NW, TK, NS>(p, smem, bh / p.H, bh % p.H, item & 1023, partials, (item >> 15) & 31, wave_has_full_blocks);
 }
 
 // Launcher for one (element type, head dim); dispatches on the mask id and takes the tile shape
@@ -506,6 +541,24 @@ int launch_fwd_shape(const FwdParams& p, hipStream_t stream) {
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
+// A launch whose long q-tiles are split along their keys (plan_fwd_split).
+template <typename E, int D, int MASK_ID>
+int launch_fwd_split(const FwdParams& p, const FwdSplit& split, hipStream_t stream) {
+    constexpr TileConfig cfg = fwd_tile_config(MASK_ID, D, Elem<E>::kDType);
+    constexpr int NS = fwd_stages(MASK_ID, D, Elem<E>::kDType, kLongSequence);
+    constexpr int kLdsBytes = fwd_lds_bytes<E, D, cfg.streamed, NS>();
+    auto kern = fwd_split_kernel<E, D, MASK_ID, cfg.waves, cfg.streamed, NS>;
+    auto merge = fwd_merge_kernel<E, D, MASK_ID, cfg.waves, cfg.streamed, NS>;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(merge), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)
+        return CHILL_ERR_HIP;
+    const int hfb = Mask<MASK_ID>::has_full_blocks(32, cfg.streamed, p.T, p.margs) ? 1 : 0;
+    const dim3 block(cfg.waves * 64);
+    hipLaunchKernelGGL(kern, dim3(p.B * p.H * split.n_items), block, kLdsBytes, stream, p, split, hfb);
+    hipLaunchKernelGGL(merge, dim3(p.B * p.H * split.n_q_tiles), block, kLdsBytes, stream, p, split, hfb);
+    return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
+}
+
 // A launch far too small for the chip: 32 query rows per workgroup, the keys split over its waves.
 template <typename E, int D, int MASK_ID>
 int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
@@ -532,7 +585,7 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
 }
 
 template <typename E, int D>
-int launch_fwd(const FwdParams& args, int mask_id, hipStream_t stream) {
+int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStream_t stream) {
     FwdParams p = args;
     p.work_block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H, p.group, 2ll * p.T * D * Elem<E>::kBytes, kWorkBlockBytes / 2);
     // the async loader keeps per-lane global offsets in 32 bits
@@ -540,6 +593,9 @@ int launch_fwd(const FwdParams& args, int mask_id, hipStream_t stream) {
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
     int status = CHILL_ERR_BAD_MASK;
     CHILL_DISPATCH_MASK(mask_id, {
+        if constexpr (fwd_split_serves(MASK_ID, D, Elem<E>::kDType)) {
+            if (split != nullptr) return launch_fwd_split<E, D, MASK_ID>(p, *split, stream);
+        }
         // the table has a row of its own for short sequences and small grids where that row differs
         constexpr bool has_short_row = fwd_tile_config(MASK_ID, D, Elem<E>::kDType, 1).waves !=
                                        fwd_tile_config(MASK_ID, D, Elem<E>::kDType).waves;

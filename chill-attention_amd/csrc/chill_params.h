@@ -28,6 +28,19 @@ struct FwdParams {
     MaskArgs margs;
 };
 
+// The forward of a launch with fewer q-tiles than the chip has room for: the keys of the long q-tiles are split into
+// parts, each an item of its own (plan_fwd_split, chill_fwd_split.h).  The items of a head, longest first:
+// q-tile | part << 10 | parts << 15 | first partial result of the q-tile << 20.
+constexpr int kFwdSplitMaxItems = CHILL_FWD_SPLIT_MAX_ITEMS, kFwdSplitMaxQTiles = 256, kFwdSplitMaxParts = 16;
+struct FwdSplit {
+    float* partials;      // [head][partials_per_head] results of one part each
+    int32_t n_items, n_q_tiles, partials_per_head, partial_floats;
+    int32_t part_tiles;   // tiles of keys in every part of a q-tile but the last
+    uint32_t item[kFwdSplitMaxItems];
+    uint32_t merge[kFwdSplitMaxQTiles];  // any item of every q-tile
+    uint32_t* again;  // [head][q-tile]: a q-tile of one part whose sums left the range (written for every such q-tile)
+};
+
 struct DeltaParams {
     const void* o;
     const void* d_o;

@@ -34,7 +34,8 @@ struct EntryPoints {
     uint64_t magic;        // kEntryPointsMagic
     uint32_t abi_version;  // CHILL_ABI_VERSION of the header the table was filled against
     uint32_t bytes;        // sizeof(EntryPoints)
-    decltype(&chill_fwd) fwd;
+    decltype(&chill_fwd_workspace) fwd;
+    decltype(&chill_fwd_workspace_bytes) fwd_workspace_bytes;
     decltype(&chill_bwd_dq_delta) dq_delta;
     decltype(&chill_bwd_dkdv) dkdv;
     decltype(&chill_status_string) status_string;
@@ -120,11 +121,17 @@ std::tuple<at::Tensor, at::Tensor> forward_impl(const at::Tensor& q, const at::T
     const ChillMaskDesc desc = mask_desc(mask_id, mask_args);
     const int64_t lse_stride[3] = {return_lse ? lse.stride(0) : 0, return_lse ? lse.stride(1) : 0, return_lse ? lse.stride(2) : 0};
     const bool has_lens = lens.has_value() && lens->defined();
+    // room for the partial results of a launch that splits its keys (none for most launches); the caching allocator hands
+    // it to a later call on this stream only after this one
+    const int64_t bytes = ep->fwd_workspace_bytes((int32_t)q.size(0), (int32_t)q.size(1), (int32_t)q.size(2), (int32_t)q.size(3),
+                                                  dtype_code(q), &desc, has_lens);
+    const at::Tensor workspace = bytes > 0 ? at::empty({bytes}, q.options().dtype(at::kByte)) : at::Tensor();
     check(ep, "chill_fwd",
           ep->fwd(&tq, &tk, &tv, &to, return_lse ? lse.data_ptr<float>() : nullptr, return_lse ? lse_stride : nullptr,
                   has_lens ? lens->data_ptr<int32_t>() : nullptr, has_lens ? lens->stride(0) : 0, (int32_t)q.size(0),
                   (int32_t)q.size(1), (int32_t)k.size(1), (int32_t)q.size(2), (int32_t)q.size(3), dtype_code(q),
-                  (float)sm_scale, &desc, c10::hip::getCurrentHIPStream(q.device().index()).stream()));
+                  (float)sm_scale, &desc, bytes > 0 ? workspace.data_ptr() : nullptr, bytes > 0 ? bytes : 0,
+                  c10::hip::getCurrentHIPStream(q.device().index()).stream()));
     return {o, lse};
 }
 
@@ -232,7 +239,7 @@ extern "C" int64_t chill_torch_register_entry_points(const void* table) {
     if (t.magic != kEntryPointsMagic || t.bytes != sizeof(EntryPoints)) return -1;
     if (t.abi_version != CHILL_ABI_VERSION) return -2;
     std::memcpy(&t, table, sizeof(EntryPoints));
-    if (!t.fwd || !t.dq_delta || !t.dkdv || !t.status_string) return -1;
+    if (!t.fwd || !t.fwd_workspace_bytes || !t.dq_delta || !t.dkdv || !t.status_string) return -1;
     std::lock_guard<std::mutex> lock(g_tables_mutex);
     g_tables.push_back(t);
     return (int64_t)g_tables.size() - 1;

@@ -104,6 +104,29 @@ int chill_fwd(const ChillTensor4* q, const ChillTensor4* k, const ChillTensor4* 
               int32_t dtype, float sm_scale,
               const ChillMaskDesc* mask, void* stream);
 
+/* The same with a workspace from the caller (16-byte aligned device memory, used until the launches on `stream` are done).
+ * A launch whose q-tiles are too few or too unequal to fill the chip splits the keys of the long ones over several
+ * workgroups and needs room for their partial results: chill_fwd_workspace_bytes says how much (0: none; negative: an
+ * error code as from chill_fwd).  Without a workspace (NULL) this is chill_fwd; a workspace smaller than that is
+ * CHILL_ERR_BAD_ARGUMENT.  Results are those of chill_fwd up to the rounding of sums in another order, and the same from
+ * launch to launch. */
+int chill_fwd_workspace(const ChillTensor4* q, const ChillTensor4* k, const ChillTensor4* v,
+                        const ChillTensor4* o,
+                        float* lse, const int64_t lse_stride[3],
+                        const int32_t* lens, int64_t lens_stride,
+                        int32_t B, int32_t H, int32_t H_kv, int32_t T, int32_t D,
+                        int32_t dtype, float sm_scale,
+                        const ChillMaskDesc* mask, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t chill_fwd_workspace_bytes(int32_t B, int32_t H, int32_t T, int32_t D, int32_t dtype,
+                                  const ChillMaskDesc* mask, int32_t has_lens);
+
+/* How such a launch is split: the items of every head in the order they are taken, each {q-tile, part, parts of the
+ * q-tile, index of the q-tile's first partial result (parts > 1)}.  Returns their number, 0 for a launch that is not
+ * split, or an error code.  Host code; the kernel is launched from the same list. */
+#define CHILL_FWD_SPLIT_MAX_ITEMS 512
+int chill_fwd_split_items(int32_t B, int32_t H, int32_t T, int32_t D, int32_t dtype, const ChillMaskDesc* mask,
+                          int32_t items[CHILL_FWD_SPLIT_MAX_ITEMS][4]);
+
 /* Backward preprocessing: delta[b,h,t] = sum_d float(O[b,h,t,d]) * float(dO[b,h,t,d]).
  * Replaces the launch of _chill_attn_bwd_precompute (utils.py:94-217) at chill.py:278-290. */
 int chill_bwd_delta(const ChillTensor4* o, const ChillTensor4* d_o,

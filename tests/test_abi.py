@@ -441,3 +441,35 @@ def test_eager_operator_library_loads():
         op(q, q, q, None, handle + 1000, 1, [], 0.25, False)
     with pytest.raises((RuntimeError, NotImplementedError)):
         op(q, q, q, None, handle, 1, [], 0.25, False)  # CPU tensors: no kernel for them, no crash
+
+
+@pytest.mark.parametrize("mask_id,args", [(0, ()), (1, ()), (4, (700,))], ids=["full", "causal", "prefix-lm"])
+@pytest.mark.parametrize("D,rows", [(64, 128), (128, 256)])
+def test_split_forward_items_cover_every_q_tile(mask_id, args, D, rows):
+    """The items of a forward that splits its keys: every part of every q-tile exactly once, partial results that do not
+    overlap and fit the workspace; no launch that other kernels take or that fills the chip."""
+    L, cap = _lib.lib, 512
+    buf = (ctypes.c_int32 * (4 * cap))()
+    desc = _lib.mask_desc(mask_id, args)
+    split = 0
+    for H in (1, 2, 3, 5, 8, 16, 40):
+        for T in (100, 1030, 4042, 5501, 8192, 12000, 16385, 33000, 70000):
+            n = L.chill_fwd_split_items(1, H, T, D, 2, ctypes.byref(desc), buf)
+            size = L.chill_fwd_workspace_bytes(1, H, T, D, 2, ctypes.byref(desc), 0)
+            assert 0 <= n <= cap and (n > 0) == (size > 0), (H, T, n, size)
+            assert L.chill_fwd_workspace_bytes(1, H, T, D, 2, ctypes.byref(desc), 1) == 0  # padded batches are left whole
+            assert L.chill_fwd_workspace_bytes(1, H, T, D, 0, ctypes.byref(desc), 0) == 0  # and fp32
+            if n == 0:
+                continue
+            split += 1
+            items = [tuple(buf[4 * i : 4 * i + 4]) for i in range(n)]
+            n_q = -(-T // rows)
+            parts = {qt: c for qt, _, c, _ in items}
+            assert sorted((qt, j) for qt, j, _, _ in items) == [(qt, j) for qt in range(n_q) for j in range(parts[qt])]
+            assert max(parts.values()) > 1
+            slots = [first + j for _, j, c, first in items if c > 1]
+            assert sorted(slots) == list(range(len(slots)))
+            assert size == H * (len(slots) * 4 * (rows * D + 4 * rows) + 4 * n_q)
+    assert split >= 5
+    assert L.chill_fwd_split_items(1, 2, 8192, 48, 2, ctypes.byref(desc), buf) < 0
+    assert L.chill_fwd_split_items(1, 2, 8192, 64, 2, ctypes.byref(desc), None) == -1

@@ -7,6 +7,7 @@ the reference's own tolerances.  The oracle (dense mask -> torch SDPA on fp32-up
 for the gradients) runs on the same device tensors.
 """
 
+import ctypes
 import math
 import zlib
 
@@ -1046,3 +1047,49 @@ def test_padded_batches_in_order_of_length(m, D, dtype, B, H, Hkv, T):
         check_close(out.detach()[b : b + 1, :, :n], ref.detach(), dtype, OUT_TOL[dtype], D, f"O[{b}]")
         for name, got, want in (("dq", q.grad, qf.grad), ("dk", k.grad, kf.grad), ("dv", v.grad, vf.grad)):
             check_close(got[b : b + 1, :, :n], want, dtype, GRAD_TOL[dtype], D, f"{name}[{b}]")
+
+
+# D, dtype, H, H_kv, T, mask: q-tiles of one, two and more parts, a part that ends in a ragged tile, GQA
+SPLIT_CASES = [(128, torch.bfloat16, 3, 1, 5501, ("CausalChillMask", ())), (128, torch.float16, 8, 4, 4096, ("PrefixLMChillMask", (700,))),
+               (128, torch.bfloat16, 4, 4, 5121, ("FullChillMask", ())), (64, torch.float16, 6, 6, 4042, ("CausalChillMask", ())),
+               (64, torch.bfloat16, 3, 3, 5505, ("FullChillMask", ())), (64, torch.bfloat16, 3, 3, 8192, ("PrefixLMChillMask", (1000,)))]
+
+
+@pytest.mark.parametrize("jump", [False, True], ids=["", "jump"])
+@pytest.mark.parametrize("D,dtype,H,Hkv,T,m", SPLIT_CASES)
+def test_forward_split_along_the_keys(D, dtype, H, Hkv, T, m, jump):
+    """Launches whose long q-tiles are split along their keys over several workgroups (chill_fwd_split.h): O and LSE2
+    against the dense reference, the same bits from a second call and from replays of a captured graph.  jump: scores that
+    rise by 300 log2 units inside one tile, so that parts and q-tiles of one part leave the range of the reference-free
+    softmax and the q-tiles are computed again."""
+    mask = make_mask(m)
+    desc = _lib.mask_desc(mask.mask_id, m[1])
+    code = {torch.float16: 1, torch.bfloat16: 2}[dtype]
+    assert _lib.lib.chill_fwd_workspace_bytes(1, H, T, D, code, ctypes.byref(desc), 0) > 0, "this shape is not split"
+    torch.manual_seed(stable_seed(D, H, T, m, "split") % 2**31)
+    q, k, v = (torch.randn(1, h, T, D, device=DEV) * (0.5 if jump else 1.0) for h in (H, Hkv, Hkv))
+    if jump:
+        # the jump at key 700 lies inside a tile of the first part and of the short q-tiles
+        u = torch.nn.functional.normalize(torch.randn(D, device=DEV), dim=0)
+        q = q - (q @ u)[..., None] * u + 4.0 * u
+        k = k + (300.0 * D**0.5 / (4.0 * 1.4427)) * (torch.arange(T, device=DEV) >= 700).float()[None, None, :, None] * u
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    print(f"split {mask} {dtype} D={D} H={H}/{Hkv} T={T} jump={jump}", flush=True)
+    out, lse = ca.chill_attention(q, k, v, mask=mask, return_lse=True)
+    ref, _ = orc.reference_naive(m[0], m[1], q.float(), k.float(), v.float(), None)
+    want_lse = orc.lse2_dense(m[0], m[1], q, k, None)
+    torch.testing.assert_close(out, ref.to(dtype), atol=OUT_TOL[dtype][0], rtol=OUT_TOL[dtype][1])
+    # Q times the scale is rounded to the input type: eps * |q| * |k| * scale * log2(e) at most (see the ramp test above)
+    eps = {torch.bfloat16: 2.0**-9, torch.float16: 2.0**-12}[dtype]
+    loose = eps * (D**-0.5 * 1.4427) * q.float().norm(dim=-1) * k.float().norm(dim=-1).max()
+    assert ((lse.double() - want_lse).abs() <= 1e-2 + loose).all()
+    again, lse_again = ca.chill_attention(q, k, v, mask=mask, return_lse=True)
+    assert torch.equal(out, again) and torch.equal(lse, lse_again)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured, captured_lse = ca.chill_attention(q, k, v, mask=mask, return_lse=True)
+    for _ in range(3):
+        captured.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, captured) and torch.equal(lse, captured_lse)
