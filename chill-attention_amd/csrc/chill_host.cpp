@@ -161,7 +161,8 @@ int chill_launch_item(int32_t workgroup, int32_t heads, int32_t per_head, int32_
     if (workgroup < 0 || heads < 1 || per_head < 1 || block < 0 || streams < 1 || heads % streams != 0 || resident < 1 ||
         (int64_t)heads * per_head > (1 << 30))
         return CHILL_ERR_BAD_ARGUMENT;
-    return work_item(workgroup, heads, per_head, block, streams, resident, &out[0], &out[1]) ? 1 : 0;
+    const WorkOrder order = work_order(false, heads, streams, block);
+    return work_item(workgroup, heads, per_head, order, streams, resident, &out[0], &out[1]) ? 1 : 0;
 }
 
 const char* chill_status_string(int32_t status) {

@@ -11,6 +11,13 @@ struct Strides3 {  // element strides of a [B, H, T, D] tensor with unit inner s
     int64_t b, h, t;
 };
 
+// The order in which a launch's workgroups take their (head, tile) items (work_order, chill_tiles.h).
+struct WorkOrder {
+    int32_t sets;     // sets of heads of a block; 0: contiguous runs of heads
+    int32_t all;      // ... and of the launch
+    int32_t in_turn;  // a block of no whole number of rounds takes its heads in turn
+};
+
 struct FwdParams {
     const void* q;
     const void* k;
@@ -23,7 +30,7 @@ struct FwdParams {
     int64_t lens_stride;
     int32_t B, H, H_kv, T;
     int32_t group;         // H / H_kv
-    int32_t work_block;    // order of the workgroups (work_block, chill_tiles.h)
+    WorkOrder order;
     float scale_log2;      // sm_scale * log2(e)
     MaskArgs margs;
 };
@@ -71,7 +78,7 @@ struct BwdParams {
     int64_t lens_stride;
     int32_t B, H, H_kv, T;
     int32_t group;
-    int32_t work_block;  // order of the workgroups (work_block, chill_tiles.h)
+    WorkOrder order;
     float sm_scale;
     float scale_log2;
     MaskArgs margs;

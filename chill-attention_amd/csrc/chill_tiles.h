@@ -485,8 +485,8 @@ CHILL_HD int xcd_contiguous_item(int wg, int total, int resident = 1) {
 }
 
 // The order in which a launch's workgroups take their (head, tile) items, as the number of heads of a BLOCK: the blocks
-// follow each other, inside one the workgroups take tile 0 of every head, then tile 1 of every head, and so on, and head
-// u of a block belongs to XCD u % 8 (work_item).  The kernels number a head's tiles from the heavy end of a causal-like
+// follow each other, inside one the workgroups take tile 0 of every head, then tile 1 of every head, and so on, and the
+// heads keep to their XCDs as work_item says.  The kernels number a head's tiles from the heavy end of a causal-like
 // mask, so a block, the last one above all, ends with its short tiles; a whole launch as one block is longest first, but
 // streams the K and V (in dK/dV the Q and dO) of all its heads at once through an XCD's L2 (4 MiB) and the last-level
 // cache (256 MiB).  So a block holds as many heads per XCD as stream about 16 MiB, two at the least.
@@ -518,13 +518,32 @@ constexpr int work_block(int mask_id, bool padded, long long heads, int streams,
     return (int)((rounds + blocks - 1) / blocks * 8 * streams);
 }
 
+// The same for the device, in sets of `streams` heads.  A padded launch takes the heads of a block of no whole number of
+// rounds in turn: with sets that keep to their XCDs some XCDs get the long elements and others the short ones (causal D128
+// B3 H32/4, lengths 4096, 3000 and 1024, forward / dQ / dK/dV: 214 / 288 / 720 us in turn, 264 / 366 / 756 in groups).
+constexpr WorkOrder work_order(bool padded, long long heads, int streams, int block) {
+    const long long sets = heads / streams, most = (block + streams - 1ll) / streams;
+    return WorkOrder{(int32_t)(most < sets ? most : sets), (int32_t)sets, padded ? 1 : 0};
+}
+
 // Workgroup `wg` of a launch of `heads` heads (query heads, or key / value heads in dK/dV; `streams` of them share what
-// they stream) of `per_head` tiles each, in the order `block`: its head and tile, or false if it has nothing to do.
+// they stream, a set) of `per_head` tiles each, in the order `order`: its head and tile, or false if it has nothing to do.
 // `resident` as in xcd_contiguous_item.
-CHILL_HD bool work_item(int wg, int heads, int per_head, int block, int streams, int resident, int* head, int* tile) {
+// Workgroups are dealt round-robin to the XCDs.  The sets of a block are taken in groups of 1, 2 and 4, the bits of their
+// number modulo 8, and one of the rest, a multiple of 8; inside a group of n the workgroups alike modulo min(n, 8), the
+// same ones for every tile, take the same sets.  So a set of the large group stays on one XCD, one of a small group on
+// 8 / n of them, and an XCD streams one set of each small group, whatever the number of heads (with the heads of a tile
+// simply in turn it streams all 25 of B1 H25).  Measured, forward / dQ / dK/dV in us, in turn -> in groups (bf16):
+//   causal D64  B1 H25 T8192 227 / 296 / 405 -> 214 / 292 / 403   B1 H12 T4042 41 / 59 / 71 -> 39 / 58 / 72
+//               B1 H5 T4042  40.3 / 56.0 / 59.0 -> 35.8 / 55.2 / 59.0   full D64 B5 H5 T1500 27.6 / 35.8 / 48.1 -> 27.0 / 35.1 / 45.8
+//   causal D128 B1 H15 T8192 216 / 324 / 466 -> 215 / 325 / 466   B3 H28/4 T4096 331 / 462 / 745 -> 328 / 464 / 743
+// Contiguous runs keep the sets together as well and are slower than both where tiles differ (B1 H25: 241 / 351 / 456; H15:
+// 296 / 477 / 549; under a full mask, fp16 B1 H25, 451 / 633 / 864 against 451 / 627 / 862).  The small groups ahead of the
+// blocks instead of inside them, tile by tile, lose what longest first gains (H15: 244 / 375 / 514).
+CHILL_HD bool work_item(int wg, int heads, int per_head, WorkOrder order, int streams, int resident, int* head, int* tile) {
     constexpr int kXcds = 8, kCusPerXcd = 32;
     const int total = heads * per_head;
-    if (block == 0) {
+    if (order.sets == 0) {
         const int item = xcd_contiguous_item(wg, total, resident);
         if (item < 0) return false;
         *head = item / per_head;
@@ -540,17 +559,28 @@ CHILL_HD bool work_item(int wg, int heads, int per_head, int block, int streams,
             wg = (pass * kCusPerXcd + len - 1 - (local - pass * kCusPerXcd)) * kXcds + xcd;
         }
     }
-    const int first = block < heads ? wg / (block * per_head) * block : 0;  // first head of the block
-    const int size = heads - first < block ? heads - first : block;
-    const int i = wg - first * per_head;
+    const int block_items = order.sets * streams * per_head;
+    const int block = order.sets < order.all ? wg / block_items : 0;
+    const int first = block * order.sets;  // first set of the block
+    const int sets = imin(order.sets, order.all - first), size = sets * streams;
+    const int i = wg - block * block_items;
     *tile = i / size;
-    int u = i - *tile * size;
-    // in whole rounds of sets the heads of a set stay on one XCD
-    if (streams > 1 && size % (kXcds * streams) == 0) {
-        const int xcd = u % kXcds, k = u / kXcds;
-        u = (xcd + kXcds * (k / streams)) * streams + k % streams;
+    int in_group = i - *tile * size;
+    int before = 0, shift = 3;  // sets of the block's groups before this one; min(n, 8) = 1 << shift
+    if (const int rest = sets % kXcds) {
+        if (order.in_turn) {
+            *head = first * streams + in_group;
+            return true;
+        }
+        if (in_group < rest * streams)
+            for (shift = 0; !(rest >> shift & 1) || in_group >= (before + (1 << shift)) * streams; shift++) before += rest & 1 << shift;
+        else
+            before = rest;
+        in_group -= before * streams;
     }
-    *head = first + u;
+    const int k = in_group >> shift, round = streams > 1 ? k / streams : k;  // (the heads of a set follow each other)
+    const int set = first + before + (wg & ((1 << shift) - 1)) + (round << shift);
+    *head = set * streams + k - round * streams;
     return true;
 }
 

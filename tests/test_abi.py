@@ -315,6 +315,29 @@ def test_launch_items_are_a_permutation(streams, resident):
     assert f(-1, 8, 1, 0, 1, 1, out) == -8 and f(0, 6, 1, 0, 4, 1, out) == -8 and f(0, 8, 1, 0, 1, 1, None) == -1
 
 
+@pytest.mark.parametrize("resident", [1, 2, 3])
+@pytest.mark.parametrize("streams", [1, 4, 7])
+def test_launch_items_keep_a_set_of_heads_on_its_xcds(streams, resident):
+    """The heads that share what they stream are one set.  Whatever the number of sets, 8 * (sets // 8) of them stay on one
+    XCD, the same number on each, and the others, in groups of n = 1, 2 or 4, on 8 / n XCDs, one of a group per XCD; where
+    the tiles of a set go to several XCDs they go there in equal shares.  (Workgroup w runs on XCD w % 8.)"""
+    out = (ctypes.c_int32 * 2)()
+    f = _lib.lib.chill_launch_item
+    per_head = 16
+    for sets in (1, 2, 3, 5, 7, 8, 12, 25, 30, 40):
+        heads = sets * streams
+        for block in (8 * streams, 16 * streams, 24 * streams):
+            items = [[0] * 8 for _ in range(sets)]  # of a set on an XCD
+            for w in range(heads * per_head):
+                assert f(w, heads, per_head, block, streams, resident, out) == 1
+                items[out[0] // streams][w % 8] += 1
+            spread = [sum(i > 0 for i in row) for row in items]
+            assert sorted(spread) == sorted([1] * (sets // 8 * 8) + [8 // n for n in (1, 2, 4) if sets & n for _ in range(n)])
+            assert all(max(row) * n <= per_head * streams + 8 for row, n in zip(items, spread)), (sets, block, items)
+            per_xcd = [sum(row[x] > 0 for row in items) for x in range(8)]
+            assert per_xcd == [sets // 8 + bin(sets % 8).count("1")] * 8, (sets, block, per_xcd)
+
+
 def test_cpu_tensors_are_refused():
     import torch
 
