@@ -450,8 +450,7 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
 template <typename E, int D>
 int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
-    const long long streamed = 2ll * p.T * D * Elem<E>::kBytes;
-    const int block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H, p.group, streamed, kWorkBlockBytes);
+    const int block = work_block(mask_id, CHILL_PASS_DQ, p.lens != nullptr, p.B, p.H, p.H_kv, p.T, D, Elem<E>::kBytes);
     p.order = work_order(p.lens != nullptr, (long long)p.B * p.H, p.group, block);
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
@@ -1396,8 +1395,7 @@ int launch_dkdv_shape(const BwdParams& p, hipStream_t stream) {
 template <typename E, int D>
 int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
-    const long long streamed = 2ll * p.group * p.T * D * Elem<E>::kBytes;
-    const int block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H_kv, 1, streamed, kWorkBlockBytes);
+    const int block = work_block(mask_id, CHILL_PASS_DKDV, p.lens != nullptr, p.B, p.H, p.H_kv, p.T, D, Elem<E>::kBytes);
     p.order = work_order(p.lens != nullptr, (long long)p.B * p.H_kv, 1, block);
     int64_t max_stride = p.sq.t > p.sdo.t ? p.sq.t : p.sdo.t;
     if (p.sk.t > max_stride) max_stride = p.sk.t;

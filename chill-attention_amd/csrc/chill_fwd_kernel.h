@@ -587,8 +587,7 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
 template <typename E, int D>
 int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStream_t stream) {
     FwdParams p = args;
-    const long long streamed = 2ll * p.T * D * Elem<E>::kBytes;
-    const int block = work_block(mask_id, p.lens != nullptr, (long long)p.B * p.H, p.group, streamed, kWorkBlockBytes / 2);
+    const int block = work_block(mask_id, CHILL_PASS_FWD, p.lens != nullptr, p.B, p.H, p.H_kv, p.T, D, Elem<E>::kBytes);
     p.order = work_order(p.lens != nullptr, (long long)p.B * p.H, p.group, block);
     // the async loader keeps per-lane global offsets in 32 bits
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;

@@ -165,6 +165,18 @@ int chill_launch_item(int32_t workgroup, int32_t heads, int32_t per_head, int32_
     return work_item(workgroup, heads, per_head, order, streams, resident, &out[0], &out[1]) ? 1 : 0;
 }
 
+int chill_launch_block(const ChillMaskDesc* mask, int32_t pass, int32_t has_lens, int32_t B, int32_t H, int32_t H_kv,
+                       int32_t T, int32_t D, int32_t dtype) {
+    MaskArgs a;
+    const int st = lower_mask(mask, &a);
+    if (st != CHILL_OK) return st;
+    if (dtype != CHILL_F32 && dtype != CHILL_F16 && dtype != CHILL_BF16) return CHILL_ERR_BAD_DTYPE;
+    if (D != 16 && D != 32 && D != 64 && D != 128 && D != 256) return CHILL_ERR_BAD_HEAD_DIM;
+    if (B < 1 || H < 1 || H_kv < 1 || T < 1 || H % H_kv != 0 || (int64_t)B * H > (1 << 30)) return CHILL_ERR_BAD_SHAPE;
+    if (pass != CHILL_PASS_FWD && pass != CHILL_PASS_DQ && pass != CHILL_PASS_DKDV) return CHILL_ERR_BAD_ARGUMENT;
+    return work_block(mask->id, pass, has_lens != 0, B, H, H_kv, T, D, dtype == CHILL_F32 ? 4 : 2);
+}
+
 const char* chill_status_string(int32_t status) {
     switch (status) {
         case CHILL_OK: return "ok";

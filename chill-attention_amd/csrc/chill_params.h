@@ -13,8 +13,9 @@ struct Strides3 {  // element strides of a [B, H, T, D] tensor with unit inner s
 
 // The order in which a launch's workgroups take their (head, tile) items (work_order, chill_tiles.h).
 struct WorkOrder {
-    int32_t sets;     // sets of heads of a block; 0: contiguous runs of heads
-    int32_t all;      // ... and of the launch
+    int32_t small;    // blocks that come first, of `sets` sets of heads each; the others have 8 more.  0: contiguous runs
+    int32_t sets;     // a multiple of 8; the first block also has the sets of an incomplete round (all % 8)
+    int32_t all;      // sets of the launch
     int32_t in_turn;  // a block of no whole number of rounds takes its heads in turn
 };
 

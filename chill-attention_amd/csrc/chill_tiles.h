@@ -505,25 +505,37 @@ CHILL_HD int xcd_contiguous_item(int wg, int total, int resident = 1) {
 // D128 B4 H32/8 T2085 197 / 219 / 340 -> 116 / 139 / 210, B8 H16 T8192 1456 / 2199 / 2935 -> 969 / 1368 / 1830,
 // full mask B8 H16 T2085 303 / 348 / 446 -> 172 / 229 / 290, sliding window 128 + 128 B8 H16 T4042 154 / 183 / 271 ->
 // 127 / 158 / 217.
-// `heads` = heads of the launch; `streams` = heads that share what they stream (H / H_kv in the forward and dQ, 1 in dK/dV); `bytes` = what is streamed
-// for one such set of heads.
+// `es` = bytes of an element; the heads of a launch are query heads, in dK/dV key / value heads, and `streams` of them
+// share what they stream (work_streams).
 constexpr long long kWorkBlockBytes = 16ll << 20;
-// Blocks of one size: a last block of fewer heads would end the launch on a part of the XCDs' CUs (causal D128 B4 H32/8
-// T2085 dK/dV, four heads per XCD: 290 us as one block of four, 373 as three and one).
-constexpr int work_block(int mask_id, bool padded, long long heads, int streams, long long bytes, long long budget) {
+constexpr int work_streams(int pass, int H, int H_kv) { return pass == CHILL_PASS_DKDV ? 1 : H / H_kv; }
+constexpr int work_block(int mask_id, int pass, bool padded, int B, int H, int H_kv, int T, int D, int es) {
     if (!padded && mask_is_banded(mask_id)) return 0;
-    const long long rounds = (heads + 8 * streams - 1) / (8 * streams);  // sets per XCD
-    const long long most = padded || budget / bytes < 2 ? 2 : budget / bytes;
+    const int streams = work_streams(pass, H, H_kv);
+    const long long sets = (long long)B * H_kv, rounds = (sets + 7) / 8;  // sets per XCD
+    const long long bytes = 2ll * T * D * es * (pass == CHILL_PASS_DKDV ? H / H_kv : 1);
+    const long long budget = (pass == CHILL_PASS_FWD ? kWorkBlockBytes / 2 : kWorkBlockBytes) / bytes;
+    const long long most = padded || budget < 2 ? 2 : budget;
     const long long blocks = rounds / most < 1 ? 1 : rounds / most;
     return (int)((rounds + blocks - 1) / blocks * 8 * streams);
 }
 
-// The same for the device, in sets of `streams` heads.  A padded launch takes the heads of a block of no whole number of
-// rounds in turn: with sets that keep to their XCDs some XCDs get the long elements and others the short ones (causal D128
-// B3 H32/4, lengths 4096, 3000 and 1024, forward / dQ / dK/dV: 214 / 288 / 720 us in turn, 264 / 366 / 756 in groups).
+// The same for the device: as many blocks as that makes, equal up to one round, because a last block of fewer heads would
+// end the launch on a part of the CUs.  The smaller blocks come first, and an incomplete round goes with the first of them.
+// (causal D128: B4 H32/8 T2085, dK/dV, one block of four heads per XCD 290 us, three and one 373.  Forward / dQ / dK/dV,
+// the last block what is left over -> equal blocks: B2 H25 T6000 453 / 587 / 808 -> 386 / 586 / 803, B8 H16 T6000 1000 /
+// 1453 / 1942 -> 1000 / 1463 / 1966, B8 H32 T6000 1995 / 2945 / 3927 -> 1992 / 2922 / 3916; padded, lengths of T/4 .. T,
+// B13 H8 T4096 240 / 322 / 463 -> 238 / 320 / 454, B5 H9 T4096 141 / 179 / 277 -> 133 / 173 / 254.)
+// A padded launch takes the heads of a block of no whole number of rounds in turn: with sets that keep to their XCDs some
+// XCDs get the long elements and others the short ones (causal D128 B3 H32/4, lengths 4096, 3000 and 1024, forward / dQ /
+// dK/dV: 214 / 288 / 720 us in turn, 264 / 366 / 756 in groups).
 constexpr WorkOrder work_order(bool padded, long long heads, int streams, int block) {
-    const long long sets = heads / streams, most = (block + streams - 1ll) / streams;
-    return WorkOrder{(int32_t)(most < sets ? most : sets), (int32_t)sets, padded ? 1 : 0};
+    if (block == 0) return WorkOrder{0, 0, 0, 0};
+    const long long sets = heads / streams, rounds = sets / 8;
+    const long long most = block < 16ll * streams ? 1 : block / (8ll * streams);  // rounds of a block
+    const long long wanted = ((sets + 7) / 8 + most - 1) / most;
+    const long long blocks = wanted > rounds ? (rounds > 1 ? rounds : 1) : wanted;
+    return WorkOrder{(int32_t)(blocks - rounds % blocks), (int32_t)(rounds / blocks * 8), (int32_t)sets, padded ? 1 : 0};
 }
 
 // Workgroup `wg` of a launch of `heads` heads (query heads, or key / value heads in dK/dV; `streams` of them share what
@@ -543,7 +555,7 @@ constexpr WorkOrder work_order(bool padded, long long heads, int streams, int bl
 CHILL_HD bool work_item(int wg, int heads, int per_head, WorkOrder order, int streams, int resident, int* head, int* tile) {
     constexpr int kXcds = 8, kCusPerXcd = 32;
     const int total = heads * per_head;
-    if (order.sets == 0) {
+    if (order.small == 0) {
         const int item = xcd_contiguous_item(wg, total, resident);
         if (item < 0) return false;
         *head = item / per_head;
@@ -559,15 +571,25 @@ CHILL_HD bool work_item(int wg, int heads, int per_head, WorkOrder order, int st
             wg = (pass * kCusPerXcd + len - 1 - (local - pass * kCusPerXcd)) * kXcds + xcd;
         }
     }
-    const int block_items = order.sets * streams * per_head;
-    const int block = order.sets < order.all ? wg / block_items : 0;
-    const int first = block * order.sets;  // first set of the block
-    const int sets = imin(order.sets, order.all - first), size = sets * streams;
-    const int i = wg - block * block_items;
+    const int rest = order.all % kXcds, set_items = streams * per_head;
+    int first = 0, sets = order.sets + rest;  // first set and number of sets of the block
+    if (wg >= sets * set_items) {
+        int later = wg - sets * set_items;  // items since the end of the first block
+        first = sets;
+        sets = order.sets;
+        const int small_items = (order.small - 1) * sets * set_items;
+        if (later >= small_items) {
+            later -= small_items;
+            first += (order.small - 1) * sets;
+            sets += 8;
+        }
+        first += later / (sets * set_items) * sets;
+    }
+    const int size = sets * streams, i = wg - first * set_items;
     *tile = i / size;
     int in_group = i - *tile * size;
     int before = 0, shift = 3;  // sets of the block's groups before this one; min(n, 8) = 1 << shift
-    if (const int rest = sets % kXcds) {
+    if (rest > 0 && first == 0) {
         if (order.in_turn) {
             *head = first * streams + in_group;
             return true;

@@ -234,11 +234,16 @@ int chill_mask_limits(const ChillMaskDesc* mask, int32_t which, int32_t n, int32
 int chill_work_item(int32_t workgroup, int32_t total, int32_t resident);
 
 /* The head and the tile (out[0], out[1]) that workgroup `workgroup` of a launch of `heads` heads of `per_head` tiles
- * each takes, and 1; 0 when it has none.  `block` = heads taken together, tile by tile (0: head by head, in the order of
- * chill_work_item); `streams` = neighbouring heads that share what they stream.  Over the workgroups of a grid the
+ * each takes, and 1; 0 when it has none.  `block` = heads taken together, tile by tile, at most: the heads are cut into
+ * blocks equal up to one round of 8 * streams heads (0: head by head, in the order of chill_work_item).  `streams` =
+ * neighbouring heads that share what they stream.  Over the workgroups of a grid the
  * (head, tile) pairs are a permutation of all of them. */
 int chill_launch_item(int32_t workgroup, int32_t heads, int32_t per_head, int32_t block, int32_t streams,
                       int32_t resident, int32_t out[2]);
+
+/* The `block` of chill_launch_item that the launches of one pass (ChillPass) take for these operands, or an error code. */
+int chill_launch_block(const ChillMaskDesc* mask, int32_t pass, int32_t has_lens, int32_t B, int32_t H, int32_t H_kv,
+                       int32_t T, int32_t D, int32_t dtype);
 
 /* Host twin of chill_tile_ranges_device (same functors compiled for the host). */
 int chill_tile_ranges(const ChillMaskDesc* mask, int32_t pass, int32_t T, int32_t seq_len,

@@ -338,6 +338,35 @@ def test_launch_items_keep_a_set_of_heads_on_its_xcds(streams, resident):
             assert per_xcd == [sets // 8 + bin(sets % 8).count("1")] * 8, (sets, block, per_xcd)
 
 
+@pytest.mark.parametrize("lens", [0, 1])
+@pytest.mark.parametrize("mask_id,args", [(1, ()), (2, (128, 128))], ids=["causal", "window"])
+def test_blocks_of_a_launch_are_of_one_size(mask_id, args, lens):
+    """The blocks of heads that the launches of every pass take (chill_launch_block) differ by at most one round of 8 sets,
+    and none of them, the last one above all, is smaller than the first by more than the sets of an incomplete round."""
+    L, out = _lib.lib, (ctypes.c_int32 * 2)()
+    desc = _lib.mask_desc(mask_id, args)
+    several = 0
+    for B, H, H_kv in ((8, 32, 32), (8, 16, 16), (8, 32, 8), (13, 8, 8), (7, 8, 8), (5, 9, 9), (3, 20, 4), (2, 25, 25), (1, 4, 4)):
+        for T in (700, 2085, 3000, 6000, 16384):
+            for D, dtype in ((64, 2), (128, 1), (128, 0)):
+                for pass_id in (0, 1, 2):
+                    block = L.chill_launch_block(ctypes.byref(desc), pass_id, lens, B, H, H_kv, T, D, dtype)
+                    if block == 0:
+                        assert mask_id == 2 and not lens
+                        continue
+                    heads, streams = (B * H_kv, 1) if pass_id == 2 else (B * H, H // H_kv)
+                    # three tiles a head: a block begins where tile 0 is taken again
+                    tiles = [L.chill_launch_item(w, heads, 3, block, streams, 1, out) and out[1] for w in range(3 * heads)]
+                    starts = [w for w in range(3 * heads) if tiles[w] == 0 and (w == 0 or tiles[w - 1] == 2)] + [3 * heads]
+                    sets = [(b - a) // 3 // streams for a, b in zip(starts, starts[1:])]
+                    assert sum(sets) * streams == heads
+                    assert max(sets) - min(sets) <= 8 and sets[-1] >= max(sets) - B * H_kv % 8, (B, H, H_kv, T, D, dtype, pass_id, sets)
+                    several += len(sets) > 1
+    assert several > (0 if mask_id == 1 or lens else -1)
+    assert L.chill_launch_block(ctypes.byref(desc), 3, 0, 1, 4, 4, 64, 64, 2) == -8
+    assert L.chill_launch_block(ctypes.byref(desc), 0, 0, 1, 4, 3, 64, 64, 2) < 0
+
+
 def test_cpu_tensors_are_refused():
     import torch
 
