@@ -14,7 +14,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # CHILL_ATTENTION_LIB names another build of the same library (for A/B measurements)
 LIB_PATH = os.environ.get("CHILL_ATTENTION_LIB") or os.path.join(os.path.dirname(_PKG_DIR), "lib", "libchill_attention_hip.so")
 
-ABI_VERSION = 1
+ABI_VERSION = 2  # CHILL_ABI_VERSION of the header: raised with every change of a signature or of EntryPoints
 
 # ChillDType / ChillMaskId / ChillPass of the header
 F32, F16, BF16 = 0, 1, 2
@@ -49,6 +49,12 @@ def load_library(path: str) -> ctypes.CDLL:
             "There is no fallback implementation."
         )
     lib = ctypes.CDLL(path)
+    # (before the symbols below: a library of another version may lack some)
+    if not hasattr(lib, "chill_abi_version"):
+        raise ImportError(f"chill_attention: {path} does not export chill_abi_version")
+    got = lib.chill_abi_version()
+    if got != ABI_VERSION:
+        raise ImportError(f"chill_attention: library ABI version {got}, binding expects {ABI_VERSION} (rebuild {path})")
     P = POINTER
     T4 = P(ChillTensor4)
     MD = P(ChillMaskDesc)
@@ -91,9 +97,6 @@ def load_library(path: str) -> ctypes.CDLL:
         fn = getattr(lib, name)  # AttributeError if the library lacks a declared symbol
         fn.restype = restype
         fn.argtypes = argtypes
-    got = lib.chill_abi_version()
-    if got != ABI_VERSION:
-        raise ImportError(f"chill_attention: library ABI version {got}, binding expects {ABI_VERSION}")
     return lib
 
 

@@ -75,6 +75,8 @@ def _kernel_sources_digest() -> bytes:
         if name.endswith((".h", ".hip", ".cpp", ".py")) or name == "Makefile":
             with open(os.path.join(CSRC_DIR, name), "rb") as f:
                 h.update(name.encode() + b"\0" + f.read())
+    # a library of another ABI version is refused (_lib.load_library), so a new version builds a new one
+    h.update(b"abi %d" % _lib.ABI_VERSION)
     return h.digest()
 
 

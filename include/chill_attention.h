@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define CHILL_ABI_VERSION 1
+#define CHILL_ABI_VERSION 2
 
 typedef enum ChillStatus {
     CHILL_OK = 0,

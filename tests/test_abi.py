@@ -4,6 +4,7 @@ argument validation answers with error codes before anything is launched (no GPU
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -365,6 +366,24 @@ def test_blocks_of_a_launch_are_of_one_size(mask_id, args, lens):
     assert several > (0 if mask_id == 1 or lens else -1)
     assert L.chill_launch_block(ctypes.byref(desc), 3, 0, 1, 4, 4, 64, 64, 2) == -8
     assert L.chill_launch_block(ctypes.byref(desc), 0, 0, 1, 4, 3, 64, 64, 2) < 0
+
+
+def test_library_of_another_abi_version_is_refused_by_name(tmp_path):
+    """A library built before the present entry points existed is told by its version, not by the first symbol it lacks;
+    the header and the binding name the same version."""
+    src = tmp_path / "old.c"
+    src.write_text("int chill_abi_version(void) { return 1; }\n")
+    old = tmp_path / "libold.so"
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(old), str(src)])
+    with pytest.raises(ImportError, match=f"ABI version 1, binding expects {_lib.ABI_VERSION}"):
+        _lib.load_library(str(old))
+    src.write_text("int something_else(void) { return 1; }\n")
+    other = tmp_path / "libother.so"
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(other), str(src)])
+    with pytest.raises(ImportError, match="chill_abi_version"):
+        _lib.load_library(str(other))
+    header = open(os.path.join(ROOT, "include", "chill_attention.h")).read()
+    assert f"#define CHILL_ABI_VERSION {_lib.ABI_VERSION}\n" in header
 
 
 def test_cpu_tensors_are_refused():

@@ -99,6 +99,13 @@ def test_a_mask_without_functor_is_refused():
         Bare().descriptor()
 
 
+def test_library_is_keyed_by_the_abi_version(monkeypatch):
+    """A library of another ABI version is refused when it is loaded, so a new version must build a new one."""
+    key = user_mask._key(SinkWindowChillMask)
+    monkeypatch.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)
+    assert user_mask._key(SinkWindowChillMask) != key
+
+
 def test_functor_text_is_wrapped_and_keyed_by_content():
     class A(ca.ChillMask):
         hip_functor = "static constexpr int kNumArgs = 0; /* ... */"
