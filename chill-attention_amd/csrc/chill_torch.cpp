@@ -203,11 +203,12 @@ class Attention : public torch::autograd::Function<Attention> {
 
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                    torch::autograd::variable_list grads) {
-        if (!grads[0].defined()) return torch::autograd::variable_list(9);
         const auto saved = ctx->get_saved_variables();
+        // (nothing is filled in for an O that got no gradient either: zeros, as the torch.library operators take it)
+        const at::Tensor d_o = grads[0].defined() ? grads[0] : at::zeros_like(saved[3]);
         const std::vector<int64_t> launch = ctx->saved_data["launch"].toIntVector();
         const c10::optional<at::Tensor> lens = saved[5].defined() ? c10::optional<at::Tensor>(saved[5]) : c10::nullopt;
-        auto [dq, dk, dv] = backward_impl(saved[0], saved[1], saved[2], lens, saved[3], saved[4], grads[0],
+        auto [dq, dk, dv] = backward_impl(saved[0], saved[1], saved[2], lens, saved[3], saved[4], d_o,
                                           launch[0], launch[1], at::IntArrayRef(launch).slice(2),
                                           ctx->saved_data["sm_scale"].toDouble());
         return {dq, dk, dv, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};

@@ -1093,3 +1093,31 @@ def test_forward_split_along_the_keys(D, dtype, H, Hkv, T, m, jump):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, captured) and torch.equal(lse, captured_lse)
+
+
+class _NoGradient(torch.autograd.Function):
+    """Passes its input on and gives it no gradient."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.parametrize("return_lse", [False, True])
+def test_an_undefined_gradient_of_the_output_counts_as_zeros(return_lse):
+    """What consumes O may give it no gradient at all: the gradients of q, k and v are zeros then, as those of the
+    torch.library operators are, and neither missing nor an error."""
+    mask = ca.CausalChillMask()
+    q, k, v = (make_qkv((2, h, 300, 64), torch.bfloat16, False).requires_grad_() for h in (4, 2, 2))
+    out = ca.chill_attention(q, k, v, mask=mask, return_lse=return_lse)
+    got = torch.autograd.grad(_NoGradient.apply(out[0] if return_lse else out).sum(), (q, k, v))
+    from chill_attention import chill as chill_mod
+
+    via_library = chill_mod._chill_attention(q, k, v, None, mask.name, mask.constargs, 0.125, return_lse, False, "ieee", False)
+    want = torch.autograd.grad(_NoGradient.apply(via_library[0] if return_lse else via_library).sum(), (q, k, v))
+    for x, g, w in zip((q, k, v), got, want):
+        assert torch.equal(g, torch.zeros_like(x)) and torch.equal(w, g)
