@@ -76,6 +76,27 @@ def test_forward_validation_returns_codes_without_launching():
     assert ei.value.status == E["dim"] and "head dim" in str(ei.value)
 
 
+def test_workspace_of_the_forward_is_checked_before_a_launch():
+    """chill_fwd_workspace: a workspace smaller than the launch needs is refused, and so is a misaligned one, also where the
+    launch needs none; what chill_fwd refuses stays refused."""
+    mask = _lib.mask_desc(_lib.MASK_CAUSAL, [])
+
+    def call(T, workspace, size, D=128):
+        t, s3 = _t4(strides=(1 << 24, 1 << 22, 128, 1)), (ctypes.c_int64 * 3)(8 * T, T, 1)
+        r = ctypes.byref(t)
+        return _lib.lib.chill_fwd_workspace(r, r, r, r, None, s3, None, 0, 1, 8, 8, T, D, _lib.BF16, 0.1, ctypes.byref(mask), workspace, size, None)
+
+    need = _lib.lib.chill_fwd_workspace_bytes(1, 8, 8192, 128, _lib.BF16, ctypes.byref(mask), 0)
+    assert need > 0
+    for size in (need - 1, 0, -1):
+        assert call(8192, 0x1000, size) == -8
+    assert call(8192, 0x1008, need) == -6
+    assert _lib.lib.chill_fwd_workspace_bytes(1, 8, 64, 128, _lib.BF16, ctypes.byref(mask), 0) == 0
+    assert call(64, 0x1008, 64) == -6
+    assert call(8192, 0x1000, need, D=48) == -3
+    assert _lib.lib.chill_fwd_workspace_bytes(1, 8, 8192, 48, _lib.BF16, ctypes.byref(mask), 0) == -3
+
+
 def test_backward_and_debug_validation():
     t = _t4()
     s3 = (ctypes.c_int64 * 3)(128, 64, 1)

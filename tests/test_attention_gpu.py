@@ -1121,3 +1121,154 @@ def test_an_undefined_gradient_of_the_output_counts_as_zeros(return_lse):
     want = torch.autograd.grad(_NoGradient.apply(via_library[0] if return_lse else via_library).sum(), (q, k, v))
     for x, g, w in zip((q, k, v), got, want):
         assert torch.equal(g, torch.zeros_like(x)) and torch.equal(w, g)
+
+
+def split_forward(q, k, v, mask, guard=0):
+    """chill_fwd_workspace with a workspace of exactly the size it asks for, `guard` bytes of 0xA5 on either side:
+    O, LSE2, the bytes around the workspace and the sums l that every part of a split q-tile left for its rows
+    ({(head, q-tile, part): [lanes of the workgroup]}; chill_fwd_split.h: per part O^T, then m0, then l)."""
+    B, H, T, D = q.shape
+    code, desc = {torch.float16: 1, torch.bfloat16: 2}[q.dtype], mask.descriptor()
+    rows = tile_config(mask, D, q.dtype, _lib.PASS_FWD, seq_len=T, batch_heads=B * H)["rows"]
+    size = _lib.lib.chill_fwd_workspace_bytes(B, H, T, D, code, ctypes.byref(desc), 0)
+    assert size > 0, "this shape is not split"
+    memory = torch.full((guard + size + guard,), 0xA5, dtype=torch.uint8, device=DEV)
+    out, lse = torch.empty(B, H, T, D, dtype=q.dtype, device=DEV), torch.empty(B, H, T, device=DEV)
+    tensors = [_lib.tensor4(x) for x in (q, k, v, out)]
+    _lib.check("chill_fwd_workspace", _lib.lib.chill_fwd_workspace(
+        *(ctypes.byref(t) for t in tensors), ctypes.c_void_p(lse.data_ptr()), _lib.strides3(lse), None, 0, B, H, k.shape[1], T, D, code,
+        D**-0.5, ctypes.byref(desc), ctypes.c_void_p(memory.data_ptr() + guard), size,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    buf = (ctypes.c_int32 * (4 * 512))()
+    n = _lib.lib.chill_fwd_split_items(B, H, T, D, code, ctypes.byref(desc), buf)
+    items = [tuple(buf[4 * i : 4 * i + 4]) for i in range(n)]
+    parts = sum(c > 1 for _, _, c, _ in items)
+    floats = rows * D + 4 * rows
+    partial = memory[guard : guard + 4 * B * H * parts * floats].view(torch.float32).view(B * H, parts, floats)
+    sums = {(h, qt, j): partial[h, first + j, rows * D + 2 * rows :] for qt, j, c, first in items if c > 1 for h in range(B * H)}
+    return out, lse, torch.cat([memory[:guard], memory[guard + size :]]), sums
+
+
+def split_reference(q, k, v, m):
+    """O and LSE2 of the dense reference, and how far LSE2 may be off: Q times the scale is rounded to the input type, so
+    eps * |q| * |k| * scale * log2(e) at most (see the ramp test above)."""
+    D, eps = q.shape[-1], {torch.bfloat16: 2.0**-9, torch.float16: 2.0**-12}[q.dtype]
+    ref, _ = orc.reference_naive(m[0], m[1], q.float(), k.float(), v.float(), None)
+    loose = eps * (D**-0.5 * 1.4427) * q.float().norm(dim=-1) * k.float().norm(dim=-1).max()
+    return ref.to(q.dtype), orc.lse2_dense(m[0], m[1], q, k, None), loose + 1e-2
+
+
+def step_inputs(B, H, Hkv, T, D, dtype, at, units):
+    """Inputs whose scores rise (fall, `units` < 0) by that many log2 units at key `at`, the same for every row."""
+    q, k, v = (torch.randn(B, h, T, D, device=DEV) * 0.5 for h in (H, Hkv, Hkv))
+    u = torch.nn.functional.normalize(torch.randn(D, device=DEV), dim=0)
+    q = q - (q @ u)[..., None] * u + 4.0 * u
+    on = (torch.arange(T, device=DEV) >= at) == (units > 0)
+    k = k + (abs(units) * D**0.5 / (4.0 * 1.4427)) * on.float()[None, None, :, None] * u
+    return [x.to(dtype) for x in (q, k, v)]
+
+
+def part_keys(H, T, D, dtype, mask):
+    """Keys of every part of a q-tile but the last: with all scores 0 a row's sum l counts the keys it sees."""
+    zero = torch.zeros(1, H, T, D, dtype=dtype, device=DEV)
+    _, _, _, sums = split_forward(zero, zero, zero, mask)
+    last = max(qt for _, qt, _ in sums)
+    count = max(j for _, qt, j in sums if qt == last) + 1
+    keys = int(sums[0, last, 0][0].item())
+    assert keys % 64 == 0 and 0 < keys * (count - 1) < T
+    return keys, last, count
+
+
+@pytest.mark.parametrize("units", [6, 30, 300, -6, -30, -300])
+@pytest.mark.parametrize("D,dtype,H,Hkv,T,m", SPLIT_CASES)
+def test_merge_of_parts_with_distant_references(D, dtype, H, Hkv, T, m, units):
+    """Scores that rise or fall exactly where the second part of a q-tile begins: every part of every split q-tile stays in
+    range (no sum is NaN) whatever the distance, so the merge alone makes O and LSE2 of those q-tiles from references m0 that
+    far apart; a weight underflows to 0 at 300 units and is far from 0 and 1 at 6."""
+    mask = make_mask(m)
+    torch.manual_seed(stable_seed(D, H, T, m, units, "merge") % 2**31)
+    at, last, count = part_keys(H, T, D, dtype, mask)
+    print(f"merge {mask} {dtype} D={D} H={H}/{Hkv} T={T} step of {units} at key {at}", flush=True)
+    q, k, v = step_inputs(1, H, Hkv, T, D, dtype, at, units)
+    out, lse, _, sums = split_forward(q, k, v, mask)
+    assert not any(torch.isnan(l).any().item() for l in sums.values())
+    ref, want_lse, loose = split_reference(q, k, v, m)
+    torch.testing.assert_close(out, ref, atol=OUT_TOL[dtype][0], rtol=OUT_TOL[dtype][1])
+    assert ((lse.double() - want_lse).abs() <= loose).all()
+
+
+@pytest.mark.parametrize("part", ["second", "last"])
+@pytest.mark.parametrize("D,dtype,H,Hkv,T,m", SPLIT_CASES)
+def test_a_later_part_leaves_the_range(D, dtype, H, Hkv, T, m, part):
+    """Scores that rise by 300 log2 units inside a tile of the second or of the last part of the last q-tile: that part and
+    no earlier one marks its sums NaN, and the q-tile is computed again."""
+    mask = make_mask(m)
+    torch.manual_seed(stable_seed(D, H, T, m, part, "later") % 2**31)
+    keys, last, count = part_keys(H, T, D, dtype, mask)
+    index = 1 if part == "second" else count - 1
+    at = index * keys + 64 + 30
+    print(f"later part {mask} {dtype} D={D} H={H}/{Hkv} T={T} part {index} of {count}, step at key {at}", flush=True)
+    q, k, v = step_inputs(1, H, Hkv, T, D, dtype, at, 300)
+    out, lse, _, sums = split_forward(q, k, v, mask)
+    assert all(torch.isnan(sums[h, last, index]).any() for h in range(H))
+    assert not any(torch.isnan(sums[h, last, j]).any() for h in range(H) for j in range(index))
+    ref, want_lse, loose = split_reference(q, k, v, m)
+    torch.testing.assert_close(out, ref, atol=OUT_TOL[dtype][0], rtol=OUT_TOL[dtype][1])
+    assert ((lse.double() - want_lse).abs() <= loose).all()
+
+
+@pytest.mark.parametrize("D,dtype,B,H,Hkv,T,m", [(128, torch.bfloat16, 2, 3, 3, 4229, ("CausalChillMask", ())),
+                                                 (128, torch.float16, 3, 2, 1, 4097, ("FullChillMask", ())),
+                                                 (64, torch.bfloat16, 2, 2, 1, 5001, ("PrefixLMChillMask", (635,)))])
+def test_split_forward_of_a_batch_and_its_gradients(D, dtype, B, H, Hkv, T, m):
+    """Several batch elements, shared key / value heads and heads interleaved in storage ([B, T, H, D]); the gradients come
+    from the LSE2 that the merge wrote."""
+    mask = make_mask(m)
+    code, desc = {torch.float16: 1, torch.bfloat16: 2}[dtype], mask.descriptor()
+    assert _lib.lib.chill_fwd_workspace_bytes(B, H, T, D, code, ctypes.byref(desc), 0) > 0, "this shape is not split"
+    print(f"split batch {mask} {dtype} D={D} B={B} H={H}/{Hkv} T={T}", flush=True)
+    q, k, v = (torch.randn(B, T, h, D, device=DEV).to(dtype).transpose(1, 2).requires_grad_() for h in (H, Hkv, Hkv))
+    dout = torch.randn(B, H, T, D, device=DEV).to(dtype)
+    out, lse = ca.chill_attention(q, k, v, mask=mask, return_lse=True)
+    out.backward(dout)
+    qf, kf, vf = (x.detach().float().clone().requires_grad_() for x in (q, k, v))
+    ref, _ = orc.reference_naive(m[0], m[1], qf, kf, vf, None)
+    ref.backward(dout.float())
+    check_close(out.detach(), ref.detach(), dtype, OUT_TOL[dtype], D, "O")
+    assert (lse.double() - orc.lse2_dense(m[0], m[1], q.detach(), k.detach(), None)).abs().max() <= 1e-2
+    for name, got, want in (("dq", q.grad, qf.grad), ("dk", k.grad, kf.grad), ("dv", v.grad, vf.grad)):
+        check_close(got, want, dtype, GRAD_TOL[dtype], D, name)
+
+
+@pytest.mark.parametrize("D,dtype,H,Hkv,T,m", SPLIT_CASES)
+def test_workspace_of_a_split_forward(D, dtype, H, Hkv, T, m):
+    """A split forward writes nothing outside the bytes it asked for.  With lens the workspace is not touched and the launch
+    is the whole one, as it is without a workspace: the same bits from chill_fwd and from chill_fwd_workspace with NULL."""
+    mask = make_mask(m)
+    print(f"workspace {mask} {dtype} D={D} H={H}/{Hkv} T={T}", flush=True)
+    q, k, v = (make_qkv((1, h, T, D), dtype, False) for h in (H, Hkv, Hkv))
+    out, lse, around, _ = split_forward(q, k, v, mask, guard=4096)
+    assert (around == 0xA5).all()
+    code, desc = {torch.float16: 1, torch.bfloat16: 2}[dtype], mask.descriptor()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    size = _lib.lib.chill_fwd_workspace_bytes(1, H, T, D, code, ctypes.byref(desc), 0)
+    memory = torch.full((size,), 0xA5, dtype=torch.uint8, device=DEV)
+    lens = torch.full((1,), T, dtype=torch.int32, device=DEV)
+    results = []
+    for workspace, lens_args in ((None, (None, 0)), (memory, (ctypes.c_void_p(lens.data_ptr()), 1)), ("chill_fwd", (None, 0))):
+        o, l = torch.full_like(out, float("nan")), torch.full_like(lse, float("nan"))
+        t = [_lib.tensor4(x) for x in (q, k, v, o)]
+        args = [*(ctypes.byref(x) for x in t), ctypes.c_void_p(l.data_ptr()), _lib.strides3(l), *lens_args, 1, H, Hkv, T, D, code, D**-0.5,
+                ctypes.byref(desc)]
+        if workspace == "chill_fwd":
+            _lib.check("chill_fwd", _lib.lib.chill_fwd(*args, stream))
+        else:
+            ptr = ctypes.c_void_p(workspace.data_ptr()) if workspace is not None else None
+            _lib.check("chill_fwd_workspace", _lib.lib.chill_fwd_workspace(*args, ptr, size if ptr else 0, stream))
+        results.append((o, l))
+    torch.cuda.synchronize()
+    assert (memory == 0xA5).all()
+    for o, l in results:
+        assert torch.equal(o, results[0][0]) and torch.equal(l, results[0][1])
+    torch.testing.assert_close(out, results[0][0], atol=OUT_TOL[dtype][0], rtol=OUT_TOL[dtype][1])
