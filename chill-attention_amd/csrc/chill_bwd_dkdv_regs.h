@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void dkdv_regs_kernel(BwdParams p, int n_k_til
 
     // key tiles first-to-last: for causal-like masks the longest run first
     int bh, ktile;
-    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, p.order, 1, 1, &bh, &ktile)) return;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, 1, &bh, &ktile)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 

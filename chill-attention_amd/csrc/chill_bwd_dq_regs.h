@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256) void dq_regs_kernel(BwdParams p, int n_q_tiles
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     int bh, qt;
-    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.order, p.group, 1, &bh, &qt)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, 1, &bh, &qt)) return;
     qt = n_q_tiles - 1 - qt;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;

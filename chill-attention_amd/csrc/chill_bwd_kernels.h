@@ -135,7 +135,7 @@ void dq_kernel(BwdParams p, int n_q_tiles,
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     int bh, qt;
-    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.order, p.group, dq_waves_per_simd<E, D, NW, TK, NS>(), &bh, &qt)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, dq_waves_per_simd<E, D, NW, TK, NS>(), &bh, &qt)) return;
     qt = n_q_tiles - 1 - qt;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
@@ -451,7 +451,7 @@ template <typename E, int D>
 int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
     const int block = work_block(mask_id, CHILL_PASS_DQ, p.lens != nullptr, p.B, p.H, p.H_kv, p.T, D, Elem<E>::kBytes);
-    p.order = work_order(p.lens != nullptr, (long long)p.B * p.H, p.group, block);
+    set_order(p, work_order(p.lens != nullptr, (long long)p.B * p.H, p.group, block));
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
     int status = CHILL_ERR_BAD_MASK;
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     int bh, qt;
-    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, p.order, p.group, 1, &bh, &qt)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, 1, &bh, &qt)) return;
     qt = n_q_tiles - 1 - qt;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
@@ -714,7 +714,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
     // (the 64-row workgroups of head dims up to 64 run three to a CU)
     // key tiles first-to-last: for causal-like masks the longest run first
     int bh, ktile;
-    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, p.order, 1, (NW == 4 && D <= 64) ? 3 : 1, &bh, &ktile)) return;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, (NW == 4 && D <= 64) ? 3 : 1, &bh, &ktile)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 
@@ -1129,7 +1129,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D >= 25
 
     // key tiles first-to-last: for causal-like masks the longest run first
     int bh, ktile;
-    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, p.order, 1, 1, &bh, &ktile)) return;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, 1, &bh, &ktile)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 
@@ -1396,7 +1396,7 @@ template <typename E, int D>
 int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
     const int block = work_block(mask_id, CHILL_PASS_DKDV, p.lens != nullptr, p.B, p.H, p.H_kv, p.T, D, Elem<E>::kBytes);
-    p.order = work_order(p.lens != nullptr, (long long)p.B * p.H_kv, 1, block);
+    set_order(p, work_order(p.lens != nullptr, (long long)p.B * p.H_kv, 1, block));
     int64_t max_stride = p.sq.t > p.sdo.t ? p.sq.t : p.sdo.t;
     if (p.sk.t > max_stride) max_stride = p.sk.t;
     if (p.sv.t > max_stride) max_stride = p.sv.t;

@@ -441,7 +441,7 @@ void fwd_kernel(FwdParams p, int n_q_tiles,
     // causal-like masks); unpaired: one q-tile per workgroup, last tiles first
     const int per_head = paired ? (n_q_tiles + 1) / 2 : n_q_tiles;
     int bh, j;
-    if (!work_item(blockIdx.x, p.B * p.H, per_head, p.order, p.group, paired ? 1 : fwd_waves_per_simd<E, D, NW, TK, NS>(), &bh, &j)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, per_head, order_of(p), p.group, paired ? 1 : fwd_waves_per_simd<E, D, NW, TK, NS>(), &bh, &j)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int qt_hi = n_q_tiles - 1 - j;
@@ -588,7 +588,7 @@ template <typename E, int D>
 int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStream_t stream) {
     FwdParams p = args;
     const int block = work_block(mask_id, CHILL_PASS_FWD, p.lens != nullptr, p.B, p.H, p.H_kv, p.T, D, Elem<E>::kBytes);
-    p.order = work_order(p.lens != nullptr, (long long)p.B * p.H, p.group, block);
+    set_order(p, work_order(p.lens != nullptr, (long long)p.B * p.H, p.group, block));
     // the async loader keeps per-lane global offsets in 32 bits
     const int64_t max_stride = p.sk.t > p.sv.t ? p.sk.t : p.sv.t;
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;

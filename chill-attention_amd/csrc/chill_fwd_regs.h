@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void fwd_regs_kernel(FwdParams p, int n_q_tile
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int per_head = paired ? (n_q_tiles + 1) / 2 : n_q_tiles;
     int bh, j;
-    if (!work_item(blockIdx.x, p.B * p.H, per_head, p.order, p.group, 1, &bh, &j)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, per_head, order_of(p), p.group, 1, &bh, &j)) return;
     agpr_reserve();
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;

@@ -14,9 +14,8 @@ struct Strides3 {  // element strides of a [B, H, T, D] tensor with unit inner s
 // The order in which a launch's workgroups take their (head, tile) items (work_order, chill_tiles.h).
 struct WorkOrder {
     int32_t small;    // blocks that come first, of `sets` sets of heads each; the others have 8 more.  0: contiguous runs
-    int32_t sets;     // a multiple of 8; the first block also has the sets of an incomplete round (all % 8)
-    int32_t all;      // sets of the launch
-    int32_t in_turn;  // a block of no whole number of rounds takes its heads in turn
+    int32_t sets;     // a multiple of 8
+    int32_t rest;     // sets of an incomplete round, which go with the first block; + 8: such a block takes its heads in turn
 };
 
 struct FwdParams {
@@ -31,9 +30,10 @@ struct FwdParams {
     int64_t lens_stride;
     int32_t B, H, H_kv, T;
     int32_t group;         // H / H_kv
-    WorkOrder order;
+    int32_t order_small;   // the WorkOrder; what only a launch in blocks reads is the struct's end, see order_of
     float scale_log2;      // sm_scale * log2(e)
     MaskArgs margs;
+    int32_t order_sets, order_rest;
 };
 
 // The forward of a launch with fewer q-tiles than the chip has room for: the keys of the long q-tiles are split into
@@ -79,11 +79,26 @@ struct BwdParams {
     int64_t lens_stride;
     int32_t B, H, H_kv, T;
     int32_t group;
-    WorkOrder order;
+    int32_t order_small;
     float sm_scale;
     float scale_log2;
     MaskArgs margs;
+    int32_t order_sets, order_rest;
 };
+
+// Three fields side by side cost the banded forward 300 moves of its pointers to vector lanes and back (scalar loads of eight
+// words in the middle of the struct leave no room for those of sixteen), and moved the code of the kernels that do not read
+// them: SlidingWindow(16, 16) from cold caches, fp16 B8 H4 T6000 D128 61 -> 64 us, fp32 B8 H8 T6000 D64 234 -> 242.
+template <typename P>
+CHILL_HD WorkOrder order_of(const P& p) {
+    return WorkOrder{p.order_small, p.order_sets, p.order_rest};
+}
+template <typename P>
+inline void set_order(P& p, WorkOrder order) {
+    p.order_small = order.small;
+    p.order_sets = order.sets;
+    p.order_rest = order.rest;
+}
 
 // One row of the static tile table (the replacement for the reference's autotune tables,
 // autotune.py:11-119): rows per workgroup = 32 * waves, streamed tile size.

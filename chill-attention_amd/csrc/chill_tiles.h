@@ -530,12 +530,12 @@ constexpr int work_block(int mask_id, int pass, bool padded, int B, int H, int H
 // XCDs get the long elements and others the short ones (causal D128 B3 H32/4, lengths 4096, 3000 and 1024, forward / dQ /
 // dK/dV: 214 / 288 / 720 us in turn, 264 / 366 / 756 in groups).
 constexpr WorkOrder work_order(bool padded, long long heads, int streams, int block) {
-    if (block == 0) return WorkOrder{0, 0, 0, 0};
+    if (block == 0) return WorkOrder{0, 0, 0};
     const long long sets = heads / streams, rounds = sets / 8;
     const long long most = block < 16ll * streams ? 1 : block / (8ll * streams);  // rounds of a block
     const long long wanted = ((sets + 7) / 8 + most - 1) / most;
     const long long blocks = wanted > rounds ? (rounds > 1 ? rounds : 1) : wanted;
-    return WorkOrder{(int32_t)(blocks - rounds % blocks), (int32_t)(rounds / blocks * 8), (int32_t)sets, padded ? 1 : 0};
+    return WorkOrder{(int32_t)(blocks - rounds % blocks), (int32_t)(rounds / blocks * 8), (int32_t)(sets % 8) + (padded ? 8 : 0)};
 }
 
 // Workgroup `wg` of a launch of `heads` heads (query heads, or key / value heads in dK/dV; `streams` of them share what
@@ -571,13 +571,14 @@ CHILL_HD bool work_item(int wg, int heads, int per_head, WorkOrder order, int st
             wg = (pass * kCusPerXcd + len - 1 - (local - pass * kCusPerXcd)) * kXcds + xcd;
         }
     }
-    const int rest = order.all % kXcds, set_items = streams * per_head;
-    int first = 0, sets = order.sets + rest;  // first set and number of sets of the block
-    if (wg >= sets * set_items) {
-        int later = wg - sets * set_items;  // items since the end of the first block
+    // (all of it is non-negative: unsigned divisions are the shorter ones)
+    const unsigned w = wg, rest = order.rest % kXcds, set_items = streams * per_head;
+    unsigned first = 0, sets = order.sets + rest;  // first set and number of sets of the block
+    if (w >= sets * set_items) {
+        unsigned later = w - sets * set_items;  // items since the end of the first block
         first = sets;
         sets = order.sets;
-        const int small_items = (order.small - 1) * sets * set_items;
+        const unsigned small_items = (order.small - 1) * sets * set_items;
         if (later >= small_items) {
             later -= small_items;
             first += (order.small - 1) * sets;
@@ -585,13 +586,13 @@ CHILL_HD bool work_item(int wg, int heads, int per_head, WorkOrder order, int st
         }
         first += later / (sets * set_items) * sets;
     }
-    const int size = sets * streams, i = wg - first * set_items;
+    const unsigned size = sets * streams, i = w - first * set_items;
     *tile = i / size;
-    int in_group = i - *tile * size;
-    int before = 0, shift = 3;  // sets of the block's groups before this one; min(n, 8) = 1 << shift
+    unsigned in_group = i - *tile * size;
+    unsigned before = 0, shift = 3;  // sets of the block's groups before this one; min(n, 8) = 1 << shift
     if (rest > 0 && first == 0) {
-        if (order.in_turn) {
-            *head = first * streams + in_group;
+        if (order.rest >= kXcds) {
+            *head = in_group;
             return true;
         }
         if (in_group < rest * streams)
@@ -600,8 +601,8 @@ CHILL_HD bool work_item(int wg, int heads, int per_head, WorkOrder order, int st
             before = rest;
         in_group -= before * streams;
     }
-    const int k = in_group >> shift, round = streams > 1 ? k / streams : k;  // (the heads of a set follow each other)
-    const int set = first + before + (wg & ((1 << shift) - 1)) + (round << shift);
+    const unsigned k = in_group >> shift, round = streams > 1 ? k / streams : k;  // (the heads of a set follow each other)
+    const unsigned set = first + before + (w & ((1 << shift) - 1)) + (round << shift);
     *head = set * streams + k - round * streams;
     return true;
 }
