@@ -17,7 +17,7 @@ namespace chill {
     X(bf16, 16) X(bf16, 32) X(bf16, 64) X(bf16, 128) X(bf16, 256)
 
 #define CHILL_DECLARE(name, d)                                                              \
-    int launch_fwd_##name##_##d(const FwdParams&, int, const FwdSplit*, hipStream_t);                        \
+    int launch_fwd_##name##_##d(const FwdParams&, int, const FwdSplit*, hipStream_t);       \
     int launch_delta_##name##_##d(const DeltaParams&, hipStream_t);                         \
     int launch_dq_##name##_##d(const BwdParams&, int, hipStream_t);                         \
     int launch_dkdv_##name##_##d(const BwdParams&, int, hipStream_t);

@@ -135,7 +135,8 @@ void dq_kernel(BwdParams p, int n_q_tiles,
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     int bh, qt;
-    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, dq_waves_per_simd<E, D, NW, TK, NS>(), &bh, &qt)) return;
+    constexpr int kResident = dq_waves_per_simd<E, D, NW, TK, NS>();
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, kResident, &bh, &qt)) return;
     qt = n_q_tiles - 1 - qt;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;

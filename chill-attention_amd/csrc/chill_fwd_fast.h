@@ -84,6 +84,9 @@ __device__ __forceinline__ bool workgroup_any(bool mine, char* flags) {
 // One part of a q-tile's keys (FwdSplit): which of how many, and where its partial result goes: O^T as the accumulators
 // hold it, then the row's reference m0 and sum l of every lane.  l = NaN: a row left the range the reference-free softmax
 // is exact in.  A q-tile of one part leaves its result, and in `again` whether such a row makes it wrong.
+// A part rounds P to 16 bits against the m0 of its own first keys, so a split launch differs from the whole one by that
+// rounding (2.4e-4 fp16, 2.8e-3 bf16 at most, relative) and is as far from attention in 64 bits: the ratio of the two errors
+// over 26 launches (masks, both types, D 64 and 128, T 4096 to 10873) is 0.997 to 1.0002.
 struct FwdPart {
     int index, count, tiles;
     float* partial;
@@ -103,10 +106,10 @@ __device__ __forceinline__ void store_partial(float* to, const f32x16 (&o)[D / 3
     to[DB * 16 * NT + NT + tid] = l;
 }
 
-// The q-tiles qt_a and then qt_b (-1: none) of one head, start to finish, or (SPLIT) one part of q-tile qt_a's keys.  While the rows of one q-tile
-// are normalised and stored, the first K/V tiles and the Q rows of the next one are already on their
-// way.  A q-tile in which a row left the range the reference-free softmax is exact in is computed
-// again by fwd_q_tile.
+// The q-tiles qt_a and then qt_b (-1: none) of one head, start to finish, or (SPLIT) one part of q-tile
+// qt_a's keys.  While the rows of one q-tile are normalised and stored, the first K/V tiles and the Q rows
+// of the next one are already on their way.  A q-tile in which a row left the range the reference-free
+// softmax is exact in is computed again by fwd_q_tile.
 template <typename E, int D, int MASK, int NW, int TK, int NS, bool SPLIT = false>
 __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem, int b, int hd, int qt_a, int qt_b,
                                                  int wave_has_full_blocks, FwdPart part = FwdPart{0, 1, 0, nullptr, nullptr}) {
@@ -496,8 +499,8 @@ __device__ __forceinline__ void fwd_fast_q_tiles(const FwdParams& p, char* smem,
 
 // The result of q-tile qt from the partial results of its `count` parts, added up in the order of the keys.
 template <typename E, int D, int MASK, int NW, int TK, int NS>
-__device__ __forceinline__ void fwd_merge_q_tile(const FwdParams& p, char* smem, int b, int hd, int qt, const float* partials,
-                                                 int count, int wave_has_full_blocks) {
+__device__ __forceinline__ void fwd_merge_q_tile(const FwdParams& p, char* smem, int b, int hd, int qt,
+                                                 const float* partials, int count, int wave_has_full_blocks) {
     using ET = typename Elem<E>::type;
     typedef FastSoftmaxLimits<E> Lim;
     constexpr int DB = D / 32, NT = NW * 64, ROW = DB * 16 * NT, SIZE = ROW + 2 * NT;
@@ -537,8 +540,10 @@ __device__ __forceinline__ void fwd_merge_q_tile(const FwdParams& p, char* smem,
     }
     if (!in_t) return;
     const float inv = 1.f / (l == 0.f ? 1.f : l);
-    store_row_transposed<E, D>(reinterpret_cast<ET*>(p.o) + b * p.so.b + hd * p.so.h + (int64_t)q_pos * p.so.t, o, inv, true, h);
-    if (p.lse != nullptr && h == 0) p.lse[b * p.lse_b + hd * p.lse_h + q_pos] = l == 0.f ? -INFINITY : top + __log2f(l);
+    ET* row = reinterpret_cast<ET*>(p.o) + b * p.so.b + hd * p.so.h + (int64_t)q_pos * p.so.t;
+    store_row_transposed<E, D>(row, o, inv, true, h);
+    if (p.lse != nullptr && h == 0)
+        p.lse[b * p.lse_b + hd * p.lse_h + q_pos] = l == 0.f ? -INFINITY : top + __log2f(l);
 }
 
 }  // namespace chill

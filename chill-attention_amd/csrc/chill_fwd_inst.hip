@@ -6,7 +6,8 @@
 #define CHILL_CAT3(a, b, c) CHILL_CAT3_(a, b, c)
 
 namespace chill {
-int CHILL_CAT3(launch_fwd_, CHILL_ELEM_NAME, CHILL_HEAD_DIM)(const FwdParams& p, int mask_id, const FwdSplit* split, hipStream_t stream) {
+int CHILL_CAT3(launch_fwd_, CHILL_ELEM_NAME, CHILL_HEAD_DIM)(const FwdParams& p, int mask_id, const FwdSplit* split,
+                                                             hipStream_t stream) {
     return launch_fwd<CHILL_ELEM, CHILL_HEAD_DIM>(p, mask_id, split, stream);
 }
 }  // namespace chill

@@ -436,12 +436,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
 void fwd_kernel(FwdParams p, int n_q_tiles,
                                                       int wave_has_full_blocks, int paired) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    // (unpaired q-tiles differ in length: the order for a grid that is resident at once)
     // paired: a workgroup takes q-tile j from the end and q-tile j from the start (equal work under
-    // causal-like masks); unpaired: one q-tile per workgroup, last tiles first
+    // causal-like masks); unpaired: one q-tile per workgroup, last tiles first (they differ in length: the
+    // order for a grid that is resident at once)
     const int per_head = paired ? (n_q_tiles + 1) / 2 : n_q_tiles;
     int bh, j;
-    if (!work_item(blockIdx.x, p.B * p.H, per_head, order_of(p), p.group, paired ? 1 : fwd_waves_per_simd<E, D, NW, TK, NS>(), &bh, &j)) return;
+    const int resident = paired ? 1 : fwd_waves_per_simd<E, D, NW, TK, NS>();
+    if (!work_item(blockIdx.x, p.B * p.H, per_head, order_of(p), p.group, resident, &bh, &j)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H;
     const int qt_hi = n_q_tiles - 1 - j;
@@ -471,7 +472,8 @@ void fwd_split_kernel(FwdParams p, FwdSplit split, int wave_has_full_blocks) {
     part.index = (item >> 10) & 31;
     part.count = (item >> 15) & 31;
     part.tiles = split.part_tiles;
-    part.partial = split.partials + ((int64_t)bh * split.partials_per_head + (item >> 20) + part.index) * split.partial_floats;
+    const int64_t slot = (int64_t)bh * split.partials_per_head + (item >> 20) + part.index;
+    part.partial = split.partials + slot * split.partial_floats;
     part.again = split.again + bh * split.n_q_tiles + qt;
     fwd_fast_q_tiles<E, D, MASK, NW, TK, NS, true>(p, smem, bh / p.H, bh % p.H, qt, -1, wave_has_full_blocks, part);
 }
@@ -487,8 +489,10 @@ __global__ __launch_bounds__(NW * 64) void fwd_merge_kernel(FwdParams p, FwdSpli
             fwd_q_tile<E, D, MASK, NW, TK, 3>(p, smem, bh / p.H, bh % p.H, i, wave_has_full_blocks);
         return;
     }
-    const float* partials = split.partials + ((int64_t)bh * split.partials_per_head + (item >> 20)) * split.partial_floats;
-    fwd_merge_q_tile<E, D, MASK, NW, TK, NS>(p, smem, bh / p.H, bh % p.H, item & 1023, partials, (item >> 15) & 31, wave_has_full_blocks);
+    const int64_t slot = (int64_t)bh * split.partials_per_head + (item >> 20);
+    fwd_merge_q_tile<E, D, MASK, NW, TK, NS>(p, smem, bh / p.H, bh % p.H, item & 1023,
+                                             split.partials + slot * split.partial_floats, (item >> 15) & 31,
+                                             wave_has_full_blocks);
 }
 
 // Launcher for one (element type, head dim); dispatches on the mask id and takes the tile shape
@@ -500,7 +504,11 @@ constexpr int kPairedMinWorkgroups = 256;
 // longest first (work_block), fill it.  Taken where more than a fifth of the last round's share is lost (`slots` =
 // workgroups the chip holds at once: 1.5 rounds of pairs, prefix-LM D128 B4 H16 T3000, 171 -> 159 us; 2.5 rounds, causal
 // B4 H32/8 T2085, 172 / 174; whole rounds 3-4 % slower), and on padded batches, where a pair has no fixed length
-// (causal D128 B8 H16 T1000 48 -> 41 us, T8192 1004 -> 951).
+// (causal D128 B8 H16 T1000 48 -> 41 us, T8192 1004 -> 951).  The other masks gain as well, us, pairs -> single, at 1.5
+// rounds: full D128 B2 H16 T6000 551 -> 476, D256 B4 H12 T2048 285 -> 236, fp32 D64 B1 H12 T8192 2266 -> 1724; sliding
+// window 128 + 128 D64 B8 H16 T1500 44 -> 40, 1024 + 0 D128 B2 H32 T3000 134 -> 115; chunkwise 128 x 2 D128 B8 H16 T1500
+// 66 -> 59, 300 x 2 D64 B4 H16 T3000 87 -> 73.  Chunkwise 128 x 2 at D64 is within 4 % either way (B8 H16 T1500 35 -> 37,
+// B1 H32 T6000 38 -> 37); the most that any of 126 launches of 1.1 to 2.3 rounds lost.
 inline bool fwd_takes_pairs(int64_t pairs, int slots, bool padded) {
     if (pairs < kPairedMinWorkgroups || padded) return false;
     const int64_t rounds = (pairs + slots - 1) / slots;
@@ -520,8 +528,8 @@ int launch_fwd_shape(const FwdParams& p, hipStream_t stream) {
     // pairing q-tiles balances long causal runs; with few workgroups it only halves the number of
     // CUs that get work
     const int64_t pairs = (int64_t)p.B * p.H * ((n_q_tiles + 1) / 2);
-    constexpr int kSlots = kComputeUnits * (fwd_uses_regs(D, Elem<E>::kDType) ? 1 : fwd_waves_per_simd<E, D, cfg.waves, cfg.streamed, NS>());
-    const bool paired = fwd_takes_pairs(pairs, kSlots, p.lens != nullptr);
+    constexpr int kPerCu = fwd_uses_regs(D, Elem<E>::kDType) ? 1 : fwd_waves_per_simd<E, D, cfg.waves, cfg.streamed, NS>();
+    const bool paired = fwd_takes_pairs(pairs, kComputeUnits * kPerCu, p.lens != nullptr);
     const int64_t total64 = (int64_t)p.B * p.H * (paired ? (n_q_tiles + 1) / 2 : n_q_tiles);
     if (total64 > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
     const int total = (int)total64;
@@ -549,9 +557,9 @@ int launch_fwd_split(const FwdParams& p, const FwdSplit& split, hipStream_t stre
     constexpr int kLdsBytes = fwd_lds_bytes<E, D, cfg.streamed, NS>();
     auto kern = fwd_split_kernel<E, D, MASK_ID, cfg.waves, cfg.streamed, NS>;
     auto merge = fwd_merge_kernel<E, D, MASK_ID, cfg.waves, cfg.streamed, NS>;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(merge), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)
-        return CHILL_ERR_HIP;
+    for (const void* f : {reinterpret_cast<const void*>(kern), reinterpret_cast<const void*>(merge)}) {
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess) return CHILL_ERR_HIP;
+    }
     const int hfb = Mask<MASK_ID>::has_full_blocks(32, cfg.streamed, p.T, p.margs) ? 1 : 0;
     const dim3 block(cfg.waves * 64);
     hipLaunchKernelGGL(kern, dim3(p.B * p.H * split.n_items), block, kLdsBytes, stream, p, split, hfb);

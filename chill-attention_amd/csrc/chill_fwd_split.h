@@ -32,13 +32,15 @@ constexpr int kFwdItemOverhead = 8, kFwdPartOverhead = 16, kFwdMergeOverhead = 1
 //   full    D128  H2 T16384 269 -> 232   H3 T8192 135 -> 107  H4 T8192 140 -> 129  H6 T4096  74 -> 66
 //   left whole by the rule (measured split): causal D128 H16 T4096 85 (89), H12 T4042 80 (85); full H12 T8192 354 (366), D64
 //   H6 T4096 36 (40).
-inline int64_t plan_fwd_split(int mask_id, const MaskArgs& margs, int64_t heads, int T, int D, int dtype, void* workspace, FwdSplit* out) {
+inline int64_t plan_fwd_split(int mask_id, const MaskArgs& margs, int64_t heads, int T, int D, int dtype, void* workspace,
+                              FwdSplit* out) {
     if (!fwd_split_serves(mask_id, D, dtype)) return 0;
     const TileConfig cfg = fwd_tile_config(mask_id, D, dtype);
     const int n_q_tiles = cdiv(T, cfg.rows);
     // launches that fill the chip with pairs of q-tiles, and those that other kernels take
     if (n_q_tiles > kFwdSplitMaxQTiles || heads * ((n_q_tiles + 1) / 2) >= kComputeUnits) return 0;
-    if (fwd_takes_small(mask_id, heads, T, D, dtype) || (D == 128 && fwd_takes_short_row(mask_id, kWholeSequence, heads, T))) return 0;
+    if (fwd_takes_small(mask_id, heads, T, D, dtype)) return 0;
+    if (D == 128 && fwd_takes_short_row(mask_id, kWholeSequence, heads, T)) return 0;
     const int slots = D == 64 ? kComputeUnits * 3 / 2 : kComputeUnits;
     int tiles[kFwdSplitMaxQTiles];
     int longest = 0;
