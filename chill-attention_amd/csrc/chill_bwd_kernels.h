@@ -24,6 +24,7 @@
 #include "chill_bwd_dkdv_regs.h"
 #include "chill_bwd_dq_regs.h"
 #include "chill_bwd_dq_gen.h"
+#include "chill_f32.h"
 
 namespace chill {
 
@@ -419,16 +420,16 @@ int launch_dq_regs2(const BwdParams& p, hipStream_t stream) {
 // PASS 1: dQ (workgroups over query blocks), 2: dK/dV (over key blocks).
 template <typename E, int D, int MASK_ID, int PASS>
 int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
-    constexpr int kLdsOne = bwd_small_lds_bytes(D, Elem<E>::kDType, PASS);
+    constexpr int kLdsOne = bwd_small_set_bytes(D, Elem<E>::kDType, PASS);
     const int n_tiles = cdiv(p.T, 32);
     const long long heads = (long long)p.B * (PASS == 1 ? p.H : p.H_kv);  // (few by bwd_takes_small)
     // (dK/dV keeps one block per workgroup: with K, V and two accumulators a wave needs more than the 256 registers it
-    // would be left with)
-    constexpr bool kTwoFit = PASS == 1 && small_fits_two_tiles(kLdsOne);
+    // would be left with; fp32 of more tiles than CUs: dq_f32_kernel)
+    constexpr bool kTwoFit = PASS == 1 && Elem<E>::k16 && small_fits_two_tiles(kLdsOne);
     bool two = false;
     if constexpr (kTwoFit) two = small_takes_two_tiles(heads * n_tiles);
     const int total = (int)(heads * (two ? (n_tiles + 1) / 2 : n_tiles));
-    const int lds_bytes = two ? 2 * kLdsOne : kLdsOne;
+    const int lds_bytes = two ? 2 * kLdsOne : PASS == 2 ? bwd_small_lds_bytes(D, Elem<E>::kDType, 2) : kLdsOne;
     void (*kern)(BwdParams, int, int, int);
     if constexpr (PASS == 1)
         kern = dq_small_kernel<E, D, MASK_ID, 1>;
@@ -448,6 +449,25 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
+// fp32 rows of at most 512 bytes (dq_f32_kernel, dkdv_f32_kernel)
+template <int D, int MASK_ID, int PASS, int R, int S>
+int launch_bwd_f32(const BwdParams& p, int lds_bytes, hipStream_t stream) {
+    const int n_tiles = cdiv(p.T, 32), n_groups = cdiv(n_tiles, R);
+    const int64_t total = (int64_t)p.B * (PASS == 1 ? p.H : p.H_kv) * n_groups;
+    if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
+    void (*kern)(BwdParams, int, int, int);
+    if constexpr (PASS == 1)
+        kern = dq_f32_kernel<D, MASK_ID, R, S>;
+    else
+        kern = dkdv_f32_kernel<D, MASK_ID, R, S>;
+    if (f32_lds_bytes(D, R, S, PASS == 1 ? CHILL_PASS_DQ : CHILL_PASS_DKDV) > lds_bytes) return CHILL_ERR_HIP;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+        return CHILL_ERR_HIP;
+    const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
+    hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(R * S * 64), lds_bytes, stream, p, n_tiles, n_groups, hfb ? 1 : 0);
+    return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
+}
+
 template <typename E, int D>
 int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
     BwdParams p = args;
@@ -457,6 +477,24 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
     int status = CHILL_ERR_BAD_MASK;
     CHILL_DISPATCH_MASK(mask_id, {
+        if constexpr (f32_serves(D, Elem<E>::kDType)) {
+            constexpr int kLdsOne = bwd_small_lds_bytes(D, CHILL_F32, 1);
+            const long long tiles = (long long)p.B * p.H * cdiv(p.T, 32);
+            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_DQ, D, tiles, p.T);
+            const bool small = bwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, CHILL_F32, CHILL_PASS_DQ);
+            if (shape.members == 4 || !small) {
+                constexpr int kLds = f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ);
+                return launch_bwd_f32<D, MASK_ID, 1, 4, 1>(p, D > 64 && small ? kLdsOne : kLds, stream);
+            }
+            if constexpr (D <= 64) {
+                if (shape.members == 0) return launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
+                if (shape.members == 2) return launch_bwd_f32<D, MASK_ID, 1, 2, 4>(p, 2 * kLdsOne, stream);
+                if (shape.streams == 8) return launch_bwd_f32<D, MASK_ID, 1, 1, 8>(p, 2 * kLdsOne, stream);
+            } else {
+                if (shape.members == 2) return launch_bwd_f32<D, MASK_ID, 1, 2, 2>(p, kLdsOne, stream);
+            }
+            return launch_bwd_f32<D, MASK_ID, 1, 1, 4>(p, kLdsOne, stream);
+        } else {
         // the table has a row of its own for short sequences and small grids where that row differs
         constexpr bool has_short_row = dq_tile_config(MASK_ID, D, Elem<E>::kDType, 1).waves !=
                                        dq_tile_config(MASK_ID, D, Elem<E>::kDType).waves;
@@ -474,6 +512,7 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
                                                                    : launch_dq_shape<E, D, MASK_ID, false>(p, stream);
         } else {
             status = launch_dq_shape<E, D, MASK_ID, false>(p, stream);
+        }
         }
     });
     return status;
@@ -1404,6 +1443,27 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
     if (max_stride * Elem<E>::kBytes * 256 >= ((int64_t)1 << 31)) return CHILL_ERR_TOO_LARGE;
     int status = CHILL_ERR_BAD_MASK;
     CHILL_DISPATCH_MASK(mask_id, {
+        if constexpr (f32_serves(D, Elem<E>::kDType) && D <= 64) {
+            constexpr int kLds = bwd_small_lds_bytes(D, CHILL_F32, 2);
+            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_DKDV, D, (long long)p.B * p.H_kv * cdiv(p.T, 32), p.T);
+            const bool small = bwd_takes_small(MASK_ID, (long long)p.B * p.H_kv, p.T, D, CHILL_F32, CHILL_PASS_DKDV);
+            if (shape.members == 4 || !small)
+                return launch_bwd_f32<D, MASK_ID, 2, 4, 2>(p, small ? kLds : f32_lds_bytes(D, 4, 2, CHILL_PASS_DKDV), stream);
+            if (shape.members == 0) return launch_bwd_small<E, D, MASK_ID, 2>(p, stream);
+            if (shape.members == 2) return launch_bwd_f32<D, MASK_ID, 2, 2, 4>(p, kLds, stream);
+            return launch_bwd_f32<D, MASK_ID, 2, 1, 4>(p, kLds, stream);
+        } else if constexpr (f32_serves(D, Elem<E>::kDType)) {
+            const int n_tiles = cdiv(p.T, 32), n_groups = cdiv(n_tiles, 4);
+            const int64_t total = (int64_t)p.B * p.H_kv * n_groups;
+            if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
+            constexpr int kLds = f32_wide_lds_bytes(D);
+            auto kern = dkdv_f32_wide_kernel<D, MASK_ID>;
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+                return CHILL_ERR_HIP;
+            const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
+            hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(512), kLds, stream, p, n_tiles, n_groups, hfb ? 1 : 0);
+            return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
+        } else {
         // the table has a row of its own for small grids where that row differs
         constexpr bool has_small_row = dkdv_tile_config(MASK_ID, D, Elem<E>::kDType, true).waves !=
                                        dkdv_tile_config(MASK_ID, D, Elem<E>::kDType, false).waves;
@@ -1422,6 +1482,7 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
                                                                         : launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);
         } else {
             status = launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);
+        }
         }
     });
     return status;

@@ -406,6 +406,7 @@ __device__ __forceinline__ void fwd_q_tile(const FwdParams& p, char* smem, int b
 #include "chill_fwd_regs.h"
 #include "chill_fwd_fast.h"
 #include "chill_fwd_small.h"
+#include "chill_f32.h"
 #include "chill_fwd_split.h"
 namespace chill {
 
@@ -574,11 +575,11 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     const int n_q_tiles = cdiv(p.T, 32);
     // (at most kComputeUnits / 4 * 4 * 32 q-tiles by fwd_takes_small)
     bool two = false;
-    if constexpr (small_fits_two_tiles(kLdsOne)) two = small_takes_two_tiles((long long)p.B * p.H * n_q_tiles);
+    if constexpr (small_fits_two_tiles(kLdsOne) && Elem<E>::k16) two = small_takes_two_tiles((long long)p.B * p.H * n_q_tiles);
     const int total = p.B * p.H * (two ? (n_q_tiles + 1) / 2 : n_q_tiles);
     const int lds_bytes = two ? 2 * kLdsOne : kLdsOne;
     void (*kern)(FwdParams, int, int, int) = fwd_small_kernel<E, D, MASK_ID, 1>;
-    if constexpr (small_fits_two_tiles(kLdsOne)) {
+    if constexpr (small_fits_two_tiles(kLdsOne) && Elem<E>::k16) {  // (fp32 of more tiles than CUs: fwd_f32_kernel)
         if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2>;
     }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
@@ -589,6 +590,21 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     }
     hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two ? 2 : 1)), lds_bytes, stream, p, n_q_tiles, total,
                        hfb ? 1 : 0);
+    return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
+}
+
+// fp32 rows of at most 512 bytes (fwd_f32_kernel)
+template <int D, int MASK_ID, int R, int S>
+int launch_fwd_f32(const FwdParams& p, int lds_bytes, hipStream_t stream) {
+    const int n_tiles = cdiv(p.T, 32), n_groups = cdiv(n_tiles, R);
+    const int64_t total = (int64_t)p.B * p.H * n_groups;
+    if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
+    auto kern = fwd_f32_kernel<D, MASK_ID, R, S>;
+    if (f32_lds_bytes(D, R, S, CHILL_PASS_FWD) > lds_bytes) return CHILL_ERR_HIP;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+        return CHILL_ERR_HIP;
+    const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
+    hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(R * S * 64), lds_bytes, stream, p, n_tiles, n_groups, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -605,6 +621,25 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
         if constexpr (fwd_split_serves(MASK_ID, D, Elem<E>::kDType)) {
             if (split != nullptr) return launch_fwd_split<E, D, MASK_ID>(p, *split, stream);
         }
+        if constexpr (f32_serves(D, Elem<E>::kDType)) {
+            constexpr int kLdsOne = fwd_small_lds_bytes(D, CHILL_F32);
+            const long long tiles = (long long)p.B * p.H * cdiv(p.T, 32);
+            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_FWD, D, tiles, p.T);
+            const bool small = fwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, CHILL_F32);
+            if (shape.members == 4 || !small) {
+                // (up to the sizes the small launches end at, rows of 512 bytes keep their LDS)
+                constexpr int kLds = f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ);
+                return launch_fwd_f32<D, MASK_ID, 4, 1>(p, D > 64 && small ? kLdsOne : kLds, stream);
+            }
+            if constexpr (D <= 64) {
+                if (shape.members == 0) return launch_fwd_small<E, D, MASK_ID>(p, stream);
+                if (shape.members == 2) return launch_fwd_f32<D, MASK_ID, 2, 4>(p, 2 * kLdsOne, stream);
+                if (shape.streams == 8) return launch_fwd_f32<D, MASK_ID, 1, 8>(p, 2 * kLdsOne, stream);
+            } else {
+                if (shape.members == 2) return launch_fwd_f32<D, MASK_ID, 2, 2>(p, kLdsOne, stream);
+            }
+            return launch_fwd_f32<D, MASK_ID, 1, 4>(p, kLdsOne, stream);
+        } else {
         // the table has a row of its own for short sequences and small grids where that row differs
         constexpr bool has_short_row = fwd_tile_config(MASK_ID, D, Elem<E>::kDType, 1).waves !=
                                        fwd_tile_config(MASK_ID, D, Elem<E>::kDType).waves;
@@ -618,6 +653,7 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
             status = short_row ? launch_fwd_shape<E, D, MASK_ID, true>(p, stream) : launch_fwd_shape<E, D, MASK_ID, false>(p, stream);
         } else {
             status = launch_fwd_shape<E, D, MASK_ID, false>(p, stream);
+        }
         }
     });
     return status;

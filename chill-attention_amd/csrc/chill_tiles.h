@@ -189,10 +189,61 @@ constexpr bool fwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 // alone: forward 66 against 69, dQ 87 against 101 us on the prefix-LM shape.
 constexpr bool small_fits_two_tiles(int lds_bytes_one) { return 2 * lds_bytes_one <= 160 * 1024; }
 constexpr bool small_takes_two_tiles(long long tiles) { return tiles > kComputeUnits; }
-// what the report says of such a launch: 32 rows and 4 waves per tile; the LDS of the workgroup (of both tiles)
+// fp32 rows of at most 512 bytes go through fwd_f32_kernel, dq_f32_kernel and dkdv_f32_kernel (chill_f32.h): `members` row tiles
+// of 32 rows per workgroup, `streams` waves each; 0: the small-launch kernels, whose fp32 MFMAs need no preparation.
+// The report counts such a workgroup as 32 rows up to the sizes above (fwd_small_max_tiles and its like, where the fp32 MFMA
+// kernels were handed over to those of 128 rows) and as 128 rows beyond.
+// Measured in us, forward / dQ / dK/dV, the fp32 MFMA kernels first, all causal at head dim 64 where not named:
+//   few blocks per row, where splitting them costs what it saves: B1 H2 T256 9.8 / 13.4 / 15.4, eight streams 10.1 / 15.9,
+//     four streams 15.0; T512 15.2 / 20.4 / 24.6, eight streams 12.7 / 19.8, four 21.7
+//   fewer tiles than CUs: B1 H4 T1111 29.8 / 38.2 / 86, four streams 26.2 / 32.5 / 66, eight 19.4 / 27.5 (dK/dV spills)
+//   pairs (two members, four streams) against four members: prefix-LM B1 H8 T2048 (512 tiles) 57 / 77 / 119, 38 / 49 / 64, 83 / 101 /
+//     96; B3 H8 T1024 (768) 48 / 68 / 80, 37 / 50 / 60, 45 / 56 / 54; B2 H8 T3000 (1500) 179 / 244 / 390, 123 / 156 / -, 124 / 151 /
+//     154; full mask B3 H8 T1024 77 / 109 / 137, 49 / 65 / 60, 45 / 56 / 59; window 128 B4 H8 T1024 28 / 42 / 44, 23 / 35 / 24,
+//     17 / 23 / 24.  (At 2048 tiles, where the report of the pairs ends, four members are ahead: 93 / 119 against 119 / 156.)
+//   head dim 128: B1 H8 T1024 45 / 62 / 327, four streams 42 / 54, dkdv_f32_wide_kernel 112; window 128 B1 H16 T1024 (512) 31 / 49 /
+//     91, pairs 21 / 30, four members 23 / 45, wide 38; full mask B4 H16/4 T1500 660 / 1000 / 1880, four members 256 / 577, wide 635
+//   filled chip: B4 H16 T4096 1160 / 1680 / 2210, four members 509 / 659 / 925; full mask T1500 315 / 460 / 612, 153 / 196 / 260
+struct F32Shape {
+    int members, streams;
+};
+constexpr bool f32_serves(int D, int dtype) { return dtype == CHILL_F32 && D <= 128; }
+constexpr F32Shape f32_shape(int mask_id, int pass, int D, long long tiles, int T) {
+    const bool grow = mask_rows_grow(mask_id);
+    if (D <= 64) {
+        if (tiles <= kComputeUnits && T <= 384) return F32Shape{0, 0};
+        if (pass == CHILL_PASS_DKDV) return tiles <= kComputeUnits ? F32Shape{1, 4} : tiles <= 512 ? F32Shape{2, 4} : F32Shape{4, 2};
+        if (tiles < kComputeUnits) return F32Shape{1, 8};
+        if (tiles == kComputeUnits) return F32Shape{1, 4};
+        return tiles <= (grow ? 2048 : 768) ? F32Shape{2, 4} : F32Shape{4, 1};
+    }
+    if (pass == CHILL_PASS_DKDV) return F32Shape{4, 2};  // dkdv_f32_wide_kernel
+    if (tiles <= (grow ? 512 : 256)) return F32Shape{1, 4};
+    return tiles <= 512 ? F32Shape{2, 2} : F32Shape{4, 1};
+}
+// what the report says of a small launch: 32 rows and the 4 waves of a set; the LDS of the workgroup, which takes two tiles or
+// one tile with two sets
 constexpr TileConfig small_tile_config(int lds_bytes_one, long long tiles) {
     return TileConfig{32, 32, kFwdSmallWaves,
                       (small_fits_two_tiles(lds_bytes_one) && small_takes_two_tiles(tiles)) ? 2 * lds_bytes_one : lds_bytes_one};
+}
+// LDS of an fp32 workgroup: per stream two stages (one where a wave has its blocks to itself) of two 32-row tiles, the scales of
+// their slices and, in dK/dV, LSE2 and delta of the block's rows; at the end the streams' partial sums, in the forward with m
+// and l of every lane
+constexpr int f32_lds_bytes(int D, int members, int streams, int pass) {
+    const int vec = pass == CHILL_PASS_DKDV ? 64 : 0;
+    const int stages = members >= 2 ? 2 : 1, slices = members >= 2 ? members / 2 : 1;
+    const int ring = stages * streams * (2 * 32 * D * 4 + 2 * slices * 4 + vec * 4);
+    const int merge = streams > 1 ? members * streams * ((D + 31) / 32 * 16 * 64 + (pass == CHILL_PASS_FWD ? 128 : 0)) * 4 : 0;
+    return ring > merge ? ring : merge;
+}
+// (dkdv_f32_wide_kernel: the ring of eight waves, then the products the two waves of a tile trade)
+constexpr int f32_wide_ring_bytes(int D) { return (f32_lds_bytes(D, 8, 1, CHILL_PASS_DKDV) + 15) / 16 * 16; }
+constexpr int f32_wide_lds_bytes(int D) { return f32_wide_ring_bytes(D) + 8 * 16 * 64 * 4; }
+constexpr TileConfig f32_small_tile_config(F32Shape shape, int D, int lds_bytes_one) {
+    if (D <= 64 && shape.members == 4) return TileConfig{32, 32, kFwdSmallWaves, f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ)};
+    const bool two = D <= 64 && shape.members * shape.streams == 8;
+    return TileConfig{32, 32, two && shape.members == 1 ? 8 : kFwdSmallWaves, two ? 2 * lds_bytes_one : lds_bytes_one};
 }
 
 // The backward of such launches (dq_small_kernel, dkdv_small_kernel): the same split of the streamed
@@ -205,7 +256,12 @@ constexpr int bwd_small_wave_bytes(int D, int dtype, int outputs) {
     const int blocks = 2 * 32 * D * elem_bytes(dtype), partial = outputs * ((D + 31) / 32) * 16 * 64 * 4;
     return (blocks > partial ? blocks : partial) + 2 * 32 * 4;
 }
-constexpr int bwd_small_lds_bytes(int D, int dtype, int outputs) { return kFwdSmallWaves * bwd_small_wave_bytes(D, dtype, outputs); }
+constexpr int bwd_small_set_bytes(int D, int dtype, int outputs) { return kFwdSmallWaves * bwd_small_wave_bytes(D, dtype, outputs); }
+// (fp32 dK/dV: what dkdv_f32_kernel needs for two tiles side by side or four in half as many streams, in every launch)
+constexpr int bwd_small_lds_bytes(int D, int dtype, int outputs) {
+    const int set = bwd_small_set_bytes(D, dtype, outputs);
+    return dtype == CHILL_F32 && outputs == 2 ? 2 * set + 64 : set;
+}
 #ifndef CHILL_TUNE_BWD_SMALL_SCALE
 #define CHILL_TUNE_BWD_SMALL_SCALE 1
 #endif
@@ -234,6 +290,7 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 }
 
 constexpr TileConfig fwd_tile_config(int mask_id, int D, int dtype, int T = kLongSequence) {
+    if (f32_serves(D, dtype)) return TileConfig{128, 32, 4, f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ)};
     const int waves = fwd_waves(mask_id, D, dtype, T);
     const int streamed = fwd_streamed(mask_id, D, dtype, T);
     return TileConfig{waves * 32, streamed, waves,
@@ -290,6 +347,7 @@ constexpr TileConfig dq_regs2_tile_config(int D, int dtype) {
 // tiles, then one 4 KiB slot per wave for the two products of a block.
 constexpr bool dq_is_split(int D, int dtype) { return dtype == CHILL_F32 && D == 256; }
 constexpr TileConfig dq_tile_config(int mask_id, int D, int dtype, int T = kLongSequence) {
+    if (f32_serves(D, dtype)) return TileConfig{128, 32, 4, f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ)};
     const int waves = dq_waves(mask_id, D, dtype, T);
     const int streamed = dq_streamed(D, dtype);
     if (dq_is_split(D, dtype)) return TileConfig{waves * 16, 32, waves, 2 * 2 * 32 * D * 4 + waves * 16 * 64 * 4};
@@ -396,6 +454,7 @@ constexpr bool dkdv_takes_regs(int mask_id, long long mask_arg0, long long band_
 
 // `regs`: the row of dkdv_regs_kernel where that kernel is an option (dkdv_regs_is_optional)
 constexpr TileConfig dkdv_tile_config(int mask_id, int D, int dtype, bool small_grid = false, bool regs = false) {
+    if (f32_serves(D, dtype)) return D <= 64 ? TileConfig{128, 64, 8, f32_lds_bytes(D, 4, 2, CHILL_PASS_DKDV)} : TileConfig{128, 32, 8, f32_wide_lds_bytes(D)};
     const int row_bytes = D * elem_bytes(dtype);
     const int blocks = (regs && dkdv_regs_is_optional(D, dtype)) ? kDkdvRegsBlocks128 : dkdv_regs_blocks(D, dtype);
     if (blocks > 0) {
@@ -423,14 +482,18 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
     switch (pass) {
         case CHILL_PASS_FWD:
             if (T != kLongSequence && fwd_takes_small(mask_id, batch_heads, T, D, dtype)) {
-                *out = small_tile_config(fwd_small_lds_bytes(D, dtype), batch_heads * ((T + 31) / 32));
+                const long long tiles = batch_heads * ((T + 31) / 32);
+                *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T), D, fwd_small_lds_bytes(D, dtype))
+                                            : small_tile_config(fwd_small_lds_bytes(D, dtype), tiles);
                 return CHILL_OK;
             }
             *out = fwd_tile_config(mask_id, D, dtype, fwd_takes_short_row(mask_id, band_keys, batch_heads, T) ? 1 : kLongSequence);
             return CHILL_OK;
         case CHILL_PASS_DQ:
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DQ)) {
-                *out = small_tile_config(bwd_small_lds_bytes(D, dtype, 1), batch_heads * ((T + 31) / 32));
+                const long long tiles = batch_heads * ((T + 31) / 32);
+                *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T), D, bwd_small_lds_bytes(D, dtype, 1))
+                                            : small_tile_config(bwd_small_lds_bytes(D, dtype, 1), tiles);
                 return CHILL_OK;
             }
             if (dq_regs2_is_optional(D, dtype) && (T == kLongSequence ? !mask_is_banded(mask_id) : dq_takes_regs2(mask_id, batch_heads, T))) {
