@@ -424,19 +424,25 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     const int n_tiles = cdiv(p.T, 32);
     const long long heads = (long long)p.B * (PASS == 1 ? p.H : p.H_kv);  // (few by bwd_takes_small)
     // (dK/dV keeps one block per workgroup: with K, V and two accumulators a wave needs more than the 256 registers it
-    // would be left with; fp32 of more tiles than CUs: dq_f32_kernel)
-    constexpr bool kTwoFit = PASS == 1 && Elem<E>::k16 && small_fits_two_tiles(kLdsOne);
-    bool two = false;
-    if constexpr (kTwoFit) two = small_takes_two_tiles(heads * n_tiles);
+    // would be left with; fp32 beyond a few blocks per row: dq_f32_kernel, dkdv_f32_kernel)
+    constexpr bool kDouble = Elem<E>::k16 && small_fits_two_tiles(kLdsOne);
+    bool two = false, sets = false;
+    if constexpr (kDouble) {
+        two = PASS == 1 && small_takes_two_tiles(heads * n_tiles);
+        sets = small_takes_two_sets(PASS == 1 ? CHILL_PASS_DQ : CHILL_PASS_DKDV, heads * n_tiles, p.T, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
+    }
     const int total = (int)(heads * (two ? (n_tiles + 1) / 2 : n_tiles));
-    const int lds_bytes = two ? 2 * kLdsOne : PASS == 2 ? bwd_small_lds_bytes(D, Elem<E>::kDType, 2) : kLdsOne;
+    const int lds_bytes = two || sets ? 2 * kLdsOne : PASS == 2 ? bwd_small_lds_bytes(D, Elem<E>::kDType, 2) : kLdsOne;
     void (*kern)(BwdParams, int, int, int);
     if constexpr (PASS == 1)
-        kern = dq_small_kernel<E, D, MASK_ID, 1>;
+        kern = dq_small_kernel<E, D, MASK_ID, 1, 1>;
     else
-        kern = dkdv_small_kernel<E, D, MASK_ID>;
-    if constexpr (kTwoFit) {
-        if (two) kern = dq_small_kernel<E, D, MASK_ID, 2>;
+        kern = dkdv_small_kernel<E, D, MASK_ID, 1>;
+    if constexpr (kDouble && PASS == 1) {
+        if (two) kern = dq_small_kernel<E, D, MASK_ID, 2, 1>;
+        if (sets) kern = dq_small_kernel<E, D, MASK_ID, 1, 2>;
+    } else if constexpr (kDouble) {
+        if (sets) kern = dkdv_small_kernel<E, D, MASK_ID, 2>;
     }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
     if (lds_bytes > 48 * 1024) {
@@ -444,7 +450,7 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
                                 lds_bytes) != hipSuccess)
             return CHILL_ERR_HIP;
     }
-    hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two ? 2 : 1)), lds_bytes, stream, p, n_tiles, total,
+    hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two || sets ? 2 : 1)), lds_bytes, stream, p, n_tiles, total,
                        hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }

@@ -21,12 +21,11 @@ namespace chill {
 // wave: register r of block i of lane l at ((i * 16 + r) * 64 + l) * 4) and stores this wave's share of
 // the finished row blocks: lane (n, h) holds, of row n, the columns 32 * db + 8 * (r / 4) + 4 * h + r % 4.
 // Block i of the accumulators goes to out[i / DB] (dQ: one output; dK/dV: two).
-template <typename E, int D, int NOUT>
+template <typename E, int D, int NOUT, int NW>
 __device__ __forceinline__ void bwd_small_merge(const char* smem, int wave_bytes, int wave, int lane,
                                                 typename Elem<E>::type* const (&row)[NOUT], const float (&mult)[NOUT],
                                                 bool in_tensor, bool valid) {
     using ET = typename Elem<E>::type;
-    constexpr int NW = kFwdSmallWaves;
     constexpr int DB = (D + 31) / 32;
     const int h = lane >> 5;
     if (!in_tensor) return;
@@ -54,12 +53,13 @@ __device__ __forceinline__ void bwd_small_merge(const char* smem, int wave_bytes
 // TILES = 2: a workgroup of eight waves takes two 32-row blocks side by side, block j from the long end and block j
 // from the short end of one head, four waves each with an LDS area of their own, as fwd_small_kernel does; the two
 // halves meet at the one barrier of the kernel and nowhere else.
-template <typename E, int D, int MASK, int TILES>
-__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) void dq_small_kernel(BwdParams p, int n_q_tiles, int total_items,
-                                                                               int has_full_blocks) {
+// SETS = 2 (and TILES = 1): eight waves share the keys of one block.
+template <typename E, int D, int MASK, int TILES, int SETS>
+__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void dq_small_kernel(BwdParams p, int n_q_tiles, int total_items,
+                                                                                      int has_full_blocks) {
     using ET = typename Elem<E>::type;
     typedef LdsTile<E, D> L;
-    constexpr int NW = kFwdSmallWaves;
+    constexpr int NW = kFwdSmallWaves * SETS;
     constexpr int NT = NW * 64;
     constexpr int DB = (D + 31) / 32;
     constexpr int TILE_BYTES = L::bytes(32);
@@ -190,16 +190,16 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) void dq_small_kernel(B
     __syncthreads();
     ET* const rows[1] = {dqbase + (int64_t)q_pos * p.sdq.t};
     const float mult[1] = {p.sm_scale};
-    bwd_small_merge<E, D, 1>(smem, WAVE_BYTES, wave, lane, rows, mult, q_pos < p.T, q_pos < seq_len);
+    bwd_small_merge<E, D, 1, NW>(smem, WAVE_BYTES, wave, lane, rows, mult, q_pos < p.T, q_pos < seq_len);
 }
 
 // ------------------------------------------------------------------------------------------ dK, dV
-template <typename E, int D, int MASK>
-__global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_kernel(BwdParams p, int n_k_tiles, int total_items,
-                                                                         int has_full_blocks) {
+template <typename E, int D, int MASK, int SETS>
+__global__ __launch_bounds__(kFwdSmallWaves * 64 * SETS) void dkdv_small_kernel(BwdParams p, int n_k_tiles, int total_items,
+                                                                                int has_full_blocks) {
     using ET = typename Elem<E>::type;
     typedef LdsTile<E, D> L;
-    constexpr int NW = kFwdSmallWaves;
+    constexpr int NW = kFwdSmallWaves * SETS;
     constexpr int NT = NW * 64;
     constexpr int DB = (D + 31) / 32;
     constexpr int TILE_BYTES = L::bytes(32);
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_kernel(BwdPara
     __syncthreads();
     ET* const rows[2] = {dkbase + (int64_t)k_pos * p.sdk.t, dvbase + (int64_t)k_pos * p.sdv.t};
     const float mult[2] = {p.sm_scale, 1.f};
-    bwd_small_merge<E, D, 2>(smem, WAVE_BYTES, wave, lane, rows, mult, k_pos < p.T, k_pos < seq_len);
+    bwd_small_merge<E, D, 2, NW>(smem, WAVE_BYTES, wave, lane, rows, mult, k_pos < p.T, k_pos < seq_len);
 }
 
 }  // namespace chill

@@ -574,13 +574,20 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     constexpr int kLdsOne = fwd_small_lds_bytes(D, Elem<E>::kDType);
     const int n_q_tiles = cdiv(p.T, 32);
     // (at most kComputeUnits / 4 * 4 * 32 q-tiles by fwd_takes_small)
-    bool two = false;
-    if constexpr (small_fits_two_tiles(kLdsOne) && Elem<E>::k16) two = small_takes_two_tiles((long long)p.B * p.H * n_q_tiles);
+    bool two = false, sets = false;
+    // (fp32 beyond a few blocks per row: fwd_f32_kernel)
+    constexpr bool kDouble = Elem<E>::k16 && small_fits_two_tiles(kLdsOne);
+    if constexpr (kDouble) {
+        const long long tiles = (long long)p.B * p.H * n_q_tiles;
+        two = small_takes_two_tiles(tiles);
+        sets = small_takes_two_sets(CHILL_PASS_FWD, tiles, p.T, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
+    }
     const int total = p.B * p.H * (two ? (n_q_tiles + 1) / 2 : n_q_tiles);
-    const int lds_bytes = two ? 2 * kLdsOne : kLdsOne;
-    void (*kern)(FwdParams, int, int, int) = fwd_small_kernel<E, D, MASK_ID, 1>;
-    if constexpr (small_fits_two_tiles(kLdsOne) && Elem<E>::k16) {  // (fp32 of more tiles than CUs: fwd_f32_kernel)
-        if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2>;
+    const int lds_bytes = two || sets ? 2 * kLdsOne : kLdsOne;
+    void (*kern)(FwdParams, int, int, int) = fwd_small_kernel<E, D, MASK_ID, 1, 1>;
+    if constexpr (kDouble) {
+        if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
+        if (sets) kern = fwd_small_kernel<E, D, MASK_ID, 1, 2>;
     }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
     if (lds_bytes > 48 * 1024) {
@@ -588,7 +595,7 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
                                 lds_bytes) != hipSuccess)
             return CHILL_ERR_HIP;
     }
-    hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two ? 2 : 1)), lds_bytes, stream, p, n_q_tiles, total,
+    hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two || sets ? 2 : 1)), lds_bytes, stream, p, n_q_tiles, total,
                        hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }

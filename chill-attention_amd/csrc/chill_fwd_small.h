@@ -25,13 +25,15 @@ namespace chill {
 // for every workgroup, where workgroups of one q-tile each leave the CUs that drew two long ones to finish alone
 // (taken when the launch has more workgroups than the chip has CUs: fwd_small_tiles).  The two halves meet at the
 // one barrier of the kernel and nowhere else.
-template <typename E, int D, int MASK, int TILES>
-__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) void fwd_small_kernel(FwdParams p, int n_q_tiles, int total_items,
-                                                                                int has_full_blocks) {
+// SETS = 2 (and TILES = 1): eight waves share the keys of one q-tile, where a launch leaves half of the CUs idle.
+template <typename E, int D, int MASK, int TILES, int SETS>
+__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_kernel(FwdParams p, int n_q_tiles, int total_items,
+                                                                                       int has_full_blocks) {
     using ET = typename Elem<E>::type;
     using M = Mask<MASK>;
     typedef LdsTile<E, D> L;
-    constexpr int NW = kFwdSmallWaves;
+    constexpr int NW = kFwdSmallWaves * SETS;
+    static_assert(TILES == 1 || SETS == 1, "two tiles or two sets of waves");
     constexpr int NT = NW * 64;
     constexpr int DB = (D + 31) / 32;
     constexpr int TILE_BYTES = L::bytes(32);

@@ -221,11 +221,23 @@ constexpr F32Shape f32_shape(int mask_id, int pass, int D, long long tiles, int 
     if (tiles <= (grow ? 512 : 256)) return F32Shape{1, 4};
     return tiles <= 512 ? F32Shape{2, 2} : F32Shape{4, 1};
 }
+// With no more tiles than CUs a workgroup has its CU to itself, and two sets of four waves share the streamed blocks of its tile
+// (16-bit inputs; fp32: f32_shape), where a row reaches over enough of them to pay for the longer merge.  us, one set -> two, bf16
+// causal where not named: forward D64 B1 H8 T256 5.7 -> 5.9, T512 7.7 -> 7.0, T1024 11.2 -> 9.1, fp16 H4 T300 7.2 -> 6.3, full mask
+// H2 T2048 17.2 -> 12.7, window 64 H4 T1024 5.4 -> 5.6, D128 H4 T512 9.7 -> 9.2, T2048 24.0 -> 17.2, prefix-LM H1 T8192 86 -> 48;
+// dK/dV D64 H8 T160 7.7 -> 7.4, T512 9.9 -> 8.8, T1024 14.6 -> 11.2, window 64 7.4 -> 7.8, prefix-LM H1 T8192 78 -> 45; dQ D64 H8 T512
+// 8.5 -> 8.8, T1024 11.5 -> 10.5, D128 H4 T512 12.7 -> 13.9, B2 H4 T800 16.2 -> 15.3, T2048 25.8 -> 21.5, prefix-LM H1 T8192 85 -> 54,
+// window 32 of T3000 9.6 -> 11.1.
+constexpr bool small_takes_two_sets(int pass, long long tiles, int T, long long band_keys) {
+    const long long reach = T < band_keys ? T : band_keys;
+    return tiles <= kComputeUnits && reach > (pass == CHILL_PASS_FWD ? 256 : pass == CHILL_PASS_DQ ? 768 : 128);
+}
 // what the report says of a small launch: 32 rows and the 4 waves of a set; the LDS of the workgroup, which takes two tiles or
 // one tile with two sets
-constexpr TileConfig small_tile_config(int lds_bytes_one, long long tiles) {
+constexpr TileConfig small_tile_config(int pass, int lds_bytes_one, long long tiles, int T, long long band_keys) {
     return TileConfig{32, 32, kFwdSmallWaves,
-                      (small_fits_two_tiles(lds_bytes_one) && small_takes_two_tiles(tiles)) ? 2 * lds_bytes_one : lds_bytes_one};
+                      (small_fits_two_tiles(lds_bytes_one) && ((pass != CHILL_PASS_DKDV && small_takes_two_tiles(tiles)) ||
+                                                               small_takes_two_sets(pass, tiles, T, band_keys))) ? 2 * lds_bytes_one : lds_bytes_one};
 }
 // LDS of an fp32 workgroup: per stream two stages (one where a wave has its blocks to itself) of two 32-row tiles, the scales of
 // their slices and, in dK/dV, LSE2 and delta of the block's rows; at the end the streams' partial sums, in the forward with m
@@ -484,7 +496,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
             if (T != kLongSequence && fwd_takes_small(mask_id, batch_heads, T, D, dtype)) {
                 const long long tiles = batch_heads * ((T + 31) / 32);
                 *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T), D, fwd_small_lds_bytes(D, dtype))
-                                            : small_tile_config(fwd_small_lds_bytes(D, dtype), tiles);
+                                            : small_tile_config(pass, fwd_small_lds_bytes(D, dtype), tiles, T, band_keys);
                 return CHILL_OK;
             }
             *out = fwd_tile_config(mask_id, D, dtype, fwd_takes_short_row(mask_id, band_keys, batch_heads, T) ? 1 : kLongSequence);
@@ -493,7 +505,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DQ)) {
                 const long long tiles = batch_heads * ((T + 31) / 32);
                 *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T), D, bwd_small_lds_bytes(D, dtype, 1))
-                                            : small_tile_config(bwd_small_lds_bytes(D, dtype, 1), tiles);
+                                            : small_tile_config(pass, bwd_small_lds_bytes(D, dtype, 1), tiles, T, band_keys);
                 return CHILL_OK;
             }
             if (dq_regs2_is_optional(D, dtype) && (T == kLongSequence ? !mask_is_banded(mask_id) : dq_takes_regs2(mask_id, batch_heads, T))) {
@@ -505,7 +517,8 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
         case CHILL_PASS_DKDV:
             // (for this pass batch_heads counts the key / value heads)
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DKDV)) {
-                *out = TileConfig{32, 32, kFwdSmallWaves, bwd_small_lds_bytes(D, dtype, 2)};
+                *out = f32_serves(D, dtype) ? TileConfig{32, 32, kFwdSmallWaves, bwd_small_lds_bytes(D, dtype, 2)}
+                                            : small_tile_config(pass, bwd_small_lds_bytes(D, dtype, 2), batch_heads * ((T + 31) / 32), T, band_keys);
                 return CHILL_OK;
             }
             // (the row of long sequences on a full chip: the generated loop where there is one)
