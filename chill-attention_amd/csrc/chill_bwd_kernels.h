@@ -1484,7 +1484,7 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         } else if (regs) {
             if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType)) status = launch_dkdv_shape<E, D, MASK_ID, false, true>(p, stream);
         } else if constexpr (has_small_row) {
-            status = dkdv_takes_small_row((long long)p.B * p.H_kv, p.T) ? launch_dkdv_shape<E, D, MASK_ID, true>(p, stream)
+            status = dkdv_takes_small_row(MASK_ID, (long long)p.B * p.H_kv, p.T) ? launch_dkdv_shape<E, D, MASK_ID, true>(p, stream)
                                                                         : launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);
         } else {
             status = launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);

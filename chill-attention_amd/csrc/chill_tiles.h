@@ -377,15 +377,19 @@ constexpr bool dkdv_is_paired(int D, int dtype) { return D * elem_bytes(dtype) <
 // (measured: sliding window dK/dV -32 %, prefix-LM at D = 64 -17 %).  At D = 128 the two-stage ring of
 // such a workgroup takes 99 KiB; with a one-stage ring it fits twice but runs 8 % slower than the
 // 8-wave workgroup.
-// `small_grid`: the 8-wave grid would cover at most half of the CUs (dkdv_takes_small_row); then the
-// 64-row workgroup is taken at every 16-bit head dim (B1 H8 T2048 D128: -17 %).
+// `small_grid`: the 8-wave grid would cover at most half of the CUs, or not all of them under a mask whose rows grow with their
+// index, where one round of 8-wave workgroups lasts as long as the longest of them (dkdv_takes_small_row); then the
+// 64-row workgroup is taken at every 16-bit head dim.  D128 bf16, 8-wave workgroups, us, 8 waves -> 4: 128 causal B1 H8 T2048 -17 %; 160
+// 61 -> 49; 192 B2 H32/4 T3000 510 -> 406; 224 B1 H8 T3500 83 -> 66, prefix-LM 88 -> 75, full mask 20 workgroups a head, 160, 62 -> 91,
+// window 512 24 -> 32; 288 B1 H9 T4000 99 -> 100; 320 B2 H32/8 T2500 249 -> 269.  (A grid of exactly 256, B1 H8 T4096 98 -> 83, keeps
+// the 8-wave entry that the tile table has always given for it.)
 constexpr int dkdv_paired_waves(int mask_id, int D, int dtype, bool small_grid = false) {
     (void)mask_id;
     if (CHILL_TUNE_DKDV_WAVES) return CHILL_TUNE_DKDV_WAVES;
     return (dtype != CHILL_F32 && (D <= 64 || small_grid)) ? 4 : 8;
 }
-constexpr bool dkdv_takes_small_row(long long batch_kv_heads, int T) {
-    return batch_kv_heads * ((T + 127) / 128) <= kComputeUnits / 2;
+constexpr bool dkdv_takes_small_row(int mask_id, long long batch_kv_heads, int T) {
+    return batch_kv_heads * ((T + 127) / 128) <= (mask_rows_grow(mask_id) ? kComputeUnits - 1 : kComputeUnits / 2);
 }
 // at the end the waves of a pair exchange one fp32 accumulator each through LDS: 8 waves x (D rounded
 // up to 32) x 32 floats
@@ -522,7 +526,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 return CHILL_OK;
             }
             // (the row of long sequences on a full chip: the generated loop where there is one)
-            *out = dkdv_tile_config(mask_id, D, dtype, T != kLongSequence && dkdv_takes_small_row(batch_heads, T),
+            *out = dkdv_tile_config(mask_id, D, dtype, T != kLongSequence && dkdv_takes_small_row(mask_id, batch_heads, T),
                                     T == kLongSequence ? (!mask_is_banded(mask_id) || dkdv_regs_serves_band(mask_id, mask_arg0, band_keys, D))
                                                        : dkdv_takes_regs(mask_id, mask_arg0, band_keys, D, batch_heads, T));
             return CHILL_OK;
