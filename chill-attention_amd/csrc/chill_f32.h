@@ -193,7 +193,7 @@ void fwd_f32_kernel(FwdParams p, int n_tiles, int n_groups, int has_full_blocks)
 #pragma unroll
         for (int i = 0; i < Lds::TENSORS; i++) {
             const bool is_v = my_tensor + i == 1;
-            rows[i].fetch(is_v ? vptr : kptr, is_v ? p.sv.t : p.sk.t, row0, p.T, lane);
+            rows[i].fetch(is_v ? vptr : kptr, is_v ? p.sv.t : p.sk.t, row0, seq_len, lane);
         }
     };
     // what was fetched to LDS, as block `it`: first its scale, then the parts, in STEPS shares
@@ -219,7 +219,7 @@ void fwd_f32_kernel(FwdParams p, int n_tiles, int n_groups, int has_full_blocks)
     fetch(0);
     ResidentParts<D> qf;
     // a negative scale reverses the order of the scores: its sign goes into Q
-    qf.load(qptr, p.sq.t, tile >= 0 ? p.T - qb : 0, lane, p.scale_log2 < 0.f ? -1.f : 1.f);
+    qf.load(qptr, p.sq.t, tile >= 0 ? seq_len - qb : 0, lane, p.scale_log2 < 0.f ? -1.f : 1.f);
     OperandOffsets<f16_t, D> ofs;
     ofs.init(lane);
     commit_all(0);
@@ -316,14 +316,14 @@ void fwd_f32_kernel(FwdParams p, int n_tiles, int n_groups, int has_full_blocks)
         for (int blk = hull.lo + stream; blk < wr.end; blk += S) {
             if (blk < wr.start) continue;
             const int k0 = blk * 32;
-            f32x16 s = native_rowwise<D>(kptr + k0 * p.sk.t, p.sk.t, p.T - k0, qptr, p.sq.t, p.T - qb, lane);
+            f32x16 s = native_rowwise<D>(kptr + k0 * p.sk.t, p.sk.t, seq_len - k0, qptr, p.sq.t, seq_len - qb, lane);
             float f[1] = {scale};
             if (p.scale_log2 < 0.f) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) s[r] = -s[r];
             }
             softmax(s, f, blk);
-            native_transposed<D>(vptr + k0 * p.sv.t, p.sv.t, p.T - k0, s, o, lane);
+            native_transposed<D>(vptr + k0 * p.sv.t, p.sv.t, seq_len - k0, s, o, lane);
         }
     }
 
@@ -456,7 +456,7 @@ void dq_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks) 
     const int tile = group.tile(member);
     const int qb = 32 * (tile < 0 ? 0 : tile);
     const int q_pos = qb + n;
-    const int q_rows = tile >= 0 ? p.T - qb : 0;
+    const int q_rows = tile >= 0 ? p.T - qb : 0, q_seen = tile >= 0 ? seq_len - qb : 0;  // (of the tensor, of the sequence)
     TileRange wr = {0, 0, 0, 0};
     if (tile >= 0 && qb < seq_len) wr = tile_range_rows_discarded<MASK, true>(qb, 32, 32, seq_len, has_full_blocks != 0, p.margs);
 
@@ -476,7 +476,7 @@ void dq_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks) 
 #pragma unroll
         for (int i = 0; i < Lds::TENSORS; i++) {
             const bool is_v = my_tensor + i == 1;
-            rows[i].fetch(is_v ? vptr : kptr, is_v ? p.sv.t : p.sk.t, row0, p.T, lane);
+            rows[i].fetch(is_v ? vptr : kptr, is_v ? p.sv.t : p.sk.t, row0, seq_len, lane);
         }
     };
     // what was fetched to LDS, as block `it`: first its scale, then the parts, in STEPS shares
@@ -515,8 +515,8 @@ void dq_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks) 
         delta_q = p.delta[b * p.delta_b + hd * p.delta_h + q_pos];
     }
     ResidentParts<D> qf, dof;
-    qf.load(qptr, p.sq.t, q_rows, lane);
-    dof.load(doptr, p.sdo.t, q_rows, lane);
+    qf.load(qptr, p.sq.t, q_seen, lane);
+    dof.load(doptr, p.sdo.t, q_seen, lane);
     OperandOffsets<f16_t, D> ofs;
     ofs.init(lane);
     commit_all(0);
@@ -588,14 +588,14 @@ void dq_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks) 
         for (int blk = hull.lo + stream; blk < wr.end; blk += S) {
             if (blk < wr.start) continue;
             const int k0 = blk * 32;
-            f32x16 s = native_rowwise<D>(kptr + k0 * p.sk.t, p.sk.t, p.T - k0, qptr, p.sq.t, q_rows, lane);
-            f32x16 dp = native_rowwise<D>(vptr + k0 * p.sv.t, p.sv.t, p.T - k0, doptr, p.sdo.t, q_rows, lane);
+            f32x16 s = native_rowwise<D>(kptr + k0 * p.sk.t, p.sk.t, seq_len - k0, qptr, p.sq.t, q_seen, lane);
+            f32x16 dp = native_rowwise<D>(vptr + k0 * p.sv.t, p.sv.t, seq_len - k0, doptr, p.sdo.t, q_seen, lane);
 #pragma unroll
             for (int r = 0; r < 16; r++) s[r] = fast_exp2(s[r] * p.scale_log2 - lse_q);
             mask(s, blk);
 #pragma unroll
             for (int r = 0; r < 16; r++) dp[r] = s[r] * (dp[r] - delta_q);
-            native_transposed<D>(kptr + k0 * p.sk.t, p.sk.t, p.T - k0, dp, dq, lane);
+            native_transposed<D>(kptr + k0 * p.sk.t, p.sk.t, seq_len - k0, dp, dq, lane);
         }
     }
     const f32x16* const acc[1] = {dq};
@@ -632,7 +632,7 @@ void dkdv_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks
     const int tile = group.tile(member);
     const int kb0 = 32 * (tile < 0 ? 0 : tile);
     const int k_pos = kb0 + n;
-    const int k_rows = tile >= 0 ? p.T - kb0 : 0;
+    const int k_rows = tile >= 0 ? p.T - kb0 : 0, k_seen = tile >= 0 ? seq_len - kb0 : 0;  // (of the tensor, of the sequence)
     TileRange wr = {0, 0, 0, 0};
     if (tile >= 0 && kb0 < seq_len) wr = tile_range_rows_discarded<MASK, false>(kb0, 32, 32, seq_len, has_full_blocks != 0, p.margs);
 
@@ -655,13 +655,13 @@ void dkdv_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks
 #pragma unroll
             for (int i = 0; i < Lds::TENSORS; i++) {
                 const bool is_do = my_tensor + i == 1;
-                rows[i].fetch(is_do ? do_of(next_head) : q_of(next_head), is_do ? p.sdo.t : p.sq.t, row0, p.T, lane);
+                rows[i].fetch(is_do ? do_of(next_head) : q_of(next_head), is_do ? p.sdo.t : p.sq.t, row0, seq_len, lane);
             }
             if (member == 0) {
-                // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the end read as zero
+                // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the sequence read as zero
                 const int hq = hkv * p.group + next_head;
                 const float* src = h == 0 ? p.lse + b * p.lse_b + hq * p.lse_h : p.delta + b * p.delta_b + hq * p.delta_h;
-                vec_next = q0 + n < p.T ? src[q0 + n] : 0.f;
+                vec_next = q0 + n < seq_len ? src[q0 + n] : 0.f;
             }
         }
         next_it++;
@@ -693,8 +693,8 @@ void dkdv_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks
     };
     fetch();
     ResidentParts<D> kf, vf;
-    kf.load(kptr, p.sk.t, k_rows, lane);
-    vf.load(vptr, p.sv.t, k_rows, lane);
+    kf.load(kptr, p.sk.t, k_seen, lane);
+    vf.load(vptr, p.sv.t, k_seen, lane);
     OperandOffsets<f16_t, D> ofs;
     ofs.init(lane);
     commit_all(0);
@@ -792,19 +792,19 @@ void dkdv_f32_kernel(BwdParams p, int n_tiles, int n_groups, int has_full_blocks
                 if (blk < wr.start) continue;
                 const int q0 = blk * 32;
                 const float *qp = q_of(gh) + q0 * p.sq.t, *dop = do_of(gh) + q0 * p.sdo.t;
-                f32x16 s = native_rowwise<D>(qp, p.sq.t, p.T - q0, kptr, p.sk.t, k_rows, lane);
-                f32x16 dp = native_rowwise<D>(dop, p.sdo.t, p.T - q0, vptr, p.sv.t, k_rows, lane);
+                f32x16 s = native_rowwise<D>(qp, p.sq.t, seq_len - q0, kptr, p.sk.t, k_seen, lane);
+                f32x16 dp = native_rowwise<D>(dop, p.sdo.t, seq_len - q0, vptr, p.sv.t, k_seen, lane);
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int q = q0 + 8 * (r / 4) + 4 * h + (r % 4);
-                    s[r] = fast_exp2(s[r] * p.scale_log2 - (q < p.T ? lse[q] : 0.f));
-                    dp[r] -= q < p.T ? delta[q] : 0.f;
+                    s[r] = fast_exp2(s[r] * p.scale_log2 - (q < seq_len ? lse[q] : 0.f));
+                    dp[r] -= q < seq_len ? delta[q] : 0.f;
                 }
                 mask(s, blk);
 #pragma unroll
                 for (int r = 0; r < 16; r++) dp[r] *= s[r];
-                native_transposed<D>(dop, p.sdo.t, p.T - q0, s, dv, lane);
-                native_transposed<D>(qp, p.sq.t, p.T - q0, dp, dk, lane);
+                native_transposed<D>(dop, p.sdo.t, seq_len - q0, s, dv, lane);
+                native_transposed<D>(qp, p.sq.t, seq_len - q0, dp, dk, lane);
             }
         }
     }
@@ -845,7 +845,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void d
     const int tile = group.tile(member);
     const int kb0 = 32 * (tile < 0 ? 0 : tile);
     const int k_pos = kb0 + n;
-    const int k_rows = tile >= 0 ? p.T - kb0 : 0;
+    const int k_rows = tile >= 0 ? p.T - kb0 : 0, k_seen = tile >= 0 ? seq_len - kb0 : 0;  // (of the tensor, of the sequence)
     TileRange wr = {0, 0, 0, 0};
     if (tile >= 0 && kb0 < seq_len) wr = tile_range_rows_discarded<MASK, false>(kb0, 32, 32, seq_len, has_full_blocks != 0, p.margs);
 
@@ -865,12 +865,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void d
         fetched = next_head < p.group && per_head > 0;
         if (!fetched) return;
         const int q0 = 32 * (hull.lo + next_it), row0 = q0 + member * (32 / NSL);
-        rows.fetch(role == 1 ? do_of(next_head) : q_of(next_head), role == 1 ? p.sdo.t : p.sq.t, row0, p.T, lane);
+        rows.fetch(role == 1 ? do_of(next_head) : q_of(next_head), role == 1 ? p.sdo.t : p.sq.t, row0, seq_len, lane);
         if (wave == 0) {
-            // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the end read as zero
+            // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the sequence read as zero
             const int hq = hkv * p.group + next_head;
             const float* src = h == 0 ? p.lse + b * p.lse_b + hq * p.lse_h : p.delta + b * p.delta_b + hq * p.delta_h;
-            vec_next = q0 + n < p.T ? src[q0 + n] : 0.f;
+            vec_next = q0 + n < seq_len ? src[q0 + n] : 0.f;
         }
         next_it++;
         if (next_it == per_head) {
@@ -889,7 +889,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void d
     };
     fetch();
     ResidentParts<D> own;
-    own.load(role == 1 ? vptr : kptr, role == 1 ? p.sv.t : p.sk.t, k_rows, lane);
+    own.load(role == 1 ? vptr : kptr, role == 1 ? p.sv.t : p.sk.t, k_seen, lane);
     OperandOffsets<f16_t, D> ofs, ofs_tr;  // of all blocks row-wise; of this wave's head-dim blocks transposed
     ofs.init(lane);
 #pragma unroll
@@ -998,19 +998,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void d
             for (int blk = wr.start; blk < wr.end; blk++) {
                 const int q0 = blk * 32;
                 const float *qp = q_of(gh) + q0 * p.sq.t, *dop = do_of(gh) + q0 * p.sdo.t;
-                f32x16 s = native_rowwise<D>(qp, p.sq.t, p.T - q0, kptr, p.sk.t, k_rows, lane);
-                f32x16 dp = native_rowwise<D>(dop, p.sdo.t, p.T - q0, vptr, p.sv.t, k_rows, lane);
+                f32x16 s = native_rowwise<D>(qp, p.sq.t, seq_len - q0, kptr, p.sk.t, k_seen, lane);
+                f32x16 dp = native_rowwise<D>(dop, p.sdo.t, seq_len - q0, vptr, p.sv.t, k_seen, lane);
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int q = q0 + 8 * (r / 4) + 4 * h + (r % 4);
-                    s[r] = fast_exp2(s[r] * p.scale_log2 - (q < p.T ? lse[q] : 0.f));
-                    dp[r] -= q < p.T ? delta[q] : 0.f;
+                    s[r] = fast_exp2(s[r] * p.scale_log2 - (q < seq_len ? lse[q] : 0.f));
+                    dp[r] -= q < seq_len ? delta[q] : 0.f;
                 }
                 mask(s, blk);
 #pragma unroll
                 for (int r = 0; r < 16; r++) dp[r] *= s[r];
-                native_transposed<D>(dop, p.sdo.t, p.T - q0, s, dv, lane, DBW * role);
-                native_transposed<D>(qp, p.sq.t, p.T - q0, dp, dk, lane, DBW * role);
+                native_transposed<D>(dop, p.sdo.t, seq_len - q0, s, dv, lane, DBW * role);
+                native_transposed<D>(qp, p.sq.t, seq_len - q0, dp, dk, lane, DBW * role);
             }
         }
     }

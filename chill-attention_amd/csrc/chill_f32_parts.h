@@ -120,8 +120,9 @@ struct PartTile {
 };
 
 // ROWS rows of a 32-row block on their way from global memory through a wave's registers to a PartTile.  `fetch` requests rows
-// row0 .. of a tensor of T rows (rows past its end repeat the last one: the caller masks what it computes from them), `measure`
-// finds their scale, `commit<I>` writes the parts of the I-th of STEPS shares to the tile.
+// row0 .. of a sequence of T rows (rows past its end repeat the last one: the caller masks what it computes from them, and what
+// a tensor holds behind a shorter sequence must not set the scale), `measure` finds their scale, `commit<I>` writes the parts of
+// the I-th of STEPS shares to the tile.
 template <int D, int ROWS>
 struct PartStager {
     static constexpr int CH = D / 4;             // 16-byte chunks of an fp32 row

@@ -87,6 +87,24 @@ def test_any_magnitude(case):
             assert torch.equal(x, y * 2.0**e), e
 
 
+@pytest.mark.parametrize("case", [c for c in CASES if c[-1] is not None], ids=lambda c: c[0])
+def test_rows_past_the_lengths(case):
+    """What the tensors hold behind a sequence, however large, does not reach the scales of the rows before it."""
+    _, m, B, H, H_kv, T, D, lens = case
+    mask = make_mask(m)
+    x = inputs(B, H, H_kv, T, D, seed=4)
+    want, lse = run(mask, *x, lens)
+    for garbage in (1e30, math.nan):
+        y = [t.clone() for t in x]
+        for t in y[:3]:
+            for i, n in enumerate(lens):
+                t[i, :, n:] = garbage
+        got, lse2 = run(mask, *y, lens)
+        assert torch.equal(lse, lse2)
+        for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+            assert torch.equal(a, b), (name, garbage)
+
+
 @pytest.mark.parametrize("case", CASES[::3] + CASES[-1:], ids=lambda c: c[0])
 def test_infinities(case):
     """Infinities have no parts: the waves that meet one compute their blocks with the fp32 instruction."""
