@@ -736,6 +736,8 @@ __global__ __launch_bounds__(NW * 64) void dq_split_kernel(BwdParams p, int n_q_
 // 32 x D accumulators, no resident MFMA operands) within 256 registers, so two waves share a SIMD
 // and one wave's vector work hides behind the other's MFMAs, with no redundant MFMA work.
 // Four-wave workgroups are compiled for two per CU, those of head dims <= 64 (50 KiB of LDS) for three: 168 registers.
+// NS = 1: the next tile is requested when every wave is done with the present one; the workgroup that shares the CU covers the
+// wait (narrow bands at head dim 128, dkdv_takes_one_stage: window 16 + 16 fp16 B8 H4 T6000 101 -> 79 us, 295 MB).
 template <typename E, int D, int MASK, int NW, int NS>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4 ? (D <= 64 ? 3 : 2) : 1))) void dkdv_kernel(BwdParams p, int n_k_tiles,
                                                        int wave_has_full_blocks) {
@@ -752,7 +754,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
     constexpr int VEC_BYTES = TQS * 4;
     constexpr int STAGE_BYTES = 2 * TILE_BYTES + 2 * VEC_BYTES;  // Q, dO, LSE2, delta
     constexpr int RING_OFF = 2 * KV_BYTES;                        // K, V tiles first
-    static_assert(NS == 2, "two ring stages");
+    static_assert(NS == 1 || NS == 2, "one or two ring stages");
     // the pair exchange at the end reuses the LDS: 2 * NKB accumulators of DB * 16 * 64 floats (the tile
     // table allocates the larger of the two needs)
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -760,7 +762,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
     // (the 64-row workgroups of head dims up to 64 run three to a CU)
     // key tiles first-to-last: for causal-like masks the longest run first
     int bh, ktile;
-    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, (NW == 4 && D <= 64) ? 3 : 1, &bh, &ktile)) return;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, (NW == 4 && D <= 64) ? 3 : NS == 1 ? 2 : 1, &bh, &ktile)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
 
@@ -919,8 +921,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
         const bool in_block = !(tile < ta || tile >= tb);
         // the two waves that share a SIMD issue their loads at different points of the iteration, so
         // that one of them keeps the matrix pipe busy while the other sits in the memory pipeline
-        const bool issue_late = in_block && half == 1;
-        if (!issue_late) {
+        const bool issue_late = NS == 2 && in_block && half == 1;
+        if (NS == 2 && !issue_late) {
             if (it + 1 < n_iters) issue_next(1 - ST);
         }
         if (!in_block) return;
@@ -1066,9 +1068,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4
             mma_transposed<E, D>(q_tile, half, ofs, dp, dk, lane);  // dK^T += Q^T dS
         }
     };
-    for (int it = 0; it < n_iters; it += 2) {
-        iteration(std::integral_constant<int, 0>{}, it);
-        if (it + 1 < n_iters) iteration(std::integral_constant<int, 1>{}, it + 1);
+    if constexpr (NS == 2) {
+        for (int it = 0; it < n_iters; it += 2) {
+            iteration(std::integral_constant<int, 0>{}, it);
+            if (it + 1 < n_iters) iteration(std::integral_constant<int, 1>{}, it + 1);
+        }
+    } else {
+        for (int it = 0; it < n_iters; it++) {
+            iteration(std::integral_constant<int, 0>{}, it);
+            if (it + 1 < n_iters) {
+                __syncthreads();  // everyone is done with the tile
+                issue_next(0);
+            }
+        }
     }
 
     // Sum the two waves of a pair through LDS and store: the waves of the second half hand their dK^T
@@ -1404,10 +1416,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D >= 25
 }
 
 // One (mask, tile shape): SMALL selects the table row for grids that would not fill the chip, REGS the one of
-// dkdv_regs_kernel where the shape has both kernels.
-template <typename E, int D, int MASK_ID, bool SMALL, bool REGS = false>
+// dkdv_regs_kernel where the shape has both kernels, ONE_STAGE that of a ring of one stage.
+template <typename E, int D, int MASK_ID, bool SMALL, bool REGS = false, bool ONE_STAGE = false>
 int launch_dkdv_shape(const BwdParams& p, hipStream_t stream) {
-    constexpr TileConfig cfg = dkdv_tile_config(MASK_ID, D, Elem<E>::kDType, SMALL, REGS);
+    constexpr TileConfig cfg = dkdv_tile_config(MASK_ID, D, Elem<E>::kDType, SMALL, REGS, ONE_STAGE);
     constexpr int CB = (REGS && dkdv_regs_is_optional(D, Elem<E>::kDType)) ? kDkdvRegsBlocks128 : dkdv_regs_blocks(D, Elem<E>::kDType);
     constexpr bool paired = dkdv_is_paired(D, Elem<E>::kDType) && CB == 0;
     static_assert(CB > 0 ? (cfg.rows == 128 * CB && cfg.streamed == 32 && cfg.waves == 4)
@@ -1424,7 +1436,7 @@ int launch_dkdv_shape(const BwdParams& p, hipStream_t stream) {
     if constexpr (CB > 0)
         kern = dkdv_regs_kernel<E, D, MASK_ID, CB, dkdv_regs_stages(D)>;
     else if constexpr (paired)
-        kern = dkdv_kernel<E, D, MASK_ID, cfg.waves, 2>;
+        kern = dkdv_kernel<E, D, MASK_ID, cfg.waves, ONE_STAGE ? 1 : 2>;
     else
         kern = dkdv_split_kernel<E, D, MASK_ID, cfg.waves, dkdv_split(D), 2>;
     // mask rule order is (q tile, k tile): the streamed tile is the q tile here
@@ -1484,8 +1496,12 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         } else if (regs) {
             if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType)) status = launch_dkdv_shape<E, D, MASK_ID, false, true>(p, stream);
         } else if constexpr (has_small_row) {
-            status = dkdv_takes_small_row(MASK_ID, (long long)p.B * p.H_kv, p.T) ? launch_dkdv_shape<E, D, MASK_ID, true>(p, stream)
-                                                                        : launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);
+            if (dkdv_takes_small_row(MASK_ID, (long long)p.B * p.H_kv, p.T)) return launch_dkdv_shape<E, D, MASK_ID, true>(p, stream);
+            if constexpr (dkdv_one_stage_serves(MASK_ID, D, Elem<E>::kDType)) {
+                if (dkdv_takes_one_stage(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1)))
+                    return launch_dkdv_shape<E, D, MASK_ID, false, false, true>(p, stream);
+            }
+            status = launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);
         } else {
             status = launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);
         }

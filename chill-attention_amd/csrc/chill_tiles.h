@@ -375,8 +375,7 @@ constexpr bool dkdv_is_paired(int D, int dtype) { return D * elem_bytes(dtype) <
 // 16-bit head dims <= 64: workgroups of 4 waves (64 key rows), small enough in LDS (50 KiB at D = 64)
 // and registers (167) for two or three of them per CU, which hide each other's start and end
 // (measured: sliding window dK/dV -32 %, prefix-LM at D = 64 -17 %).  At D = 128 the two-stage ring of
-// such a workgroup takes 99 KiB; with a one-stage ring it fits twice but runs 8 % slower than the
-// 8-wave workgroup.
+// such a workgroup takes 99 KiB; with a one-stage ring it fits twice, which pays under narrow bands (dkdv_takes_one_stage).
 // `small_grid`: the 8-wave grid would cover at most half of the CUs, or not all of them under a mask whose rows grow with their
 // index, where one round of 8-wave workgroups lasts as long as the longest of them (dkdv_takes_small_row); then the
 // 64-row workgroup is taken at every 16-bit head dim.  D128 bf16, 8-wave workgroups, us, 8 waves -> 4: 128 causal B1 H8 T2048 -17 %; 160
@@ -391,6 +390,19 @@ constexpr int dkdv_paired_waves(int mask_id, int D, int dtype, bool small_grid =
 constexpr bool dkdv_takes_small_row(int mask_id, long long batch_kv_heads, int T) {
     return batch_kv_heads * ((T + 127) / 128) <= (mask_rows_grow(mask_id) ? kComputeUnits - 1 : kComputeUnits / 2);
 }
+// Narrow bands at head dim 128, 16-bit: the 64-row workgroup with a ring of ONE stage (64.5 KiB), two of which share a CU.  Its
+// loads are exposed, but a key block of a band has a handful of query tiles, and what the 8-wave workgroup, alone on its CU, spends
+// before and after them (K and V to LDS, the exchange of the pairs, the stores) hides behind the other workgroup.  us, 8 waves ->
+// one stage: window 16 + 16 fp16 B8 H4 T6000 101 -> 79, bf16 B2 H16/4 T2085 36 -> 27; 128 + 128 115 -> 95, 44 -> 33, bf16 B2 H32
+// T4096 153 -> 128; 512 + 128 172 -> 160, 75 -> 57; 1024 + 0 231 -> 219; 2047 + 0 352 -> 346, B2 H16/4 T16000 917 -> 905; 3000 + 500
+// 523 -> 529; chunkwise 100 x 3 129 -> 113, 128 x 3 114 -> 105, B2 H16 T3000 55 -> 49, 1000 x 2 392 -> 385 (T3000 180 -> 183),
+// 1000 x 5 640 -> 642 (T3000 192 -> 200).  Masks that are not banded are within 4 % either way.  Letting dO's half of the next tile go
+// out behind the dV^T MFMAs, with a barrier of its own, costs 2-10 %.  Grids that leave CUs idle keep the two-stage 64-row
+// workgroups (dkdv_takes_small_row).
+// The report gives the two workgroups of a CU as one, 128 rows and 8 waves, which is also what they take of its LDS.
+constexpr int kDkdvOneStageBand = 2048;
+constexpr bool dkdv_one_stage_serves(int mask_id, int D, int dtype) { return dtype != CHILL_F32 && D == 128 && mask_is_banded(mask_id); }
+constexpr bool dkdv_takes_one_stage(long long band_keys) { return band_keys <= kDkdvOneStageBand; }
 // at the end the waves of a pair exchange one fp32 accumulator each through LDS: 8 waves x (D rounded
 // up to 32) x 32 floats
 constexpr int dkdv_paired_exchange_bytes(int D) { return 8 * ((D + 31) / 32) * 16 * 64 * 4; }
@@ -463,13 +475,23 @@ constexpr bool dkdv_regs_serves_band(int mask_id, long long mask_arg0, long long
     return (mask_id == CHILL_MASK_CHUNKWISE && mask_arg0 % (32 * kDkdvRegsBlocks128) == 0 && (D >= 128 || mask_arg0 >= 320)) ||
            (mask_id == CHILL_MASK_SLIDING_WINDOW && band_keys >= kDkdvRegsWideBand);
 }
+// (at head dim 128 chunks of fewer than 256 rows whose band has at most 256 keys go through the workgroups that share a CU,
+// dkdv_takes_one_stage, instead: bf16 B2 H16 T8192, this kernel -> that, us, 64 x 1 112 -> 84, 64 x 3 126 -> 100, 128 x 1 113 -> 92,
+// 128 x 2 129 -> 118, 192 x 1 128 -> 106; B2 H32 T16384 398 -> 289, 471 -> 382, 396 -> 333, 466 -> 462, 457 -> 407.  Wider: 128 x 3
+// 151 -> 140, 549 -> 575, 64 x 9 190 -> 175, 704 -> 737, 192 x 3 189 -> 177, 694 -> 752, 256 x 1 122 -> 123, 420 -> 473.  The smallest
+// grid this kernel takes keeps it, as the report has always said.)
+constexpr bool dkdv_regs_leaves_band(int mask_id, long long mask_arg0, long long band_keys, int D, long long workgroups) {
+    return mask_id == CHILL_MASK_CHUNKWISE && D == 128 && mask_arg0 < 256 && band_keys <= 256 && workgroups > kDkdvRegsMinWorkgroups;
+}
 constexpr bool dkdv_takes_regs(int mask_id, long long mask_arg0, long long band_keys, int D, long long batch_kv_heads, int T) {
+    const long long workgroups = batch_kv_heads * ((T + 128 * kDkdvRegsBlocks128 - 1) / (128 * kDkdvRegsBlocks128));
     return (!mask_is_banded(mask_id) || dkdv_regs_serves_band(mask_id, mask_arg0, band_keys, D)) && T >= dkdv_regs_min_sequence(mask_id, D) &&
-           batch_kv_heads * ((T + 128 * kDkdvRegsBlocks128 - 1) / (128 * kDkdvRegsBlocks128)) >= dkdv_regs_min_workgroups(mask_id, D, T);
+           workgroups >= dkdv_regs_min_workgroups(mask_id, D, T) && !dkdv_regs_leaves_band(mask_id, mask_arg0, band_keys, D, workgroups);
 }
 
-// `regs`: the row of dkdv_regs_kernel where that kernel is an option (dkdv_regs_is_optional)
-constexpr TileConfig dkdv_tile_config(int mask_id, int D, int dtype, bool small_grid = false, bool regs = false) {
+// `regs`: the row of dkdv_regs_kernel where that kernel is an option (dkdv_regs_is_optional); `one_stage`: that of the paired
+// kernel with a ring of one stage (dkdv_takes_one_stage)
+constexpr TileConfig dkdv_tile_config(int mask_id, int D, int dtype, bool small_grid = false, bool regs = false, bool one_stage = false) {
     if (f32_serves(D, dtype)) return D <= 64 ? TileConfig{128, 64, 8, f32_lds_bytes(D, 4, 2, CHILL_PASS_DKDV)} : TileConfig{128, 32, 8, f32_wide_lds_bytes(D)};
     const int row_bytes = D * elem_bytes(dtype);
     const int blocks = (regs && dkdv_regs_is_optional(D, dtype)) ? kDkdvRegsBlocks128 : dkdv_regs_blocks(D, dtype);
@@ -478,9 +500,9 @@ constexpr TileConfig dkdv_tile_config(int mask_id, int D, int dtype, bool small_
         return TileConfig{rows, 32, 4, rows * row_bytes + dkdv_regs_stages(D) * (2 * 32 * row_bytes + 2 * 32 * 4)};
     }
     if (dkdv_is_paired(D, dtype)) {
-        const int waves = dkdv_paired_waves(mask_id, D, dtype, small_grid);
+        const int waves = dkdv_paired_waves(mask_id, D, dtype, small_grid || one_stage);
         const int rows = 16 * waves;
-        const int ring = 2 * rows * row_bytes + 2 * (2 * 64 * row_bytes + 2 * 64 * 4);
+        const int ring = 2 * rows * row_bytes + (one_stage ? 1 : 2) * (2 * 64 * row_bytes + 2 * 64 * 4);
         const int exchange = dkdv_paired_exchange_bytes(D) * waves / 8;
         return TileConfig{rows, 64, waves, ring > exchange ? ring : exchange};
     }
