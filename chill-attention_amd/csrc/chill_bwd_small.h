@@ -17,10 +17,19 @@
 
 namespace chill {
 
-// Adds up the waves' partial accumulators (NB blocks of 16 registers per lane, staged at `area` of every
-// wave: register r of block i of lane l at ((i * 16 + r) * 64 + l) * 4) and stores this wave's share of
-// the finished row blocks: lane (n, h) holds, of row n, the columns 32 * db + 8 * (r / 4) + 4 * h + r % 4.
-// Block i of the accumulators goes to out[i / DB] (dQ: one output; dK/dV: two).
+// A wave's partial accumulators (NB blocks of 16 registers per lane) over its staging area, four registers at a time: registers
+// 4 * (u % 4) .. + 3 of block u / 4 of lane l at (u * 64 + l) * 16.
+template <int NB>
+__device__ __forceinline__ void bwd_small_leave(char* area, int first, const f32x16 (&acc)[NB], int lane) {
+    f32x4* my = reinterpret_cast<f32x4*>(area);
+#pragma unroll
+    for (int u = 0; u < 4 * NB; u++)
+        my[(4 * first + u) * 64 + lane] =
+            f32x4{acc[u / 4][4 * (u % 4)], acc[u / 4][4 * (u % 4) + 1], acc[u / 4][4 * (u % 4) + 2], acc[u / 4][4 * (u % 4) + 3]};
+}
+
+// Adds them up and stores this wave's share of the finished rows: lane (n, h) holds, of row n, the columns 8 * u + 4 * h .. + 3 of
+// an output, and the groups of four columns go round the waves.  (dQ has one output, dK/dV two, one after the other.)
 template <typename E, int D, int NOUT, int NW>
 __device__ __forceinline__ void bwd_small_merge(const char* smem, int wave_bytes, int wave, int lane,
                                                 typename Elem<E>::type* const (&row)[NOUT], const float (&mult)[NOUT],
@@ -29,22 +38,20 @@ __device__ __forceinline__ void bwd_small_merge(const char* smem, int wave_bytes
     constexpr int DB = (D + 31) / 32;
     const int h = lane >> 5;
     if (!in_tensor) return;
-    for (int i = wave; i < NOUT * DB; i += NW) {
-        const int o = i / DB, db = i % DB;
+    for (int i = wave; i < NOUT * 4 * DB; i += NW) {
+        const bool last = i >= (NOUT - 1) * 4 * DB;  // (of the outputs)
+        const int d0 = 8 * (i % (4 * DB)) + 4 * h;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int g4 = 0; g4 < 4; g4++) {
-            float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int w = 0; w < NW; w++) {
+            const f32x4 part = reinterpret_cast<const f32x4*>(smem + w * wave_bytes)[i * 64 + lane];
 #pragma unroll
-            for (int w = 0; w < NW; w++) {
-                const float* part = reinterpret_cast<const float*>(smem + w * wave_bytes);
+            for (int e = 0; e < 4; e++) acc[e] += part[e];
+        }
+        if (D >= 32 || d0 < D) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) acc[e] += part[(i * 16 + 4 * g4 + e) * 64 + lane];
-            }
-            const int d0 = 32 * db + 8 * g4 + 4 * h;
-            if (D >= 32 || d0 < D) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) row[o][d0 + e] = (ET)(valid ? acc[e] * mult[o] : 0.f);
-            }
+            for (int e = 0; e < 4; e++)
+                (last ? row[NOUT - 1] : row[0])[d0 + e] = (ET)(valid ? acc[e] * (last ? mult[NOUT - 1] : mult[0]) : 0.f);
         }
     }
 }
@@ -180,13 +187,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void dq_small_k
         if (blk + NW < wr.end) issue_block(blk + NW);
     }
 
-    {
-        float* my = reinterpret_cast<float*>(mine);
-#pragma unroll
-        for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) my[(db * 16 + r) * 64 + lane] = dq[db][r];
-    }
+    bwd_small_leave<DB>(mine, 0, dq, lane);
     __syncthreads();
     ET* const rows[1] = {dqbase + (int64_t)q_pos * p.sdq.t};
     const float mult[1] = {p.sm_scale};
@@ -318,16 +319,8 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * SETS) void dkdv_small_kernel(
         if (it + NW < n_iters) issue_iter(it + NW);
     }
 
-    {
-        float* my = reinterpret_cast<float*>(mine);
-#pragma unroll
-        for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                my[(db * 16 + r) * 64 + lane] = dk[db][r];
-                my[((DB + db) * 16 + r) * 64 + lane] = dv[db][r];
-            }
-    }
+    bwd_small_leave<DB>(mine, 0, dk, lane);
+    bwd_small_leave<DB>(mine, DB, dv, lane);
     __syncthreads();
     ET* const rows[2] = {dkbase + (int64_t)k_pos * p.sdk.t, dvbase + (int64_t)k_pos * p.sdv.t};
     const float mult[2] = {p.sm_scale, 1.f};

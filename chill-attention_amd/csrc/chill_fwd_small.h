@@ -162,18 +162,17 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_
     }
 
     // ---- merge the waves' partial results
-    // m and the row sum (both halves of a row added up) of every wave; then O^T of every wave over its
-    // own staging area: register r of head-dim block db of lane l at ((db * 16 + r) * 64 + l) * 4
+    // m and the row sum (both halves of a row added up) of every wave; then O^T of every wave over its own staging area, four
+    // registers at a time: columns d0 .. d0 + 3, d0 = 8 * u + 4 * h, of lane l's row at (u * 64 + l) * 16
     const float l_row = sum_across_halves(l_run);
     float* my_ml = reinterpret_cast<float*>(mine + ML_OFF);
     my_ml[lane] = m_run;
     my_ml[64 + lane] = l_row;
     {
-        float* my_o = reinterpret_cast<float*>(mine);
+        f32x4* my_o = reinterpret_cast<f32x4*>(mine);
 #pragma unroll
-        for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) my_o[(db * 16 + r) * 64 + lane] = o[db][r];
+        for (int u = 0; u < 4 * DB; u++)
+            my_o[u * 64 + lane] = f32x4{o[u / 4][4 * (u % 4)], o[u / 4][4 * (u % 4) + 1], o[u / 4][4 * (u % 4) + 2], o[u / 4][4 * (u % 4) + 3]};
     }
     __syncthreads();
     float m_all = -INFINITY;
@@ -192,25 +191,21 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_
     const float l_safe = (l_all == 0.f) ? 1.f : l_all;
     const float inv = 1.f / l_safe;
     const bool valid = q_pos < seq_len;
-    // wave w finishes the head-dim blocks w, w + NW, ...: lane (n, h) holds, of ITS row, the columns
-    // d = 32 * db + 8 * (r / 4) + 4 * h + r % 4
+    // the groups of four columns go round the waves
     if (q_pos < p.T) {
         ET* orow = obase + (int64_t)q_pos * p.so.t;
-        for (int db = wave; db < DB; db += NW) {
+        for (int u = wave; u < 4 * DB; u += NW) {
+            const int d0 = 8 * u + 4 * h;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int g4 = 0; g4 < 4; g4++) {
-                float acc[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int w = 0; w < NW; w++) {
+                const f32x4 part = reinterpret_cast<const f32x4*>(smem + w * WAVE_BYTES)[u * 64 + lane];
 #pragma unroll
-                for (int w = 0; w < NW; w++) {
-                    const float* wo = reinterpret_cast<const float*>(smem + w * WAVE_BYTES);
+                for (int e = 0; e < 4; e++) acc[e] += part[e] * weight[w];
+            }
+            if (D >= 32 || d0 < D) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[e] += wo[(db * 16 + 4 * g4 + e) * 64 + lane] * weight[w];
-                }
-                const int d0 = 32 * db + 8 * g4 + 4 * h;
-                if (D >= 32 || d0 < D) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) orow[d0 + e] = (ET)(valid ? acc[e] * inv : 0.f);
-                }
+                for (int e = 0; e < 4; e++) orow[d0 + e] = (ET)(valid ? acc[e] * inv : 0.f);
             }
         }
         // LSE2 = m + log2(l) (chill_fwd.py:288-289); -inf for a row that saw no key, 0 for rows past lens
