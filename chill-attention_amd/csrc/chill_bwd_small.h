@@ -126,10 +126,11 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void dq_small_k
     AsyncSwizzledLoader<E, D, 32, 64> load_k, load_v;
     load_k.init(p.sk.t, 0, lane);
     load_v.init(p.sv.t, 0, lane);
+    // (rows behind the sequence read as zero: a masked weight of 0 does not keep the NaN of a tensor's padding out)
     auto issue_block = [&](int blk) {
         const int k0 = blk * 32;
-        load_k.issue(kptr + (int64_t)k0 * p.sk.t, p.T - k0, mine, 0, lane);
-        load_v.issue(vptr + (int64_t)k0 * p.sv.t, p.T - k0, mine + TILE_BYTES, 0, lane);
+        load_k.issue(kptr + (int64_t)k0 * p.sk.t, seq_len - k0, mine, 0, lane);
+        load_v.issue(vptr + (int64_t)k0 * p.sv.t, seq_len - k0, mine + TILE_BYTES, 0, lane);
     };
     const int first = wr.start + wave;
     if (first < wr.end) issue_block(first);
@@ -247,14 +248,14 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * SETS) void dkdv_small_kernel(
     AsyncSwizzledLoader<E, D, 32, 64> load_q, load_do;
     load_q.init(p.sq.t, 0, lane);
     load_do.init(p.sdo.t, 0, lane);
-    // iteration it = (group head, query block)
+    // iteration it = (group head, query block); rows behind the sequence read as zero, as above
     auto issue_iter = [&](int it) {
         const int hq = hkv * p.group + it / n_blocks;
         const int q0 = (wr.start + it % n_blocks) * 32;
         const ET* qptr = reinterpret_cast<const ET*>(p.q) + b * p.sq.b + hq * p.sq.h;
         const ET* doptr = reinterpret_cast<const ET*>(p.d_o) + b * p.sdo.b + hq * p.sdo.h;
-        load_q.issue(qptr + (int64_t)q0 * p.sq.t, p.T - q0, mine, 0, lane);
-        load_do.issue(doptr + (int64_t)q0 * p.sdo.t, p.T - q0, mine + TILE_BYTES, 0, lane);
+        load_q.issue(qptr + (int64_t)q0 * p.sq.t, seq_len - q0, mine, 0, lane);
+        load_do.issue(doptr + (int64_t)q0 * p.sdo.t, seq_len - q0, mine + TILE_BYTES, 0, lane);
         // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the end read as zero
         const int qq = q0 + n;
         const float* src = h == 0 ? p.lse + b * p.lse_b + hq * p.lse_h : p.delta + b * p.delta_b + hq * p.delta_h;

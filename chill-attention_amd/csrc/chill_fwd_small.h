@@ -94,10 +94,11 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_
     AsyncSwizzledLoader<E, D, 32, 64> load_k, load_v;
     load_k.init(p.sk.t, 0, lane);
     load_v.init(p.sv.t, 0, lane);
+    // (rows behind the sequence read as zero: a masked weight of 0 does not keep the NaN of a tensor's padding out)
     auto issue_block = [&](int blk) {
         const int k0 = blk * 32;
-        load_k.issue(kptr + (int64_t)k0 * p.sk.t, p.T - k0, mine, 0, lane);
-        load_v.issue(vptr + (int64_t)k0 * p.sv.t, p.T - k0, mine + TILE_BYTES, 0, lane);
+        load_k.issue(kptr + (int64_t)k0 * p.sk.t, seq_len - k0, mine, 0, lane);
+        load_v.issue(vptr + (int64_t)k0 * p.sv.t, seq_len - k0, mine + TILE_BYTES, 0, lane);
     };
     const int first = wr.start + wave;
     if (first < wr.end) issue_block(first);
