@@ -486,14 +486,14 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
         if constexpr (f32_serves(D, Elem<E>::kDType)) {
             constexpr int kLdsOne = bwd_small_lds_bytes(D, CHILL_F32, 1);
             const long long tiles = (long long)p.B * p.H * cdiv(p.T, 32);
-            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_DQ, D, tiles, p.T);
+            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_DQ, D, tiles, p.T, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
             const bool small = bwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, CHILL_F32, CHILL_PASS_DQ);
             if (shape.members == 4 || !small) {
                 constexpr int kLds = f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ);
                 return launch_bwd_f32<D, MASK_ID, 1, 4, 1>(p, D > 64 && small ? kLdsOne : kLds, stream);
             }
+            if (shape.members == 0) return launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
             if constexpr (D <= 64) {
-                if (shape.members == 0) return launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
                 if (shape.members == 2) return launch_bwd_f32<D, MASK_ID, 1, 2, 4>(p, 2 * kLdsOne, stream);
                 if (shape.streams == 8) return launch_bwd_f32<D, MASK_ID, 1, 1, 8>(p, 2 * kLdsOne, stream);
             } else {
@@ -1463,7 +1463,8 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
     CHILL_DISPATCH_MASK(mask_id, {
         if constexpr (f32_serves(D, Elem<E>::kDType) && D <= 64) {
             constexpr int kLds = bwd_small_lds_bytes(D, CHILL_F32, 2);
-            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_DKDV, D, (long long)p.B * p.H_kv * cdiv(p.T, 32), p.T);
+            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_DKDV, D, (long long)p.B * p.H_kv * cdiv(p.T, 32), p.T,
+                                             mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
             const bool small = bwd_takes_small(MASK_ID, (long long)p.B * p.H_kv, p.T, D, CHILL_F32, CHILL_PASS_DKDV);
             if (shape.members == 4 || !small)
                 return launch_bwd_f32<D, MASK_ID, 2, 4, 2>(p, small ? kLds : f32_lds_bytes(D, 4, 2, CHILL_PASS_DKDV), stream);

@@ -575,18 +575,23 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     const int n_q_tiles = cdiv(p.T, 32);
     // (at most kComputeUnits / 4 * 4 * 32 q-tiles by fwd_takes_small)
     bool two = false, sets = false;
-    // (fp32 beyond a few blocks per row: fwd_f32_kernel)
-    constexpr bool kDouble = Elem<E>::k16 && small_fits_two_tiles(kLdsOne);
+    constexpr bool kDouble = small_fits_two_tiles(kLdsOne);
     if constexpr (kDouble) {
-        const long long tiles = (long long)p.B * p.H * n_q_tiles;
-        two = small_takes_two_tiles(tiles);
-        sets = small_takes_two_sets(CHILL_PASS_FWD, tiles, p.T, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
+        const long long tiles = (long long)p.B * p.H * n_q_tiles, band_keys = mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1);
+        if constexpr (Elem<E>::k16) {
+            two = small_takes_two_tiles(tiles);
+            sets = small_takes_two_sets(CHILL_PASS_FWD, tiles, p.T, band_keys);
+        } else {
+            // (fp32 with more blocks per row or more tiles than CUs: fwd_f32_kernel)
+            sets = f32_shape(MASK_ID, CHILL_PASS_FWD, D, tiles, p.T, band_keys).streams == 8;
+        }
     }
     const int total = p.B * p.H * (two ? (n_q_tiles + 1) / 2 : n_q_tiles);
     const int lds_bytes = two || sets ? 2 * kLdsOne : kLdsOne;
     void (*kern)(FwdParams, int, int, int) = fwd_small_kernel<E, D, MASK_ID, 1, 1>;
     if constexpr (kDouble) {
-        if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
+        if constexpr (Elem<E>::k16)
+            if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
         if (sets) kern = fwd_small_kernel<E, D, MASK_ID, 1, 2>;
     }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
@@ -631,15 +636,15 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
         if constexpr (f32_serves(D, Elem<E>::kDType)) {
             constexpr int kLdsOne = fwd_small_lds_bytes(D, CHILL_F32);
             const long long tiles = (long long)p.B * p.H * cdiv(p.T, 32);
-            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_FWD, D, tiles, p.T);
+            const F32Shape shape = f32_shape(MASK_ID, CHILL_PASS_FWD, D, tiles, p.T, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
             const bool small = fwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, CHILL_F32);
             if (shape.members == 4 || !small) {
                 // (up to the sizes the small launches end at, rows of 512 bytes keep their LDS)
                 constexpr int kLds = f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ);
                 return launch_fwd_f32<D, MASK_ID, 4, 1>(p, D > 64 && small ? kLdsOne : kLds, stream);
             }
+            if (shape.members == 0) return launch_fwd_small<E, D, MASK_ID>(p, stream);
             if constexpr (D <= 64) {
-                if (shape.members == 0) return launch_fwd_small<E, D, MASK_ID>(p, stream);
                 if (shape.members == 2) return launch_fwd_f32<D, MASK_ID, 2, 4>(p, 2 * kLdsOne, stream);
                 if (shape.streams == 8) return launch_fwd_f32<D, MASK_ID, 1, 8>(p, 2 * kLdsOne, stream);
             } else {

@@ -190,12 +190,18 @@ constexpr bool fwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 constexpr bool small_fits_two_tiles(int lds_bytes_one) { return 2 * lds_bytes_one <= 160 * 1024; }
 constexpr bool small_takes_two_tiles(long long tiles) { return tiles > kComputeUnits; }
 // fp32 rows of at most 512 bytes go through fwd_f32_kernel, dq_f32_kernel and dkdv_f32_kernel (chill_f32.h): `members` row tiles
-// of 32 rows per workgroup, `streams` waves each; 0: the small-launch kernels, whose fp32 MFMAs need no preparation.
+// of 32 rows per workgroup, `streams` waves each; no members: the small-launch kernels, whose fp32 MFMAs need no preparation.
 // The report counts such a workgroup as 32 rows up to the sizes above (fwd_small_max_tiles and its like, where the fp32 MFMA
 // kernels were handed over to those of 128 rows) and as 128 rows beyond.
 // Measured in us, forward / dQ / dK/dV, the fp32 MFMA kernels first, all causal at head dim 64 where not named:
-//   few blocks per row, where splitting them costs what it saves: B1 H2 T256 9.8 / 13.4 / 15.4, eight streams 10.1 / 15.9,
-//     four streams 15.0; T512 15.2 / 20.4 / 24.6, eight streams 12.7 / 19.8, four 21.7
+//   few blocks per row (`reach` keys), where splitting them costs what it saves; one set of waves with the fp32 MFMA, two sets,
+//     four streams, eight, by graph replay; whole training step for dQ and dK/dV.  Forward: B1 H2 T256 9.78 / 9.83 / 10.75 / 10.44,
+//     B2 H8 T384 12.97 / 12.16 / 13.24 / 11.43, T512 15.28 / 14.15 / 15.67 / 13.21, full mask T256 10.05 / 9.87 / 10.76 / 10.41, window
+//     32 + 0 T1024 7.74 / 8.45 / 8.75 / 8.59, 64 + 64 10.87 / 10.28 / 11.35 / 10.98, 128 + 128 13.65 / 12.75 / 13.69 / 11.77.  dQ: T384
+//     49.2 / 49.3 / 48.9 / 50.4, T512 54.9 / 54.5 / 54.2 / 54.8, window 32 + 0 T640 30.0 / 31.7 / 30.7 / 35.0, 64 + 64 40.7 / 41.5 /
+//     40.6 / 43.5.  dK/dV, one set and four streams: T256 37.6 / 37.7, T384 49.1 / 48.2, T512 57.2 / 55.0, window 32 + 0 T512 33.5 /
+//     34.0, 64 + 64 43.0 / 42.3.  Head dim 128, one set and four streams: forward T128 10.9 / 12.9, T256 16.0 / 17.3, T512 25.8 / 25.9,
+//     window 64 + 64 T512 16.4 / 17.8; dQ T128 52.9 / 55.2, T256 76.5 / 77.4, T384 99.8 / 99.2, window 64 + 64 T512 77.3 / 78.5
 //   fewer tiles than CUs: B1 H4 T1111 29.8 / 38.2 / 86, four streams 26.2 / 32.5 / 66, eight 19.4 / 27.5 (dK/dV spills)
 //   pairs (two members, four streams) against four members: prefix-LM B1 H8 T2048 (512 tiles) 57 / 77 / 119, 38 / 49 / 64, 83 / 101 /
 //     96; B3 H8 T1024 (768) 48 / 68 / 80, 37 / 50 / 60, 45 / 56 / 54; B2 H8 T3000 (1500) 179 / 244 / 390, 123 / 156 / -, 124 / 151 /
@@ -208,16 +214,22 @@ struct F32Shape {
     int members, streams;
 };
 constexpr bool f32_serves(int D, int dtype) { return dtype == CHILL_F32 && D <= 128; }
-constexpr F32Shape f32_shape(int mask_id, int pass, int D, long long tiles, int T) {
+constexpr F32Shape f32_shape(int mask_id, int pass, int D, long long tiles, int T, long long band_keys) {
     const bool grow = mask_rows_grow(mask_id);
+    const long long reach = T - 31 < band_keys ? T : band_keys + 31;  // keys that the rows of a tile see
     if (D <= 64) {
-        if (tiles <= kComputeUnits && T <= 384) return F32Shape{0, 0};
+        if (tiles <= kComputeUnits) {
+            if (pass == CHILL_PASS_FWD && reach <= 256) return F32Shape{0, reach <= 128 || grow ? 4 : 8};
+            if (pass == CHILL_PASS_DQ && reach <= 384) return F32Shape{0, 4};
+            if (pass == CHILL_PASS_DKDV && (T <= 256 || reach <= 128)) return F32Shape{0, 4};
+        }
         if (pass == CHILL_PASS_DKDV) return tiles <= kComputeUnits ? F32Shape{1, 4} : tiles <= 512 ? F32Shape{2, 4} : F32Shape{4, 2};
-        if (tiles < kComputeUnits) return F32Shape{1, 8};
+        if (tiles < kComputeUnits) return F32Shape{1, pass == CHILL_PASS_DQ && reach <= 512 ? 4 : 8};
         if (tiles == kComputeUnits) return F32Shape{1, 4};
         return tiles <= (grow ? 2048 : 768) ? F32Shape{2, 4} : F32Shape{4, 1};
     }
     if (pass == CHILL_PASS_DKDV) return F32Shape{4, 2};  // dkdv_f32_wide_kernel
+    if (tiles <= kComputeUnits && reach <= (pass == CHILL_PASS_FWD ? 384 : 256)) return F32Shape{0, 4};
     if (tiles <= (grow ? 512 : 256)) return F32Shape{1, 4};
     return tiles <= 512 ? F32Shape{2, 2} : F32Shape{4, 1};
 }
@@ -254,8 +266,8 @@ constexpr int f32_wide_ring_bytes(int D) { return (f32_lds_bytes(D, 8, 1, CHILL_
 constexpr int f32_wide_lds_bytes(int D) { return f32_wide_ring_bytes(D) + 8 * 16 * 64 * 4; }
 constexpr TileConfig f32_small_tile_config(F32Shape shape, int D, int lds_bytes_one) {
     if (D <= 64 && shape.members == 4) return TileConfig{32, 32, kFwdSmallWaves, f32_lds_bytes(D, 4, 1, CHILL_PASS_DQ)};
-    const bool two = D <= 64 && shape.members * shape.streams == 8;
-    return TileConfig{32, 32, two && shape.members == 1 ? 8 : kFwdSmallWaves, two ? 2 * lds_bytes_one : lds_bytes_one};
+    const bool two = D <= 64 && (shape.members * shape.streams == 8 || (shape.members == 0 && shape.streams == 8));
+    return TileConfig{32, 32, two && shape.members <= 1 ? 8 : kFwdSmallWaves, two ? 2 * lds_bytes_one : lds_bytes_one};
 }
 
 // The backward of such launches (dq_small_kernel, dkdv_small_kernel): the same split of the streamed
@@ -521,7 +533,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
         case CHILL_PASS_FWD:
             if (T != kLongSequence && fwd_takes_small(mask_id, batch_heads, T, D, dtype)) {
                 const long long tiles = batch_heads * ((T + 31) / 32);
-                *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T), D, fwd_small_lds_bytes(D, dtype))
+                *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T, band_keys), D, fwd_small_lds_bytes(D, dtype))
                                             : small_tile_config(pass, fwd_small_lds_bytes(D, dtype), tiles, T, band_keys);
                 return CHILL_OK;
             }
@@ -530,7 +542,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
         case CHILL_PASS_DQ:
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DQ)) {
                 const long long tiles = batch_heads * ((T + 31) / 32);
-                *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T), D, bwd_small_lds_bytes(D, dtype, 1))
+                *out = f32_serves(D, dtype) ? f32_small_tile_config(f32_shape(mask_id, pass, D, tiles, T, band_keys), D, bwd_small_lds_bytes(D, dtype, 1))
                                             : small_tile_config(pass, bwd_small_lds_bytes(D, dtype, 1), tiles, T, band_keys);
                 return CHILL_OK;
             }

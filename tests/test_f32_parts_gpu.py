@@ -73,6 +73,36 @@ def test_against_64_bits(case):
                 assert (a[i, :, n:] == 0).all(), name
 
 
+# rows of few blocks, where the choice between the fp32 instruction (one or two sets of waves) and the parts lies: a mask and a T on
+# either side of each limit, with ragged ends, shared heads and lengths
+FEW_BLOCKS = [
+    ("one-block", ("CausalChillMask", ()), 1, 1, 1, 31, 64, None),
+    ("128-keys", ("FullChillMask", ()), 1, 2, 2, 128, 64, None),
+    ("129-keys", ("FullChillMask", ()), 2, 2, 1, 129, 64, (129, 1)),
+    ("two-sets-32", ("FullChillMask", ()), 1, 4, 2, 255, 32, (200,)),
+    ("two-sets-16", ("SlidingWindowChillMask", (64, 64)), 2, 3, 3, 333, 16, (333, 40)),
+    ("two-sets-all-units", ("SlidingWindowChillMask", (100, 60)), 1, 8, 4, 1023, 64, None),
+    ("growing-rows-257", ("CausalChillMask", ()), 1, 3, 3, 257, 64, None),
+    ("dq-385", ("PrefixLMChillMask", (30,)), 1, 3, 1, 385, 64, None),
+    ("dq-513", ("CausalChillMask", ()), 1, 2, 2, 513, 64, (511,)),
+    ("chunks", ("ChunkwiseChillMask", (32, 1)), 1, 4, 2, 700, 64, None),
+    ("wide-256", ("CausalChillMask", ()), 1, 2, 1, 256, 128, (250,)),
+    ("wide-385", ("FullChillMask", ()), 1, 2, 2, 385, 128, None),
+    ("wide-window", ("SlidingWindowChillMask", (40, 0)), 1, 8, 2, 1001, 128, None),
+]
+
+
+@pytest.mark.parametrize("case", FEW_BLOCKS, ids=lambda c: c[0])
+def test_few_blocks(case):
+    _, m, B, H, H_kv, T, D, lens = case
+    q, k, v, d_out = inputs(B, H, H_kv, T, D)
+    got, _ = run(make_mask(m), q, k, v, d_out, lens)
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, reference(m, q, k, v, d_out, lens)):
+        # as above (a row of one key has a dQ and dK of rounding alone: the difference over that of the inputs then)
+        err = ((a.double() - b).norm() / torch.maximum(b.norm(), 0.1 * q.double().norm())).item()
+        assert err < 1e-6, (name, err)
+
+
 @pytest.mark.parametrize("case", CASES[::2], ids=lambda c: c[0])
 def test_any_magnitude(case):
     """Powers of two pass through the scaled parts exactly: inputs scaled by them give the same bits, scaled."""
