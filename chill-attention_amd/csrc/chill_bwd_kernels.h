@@ -1499,7 +1499,7 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         } else if constexpr (has_small_row) {
             if (dkdv_takes_small_row(MASK_ID, (long long)p.B * p.H_kv, p.T)) return launch_dkdv_shape<E, D, MASK_ID, true>(p, stream);
             if constexpr (dkdv_one_stage_serves(MASK_ID, D, Elem<E>::kDType)) {
-                if (dkdv_takes_one_stage(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1)))
+                if (dkdv_takes_one_stage(MASK_ID, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, p.lens != nullptr))
                     return launch_dkdv_shape<E, D, MASK_ID, false, false, true>(p, stream);
             }
             status = launch_dkdv_shape<E, D, MASK_ID, false>(p, stream);

@@ -387,13 +387,13 @@ constexpr bool dkdv_is_paired(int D, int dtype) { return D * elem_bytes(dtype) <
 // 16-bit head dims <= 64: workgroups of 4 waves (64 key rows), small enough in LDS (50 KiB at D = 64)
 // and registers (167) for two or three of them per CU, which hide each other's start and end
 // (measured: sliding window dK/dV -32 %, prefix-LM at D = 64 -17 %).  At D = 128 the two-stage ring of
-// such a workgroup takes 99 KiB; with a one-stage ring it fits twice, which pays under narrow bands (dkdv_takes_one_stage).
+// such a workgroup takes 99 KiB; with a one-stage ring it fits twice (dkdv_takes_one_stage).
 // `small_grid`: the 8-wave grid would cover at most half of the CUs, or not all of them under a mask whose rows grow with their
 // index, where one round of 8-wave workgroups lasts as long as the longest of them (dkdv_takes_small_row); then the
 // 64-row workgroup is taken at every 16-bit head dim.  D128 bf16, 8-wave workgroups, us, 8 waves -> 4: 128 causal B1 H8 T2048 -17 %; 160
 // 61 -> 49; 192 B2 H32/4 T3000 510 -> 406; 224 B1 H8 T3500 83 -> 66, prefix-LM 88 -> 75, full mask 20 workgroups a head, 160, 62 -> 91,
-// window 512 24 -> 32; 288 B1 H9 T4000 99 -> 100; 320 B2 H32/8 T2500 249 -> 269.  (A grid of exactly 256, B1 H8 T4096 98 -> 83, keeps
-// the 8-wave entry that the tile table has always given for it.)
+// window 512 24 -> 32; 288 B1 H9 T4000 99 -> 100; 320 B2 H32/8 T2500 249 -> 269.  (A grid of exactly 256 keeps the 8-wave entry that
+// the tile table has always given for it.)
 constexpr int dkdv_paired_waves(int mask_id, int D, int dtype, bool small_grid = false) {
     (void)mask_id;
     if (CHILL_TUNE_DKDV_WAVES) return CHILL_TUNE_DKDV_WAVES;
@@ -408,13 +408,27 @@ constexpr bool dkdv_takes_small_row(int mask_id, long long batch_kv_heads, int T
 // one stage: window 16 + 16 fp16 B8 H4 T6000 101 -> 79, bf16 B2 H16/4 T2085 36 -> 27; 128 + 128 115 -> 95, 44 -> 33, bf16 B2 H32
 // T4096 153 -> 128; 512 + 128 172 -> 160, 75 -> 57; 1024 + 0 231 -> 219; 2047 + 0 352 -> 346, B2 H16/4 T16000 917 -> 905; 3000 + 500
 // 523 -> 529; chunkwise 100 x 3 129 -> 113, 128 x 3 114 -> 105, B2 H16 T3000 55 -> 49, 1000 x 2 392 -> 385 (T3000 180 -> 183),
-// 1000 x 5 640 -> 642 (T3000 192 -> 200).  Masks that are not banded are within 4 % either way.  Letting dO's half of the next tile go
-// out behind the dV^T MFMAs, with a barrier of its own, costs 2-10 %.  Grids that leave CUs idle keep the two-stage 64-row
-// workgroups (dkdv_takes_small_row).
+// 1000 x 5 640 -> 642 (T3000 192 -> 200).  Letting dO's half of the next tile go out behind the dV^T MFMAs, with a barrier of its own,
+// costs 2-10 %.
+// Under masks whose rows grow with their index the smaller workgroups end a launch more evenly, the more so over the unequal
+// sequences of a padded batch.  Training step, us, 8 waves -> one stage (bf16; the number is that of 8-wave workgroups): causal 256
+// B1 H16/4 T8192 1272 -> 1216, B4 H32/8 T1000 226 -> 210; 272 B2 H32/8 T2085 411 -> 388; 384 B1 H12 T4000 280 -> 274; 512 B1 H32 T2048
+// 194 -> 195; 752 B2 H8 T6000 649 -> 644; 960 B4 H12 T2500 386 -> 384; 1536 B8 H16 T1500 424 -> 430; 2176 B8 H16 T2085 739 -> 737;
+// prefix-LM 384 285 -> 272, 512 199 -> 196, 960 394 -> 385, 1536 434 -> 435; padded to T/4 .. T, causal B8 H16 T300 56 -> 50, B4 H32/8
+// T2085 479 -> 463, B8 H16 T1500 285 -> 273, T2085 448 -> 435, B4 H32 T2900 817 -> 823, prefix-LM 344 -> 317, 297 -> 284, 463 -> 450,
+// 835 -> 831.  Full masks are within 1 % either way.
+// Grids that leave CUs idle keep the two-stage 64-row workgroups (dkdv_takes_small_row; one stage: causal B2 H16/2 T2900, 92, 568 ->
+// 584, B3 H16/4 T2048, 192, 305 -> 307, prefix-LM 574 -> 621).
 // The report gives the two workgroups of a CU as one, 128 rows and 8 waves, which is also what they take of its LDS.
 constexpr int kDkdvOneStageBand = 2048;
-constexpr bool dkdv_one_stage_serves(int mask_id, int D, int dtype) { return dtype != CHILL_F32 && D == 128 && mask_is_banded(mask_id); }
-constexpr bool dkdv_takes_one_stage(long long band_keys) { return band_keys <= kDkdvOneStageBand; }
+constexpr int kDkdvOneStageMaxGrid = 4 * kComputeUnits;
+constexpr bool dkdv_one_stage_serves(int mask_id, int D, int dtype) {
+    return dtype != CHILL_F32 && D == 128 && (mask_is_banded(mask_id) || mask_rows_grow(mask_id));
+}
+constexpr bool dkdv_takes_one_stage(int mask_id, long long band_keys, long long batch_kv_heads, int T, bool padded) {
+    return mask_is_banded(mask_id) ? band_keys <= kDkdvOneStageBand
+                                   : padded || batch_kv_heads * ((T + 127) / 128) < kDkdvOneStageMaxGrid;
+}
 // at the end the waves of a pair exchange one fp32 accumulator each through LDS: 8 waves x (D rounded
 // up to 32) x 32 floats
 constexpr int dkdv_paired_exchange_bytes(int D) { return 8 * ((D + 31) / 32) * 16 * 64 * 4; }

@@ -1,6 +1,6 @@
-"""dK/dV of 16-bit inputs at head dim 128 under narrow bands (csrc/chill_tiles.h, dkdv_takes_one_stage): 64-row workgroups with a
-ring of one stage, two to a CU, at ragged lengths, with grouped heads and padding, either side of the widths and chunk sizes
-that change the route, against the oracle."""
+"""dK/dV of 16-bit inputs at head dim 128 under narrow bands and under masks whose rows grow (csrc/chill_tiles.h,
+dkdv_takes_one_stage): 64-row workgroups with a ring of one stage, two to a CU, at ragged lengths, with grouped heads and padding,
+either side of the widths, chunk sizes and grids that change the route, against the oracle."""
 import pytest
 import torch
 
@@ -25,6 +25,14 @@ CASES = [
     (torch.bfloat16, ("ChunkwiseChillMask", (64, 2)), 1, 33, 33, 4097, None, (128, 8)),
     (torch.float16, ("ChunkwiseChillMask", (64, 2)), 1, 32, 32, 4096, None, (256, 4)),
     (torch.float16, ("ChunkwiseChillMask", (128, 1)), 1, 34, 34, 4100, None, (128, 8)),
+    # as many 8-wave workgroups as CUs and a few more, up to four times that, and beyond with and without padding
+    (torch.bfloat16, ("CausalChillMask", ()), 1, 16, 16, 2048, None, (128, 8)),
+    (torch.float16, ("CausalChillMask", ()), 2, 16, 8, 2081, (2081, 65), (128, 8)),
+    (torch.float16, ("PrefixLMChillMask", (300,)), 3, 8, 8, 1441, (1441, 0, 299), (128, 8)),
+    (torch.bfloat16, ("PrefixLMChillMask", (100,)), 4, 16, 16, 1920, None, (128, 8)),
+    (torch.bfloat16, ("CausalChillMask", ()), 4, 16, 16, 2033, None, (128, 8)),
+    (torch.float16, ("CausalChillMask", ()), 4, 16, 16, 2033, (2033, 700, 64, 1), (128, 8)),
+    (torch.bfloat16, ("CausalChillMask", ()), 1, 8, 8, 4100, None, (128, 8)),
 ]
 
 
