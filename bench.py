@@ -39,9 +39,9 @@ PEAK_HBM_GBS = 8000.0
 # sources it was measured on (kernel_sources_digest below); with other sources the line reports null.
 TRAFFIC_SOURCE = "profiles/c3_causal_bf16_fwd_bwd_kernels.md"
 MEASURED_TRAFFIC = {
-    ("C3", "chill_fwd"): (580675 * 2.0 + 348163) * 1024,
-    ("C3", "chill_bwd_dq_delta"): (1135401 * 2.0 + 294912) * 1024,
-    ("C3", "chill_bwd_dkdv"): (1215685 * 2.0 + 581632) * 1024,
+    ("C3", "chill_fwd"): (579099 * 2.0 + 348161) * 1024,
+    ("C3", "chill_bwd_dq_delta"): (1124039 * 2.0 + 294912) * 1024,
+    ("C3", "chill_bwd_dkdv"): (1212499 * 2.0 + 581632) * 1024,
 }
 
 

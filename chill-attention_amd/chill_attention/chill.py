@@ -322,8 +322,8 @@ def chill_attention(
         return_lse: also return LSE2 ``[B, H, T]`` fp32 (base 2, scale included; ``-inf`` for rows
             that see no key, 0 for rows at or beyond ``lens``).
         prescale_qk, precision, autotune: accepted for interface compatibility.  The scale is
-            always applied to the fp32 scores; fp32 inputs always use IEEE fp32 MFMA (gfx950 has no
-            tf32 path); tile shapes come from a static table, there is no autotuner.
+            always applied to the fp32 scores; fp32 inputs always keep fp32 precision (gfx950
+            has no tf32 path); tile shapes come from a static table, there is no autotuner.
 
     Returns:
         ``O`` or ``(O, LSE2)``.

