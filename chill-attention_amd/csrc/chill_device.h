@@ -308,8 +308,9 @@ struct LdsTile {
     // +32 rows leaves the swizzle key unchanged (mod 16) when 32 rows are a multiple of 16 lines
     static constexpr bool kBlockAffine = CH >= 8;
 
-    __device__ __forceinline__ static int swz(int t) { return ((t & 3) << 2) | ((t >> 2) & 3); }
-    __device__ __forceinline__ static int phys(int L) { return L ^ swz(CH > 16 ? (L >> 5) : (L >> 4)); }
+    // (indices are non-negative)
+    __device__ __forceinline__ static unsigned swz(unsigned t) { return ((t & 3) << 2) | ((t >> 2) & 3); }
+    __device__ __forceinline__ static int phys(unsigned L) { return (int)(L ^ swz(CH > 16 ? (L >> 5) : (L >> 4))); }
     __device__ __forceinline__ static int chunk_off(int row, int c) { return phys(row * CH + c) * 16; }
     // byte offset of element (row, col)
     __device__ __forceinline__ static int elem_off(int row, int col) {
@@ -394,8 +395,9 @@ struct AsyncSwizzledLoader {
     __device__ __forceinline__ void init(int64_t row_stride, int wave, int lane) {
 #pragma unroll
         for (int i = 0; i < PER_WAVE; i++) {
-            int lg = L::phys((i * NWV + wave) * 64 + lane);
-            goff[i] = (int)((lg / L::CH) * row_stride * Elem<E>::kBytes) + (lg % L::CH) * 16;
+            // (unsigned: a signed division by a power of two is four instructions)
+            const unsigned lg = L::phys((i * NWV + wave) * 64 + lane);
+            goff[i] = (int)((lg / L::CH) * (unsigned)(row_stride * Elem<E>::kBytes) + (lg % L::CH) * 16);
         }
     }
 
@@ -415,7 +417,7 @@ struct AsyncSwizzledLoader {
                 const int slab = i * NWV + wave;
                 if (SLABS % NWV != 0 && slab >= SLABS) continue;
                 int slot = slab * 64 + lane;
-                int row = L::phys(slot) / L::CH;
+                int row = (unsigned)L::phys(slot) / L::CH;
                 if (row < rows_valid) {
                     async_load16(tile_base, goff[i], lds_base + slab * 1024);
                 } else {
@@ -482,9 +484,10 @@ struct AsyncPaddedLoader {
     __device__ __forceinline__ void init(int64_t row_stride, int wave, int lane) {
 #pragma unroll
         for (int i = 0; i < PER_WAVE; i++) {
-            int slot = (i * NWV + wave) * 64 + lane;
-            int row = slot / P::CHP, c = slot % P::CHP;
-            goff[i] = slot < SLOTS ? (int)(row * row_stride * Elem<E>::kBytes) + (c < P::CH ? c * 16 : 0) : -1;
+            const unsigned slot = (i * NWV + wave) * 64 + lane;
+            const unsigned row = slot / P::CHP, c = slot % P::CHP;
+            const int at = (int)(row * (unsigned)(row_stride * Elem<E>::kBytes) + (c < P::CH ? c * 16 : 0));
+            goff[i] = slot < SLOTS ? at : -1;
         }
     }
 
@@ -729,15 +732,19 @@ __device__ __forceinline__ void load_resident(Resident<E, D>& regs,
                                               const typename Elem<E>::type* base, int64_t row_stride,
                                               int rows_valid, int lane) {
     constexpr int NJ = Resident<E, D>::NJ;
-    int n = lane & 31, h = lane >> 5;
+    const int n = lane & 31, h = lane >> 5;
+    // (one address and one test for the row, the chunks at constant offsets: a test and an address for every chunk are ten
+    // vector instructions each; and complete blocks, which are nearly all, without the zeros)
+    const char* row = reinterpret_cast<const char*>(base + (int64_t)n * row_stride) + h * 16;
+    if (rows_valid >= 32) {
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        i32x4 val = {0, 0, 0, 0};
-        if (n < rows_valid) {
-            val = *reinterpret_cast<const i32x4*>(
-                reinterpret_cast<const char*>(base + (int64_t)n * row_stride) + (2 * j + h) * 16);
+        for (int j = 0; j < NJ; j++) regs.c[j] = *reinterpret_cast<const i32x4*>(row + j * 32);
+    } else {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            regs.c[j] = i32x4{0, 0, 0, 0};
+            if (n < rows_valid) regs.c[j] = *reinterpret_cast<const i32x4*>(row + j * 32);
         }
-        regs.c[j] = val;
     }
 }
 
@@ -785,16 +792,17 @@ __device__ __forceinline__ void store_row_transposed(typename Elem<E>::type* row
                     f32x4 va, vb;
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        va[e] = valid ? acc[db][8 * gp + e] * mult : 0.f;
-                        vb[e] = valid ? acc[db][8 * gp + 4 + e] * mult : 0.f;
+                        va[e] = acc[db][8 * gp + e] * mult;
+                        vb[e] = acc[db][8 * gp + 4 + e] * mult;
                     }
                     const i32x2 a = Elem<E>::pack4(va), b = Elem<E>::pack4(vb);
                     // first: lanes h = 0 keep their group 2 gp, lanes h = 1 receive the partner's group 2 gp + 1;
                     // second: lanes h = 0 receive the partner's group 2 gp, lanes h = 1 keep their group 2 gp + 1
                     const auto w0 = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
                     const auto w1 = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
-                    *reinterpret_cast<i32x4*>(row_ptr + 32 * db + 16 * gp + 8 * h) =
-                        i32x4{(int)w0[0], (int)w1[0], (int)w0[1], (int)w1[1]};
+                    // (the row's two lanes are valid together: the packed values are selected, half as many)
+                    const i32x4 out = {(int)w0[0], (int)w1[0], (int)w0[1], (int)w1[1]};
+                    *reinterpret_cast<i32x4*>(row_ptr + 32 * db + 16 * gp + 8 * h) = valid ? out : i32x4{0, 0, 0, 0};
                 }
             }
         } else {
