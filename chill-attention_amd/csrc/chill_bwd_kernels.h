@@ -105,6 +105,7 @@ __device__ __forceinline__ void softmax_grad_block(f32x16& s, f32x16& dp, float 
 
 }  // namespace chill
 #include "chill_bwd_small.h"
+#include "chill_f32_bwd_small.h"
 namespace chill {
 
 // ------------------------------------------------------------------------------------------ dQ
@@ -425,29 +426,40 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     const long long heads = (long long)p.B * (PASS == 1 ? p.H : p.H_kv);  // (few by bwd_takes_small)
     // (dK/dV keeps one block per workgroup: with K, V and two accumulators a wave needs more than the 256 registers it
     // would be left with; fp32 takes one set of waves)
+    constexpr int DT = Elem<E>::kDType;
     constexpr bool kDouble = small_fits_two_tiles(kLdsOne) && (PASS == 1 || Elem<E>::k16);
-    bool two = false, sets = false;
-    if constexpr (kDouble) {
-        const long long tiles = heads * n_tiles;
-        two = PASS == 1 && small_takes_two_tiles(tiles);
-        if constexpr (Elem<E>::k16)
-            sets = small_takes_two_sets(MASK_ID, Elem<E>::kDType, PASS == 1 ? CHILL_PASS_DQ : CHILL_PASS_DKDV, tiles, p.T,
-                                        mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
+    const long long tiles = heads * n_tiles;
+    const long long band = mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1);
+    const bool two = kDouble && PASS == 1 && small_takes_two_tiles(tiles);
+    bool sets = false;
+    void (*kern)(BwdParams, int, int, int) = nullptr;
+    if constexpr (f32_parts_serve(D, DT)) {
+        if (small_takes_parts(MASK_ID, band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
+            if constexpr (PASS == 1)
+                kern = two ? dq_small_f32_kernel<D, MASK_ID, 2> : dq_small_f32_kernel<D, MASK_ID, 1>;
+            else
+                kern = dkdv_small_f32_kernel<D, MASK_ID>;
+        }
+    }
+    if (kern == nullptr) {
+        if constexpr (PASS == 1)
+            kern = dq_small_kernel<E, D, MASK_ID, 1, 1>;
+        else
+            kern = dkdv_small_kernel<E, D, MASK_ID, 1>;
+        if constexpr (kDouble) {
+            if constexpr (Elem<E>::k16)
+                sets = small_takes_two_sets(MASK_ID, DT, PASS == 1 ? CHILL_PASS_DQ : CHILL_PASS_DKDV, tiles, p.T, band);
+            if constexpr (PASS == 1) {
+                if (two) kern = dq_small_kernel<E, D, MASK_ID, 2, 1>;
+                if constexpr (Elem<E>::k16)
+                    if (sets) kern = dq_small_kernel<E, D, MASK_ID, 1, 2>;
+            } else {
+                if (sets) kern = dkdv_small_kernel<E, D, MASK_ID, 2>;
+            }
+        }
     }
     const int total = (int)(heads * (two ? (n_tiles + 1) / 2 : n_tiles));
     const int lds_bytes = two || sets ? 2 * kLdsOne : kLdsOne;
-    void (*kern)(BwdParams, int, int, int);
-    if constexpr (PASS == 1)
-        kern = dq_small_kernel<E, D, MASK_ID, 1, 1>;
-    else
-        kern = dkdv_small_kernel<E, D, MASK_ID, 1>;
-    if constexpr (kDouble && PASS == 1) {
-        if (two) kern = dq_small_kernel<E, D, MASK_ID, 2, 1>;
-        if constexpr (Elem<E>::k16)
-            if (sets) kern = dq_small_kernel<E, D, MASK_ID, 1, 2>;
-    } else if constexpr (kDouble) {
-        if (sets) kern = dkdv_small_kernel<E, D, MASK_ID, 2>;
-    }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
     if (lds_bytes > 48 * 1024) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -407,6 +407,7 @@ __device__ __forceinline__ void fwd_q_tile(const FwdParams& p, char* smem, int b
 #include "chill_fwd_regs.h"
 #include "chill_fwd_fast.h"
 #include "chill_fwd_small.h"
+#include "chill_f32_fwd_small.h"
 #include "chill_fwd_split.h"
 namespace chill {
 
@@ -573,21 +574,29 @@ template <typename E, int D, int MASK_ID>
 int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     constexpr int kLdsOne = fwd_small_lds_bytes(D, Elem<E>::kDType);
     const int n_q_tiles = cdiv(p.T, 32);
-    // (at most kComputeUnits / 4 * 4 * 32 q-tiles by fwd_takes_small)
-    bool two = false, sets = false;
+    const long long tiles = (long long)p.B * p.H * n_q_tiles;
+    constexpr int DT = Elem<E>::kDType;
     constexpr bool kDouble = small_fits_two_tiles(kLdsOne);
-    if constexpr (kDouble) {
-        const long long tiles = (long long)p.B * p.H * n_q_tiles;
-        two = small_takes_two_tiles(tiles);
-        sets = small_takes_two_sets(MASK_ID, Elem<E>::kDType, CHILL_PASS_FWD, tiles, p.T, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1));
+    const bool two = kDouble && small_takes_two_tiles(tiles);
+    const long long band = mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1);
+    const bool sets = kDouble && small_takes_two_sets(MASK_ID, DT, CHILL_PASS_FWD, tiles, p.T, band);
+    void (*kern)(FwdParams, int, int, int) = nullptr;
+    if constexpr (f32_parts_serve(D, DT)) {
+        if (small_takes_parts(MASK_ID, band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
+            kern = fwd_small_f32_kernel<D, MASK_ID, 1, 1>;
+            if (two) kern = fwd_small_f32_kernel<D, MASK_ID, 2, 1>;
+            if (sets) kern = fwd_small_f32_kernel<D, MASK_ID, 1, 2>;
+        }
+    }
+    if (kern == nullptr) {
+        kern = fwd_small_kernel<E, D, MASK_ID, 1, 1>;
+        if constexpr (kDouble) {
+            if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
+            if (sets) kern = fwd_small_kernel<E, D, MASK_ID, 1, 2>;
+        }
     }
     const int total = p.B * p.H * (two ? (n_q_tiles + 1) / 2 : n_q_tiles);
     const int lds_bytes = two || sets ? 2 * kLdsOne : kLdsOne;
-    void (*kern)(FwdParams, int, int, int) = fwd_small_kernel<E, D, MASK_ID, 1, 1>;
-    if constexpr (kDouble) {
-        if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
-        if (sets) kern = fwd_small_kernel<E, D, MASK_ID, 1, 2>;
-    }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
     if (lds_bytes > 48 * 1024) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -20,6 +20,67 @@ namespace chill {
 
 // (kFwdSmallWaves, fwd_small_lds_bytes and the launches that come here: chill_tiles.h)
 
+// A wave's partial result: m and the row sum (both halves of a row added up) at the end of its area, O^T over its staging area, four
+// registers at a time: columns d0 .. d0 + 3, d0 = 8 * u + 4 * h, of lane l's row at (u * 64 + l) * 16
+template <int DB>
+__device__ __forceinline__ void fwd_small_leave(char* mine, int wave_bytes, int lane, const f32x16 (&o)[DB], float m_run, float l_row) {
+    float* my_ml = reinterpret_cast<float*>(mine + wave_bytes - 2 * 64 * 4);
+    my_ml[lane] = m_run;
+    my_ml[64 + lane] = l_row;
+    f32x4* my_o = reinterpret_cast<f32x4*>(mine);
+#pragma unroll
+    for (int u = 0; u < 4 * DB; u++)
+        my_o[u * 64 + lane] = f32x4{o[u / 4][4 * (u % 4)], o[u / 4][4 * (u % 4) + 1], o[u / 4][4 * (u % 4) + 2], o[u / 4][4 * (u % 4) + 3]};
+}
+
+// Merges the partial results of a workgroup's waves and stores the rows.
+template <typename E, int D, int NW>
+__device__ __forceinline__ void fwd_small_merge(const FwdParams& p, char* smem, int wave_bytes, int wave, int lane,
+                                                typename Elem<E>::type* obase, float* lse_base, int q_pos, int seq_len) {
+    using ET = typename Elem<E>::type;
+    constexpr int DB = (D + 31) / 32;
+    const int h = lane >> 5;
+    const int ml_off = wave_bytes - 2 * 64 * 4;
+    float m_all = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; w++) m_all = fmaxf(m_all, reinterpret_cast<const float*>(smem + w * wave_bytes + ml_off)[lane]);
+    const float m_ref = (m_all == -INFINITY) ? 0.f : m_all;
+    float weight[NW];
+    float l_all = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const float* ml = reinterpret_cast<const float*>(smem + w * wave_bytes + ml_off);
+        const float mw = ml[lane];
+        weight[w] = (mw == -INFINITY) ? 0.f : fast_exp2(mw - m_ref);
+        l_all += ml[64 + lane] * weight[w];
+    }
+    const float l_safe = (l_all == 0.f) ? 1.f : l_all;
+    const float inv = 1.f / l_safe;
+    const bool valid = q_pos < seq_len;
+    // the groups of four columns go round the waves: one to four LDS reads of 16 bytes a wave and partial result, all waves at it
+    // (whole 32-column blocks of a wave, value by value, left half of the waves idle at head dim 64: bf16 causal B1 H8 T256 5.66 ->
+    // 5.44 us, fp32 B1 H2 T256 9.55 -> 9.35)
+    if (q_pos < p.T) {
+        ET* orow = obase + (int64_t)q_pos * p.so.t;
+        for (int u = wave; u < 4 * DB; u += NW) {
+            const int d0 = 8 * u + 4 * h;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                const f32x4 part = reinterpret_cast<const f32x4*>(smem + w * wave_bytes)[u * 64 + lane];
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] += part[e] * weight[w];
+            }
+            if (D >= 32 || d0 < D) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) orow[d0 + e] = (ET)(valid ? acc[e] * inv : 0.f);
+            }
+        }
+        // LSE2 = m + log2(l) (chill_fwd.py:288-289); -inf for a row that saw no key, 0 for rows past lens
+        if (lse_base != nullptr && wave == 0 && h == 0) lse_base[q_pos] = valid ? m_all + __log2f(l_safe) : 0.f;
+    }
+}
+
 // TILES = 2: a workgroup of eight waves takes two q-tiles side by side, tile j from the end and tile j from the start of
 // one head, four waves each with an LDS area of their own.  Under causal-like masks the two add up to the same work
 // for every workgroup, where workgroups of one q-tile each leave the CUs that drew two long ones to finish alone
@@ -39,7 +100,6 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_
     constexpr int TILE_BYTES = L::bytes(32);
     // K block, V block (later the partial O^T); then m and l of the wave's lanes
     constexpr int WAVE_BYTES = fwd_small_wave_bytes(D, Elem<E>::kDType);
-    constexpr int ML_OFF = WAVE_BYTES - 2 * 64 * 4;
     extern __shared__ __attribute__((aligned(16))) char smem_all[];
 
     const int item = blockIdx.x;
@@ -163,57 +223,9 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) void fwd_small_
     }
 
     // ---- merge the waves' partial results
-    // m and the row sum (both halves of a row added up) of every wave; then O^T of every wave over its own staging area, four
-    // registers at a time: columns d0 .. d0 + 3, d0 = 8 * u + 4 * h, of lane l's row at (u * 64 + l) * 16
-    const float l_row = sum_across_halves(l_run);
-    float* my_ml = reinterpret_cast<float*>(mine + ML_OFF);
-    my_ml[lane] = m_run;
-    my_ml[64 + lane] = l_row;
-    {
-        f32x4* my_o = reinterpret_cast<f32x4*>(mine);
-#pragma unroll
-        for (int u = 0; u < 4 * DB; u++)
-            my_o[u * 64 + lane] = f32x4{o[u / 4][4 * (u % 4)], o[u / 4][4 * (u % 4) + 1], o[u / 4][4 * (u % 4) + 2], o[u / 4][4 * (u % 4) + 3]};
-    }
+    fwd_small_leave<DB>(mine, WAVE_BYTES, lane, o, m_run, sum_across_halves(l_run));
     __syncthreads();
-    float m_all = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < NW; w++) m_all = fmaxf(m_all, reinterpret_cast<const float*>(smem + w * WAVE_BYTES + ML_OFF)[lane]);
-    const float m_ref = (m_all == -INFINITY) ? 0.f : m_all;
-    float weight[NW];
-    float l_all = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-        const float* ml = reinterpret_cast<const float*>(smem + w * WAVE_BYTES + ML_OFF);
-        const float mw = ml[lane];
-        weight[w] = (mw == -INFINITY) ? 0.f : fast_exp2(mw - m_ref);
-        l_all += ml[64 + lane] * weight[w];
-    }
-    const float l_safe = (l_all == 0.f) ? 1.f : l_all;
-    const float inv = 1.f / l_safe;
-    const bool valid = q_pos < seq_len;
-    // the groups of four columns go round the waves: one to four LDS reads of 16 bytes a wave and partial result, all waves at it
-    // (whole 32-column blocks of a wave, value by value, left half of the waves idle at head dim 64: bf16 causal B1 H8 T256 5.66 ->
-    // 5.44 us, fp32 B1 H2 T256 9.55 -> 9.35)
-    if (q_pos < p.T) {
-        ET* orow = obase + (int64_t)q_pos * p.so.t;
-        for (int u = wave; u < 4 * DB; u += NW) {
-            const int d0 = 8 * u + 4 * h;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int w = 0; w < NW; w++) {
-                const f32x4 part = reinterpret_cast<const f32x4*>(smem + w * WAVE_BYTES)[u * 64 + lane];
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[e] += part[e] * weight[w];
-            }
-            if (D >= 32 || d0 < D) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) orow[d0 + e] = (ET)(valid ? acc[e] * inv : 0.f);
-            }
-        }
-        // LSE2 = m + log2(l) (chill_fwd.py:288-289); -inf for a row that saw no key, 0 for rows past lens
-        if (lse_base != nullptr && wave == 0 && h == 0) lse_base[q_pos] = valid ? m_all + __log2f(l_safe) : 0.f;
-    }
+    fwd_small_merge<E, D, NW>(p, smem, WAVE_BYTES, wave, lane, obase, lse_base, q_pos, seq_len);
 }
 
 }  // namespace chill

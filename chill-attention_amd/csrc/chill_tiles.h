@@ -152,6 +152,10 @@ constexpr int kFwdSmallWaves = 4;
 // dK/dV 110 -> 76)
 constexpr int kFwdSmallMaxT = 16384;
 // (at the end the area also takes the wave's partial O^T, 4 KiB per 32 columns of the head dim)
+// (fp32 at head dims up to 64 has kernels of the same shape whose products go through bf16 parts, chill_f32_parts.h: their
+// areas hold the parts of one 32-row block of V, in dQ of K, which are smaller, in dK/dV of Q and of dO)
+constexpr bool f32_parts_serve(int D, int dtype) { return dtype == CHILL_F32 && D <= 64; }
+constexpr int f32_planes_bytes(int D) { return 3 * 32 * D * 2; }
 constexpr int fwd_small_wave_bytes(int D, int dtype) {
     const int blocks = 2 * 32 * D * elem_bytes(dtype), partial = ((D + 31) / 32) * 16 * 64 * 4;
     return (blocks > partial ? blocks : partial) + 2 * 64 * 4;
@@ -220,7 +224,8 @@ constexpr TileConfig small_tile_config(int mask_id, int dtype, int pass, int lds
 #define CHILL_TUNE_BWD_SMALL 1
 #endif
 constexpr int bwd_small_wave_bytes(int D, int dtype, int outputs) {
-    const int blocks = 2 * 32 * D * elem_bytes(dtype), partial = outputs * ((D + 31) / 32) * 16 * 64 * 4;
+    const int rows = 2 * 32 * D * elem_bytes(dtype), parts = f32_parts_serve(D, dtype) ? outputs * f32_planes_bytes(D) : 0;
+    const int blocks = rows > parts ? rows : parts, partial = outputs * ((D + 31) / 32) * 16 * 64 * 4;
     return (blocks > partial ? blocks : partial) + 2 * 32 * 4;
 }
 constexpr int bwd_small_lds_bytes(int D, int dtype, int outputs) { return kFwdSmallWaves * bwd_small_wave_bytes(D, dtype, outputs); }
@@ -249,6 +254,22 @@ constexpr long long bwd_small_max_tiles(int mask_id, int T, int D, int dtype, in
 constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D, int dtype, int pass) {
     return bwd_small_serves(D, dtype, pass) && T <= kFwdSmallMaxT * CHILL_TUNE_BWD_SMALL_SCALE &&
            batch_heads * ((T + 31) / 32) <= bwd_small_max_tiles(mask_id, T, D, dtype, pass) * CHILL_TUNE_BWD_SMALL_SCALE;
+}
+// Small fp32 launches whose products go through bf16 parts: all at head dim 16, at head dims 32 and 64 those of more than 256 and of
+// at least 1024 rows, bands of less than 256 keys aside, where all three passes are served by the small kernels.  A forward of short
+// rows ends before the splits of a wave's first operands are paid for, and the passes go together: P comes out of a score and an
+// LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both through the fp32 instruction, 2.0e-6 with
+// both through parts, 4.2e-6 with one of each).
+// Forward / dQ / dK/dV in us, fp32 instruction -> parts:
+//   D64 causal B2 H16 T512 18 / 25 / 35 -> 20 / 24 / 30      B1 H8 T1024 24 / 35 / 44 -> 24 / 27 / 31     B1 H4 T1111 25 / 38 / 47 -> 25 / 24 / 32
+//       B2 H16 T2048 166 / 228 / 347 -> 161 / 198 / 257      full mask B1 H8 T2048 76 / 103 / 154 -> 71 / 87 / 111
+//       window 256 B1 H8 T2048 20 / 27 / 40 -> 20 / 25 / 33  window 100 + 30 B1 H4 T1111 10 / 15 / 17 -> 12 / 11 / 15
+//   D32 causal B8 H8 T256 9 / 12 / 13 -> 10 / 11 / 16        B1 H8 T512 9 / 12 / 15 -> 11 / 10 / 12       B1 H16 T1100 30 / 43 / 38 -> 30 / 32 / 35
+//   D16 causal B8 H8 T256 7 / 8 / 10 -> 7 / 7 / 9            B4 H8 T1100 32 / 37 / 47 -> 25 / 29 / 33
+constexpr bool small_takes_parts(int mask_id, long long band_keys, long long heads, long long kv_heads, int T, int D, int dtype) {
+    return f32_parts_serve(D, dtype) && (D < 32 || (T >= (D == 32 ? 257 : 1024) && band_keys >= 256)) &&
+           fwd_takes_small(mask_id, heads, T, D, dtype) && bwd_takes_small(mask_id, heads, T, D, dtype, CHILL_PASS_DQ) &&
+           bwd_takes_small(mask_id, kv_heads, T, D, dtype, CHILL_PASS_DKDV);
 }
 
 constexpr TileConfig fwd_tile_config(int mask_id, int D, int dtype, int T = kLongSequence) {
