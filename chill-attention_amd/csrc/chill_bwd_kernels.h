@@ -106,6 +106,7 @@ __device__ __forceinline__ void softmax_grad_block(f32x16& s, f32x16& dp, float 
 }  // namespace chill
 #include "chill_bwd_small.h"
 #include "chill_f32_bwd_small.h"
+#include "chill_f32_group.h"
 namespace chill {
 
 // ------------------------------------------------------------------------------------------ dQ
@@ -434,27 +435,29 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     bool sets = false;
     void (*kern)(BwdParams, int, int, int) = nullptr;
     if constexpr (f32_parts_serve(D, DT)) {
-        if (small_takes_parts(MASK_ID, band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
+        if (f32_takes_parts(band, (long long)p.B * p.H_kv, p.T, D, DT)) {
             if constexpr (PASS == 1)
                 kern = two ? dq_small_f32_kernel<D, MASK_ID, 2> : dq_small_f32_kernel<D, MASK_ID, 1>;
             else
                 kern = dkdv_small_f32_kernel<D, MASK_ID>;
         }
     }
-    if (kern == nullptr) {
-        if constexpr (PASS == 1)
-            kern = dq_small_kernel<E, D, MASK_ID, 1, 1>;
-        else
-            kern = dkdv_small_kernel<E, D, MASK_ID, 1>;
-        if constexpr (kDouble) {
-            if constexpr (Elem<E>::k16)
-                sets = small_takes_two_sets(MASK_ID, DT, PASS == 1 ? CHILL_PASS_DQ : CHILL_PASS_DKDV, tiles, p.T, band);
-            if constexpr (PASS == 1) {
-                if (two) kern = dq_small_kernel<E, D, MASK_ID, 2, 1>;
+    if constexpr (!f32_all_parts(D, DT)) {
+        if (kern == nullptr) {
+            if constexpr (PASS == 1)
+                kern = dq_small_kernel<E, D, MASK_ID, 1, 1>;
+            else
+                kern = dkdv_small_kernel<E, D, MASK_ID, 1>;
+            if constexpr (kDouble) {
                 if constexpr (Elem<E>::k16)
-                    if (sets) kern = dq_small_kernel<E, D, MASK_ID, 1, 2>;
-            } else {
-                if (sets) kern = dkdv_small_kernel<E, D, MASK_ID, 2>;
+                    sets = small_takes_two_sets(MASK_ID, DT, PASS == 1 ? CHILL_PASS_DQ : CHILL_PASS_DKDV, tiles, p.T, band);
+                if constexpr (PASS == 1) {
+                    if (two) kern = dq_small_kernel<E, D, MASK_ID, 2, 1>;
+                    if constexpr (Elem<E>::k16)
+                        if (sets) kern = dq_small_kernel<E, D, MASK_ID, 1, 2>;
+                } else {
+                    if (sets) kern = dkdv_small_kernel<E, D, MASK_ID, 2>;
+                }
             }
         }
     }
@@ -468,6 +471,27 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     }
     hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two || sets ? 2 : 1)), lds_bytes, stream, p, n_tiles, total,
                        hfb ? 1 : 0);
+    return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
+}
+
+// fp32 that fills the chip, products through bf16 parts: dQ or dK/dV.
+template <int D, int MASK_ID, int PASS>
+int launch_bwd_group(const BwdParams& p, hipStream_t stream) {
+    constexpr TileConfig cfg = f32_group_tile_config(D, PASS);
+    const int n_tiles = cdiv(p.T, cfg.rows);
+    const int64_t total = (int64_t)p.B * (PASS == CHILL_PASS_DQ ? p.H : p.H_kv) * n_tiles;
+    if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
+    void (*kern)(BwdParams, int, int);
+    if constexpr (PASS == CHILL_PASS_DQ)
+        kern = dq_group_f32_kernel<D, MASK_ID>;
+    else
+        kern = dkdv_group_f32_kernel<D, MASK_ID>;
+    const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
+    if (cfg.lds_bytes > 48 * 1024) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, cfg.lds_bytes) != hipSuccess)
+            return CHILL_ERR_HIP;
+    }
+    hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(cfg.waves * 64), cfg.lds_bytes, stream, p, n_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -488,8 +512,13 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
         if constexpr (served) small = bwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, Elem<E>::kDType, CHILL_PASS_DQ);
         bool regs2 = false;
         if constexpr (dq_regs2_is_optional(D, Elem<E>::kDType)) regs2 = dq_takes_regs2(MASK_ID, (long long)p.B * p.H, p.T);
-        if (small) {
+        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
+        if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
+        } else if (parts) {
+            if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DQ>(p, stream);
+        } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if (regs2) {
             if constexpr (dq_regs2_is_optional(D, Elem<E>::kDType)) status = launch_dq_regs2<E, D, MASK_ID>(p, stream);
         } else if constexpr (has_short_row) {
@@ -1449,8 +1478,13 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         bool regs = false;
         if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType))
             regs = dkdv_takes_regs(MASK_ID, p.margs.a0, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), D, (long long)p.B * p.H_kv, p.T);
-        if (small) {
+        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
+        if (small && !(parts && f32_takes_group((long long)p.B * p.H_kv, p.T))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 2>(p, stream);
+        } else if (parts) {
+            if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DKDV>(p, stream);
+        } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if (regs) {
             if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType)) status = launch_dkdv_shape<E, D, MASK_ID, false, true>(p, stream);
         } else if constexpr (has_small_row) {

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
         slots<6 * N>([&](auto i) {
             operand_slot(std::integral_constant<int, 6 * N + i>{});
 #pragma unroll
-            for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = fast_exp2(__builtin_fmaf(s[r], scale, -lse_q));
+            for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse_q);
             if constexpr (i == 6 * N - 3) kt[0] = Planes::transposed(planes, ofs, 0, 0, lane);
         });
 #pragma unroll
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
             f32x16 dp = native_rowwise<D>(vb, p.sv.t, seq_len - k0, doptr + (int64_t)qb * p.sdo.t, p.sdo.t, seq_len - qb, lane);
             mask(s, blk);
 #pragma unroll
-            for (int r = 0; r < 16; r++) dp[r] = fast_exp2(__builtin_fmaf(s[r], scale, -lse_q)) * (dp[r] - delta_q);
+            for (int r = 0; r < 16; r++) dp[r] = f32_probability(s[r], scale, lse_q) * (dp[r] - delta_q);
             native_transposed<D>(kb, p.sk.t, seq_len - k0, dp, dq, lane);
         }
         if (bad != bad) bwd_small_leave<DB>(mine, 0, dq, lane);
@@ -310,12 +310,12 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
         f32x16 s, dp = read_vec(32);  // (the dP chain starts from -delta)
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = 0.f;
-        // S and dP blocks: rows = queries 8 * (r / 4) + 4 * h + r % 4 of the block, column n = key.  Operand t, Q's and then
+        // S (rounded as in the forward) and dP blocks: rows = queries 8 * (r / 4) + 4 * h + r % 4 of the block, column n = key.  Operand t, Q's and then
         // dO's, in job[t % 2]; its successor is split behind its MFMAs
         auto operand_slot = [&](auto i_tag) {
             constexpr int i = decltype(i_tag)::value, t = i / 6, part = i % 6;
             if constexpr (t < N)
-                s = mma_part<part>(job[t % 2].p, k.p[t % N], s);
+                s = mma_part_transposed<part>(job[t % 2].p, k.p[t % N], s);
             else
                 dp = mma_part<part>(job[t % 2].p, v.p[t % N], dp);
             constexpr int u = t + 1;
@@ -345,14 +345,14 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
             operand_slot(std::integral_constant<int, 6 * N + i>{});
             if constexpr (N > 1) {
 #pragma unroll
-                for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = fast_exp2(__builtin_fmaf(s[r], scale, -lse[r]));
+                for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]);
                 if constexpr (i == 6 * N - 6) pj[0].x = half_of<0>(s);
                 if constexpr (i >= 6 * N - 6) pj[0].template share<i % 6>();
             }
         });
         if constexpr (N == 1) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) s[r] = fast_exp2(__builtin_fmaf(s[r], scale, -lse[r]));
+            for (int r = 0; r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]);
             pj[0].x = half_of<0>(s);
             pj[0].all();
         }
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
             mask(s, blk);
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                s[r] = fast_exp2(__builtin_fmaf(s[r], scale, -lse[r]));
+                s[r] = f32_probability(s[r], scale, lse[r]);
                 dp[r] = s[r] * (dp[r] + neg_delta[r]);
             }
             native_transposed<D>(dob, p.sdo.t, seq_len - q0, s, dv, lane);

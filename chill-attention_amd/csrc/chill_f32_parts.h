@@ -66,6 +66,12 @@ __device__ __forceinline__ f32x16 mma_part(const Parts& a, const Parts& b, f32x1
     return Elem<bf16_t>::mma(x, y, c);
 }
 
+// the same products in the same order with the operands exchanged: c is the transposed sum, bit by bit
+template <int K>
+__device__ __forceinline__ f32x16 mma_part_transposed(const Parts& a, const Parts& b, f32x16 c) {
+    return mma_part<K == 0 ? 1 : K == 1 ? 0 : K == 3 ? 4 : K == 4 ? 3 : K>(a, b, c);
+}
+
 // f(0), ..., f(N - 1), each left where it stands: one MFMA, and the vector and memory instructions that go behind it
 template <int N, typename F>
 __device__ __forceinline__ void slots(F&& f) {
@@ -154,6 +160,14 @@ __device__ __forceinline__ void mask_f32_block(f32x16& s, const Range& vis, int 
             s[r] = (q < seq_len && k < seq_len && Mask<MASK>::pred(q, k, seq_len, a)) ? s[r] : fill;
         }
     }
+}
+
+// P of a score: rounded after the scale as the forward does before it takes the largest as its reference, so that P of a row's
+// largest comes out of it as it went into LSE2 (fused, dV of scores up to 50 was off by 1.06 times what the fp32 instruction left)
+__device__ __forceinline__ float f32_probability(float s, float scale, float lse) {
+#pragma clang fp contract(off)
+    const float x = s * scale;
+    return fast_exp2(x - lse);
 }
 
 // NaN in the lanes of a row (n, 0), (n, 1) that has an accumulator that is infinite or NaN, 0 in the others

@@ -408,6 +408,7 @@ __device__ __forceinline__ void fwd_q_tile(const FwdParams& p, char* smem, int b
 #include "chill_fwd_fast.h"
 #include "chill_fwd_small.h"
 #include "chill_f32_fwd_small.h"
+#include "chill_f32_group.h"
 #include "chill_fwd_split.h"
 namespace chill {
 
@@ -582,17 +583,19 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     const bool sets = kDouble && small_takes_two_sets(MASK_ID, DT, CHILL_PASS_FWD, tiles, p.T, band);
     void (*kern)(FwdParams, int, int, int) = nullptr;
     if constexpr (f32_parts_serve(D, DT)) {
-        if (small_takes_parts(MASK_ID, band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
+        if (f32_takes_parts(band, (long long)p.B * p.H_kv, p.T, D, DT)) {
             kern = fwd_small_f32_kernel<D, MASK_ID, 1, 1>;
             if (two) kern = fwd_small_f32_kernel<D, MASK_ID, 2, 1>;
             if (sets) kern = fwd_small_f32_kernel<D, MASK_ID, 1, 2>;
         }
     }
-    if (kern == nullptr) {
-        kern = fwd_small_kernel<E, D, MASK_ID, 1, 1>;
-        if constexpr (kDouble) {
-            if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
-            if (sets) kern = fwd_small_kernel<E, D, MASK_ID, 1, 2>;
+    if constexpr (!f32_all_parts(D, DT)) {
+        if (kern == nullptr) {
+            kern = fwd_small_kernel<E, D, MASK_ID, 1, 1>;
+            if constexpr (kDouble) {
+                if (two) kern = fwd_small_kernel<E, D, MASK_ID, 2, 1>;
+                if (sets) kern = fwd_small_kernel<E, D, MASK_ID, 1, 2>;
+            }
         }
     }
     const int total = p.B * p.H * (two ? (n_q_tiles + 1) / 2 : n_q_tiles);
@@ -605,6 +608,19 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     }
     hipLaunchKernelGGL(kern, dim3(total), dim3(kFwdSmallWaves * 64 * (two || sets ? 2 : 1)), lds_bytes, stream, p, n_q_tiles, total,
                        hfb ? 1 : 0);
+    return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
+}
+
+// fp32 that fills the chip, products through bf16 parts.
+template <int D, int MASK_ID>
+int launch_fwd_group(const FwdParams& p, hipStream_t stream) {
+    constexpr TileConfig cfg = f32_group_tile_config(D, CHILL_PASS_FWD);
+    const int n_q_tiles = cdiv(p.T, cfg.rows);
+    const int64_t total = (int64_t)p.B * p.H * n_q_tiles;
+    if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
+    auto kern = fwd_group_f32_kernel<D, MASK_ID>;
+    const bool hfb = Mask<MASK_ID>::has_full_blocks(32, cfg.streamed, p.T, p.margs);
+    hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(cfg.waves * 64), cfg.lds_bytes, stream, p, n_q_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -626,8 +642,12 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
                                        fwd_tile_config(MASK_ID, D, Elem<E>::kDType).waves;
         bool small = false;
         if constexpr (D * Elem<E>::kBytes <= 512) small = fwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, Elem<E>::kDType);
+        constexpr bool parts = f32_parts_serve(D, Elem<E>::kDType);
         if (small) {
             if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, stream);
+        } else if (parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType)) {
+            if constexpr (parts) status = launch_fwd_group<D, MASK_ID>(p, stream);
+        } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if constexpr (has_short_row) {
             const bool short_row = fwd_takes_short_row(MASK_ID, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1),
                                                        (long long)p.B * p.H, p.T);

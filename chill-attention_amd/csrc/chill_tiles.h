@@ -255,21 +255,34 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
     return bwd_small_serves(D, dtype, pass) && T <= kFwdSmallMaxT * CHILL_TUNE_BWD_SMALL_SCALE &&
            batch_heads * ((T + 31) / 32) <= bwd_small_max_tiles(mask_id, T, D, dtype, pass) * CHILL_TUNE_BWD_SMALL_SCALE;
 }
-// Small fp32 launches whose products go through bf16 parts: all at head dim 16, at head dims 32 and 64 those of more than 256 and of
-// at least 1024 rows, bands of less than 256 keys aside, where all three passes are served by the small kernels.  A forward of short
-// rows ends before the splits of a wave's first operands are paid for, and the passes go together: P comes out of a score and an
-// LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both through the fp32 instruction, 2.0e-6 with
-// both through parts, 4.2e-6 with one of each).
-// Forward / dQ / dK/dV in us, fp32 instruction -> parts:
-//   D64 causal B2 H16 T512 18 / 25 / 35 -> 20 / 24 / 30      B1 H8 T1024 24 / 35 / 44 -> 24 / 27 / 31     B1 H4 T1111 25 / 38 / 47 -> 25 / 24 / 32
-//       B2 H16 T2048 166 / 228 / 347 -> 161 / 198 / 257      full mask B1 H8 T2048 76 / 103 / 154 -> 71 / 87 / 111
+// fp32 launches whose products go through bf16 parts: all at head dim 16; at head dims 32 and 64 those of more than 256 and of at least
+// 1024 rows, bands of less than 256 keys aside, and those of more than 2048 tiles of key / value heads, which no pass leaves to the
+// small kernels.  Below that a small forward ends before the splits of a wave's first operands are paid for, and the passes go
+// together: P comes out of a score and an LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both
+// through the fp32 instruction, 2.0e-6 with both through parts, 4.2e-6 with one of each).
+// Forward / dQ / dK/dV in us, fp32 instruction -> parts, in the kernels of few tiles (chill_f32_fwd_small.h, chill_f32_bwd_small.h):
+//   D64 causal B2 H16 T512 18 / 25 / 35 -> 20 / 24 / 30      B1 H8 T1024 24 / 35 / 44 -> 24 / 24 / 31     B1 H4 T1111 25 / 38 / 47 -> 25 / 24 / 32
+//       B2 H16 T2048 166 / 228 / 347 -> 157 / 197 / 251      full mask B1 H8 T2048 76 / 103 / 154 -> 71 / 87 / 109
 //       window 256 B1 H8 T2048 20 / 27 / 40 -> 20 / 25 / 33  window 100 + 30 B1 H4 T1111 10 / 15 / 17 -> 12 / 11 / 15
 //   D32 causal B8 H8 T256 9 / 12 / 13 -> 10 / 11 / 16        B1 H8 T512 9 / 12 / 15 -> 11 / 10 / 12       B1 H16 T1100 30 / 43 / 38 -> 30 / 32 / 35
 //   D16 causal B8 H8 T256 7 / 8 / 10 -> 7 / 7 / 9            B4 H8 T1100 32 / 37 / 47 -> 25 / 29 / 33
-constexpr bool small_takes_parts(int mask_id, long long band_keys, long long heads, long long kv_heads, int T, int D, int dtype) {
-    return f32_parts_serve(D, dtype) && (D < 32 || (T >= (D == 32 ? 257 : 1024) && band_keys >= 256)) &&
-           fwd_takes_small(mask_id, heads, T, D, dtype) && bwd_takes_small(mask_id, heads, T, D, dtype, CHILL_PASS_DQ) &&
-           bwd_takes_small(mask_id, kv_heads, T, D, dtype, CHILL_PASS_DKDV);
+// and in those that fill the chip (chill_f32_group.h):
+//   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 743 / 1000 / 1525   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
+//       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1442 / 1935 / 2900   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
+//   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 395 / 530 / 690   D16 498 / 552 / 886 -> 326 / 362 / 542
+constexpr long long kF32GroupTiles = 8 * kComputeUnits;
+constexpr bool f32_takes_group(long long heads, int T) { return heads * ((T + 31) / 32) > kF32GroupTiles; }
+constexpr bool f32_all_parts(int D, int dtype) { return f32_parts_serve(D, dtype) && D < 32; }
+constexpr bool f32_takes_parts(long long band_keys, long long kv_heads, int T, int D, int dtype) {
+    return f32_parts_serve(D, dtype) && (f32_all_parts(D, dtype) || (T >= (D == 32 ? 257 : 1024) && band_keys >= 256) || f32_takes_group(kv_heads, T));
+}
+// The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
+// dO with LSE2 and delta.  They take every launch that the small kernels do not, and of those launches the dQ and dK/dV of more than
+// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 1000 us, B4 H16 T2048 394 -> 270; dK/dV 498 -> 411; at 2048 tiles 197 -> 143 and
+// 251 -> 199, at 1024 103 -> 116 and 129 -> 166); the report then says the 32 rows of a tile, as it does of every small launch, and
+// the waves and the LDS of the workgroup, which holds four.
+constexpr TileConfig f32_group_tile_config(int D, int pass) {
+    return TileConfig{128, 32, 4, 2 * (2 * f32_planes_bytes(D) + (pass == CHILL_PASS_DKDV ? 2 * 32 * 4 : 0))};
 }
 
 constexpr TileConfig fwd_tile_config(int mask_id, int D, int dtype, int T = kLongSequence) {
@@ -508,11 +521,24 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 *out = small_tile_config(mask_id, dtype, pass, fwd_small_lds_bytes(D, dtype), batch_heads * ((T + 31) / 32), T, band_keys);
                 return CHILL_OK;
             }
+            if (f32_takes_parts(band_keys, batch_heads, T, D, dtype)) {
+                *out = f32_group_tile_config(D, pass);
+                return CHILL_OK;
+            }
             *out = fwd_tile_config(mask_id, D, dtype, fwd_takes_short_row(mask_id, band_keys, batch_heads, T) ? 1 : kLongSequence);
             return CHILL_OK;
         case CHILL_PASS_DQ:
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DQ)) {
+                if (f32_takes_parts(band_keys, batch_heads, T, D, dtype) && f32_takes_group(batch_heads, T)) {
+                    *out = f32_group_tile_config(D, pass);
+                    out->rows = 32;
+                    return CHILL_OK;
+                }
                 *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 1), batch_heads * ((T + 31) / 32), T, band_keys);
+                return CHILL_OK;
+            }
+            if (f32_takes_parts(band_keys, batch_heads, T, D, dtype)) {
+                *out = f32_group_tile_config(D, pass);
                 return CHILL_OK;
             }
             if (dq_regs2_is_optional(D, dtype) && (T == kLongSequence ? !mask_is_banded(mask_id) : dq_takes_regs2(mask_id, batch_heads, T))) {
@@ -524,7 +550,16 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
         case CHILL_PASS_DKDV:
             // (for this pass batch_heads counts the key / value heads)
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DKDV)) {
+                if (f32_takes_parts(band_keys, batch_heads, T, D, dtype) && f32_takes_group(batch_heads, T)) {
+                    *out = f32_group_tile_config(D, pass);
+                    out->rows = 32;
+                    return CHILL_OK;
+                }
                 *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 2), batch_heads * ((T + 31) / 32), T, band_keys);
+                return CHILL_OK;
+            }
+            if (f32_takes_parts(band_keys, batch_heads, T, D, dtype)) {
+                *out = f32_group_tile_config(D, pass);
                 return CHILL_OK;
             }
             {
