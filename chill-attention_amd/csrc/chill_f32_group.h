@@ -1,14 +1,14 @@
 // Forward, dQ and dK/dV of fp32 launches that fill the chip, with their matrix products through bf16 parts (chill_f32_parts.h).
 //
 // A workgroup owns 128 rows of a head (queries in the forward and dQ, keys in dK/dV), 32 a wave, and walks the 32-row blocks of the
-// other axis.  Its four waves share the splits of a block: each takes a quarter of the block's two tensors from global memory into
+// other axis.  Its four waves share the splits of a block: each takes a quarter of the block's rows from global memory into
 // registers two blocks ahead, splits it between the matrix instructions of the block before, and leaves the parts in LDS
 // (F32Planes), where every wave reads them row by row and transposed.  Two stages, one workgroup barrier a block.  The forward and
 // dQ fit in 256 registers, two workgroups a CU; dK/dV, with the parts of K and V and two accumulators, takes one wave a SIMD at
 // head dim 64.
-// What bounds it: issue.  At head dim 64 a block is 48, 72 and 96 MFMAs of 32 cycles and 300 to 400 vector instructions to a wave, which
-// hide behind the MFMAs in part: they are 49, 55 and 47 % of the time (causal B4 H16 T4096, 743 / 1000 / 1525 us; the fp32 instruction's
-// own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).
+// What bounds it: issue.  At head dim 64 a block is 48, 72 and 96 MFMAs of 32 cycles and 330 to 560 vector instructions to a wave, which
+// hide behind the MFMAs in part: those are 54, 65 and 48 % of the time (causal B4 H16 T4096, 704 / 936 / 1460 us; the fp32
+// instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).
 #pragma once
 
 #include "chill_device.h"
@@ -21,28 +21,30 @@ namespace chill {
 
 constexpr int kF32GroupWaves = 4;
 
-// A wave's quarter of the 2 N operands of a block: of two tensors of four operands each one, of fewer one of either (at head
-// dim 16 two waves do the same)
+// A thread's share of a block: eight columns of a row of both tensors, at head dims below 64 of one of them (at head dim 16 two
+// waves do the same).  Neighbouring lanes take neighbouring columns: whole rows from global memory and to LDS, where an operand's own
+// lanes, a row each, met in the banks for 25 cycles a write (causal D64 B4 H16 T4096 728 / 959 / 1495 -> 704 / 936 / 1460 us).
 template <int D>
 struct F32Share {
-    static constexpr int N = D / 16, JOBS = N > 2 ? N / 2 : 1;
+    static constexpr int N = D / 16, JOBS = N > 2 ? N / 2 : 1, CHUNKS = D / 8;
     typedef F32Planes<D> Planes;
-    bool second;    // (JOBS = 1: the wave's tensor)
-    int col, dst;   // first column of its operands, place of the lane's row in the planes of a tensor
+    bool second;        // (JOBS = 1: the wave's tensor)
+    int row, col, dst;  // row of the block, first column, their place in the planes of a tensor
     f32x4 x[JOBS][2];
     SplitJob job[JOBS];
-    __device__ __forceinline__ void init(int wave, int lane) {
-        static_assert(N <= kF32GroupWaves, "an operand a wave");
-        const int t = JOBS == 2 ? wave : wave % (2 * N);
-        second = t / N != 0;
-        col = 16 * (t % N) + 8 * (lane >> 5);
-        dst = (JOBS == 1 && second ? Planes::BYTES : 0) + Planes::L::chunk_off(lane & 31, 2 * (t % N) + (lane >> 5));
+    __device__ __forceinline__ void init(int tid) {
+        static_assert(JOBS * kF32GroupWaves * 64 >= 2 * 32 * CHUNKS && JOBS <= 2, "a share covers a block");
+        const int at = JOBS == 2 ? tid : tid % (2 * 32 * CHUNKS);
+        second = __builtin_amdgcn_readfirstlane(at / (32 * CHUNKS)) != 0;
+        row = at % (32 * CHUNKS) / CHUNKS;
+        col = 8 * (at % CHUNKS);
+        dst = (second ? Planes::BYTES : 0) + Planes::L::chunk_off(row, at % CHUNKS);
     }
-    // rows row0 + n of a and b (rows at and beyond `rows` repeat the last one)
+    // rows row0 .. row0 + 31 of a and b (rows at and beyond `rows` repeat the last one)
     template <int I>
-    __device__ __forceinline__ void load(const float* a, int64_t a_stride, const float* b, int64_t b_stride, int row0, int rows, int lane) {
+    __device__ __forceinline__ void load(const float* a, int64_t a_stride, const float* b, int64_t b_stride, int row0, int rows) {
         const bool other = JOBS == 2 ? I == 1 : second;
-        const float* src = (other ? b : a) + (int64_t)imin(row0 + (lane & 31), rows - 1) * (other ? b_stride : a_stride) + col;
+        const float* src = (other ? b : a) + (int64_t)imin(row0 + row, rows - 1) * (other ? b_stride : a_stride) + col;
         x[I][0] = *reinterpret_cast<const f32x4*>(src);
         x[I][1] = *reinterpret_cast<const f32x4*>(src + 4);
     }
@@ -132,8 +134,8 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     if (qw >= seq_len) wr.end = wr.start;
     const int last = imax(wg.end - 1, 0);
     F32Share<D> share;
-    share.init(wave, lane);
-    auto load = [&](auto i, int blk) { share.template load<i>(kptr, p.sk.t, vptr, p.sv.t, imin(blk, last) * 32, seq_len, lane); };
+    share.init(tid);
+    auto load = [&](auto i, int blk) { share.template load<i>(kptr, p.sk.t, vptr, p.sv.t, imin(blk, last) * 32, seq_len); };
     static_for<F32Share<D>::JOBS>([&](auto i) { load(i, wg.start); });
     F32Resident<D> q;
     {
@@ -290,8 +292,8 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     if (qw >= seq_len) wr.end = wr.start;
     const int last = imax(wg.end - 1, 0);
     F32Share<D> share;
-    share.init(wave, lane);
-    auto load = [&](auto i, int blk) { share.template load<i>(kptr, p.sk.t, vptr, p.sv.t, imin(blk, last) * 32, seq_len, lane); };
+    share.init(tid);
+    auto load = [&](auto i, int blk) { share.template load<i>(kptr, p.sk.t, vptr, p.sv.t, imin(blk, last) * 32, seq_len); };
     static_for<F32Share<D>::JOBS>([&](auto i) { load(i, wg.start); });
     const int q_pos = qw + n;
     F32Resident<D> q, d_o;
@@ -474,9 +476,9 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         }
     };
     F32Share<D> share;
-    share.init(wave, lane);
+    share.init(tid);
     auto load = [&](auto i) {
-        share.template load<i>(q0 + head_ahead * p.sq.h, p.sq.t, do0 + head_ahead * p.sdo.h, p.sdo.t, blk_ahead * 32, seq_len, lane);
+        share.template load<i>(q0 + head_ahead * p.sq.h, p.sq.t, do0 + head_ahead * p.sdo.h, p.sdo.t, blk_ahead * 32, seq_len);
     };
     // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows, through LDS (a row that attends to nothing has LSE2 = -inf and
     // only masked entries)

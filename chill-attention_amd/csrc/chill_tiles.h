@@ -267,9 +267,9 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 //   D32 causal B8 H8 T256 9 / 12 / 13 -> 10 / 11 / 16        B1 H8 T512 9 / 12 / 15 -> 11 / 10 / 12       B1 H16 T1100 30 / 43 / 38 -> 30 / 32 / 35
 //   D16 causal B8 H8 T256 7 / 8 / 10 -> 7 / 7 / 9            B4 H8 T1100 32 / 37 / 47 -> 25 / 29 / 33
 // and in those that fill the chip (chill_f32_group.h):
-//   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 743 / 1000 / 1525   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
-//       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1442 / 1935 / 2900   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
-//   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 395 / 530 / 690   D16 498 / 552 / 886 -> 326 / 362 / 542
+//   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 704 / 936 / 1460   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
+//       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1345 / 1792 / 2820   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
+//   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 383 / 512 / 704   D16 511 / 580 / 930 -> 321 / 382 / 597
 constexpr long long kF32GroupTiles = 8 * kComputeUnits;
 constexpr bool f32_takes_group(long long heads, int T) { return heads * ((T + 31) / 32) > kF32GroupTiles; }
 constexpr bool f32_all_parts(int D, int dtype) { return f32_parts_serve(D, dtype) && D < 32; }
@@ -278,7 +278,7 @@ constexpr bool f32_takes_parts(long long band_keys, long long kv_heads, int T, i
 }
 // The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
 // dO with LSE2 and delta.  They take every launch that the small kernels do not, and of those launches the dQ and dK/dV of more than
-// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 1000 us, B4 H16 T2048 394 -> 270; dK/dV 498 -> 411; at 2048 tiles 197 -> 143 and
+// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
 // 251 -> 199, at 1024 103 -> 116 and 129 -> 166); the report then says the 32 rows of a tile, as it does of every small launch, and
 // the waves and the LDS of the workgroup, which holds four.
 constexpr TileConfig f32_group_tile_config(int D, int pass) {
