@@ -512,9 +512,9 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
         if constexpr (served) small = bwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, Elem<E>::kDType, CHILL_PASS_DQ);
         bool regs2 = false;
         if constexpr (dq_regs2_is_optional(D, Elem<E>::kDType)) regs2 = dq_takes_regs2(MASK_ID, (long long)p.B * p.H, p.T);
-        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        constexpr bool served_by_parts = f32_group_serves(D, Elem<E>::kDType);
         const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
-        if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T))) {
+        if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
         } else if (parts) {
             if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DQ>(p, stream);
@@ -1478,9 +1478,9 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         bool regs = false;
         if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType))
             regs = dkdv_takes_regs(MASK_ID, p.margs.a0, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), D, (long long)p.B * p.H_kv, p.T);
-        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        constexpr bool served_by_parts = f32_group_serves(D, Elem<E>::kDType);
         const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
-        if (small && !(parts && f32_takes_group((long long)p.B * p.H_kv, p.T))) {
+        if (small && !(parts && f32_takes_group((long long)p.B * p.H_kv, p.T, D))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 2>(p, stream);
         } else if (parts) {
             if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DKDV>(p, stream);

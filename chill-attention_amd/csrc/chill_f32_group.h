@@ -4,11 +4,14 @@
 // other axis.  Its four waves share the splits of a block: each takes a quarter of the block's rows from global memory into
 // registers two blocks ahead, splits it between the matrix instructions of the block before, and leaves the parts in LDS
 // (F32Planes), where every wave reads them row by row and transposed.  Two stages, one workgroup barrier a block.  The forward and
-// dQ fit in 256 registers, two workgroups a CU; dK/dV, with the parts of K and V and two accumulators, takes one wave a SIMD at
-// head dim 64.
+// dQ fit in 256 registers, two workgroups a CU; dK/dV at head dim 64, with the parts of K and V and two accumulators, takes one wave a
+// SIMD, and so does everything at head dim 128, where the two stages are 96 KiB of LDS: 352 and 416 registers in the forward and dQ, all 512
+// and 15 to 31 spilled around the loop in dK/dV.
 // What bounds it: issue.  At head dim 64 a block is 48, 72 and 96 MFMAs of 32 cycles and 330 to 560 vector instructions to a wave, which
 // hide behind the MFMAs in part: those are 54, 65 and 48 % of the time (causal B4 H16 T4096, 704 / 936 / 1460 us; the fp32
-// instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).
+// instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).  At head dim 128 (the same sizes, 2427 / 3757 / 5406 -> 1787 /
+// 2259 / 3295 us) it is 96, 144 and 192 MFMAs, 37, 44 and 40 % of the time at 2.4 GHz: a wave
+// has its SIMD to itself.
 #pragma once
 
 #include "chill_device.h"
@@ -27,15 +30,16 @@ constexpr int kF32GroupWaves = 4;
 template <int D>
 struct F32Share {
     static constexpr int N = D / 16, JOBS = N > 2 ? N / 2 : 1, CHUNKS = D / 8;
+    static constexpr int HALVES = JOBS > 2 ? 2 : 1;  // at head dim 128 jobs 2 t and 2 t + 1 are rows 0 .. 15 and 16 .. 31 of a tensor
     typedef F32Planes<D> Planes;
     bool second;        // (JOBS = 1: the wave's tensor)
     int row, col, dst;  // row of the block, first column, their place in the planes of a tensor
     f32x4 x[JOBS][2];
     SplitJob job[JOBS];
     __device__ __forceinline__ void init(int tid) {
-        static_assert(JOBS * kF32GroupWaves * 64 >= 2 * 32 * CHUNKS && JOBS <= 2, "a share covers a block");
-        const int at = JOBS == 2 ? tid : tid % (2 * 32 * CHUNKS);
-        second = __builtin_amdgcn_readfirstlane(at / (32 * CHUNKS)) != 0;
+        static_assert(JOBS * kF32GroupWaves * 64 >= 2 * 32 * CHUNKS && JOBS <= 4, "a share covers a block");
+        const int at = JOBS >= 2 ? tid : tid % (2 * 32 * CHUNKS);
+        second = JOBS == 1 && __builtin_amdgcn_readfirstlane(at / (32 * CHUNKS)) != 0;
         row = at % (32 * CHUNKS) / CHUNKS;
         col = 8 * (at % CHUNKS);
         dst = (second ? Planes::BYTES : 0) + Planes::L::chunk_off(row, at % CHUNKS);
@@ -43,8 +47,8 @@ struct F32Share {
     // rows row0 .. row0 + 31 of a and b (rows at and beyond `rows` repeat the last one)
     template <int I>
     __device__ __forceinline__ void load(const float* a, int64_t a_stride, const float* b, int64_t b_stride, int row0, int rows) {
-        const bool other = JOBS == 2 ? I == 1 : second;
-        const float* src = (other ? b : a) + (int64_t)imin(row0 + row, rows - 1) * (other ? b_stride : a_stride) + col;
+        const bool other = JOBS >= 2 ? I / HALVES == 1 : second;
+        const float* src = (other ? b : a) + (int64_t)imin(row0 + row + 16 * (I % HALVES), rows - 1) * (other ? b_stride : a_stride) + col;
         x[I][0] = *reinterpret_cast<const f32x4*>(src);
         x[I][1] = *reinterpret_cast<const f32x4*>(src + 4);
     }
@@ -55,7 +59,9 @@ struct F32Share {
     template <int I, int PART>
     __device__ __forceinline__ void write(char* stage) const {
         const Parts& p = job[I].p;
-        *reinterpret_cast<i32x4*>(stage + I * Planes::BYTES + PART * Planes::PLANE + dst) = PART == 0 ? p.h : PART == 1 ? p.m : p.l;
+        static_assert(HALVES == 1 || OperandOffsets<bf16_t, D>::kHalfAffine, "16 rows further the swizzle is the same");
+        constexpr int half = (I % HALVES) * 16 * D * 2;
+        *reinterpret_cast<i32x4*>(stage + I / HALVES * Planes::BYTES + PART * Planes::PLANE + half + dst) = PART == 0 ? p.h : PART == 1 ? p.m : p.l;
     }
     template <typename Load>
     __device__ __forceinline__ void at_once(char* stage, Load&& load_next) {
@@ -96,7 +102,7 @@ __device__ __forceinline__ void clear_f32_blocks(f32x16 (&acc)[N]) {
 
 // ------------------------------------------------------------------------------------------ forward
 template <int D, int MASK>
-__global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void fwd_group_f32_kernel(FwdParams p, int n_q_tiles, int has_full_blocks) {
+__global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_per_eu(D < 128 ? 2 : 1))) void fwd_group_f32_kernel(FwdParams p, int n_q_tiles, int has_full_blocks) {
     constexpr int TQ = kF32GroupWaves * 32, NT = kF32GroupWaves * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
     constexpr int STAGE = 2 * Planes::BYTES;  // K, V
@@ -214,13 +220,32 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             pj[0].all();
             __builtin_amdgcn_sched_barrier(0);
             // O^T += V^T P^T; the second half of P is split beside it
-            slots<12 * DB>([&](auto i) {
-                constexpr int step = i / 6, part = i % 6, half = step / DB, db = step % DB;
-                if constexpr (part == 0 && step + 1 < 2 * DB)
-                    v[(step + 1) % 2] = Planes::transposed(v_planes, ofs, (step + 1) / DB, (step + 1) % DB, lane);
-                o[db] = mma_part<part>(v[step % 2], pj[half].p, o[db]);
-                if constexpr (step == 0) pj[1].template share<part>();
-            });
+            if constexpr (D == 128) {
+                // (a block's share of O added up by itself, as in dQ: the launches of 1024 tiles and more whose keys were shared by four
+                // waves had sums a quarter as long.  Full mask B1 H4 T8192 against 64 bits, relative: four sums 7.9e-7, one 14.2e-7, this 3.6e-7)
+                static_for<DB>([&](auto db) {
+                    f32x16 sum;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) sum[r] = 0.f;
+                    slots<12>([&](auto i) {
+                        constexpr int half = i / 6, step = 2 * db + half, part = i % 6;
+                        if constexpr (part == 0 && step + 1 < 2 * DB)
+                            v[(step + 1) % 2] = Planes::transposed(v_planes, ofs, (step + 1) % 2, (step + 1) / 2, lane);
+                        sum = mma_part<part>(v[step % 2], pj[half].p, sum);
+                        if constexpr (step == 0) pj[1].template share<part>();
+                    });
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[db][r] += sum[r];
+                });
+            } else {
+                slots<12 * DB>([&](auto i) {
+                    constexpr int step = i / 6, part = i % 6, half = step / DB, db = step % DB;
+                    if constexpr (part == 0 && step + 1 < 2 * DB)
+                        v[(step + 1) % 2] = Planes::transposed(v_planes, ofs, (step + 1) / DB, (step + 1) % DB, lane);
+                    o[db] = mma_part<part>(v[step % 2], pj[half].p, o[db]);
+                    if constexpr (step == 0) pj[1].template share<part>();
+                });
+            }
         } else {
             share.at_once(next, load_next);
         }
@@ -253,7 +278,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
 
 // ------------------------------------------------------------------------------------------ dQ
 template <int D, int MASK>
-__global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void dq_group_f32_kernel(BwdParams p, int n_q_tiles, int has_full_blocks) {
+__global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_per_eu(D < 128 ? 2 : 1))) void dq_group_f32_kernel(BwdParams p, int n_q_tiles, int has_full_blocks) {
     constexpr int TQ = kF32GroupWaves * 32, NT = kF32GroupWaves * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
     constexpr int STAGE = 2 * Planes::BYTES;  // K, V

@@ -619,6 +619,10 @@ int launch_fwd_group(const FwdParams& p, hipStream_t stream) {
     const int64_t total = (int64_t)p.B * p.H * n_q_tiles;
     if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
     auto kern = fwd_group_f32_kernel<D, MASK_ID>;
+    if (cfg.lds_bytes > 48 * 1024) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, cfg.lds_bytes) != hipSuccess)
+            return CHILL_ERR_HIP;
+    }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, cfg.streamed, p.T, p.margs);
     hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(cfg.waves * 64), cfg.lds_bytes, stream, p, n_q_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
@@ -642,11 +646,12 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
                                        fwd_tile_config(MASK_ID, D, Elem<E>::kDType).waves;
         bool small = false;
         if constexpr (D * Elem<E>::kBytes <= 512) small = fwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, Elem<E>::kDType);
-        constexpr bool parts = f32_parts_serve(D, Elem<E>::kDType);
-        if (small) {
+        constexpr bool served_by_parts = f32_group_serves(D, Elem<E>::kDType);
+        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
+        if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
             if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, stream);
-        } else if (parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType)) {
-            if constexpr (parts) status = launch_fwd_group<D, MASK_ID>(p, stream);
+        } else if (parts) {
+            if constexpr (served_by_parts) status = launch_fwd_group<D, MASK_ID>(p, stream);
         } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if constexpr (has_short_row) {
             const bool short_row = fwd_takes_short_row(MASK_ID, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1),

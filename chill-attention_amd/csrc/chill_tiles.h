@@ -255,7 +255,8 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
     return bwd_small_serves(D, dtype, pass) && T <= kFwdSmallMaxT * CHILL_TUNE_BWD_SMALL_SCALE &&
            batch_heads * ((T + 31) / 32) <= bwd_small_max_tiles(mask_id, T, D, dtype, pass) * CHILL_TUNE_BWD_SMALL_SCALE;
 }
-// fp32 launches whose products go through bf16 parts: all at head dim 16; at head dims 32 and 64 those of more than 256 and of at least
+// fp32 launches whose products go through bf16 parts: all at head dim 16; at head dim 128 those of at least 1024 tiles of key / value
+// heads; at head dims 32 and 64 those of more than 256 and of at least
 // 1024 rows, bands of less than 256 keys aside, and those of more than 2048 tiles of key / value heads, which no pass leaves to the
 // small kernels.  Below that a small forward ends before the splits of a wave's first operands are paid for, and the passes go
 // together: P comes out of a score and an LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both
@@ -270,15 +271,22 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 //   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 704 / 936 / 1460   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
 //       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1345 / 1792 / 2820   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
 //   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 383 / 512 / 704   D16 511 / 580 / 930 -> 321 / 382 / 597
-constexpr long long kF32GroupTiles = 8 * kComputeUnits;
-constexpr bool f32_takes_group(long long heads, int T) { return heads * ((T + 31) / 32) > kF32GroupTiles; }
+//   D128 causal B4 H16 T4096 2427 / 3757 / 5406 -> 1787 / 2259 / 3295   B1 H32 T2048 326 / 520 / 708 -> 270 / 356 / 415   B8 H32 T300 129 / 229 / 218 -> 93 / 122 / 144
+//       window 100 + 30 B8 H32 T800 478 / 509 / 679 -> 255 / 345 / 459   16 + 16 B8 H8 T3000 285 / 347 / 449 -> 169 / 232 / 309
+//       grouped heads B4 H32/8 T2085 1498 / 2154 / 3093 -> 1018 / 1307 / 1843
+//   D128 of 1024 tiles: causal B1 H16 T2048 202 / 279 / 667 -> 198 / 255 / 361   B1 H4 T8192 672 / 908 / 2536 -> 674 / 875 / 1270   B8 H32 T128 46 / 71 / 56 -> 24 / 33 / 43
+//       full mask B1 H16 T2048 368 / 501 / 703 -> 242 / 313 / 417   of 768: causal B1 H12 T2048 155 / 213 / 637 -> 180 / 234 / 334
+constexpr bool f32_group_serves(int D, int dtype) { return dtype == CHILL_F32 && D <= 128; }
+constexpr long long f32_group_tiles(int D) { return D == 128 ? 4 * kComputeUnits - 1 : 8 * kComputeUnits; }
+constexpr bool f32_takes_group(long long heads, int T, int D) { return heads * (((long long)T + 31) / 32) > f32_group_tiles(D); }
 constexpr bool f32_all_parts(int D, int dtype) { return f32_parts_serve(D, dtype) && D < 32; }
 constexpr bool f32_takes_parts(long long band_keys, long long kv_heads, int T, int D, int dtype) {
-    return f32_parts_serve(D, dtype) && (f32_all_parts(D, dtype) || (T >= (D == 32 ? 257 : 1024) && band_keys >= 256) || f32_takes_group(kv_heads, T));
+    if (f32_parts_serve(D, dtype) && (f32_all_parts(D, dtype) || (T >= (D == 32 ? 257 : 1024) && band_keys >= 256))) return true;
+    return f32_group_serves(D, dtype) && f32_takes_group(kv_heads, T, D);
 }
 // The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
-// dO with LSE2 and delta.  They take every launch that the small kernels do not, and of those launches the dQ and dK/dV of more than
-// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
+// dO with LSE2 and delta.  They take every launch that the small kernels do not, of those launches the dQ and dK/dV of more than
+// 2048 tiles too, and at head dim 128 all of at least 1024 (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
 // 251 -> 199, at 1024 103 -> 116 and 129 -> 166); the report then says the 32 rows of a tile, as it does of every small launch, and
 // the waves and the LDS of the workgroup, which holds four.
 constexpr TileConfig f32_group_tile_config(int D, int pass) {
@@ -515,13 +523,20 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                        int T, TileConfig* out) {
     if (dtype != CHILL_F32 && dtype != CHILL_F16 && dtype != CHILL_BF16) return CHILL_ERR_BAD_DTYPE;
     if (D != 16 && D != 32 && D != 64 && D != 128 && D != 256) return CHILL_ERR_BAD_HEAD_DIM;
+    // (the row of long sequences of fp32 at head dim 128 is that of the fp32 instruction, which the launches of few tiles take)
+    const bool takes_parts = f32_takes_parts(band_keys, batch_heads, T, D, dtype) && !(T == kLongSequence && D == 128);
     switch (pass) {
         case CHILL_PASS_FWD:
             if (T != kLongSequence && fwd_takes_small(mask_id, batch_heads, T, D, dtype)) {
+                if (takes_parts && f32_takes_group(batch_heads, T, D)) {
+                    *out = f32_group_tile_config(D, pass);
+                    out->rows = 32;
+                    return CHILL_OK;
+                }
                 *out = small_tile_config(mask_id, dtype, pass, fwd_small_lds_bytes(D, dtype), batch_heads * ((T + 31) / 32), T, band_keys);
                 return CHILL_OK;
             }
-            if (f32_takes_parts(band_keys, batch_heads, T, D, dtype)) {
+            if (takes_parts) {
                 *out = f32_group_tile_config(D, pass);
                 return CHILL_OK;
             }
@@ -529,7 +544,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
             return CHILL_OK;
         case CHILL_PASS_DQ:
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DQ)) {
-                if (f32_takes_parts(band_keys, batch_heads, T, D, dtype) && f32_takes_group(batch_heads, T)) {
+                if (takes_parts && f32_takes_group(batch_heads, T, D)) {
                     *out = f32_group_tile_config(D, pass);
                     out->rows = 32;
                     return CHILL_OK;
@@ -537,7 +552,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 1), batch_heads * ((T + 31) / 32), T, band_keys);
                 return CHILL_OK;
             }
-            if (f32_takes_parts(band_keys, batch_heads, T, D, dtype)) {
+            if (takes_parts) {
                 *out = f32_group_tile_config(D, pass);
                 return CHILL_OK;
             }
@@ -550,7 +565,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
         case CHILL_PASS_DKDV:
             // (for this pass batch_heads counts the key / value heads)
             if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DKDV)) {
-                if (f32_takes_parts(band_keys, batch_heads, T, D, dtype) && f32_takes_group(batch_heads, T)) {
+                if (takes_parts && f32_takes_group(batch_heads, T, D)) {
                     *out = f32_group_tile_config(D, pass);
                     out->rows = 32;
                     return CHILL_OK;
@@ -558,7 +573,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 2), batch_heads * ((T + 31) / 32), T, band_keys);
                 return CHILL_OK;
             }
-            if (f32_takes_parts(band_keys, batch_heads, T, D, dtype)) {
+            if (takes_parts) {
                 *out = f32_group_tile_config(D, pass);
                 return CHILL_OK;
             }
