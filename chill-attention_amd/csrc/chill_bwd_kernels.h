@@ -435,11 +435,14 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     bool sets = false;
     void (*kern)(BwdParams, int, int, int) = nullptr;
     if constexpr (f32_parts_serve(D, DT)) {
-        if (f32_takes_parts(band, (long long)p.B * p.H_kv, p.T, D, DT)) {
-            if constexpr (PASS == 1)
-                kern = two ? dq_small_f32_kernel<D, MASK_ID, 2> : dq_small_f32_kernel<D, MASK_ID, 1>;
-            else
+        if (f32_takes_parts(band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
+            if constexpr (PASS == 1) {
+                kern = dq_small_f32_kernel<D, MASK_ID, 1>;
+                if constexpr (kDouble)
+                    if (two) kern = dq_small_f32_kernel<D, MASK_ID, 2>;
+            } else {
                 kern = dkdv_small_f32_kernel<D, MASK_ID>;
+            }
         }
     }
     if constexpr (!f32_all_parts(D, DT)) {
@@ -512,8 +515,8 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
         if constexpr (served) small = bwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, Elem<E>::kDType, CHILL_PASS_DQ);
         bool regs2 = false;
         if constexpr (dq_regs2_is_optional(D, Elem<E>::kDType)) regs2 = dq_takes_regs2(MASK_ID, (long long)p.B * p.H, p.T);
-        constexpr bool served_by_parts = f32_group_serves(D, Elem<E>::kDType);
-        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
+        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
         if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
         } else if (parts) {
@@ -1478,8 +1481,8 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         bool regs = false;
         if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType))
             regs = dkdv_takes_regs(MASK_ID, p.margs.a0, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), D, (long long)p.B * p.H_kv, p.T);
-        constexpr bool served_by_parts = f32_group_serves(D, Elem<E>::kDType);
-        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
+        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
         if (small && !(parts && f32_takes_group((long long)p.B * p.H_kv, p.T, D))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 2>(p, stream);
         } else if (parts) {

@@ -16,7 +16,7 @@ namespace chill {
 
 // (TILES and SETS as in fwd_small_kernel)
 template <int D, int MASK, int TILES, int SETS>
-__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((amdgpu_waves_per_eu(2))) void fwd_small_f32_kernel(FwdParams p, int n_q_tiles, int total_items, int has_full_blocks) {
+__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((amdgpu_waves_per_eu(D < 128 ? 2 : 1))) void fwd_small_f32_kernel(FwdParams p, int n_q_tiles, int total_items, int has_full_blocks) {
     constexpr int NW = kFwdSmallWaves * SETS, NT = NW * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
     constexpr int WAVE_BYTES = fwd_small_wave_bytes(D, CHILL_F32);
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
         const int next = blk + NW < wr.end ? blk + NW : blk;
         const float* k_next = F32Rows<D>::at(kptr, p.sk.t, next * 32, seq_len, lane);
         const float* v_next = F32Rows<D>::at(vptr, p.sv.t, next * 32, seq_len, lane);
-        k.load_all(k_next);
+        if constexpr (D < 128) k.load_all(k_next);
         // S^T block: rows = keys 8 * (r / 4) + 4 * h + r % 4 of the block, column n = query row; V is split beside it
         f32x16 s;
 #pragma unroll
@@ -144,6 +144,9 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
             if constexpr (part == 0) vj[j % 2].x = v.template operand<j>();
             vj[j % 2].template share<part>();
             if constexpr (part == 2) v.template load<j>(v_next);
+            // (at head dim 128 into the registers of the operand that was due: no register is spilled, where 8 were under a causal mask, and
+            // a band of 256 + 256 took three times as long)
+            if constexpr (D == 128 && part == 5) k.template load<j>(k_next);
             if constexpr (j > 0 && part < 3) Planes::template write<j - 1, part>(mine, vj[(j + 1) % 2].p, lane);
         });
         static_for<3>([&](auto part) { Planes::template write<N - 1, part>(mine, vj[(N - 1) % 2].p, lane); });

@@ -583,10 +583,12 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     const bool sets = kDouble && small_takes_two_sets(MASK_ID, DT, CHILL_PASS_FWD, tiles, p.T, band);
     void (*kern)(FwdParams, int, int, int) = nullptr;
     if constexpr (f32_parts_serve(D, DT)) {
-        if (f32_takes_parts(band, (long long)p.B * p.H_kv, p.T, D, DT)) {
+        if (f32_takes_parts(band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
             kern = fwd_small_f32_kernel<D, MASK_ID, 1, 1>;
-            if (two) kern = fwd_small_f32_kernel<D, MASK_ID, 2, 1>;
-            if (sets) kern = fwd_small_f32_kernel<D, MASK_ID, 1, 2>;
+            if constexpr (kDouble) {
+                if (two) kern = fwd_small_f32_kernel<D, MASK_ID, 2, 1>;
+                if (sets) kern = fwd_small_f32_kernel<D, MASK_ID, 1, 2>;
+            }
         }
     }
     if constexpr (!f32_all_parts(D, DT)) {
@@ -646,8 +648,8 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
                                        fwd_tile_config(MASK_ID, D, Elem<E>::kDType).waves;
         bool small = false;
         if constexpr (D * Elem<E>::kBytes <= 512) small = fwd_takes_small(MASK_ID, (long long)p.B * p.H, p.T, D, Elem<E>::kDType);
-        constexpr bool served_by_parts = f32_group_serves(D, Elem<E>::kDType);
-        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
+        constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
+        const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
         if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
             if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, stream);
         } else if (parts) {

@@ -152,9 +152,9 @@ constexpr int kFwdSmallWaves = 4;
 // dK/dV 110 -> 76)
 constexpr int kFwdSmallMaxT = 16384;
 // (at the end the area also takes the wave's partial O^T, 4 KiB per 32 columns of the head dim)
-// (fp32 at head dims up to 64 has kernels of the same shape whose products go through bf16 parts, chill_f32_parts.h: their
-// areas hold the parts of one 32-row block of V, in dQ of K, which are smaller, in dK/dV of Q and of dO)
-constexpr bool f32_parts_serve(int D, int dtype) { return dtype == CHILL_F32 && D <= 64; }
+// (fp32 at head dims up to 128 has kernels of the same shape whose products go through bf16 parts, chill_f32_parts.h: their
+// areas hold the parts of one 32-row block of V, in dQ of K, which are smaller, in dK/dV, at head dims up to 64, of Q and of dO)
+constexpr bool f32_parts_serve(int D, int dtype) { return dtype == CHILL_F32 && D <= 128; }
 constexpr int f32_planes_bytes(int D) { return 3 * 32 * D * 2; }
 constexpr int fwd_small_wave_bytes(int D, int dtype) {
     const int blocks = 2 * 32 * D * elem_bytes(dtype), partial = ((D + 31) / 32) * 16 * 64 * 4;
@@ -255,16 +255,22 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
     return bwd_small_serves(D, dtype, pass) && T <= kFwdSmallMaxT * CHILL_TUNE_BWD_SMALL_SCALE &&
            batch_heads * ((T + 31) / 32) <= bwd_small_max_tiles(mask_id, T, D, dtype, pass) * CHILL_TUNE_BWD_SMALL_SCALE;
 }
-// fp32 launches whose products go through bf16 parts: all at head dim 16; at head dim 128 those of at least 1024 tiles of key / value
-// heads; at head dims 32 and 64 those of more than 256 and of at least
+// fp32 launches whose products go through bf16 parts: all at head dim 16; at head dims 32 and 64 those of more than 256 and of at least
 // 1024 rows, bands of less than 256 keys aside, and those of more than 2048 tiles of key / value heads, which no pass leaves to the
-// small kernels.  Below that a small forward ends before the splits of a wave's first operands are paid for, and the passes go
+// small kernels; at head dim 128 those of at least 1024 rows, or 512 with at most one tile a CU, bands of less than 512 keys aside, and
+// those of at least 1024 tiles.  Below that a small forward ends before the splits of a wave's first operands are paid for, and the passes go
 // together: P comes out of a score and an LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both
 // through the fp32 instruction, 2.0e-6 with both through parts, 4.2e-6 with one of each).
 // Forward / dQ / dK/dV in us, fp32 instruction -> parts, in the kernels of few tiles (chill_f32_fwd_small.h, chill_f32_bwd_small.h):
 //   D64 causal B2 H16 T512 18 / 25 / 35 -> 20 / 24 / 30      B1 H8 T1024 24 / 35 / 44 -> 24 / 24 / 31     B1 H4 T1111 25 / 38 / 47 -> 25 / 24 / 32
 //       B2 H16 T2048 166 / 228 / 347 -> 157 / 197 / 251      full mask B1 H8 T2048 76 / 103 / 154 -> 71 / 87 / 109
 //       window 256 B1 H8 T2048 20 / 27 / 40 -> 20 / 25 / 33  window 100 + 30 B1 H4 T1111 10 / 15 / 17 -> 12 / 11 / 15
+//   D128 (dK/dV in the kernel of launches that fill the chip, which is ahead however few tiles there are: the parts of Q and dO of four
+//        waves do not fit in LDS)   causal B1 H8 T512 26 / 37 / 167 -> 26 / 27 / 89   B1 H8 T1024 47 / 65 / 327 -> 42 / 44 / 167
+//       B1 H24 T1024 92 / 131 / 339 -> 90 / 98 / 182   B1 H8 T2048 98 / 136 / 633 -> 88 / 97 / 316   B1 H2 T8192 367 / 498 / 2536 -> 279 / 318 / 1253
+//       full mask B1 H8 T2048 177 / 242 / 643 -> 154 / 170 / 337   window 512 B1 H8 T4000 129 / 181 / 230 -> 123 / 134 / 139
+//       outside the rule, the forward: causal B1 H8 T256 15.9 -> 18.3   B4 H8 T512 37.1 -> 38.7   window 100 + 30 B1 H16 T1024 34.2 -> 37.8
+//       chunkwise 128, 2 B1 H8 T4001 85.4 -> 90.4
 //   D32 causal B8 H8 T256 9 / 12 / 13 -> 10 / 11 / 16        B1 H8 T512 9 / 12 / 15 -> 11 / 10 / 12       B1 H16 T1100 30 / 43 / 38 -> 30 / 32 / 35
 //   D16 causal B8 H8 T256 7 / 8 / 10 -> 7 / 7 / 9            B4 H8 T1100 32 / 37 / 47 -> 25 / 29 / 33
 // and in those that fill the chip (chill_f32_group.h):
@@ -275,19 +281,20 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 //       window 100 + 30 B8 H32 T800 478 / 509 / 679 -> 255 / 345 / 459   16 + 16 B8 H8 T3000 285 / 347 / 449 -> 169 / 232 / 309
 //       grouped heads B4 H32/8 T2085 1498 / 2154 / 3093 -> 1018 / 1307 / 1843
 //   D128 of 1024 tiles: causal B1 H16 T2048 202 / 279 / 667 -> 198 / 255 / 361   B1 H4 T8192 672 / 908 / 2536 -> 674 / 875 / 1270   B8 H32 T128 46 / 71 / 56 -> 24 / 33 / 43
-//       full mask B1 H16 T2048 368 / 501 / 703 -> 242 / 313 / 417   of 768: causal B1 H12 T2048 155 / 213 / 637 -> 180 / 234 / 334
-constexpr bool f32_group_serves(int D, int dtype) { return dtype == CHILL_F32 && D <= 128; }
+//       full mask B1 H16 T2048 368 / 501 / 703 -> 242 / 313 / 417
 constexpr long long f32_group_tiles(int D) { return D == 128 ? 4 * kComputeUnits - 1 : 8 * kComputeUnits; }
 constexpr bool f32_takes_group(long long heads, int T, int D) { return heads * (((long long)T + 31) / 32) > f32_group_tiles(D); }
 constexpr bool f32_all_parts(int D, int dtype) { return f32_parts_serve(D, dtype) && D < 32; }
-constexpr bool f32_takes_parts(long long band_keys, long long kv_heads, int T, int D, int dtype) {
-    if (f32_parts_serve(D, dtype) && (f32_all_parts(D, dtype) || (T >= (D == 32 ? 257 : 1024) && band_keys >= 256))) return true;
-    return f32_group_serves(D, dtype) && f32_takes_group(kv_heads, T, D);
+constexpr bool f32_takes_parts(long long band_keys, long long heads, long long kv_heads, int T, int D, int dtype) {
+    if (!f32_parts_serve(D, dtype)) return false;
+    if (f32_all_parts(D, dtype) || f32_takes_group(kv_heads, T, D)) return true;
+    if (D == 128) return band_keys >= 512 && (T >= 1024 || (T >= 512 && heads * ((T + 31) / 32) <= kComputeUnits));
+    return band_keys >= 256 && T >= (D == 32 ? 257 : 1024);
 }
 // The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
 // dO with LSE2 and delta.  They take every launch that the small kernels do not, of those launches the dQ and dK/dV of more than
-// 2048 tiles too, and at head dim 128 all of at least 1024 (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
-// 251 -> 199, at 1024 103 -> 116 and 129 -> 166); the report then says the 32 rows of a tile, as it does of every small launch, and
+// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
+// 251 -> 199, at 1024 103 -> 116 and 129 -> 166), and at head dim 128 all of at least 1024; the report then says the 32 rows of a tile, as it does of every small launch, and
 // the waves and the LDS of the workgroup, which holds four.
 constexpr TileConfig f32_group_tile_config(int D, int pass) {
     return TileConfig{128, 32, 4, 2 * (2 * f32_planes_bytes(D) + (pass == CHILL_PASS_DKDV ? 2 * 32 * 4 : 0))};
@@ -524,7 +531,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
     if (dtype != CHILL_F32 && dtype != CHILL_F16 && dtype != CHILL_BF16) return CHILL_ERR_BAD_DTYPE;
     if (D != 16 && D != 32 && D != 64 && D != 128 && D != 256) return CHILL_ERR_BAD_HEAD_DIM;
     // (the row of long sequences of fp32 at head dim 128 is that of the fp32 instruction, which the launches of few tiles take)
-    const bool takes_parts = f32_takes_parts(band_keys, batch_heads, T, D, dtype) && !(T == kLongSequence && D == 128);
+    const bool takes_parts = f32_takes_parts(band_keys, batch_heads, batch_heads, T, D, dtype) && !(T == kLongSequence && D == 128);
     switch (pass) {
         case CHILL_PASS_FWD:
             if (T != kLongSequence && fwd_takes_small(mask_id, batch_heads, T, D, dtype)) {

@@ -275,8 +275,9 @@ int chill_tile_config(int32_t mask_id, int32_t D, int32_t dtype, int32_t pass, i
  * as {32, 32, 4, lds_bytes}, lds_bytes being the workgroup's, which in the forward and dQ holds two such
  * blocks of eight waves in all when the launch has more blocks than the chip has CUs.  Where it has no more
  * and a row sees many streamed rows, eight waves split them: {32, 32, 8, lds_bytes}.
- * chill_tile_config reports the row of long sequences on a full chip (of fp32 at head dim 128 that of sequences too
- * long for the kernels of few blocks on a chip that is not full: from 1024 blocks on it takes another). */
+ * chill_tile_config reports the row of long sequences on a full chip (of fp32 at head dim 128 the row of narrow
+ * bands on grids of few blocks; other launches take another).  In fp32 a launch's kernels follow from H and from H_kv, and
+ * the report takes batch_heads for both. */
 int chill_tile_config_for_shape(int32_t mask_id, int32_t D, int32_t dtype, int32_t pass, int64_t batch_heads,
                                 int32_t T, int32_t out[4]);
 
