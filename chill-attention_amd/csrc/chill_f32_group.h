@@ -5,13 +5,12 @@
 // registers two blocks ahead, splits it between the matrix instructions of the block before, and leaves the parts in LDS
 // (F32Planes), where every wave reads them row by row and transposed.  Two stages, one workgroup barrier a block.  The forward and
 // dQ fit in 256 registers, two workgroups a CU; dK/dV at head dim 64, with the parts of K and V and two accumulators, takes one wave a
-// SIMD, and so does everything at head dim 128, where the two stages are 96 KiB of LDS: 352 and 416 registers in the forward and dQ, all 512
-// and 15 to 31 spilled around the loop in dK/dV.
+// SIMD, and so does everything at head dim 128, where the two stages are 96 KiB of LDS: 309, 425 and 510 registers in the three
+// kernels.
 // What bounds it: issue.  At head dim 64 a block is 48, 72 and 96 MFMAs of 32 cycles and 330 to 560 vector instructions to a wave, which
 // hide behind the MFMAs in part: those are 54, 65 and 48 % of the time (causal B4 H16 T4096, 704 / 936 / 1460 us; the fp32
-// instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).  At head dim 128 (the same sizes, 2427 / 3757 / 5406 -> 1787 /
-// 2259 / 3295 us) it is 96, 144 and 192 MFMAs, 37, 44 and 40 % of the time at 2.4 GHz: a wave
-// has its SIMD to itself.
+// instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).  At head dim 128 (the same sizes, 2414 / 3761 / 5432 -> 1632 /
+// 2144 / 2810 us) it is 96, 144 and 192 MFMAs, 40, 46 and 47 % of the time at 2.4 GHz: a wave has its SIMD to itself.
 #pragma once
 
 #include "chill_device.h"
