@@ -258,7 +258,7 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 // fp32 launches whose products go through bf16 parts: all at head dim 16; at head dims 32 and 64 those of more than 256 and of at least
 // 1024 rows, bands of less than 256 keys aside, and those of more than 2048 tiles of key / value heads, which no pass leaves to the
 // small kernels; at head dim 128 those of at least 1024 rows, or 512 with at most one tile a CU, bands of less than 512 keys aside, and
-// those of at least 1024 tiles.  Below that a small forward ends before the splits of a wave's first operands are paid for, and the passes go
+// those of at least 1024 tiles of query heads.  Below that a small forward ends before the splits of a wave's first operands are paid for, and the passes go
 // together: P comes out of a score and an LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both
 // through the fp32 instruction, 2.0e-6 with both through parts, 4.2e-6 with one of each).
 // Forward / dQ / dK/dV in us, fp32 instruction -> parts, in the kernels of few tiles (chill_f32_fwd_small.h, chill_f32_bwd_small.h):
@@ -266,9 +266,9 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 //       B2 H16 T2048 166 / 228 / 347 -> 157 / 197 / 251      full mask B1 H8 T2048 76 / 103 / 154 -> 71 / 87 / 109
 //       window 256 B1 H8 T2048 20 / 27 / 40 -> 20 / 25 / 33  window 100 + 30 B1 H4 T1111 10 / 15 / 17 -> 12 / 11 / 15
 //   D128 (dK/dV in the kernel of launches that fill the chip, which is ahead however few tiles there are: the parts of Q and dO of four
-//        waves do not fit in LDS)   causal B1 H8 T512 26 / 37 / 167 -> 26 / 27 / 89   B1 H8 T1024 47 / 65 / 327 -> 42 / 44 / 167
-//       B1 H24 T1024 92 / 131 / 339 -> 90 / 98 / 182   B1 H8 T2048 98 / 136 / 633 -> 88 / 97 / 316   B1 H2 T8192 367 / 498 / 2536 -> 279 / 318 / 1253
-//       full mask B1 H8 T2048 177 / 242 / 643 -> 154 / 170 / 337   window 512 B1 H8 T4000 129 / 181 / 230 -> 123 / 134 / 139
+//        waves do not fit in LDS)   causal B1 H8 T512 26 / 37 / 168 -> 25 / 27 / 80   B1 H8 T1024 47 / 66 / 329 -> 42 / 44 / 148
+//       B1 H24 T1024 92 / 131 / 339 -> 78 / 88 / 144   B1 H8 T2048 98 / 136 / 635 -> 85 / 94 / 276   B1 H2 T8192 368 / 496 / 2546 -> 262 / 303 / 1063
+//       full mask B1 H8 T2048 168 / 231 / 637 -> 155 / 167 / 306   window 256 + 256 B1 H4 T2048 35 / 47 / 212 -> 32 / 35 / 102
 //       outside the rule, the forward: causal B1 H8 T256 15.9 -> 18.3   B4 H8 T512 37.1 -> 38.7   window 100 + 30 B1 H16 T1024 34.2 -> 37.8
 //       chunkwise 128, 2 B1 H8 T4001 85.4 -> 90.4
 //   D32 causal B8 H8 T256 9 / 12 / 13 -> 10 / 11 / 16        B1 H8 T512 9 / 12 / 15 -> 11 / 10 / 12       B1 H16 T1100 30 / 43 / 38 -> 30 / 32 / 35
@@ -277,17 +277,17 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 //   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 704 / 936 / 1460   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
 //       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1345 / 1792 / 2820   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
 //   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 383 / 512 / 704   D16 511 / 580 / 930 -> 321 / 382 / 597
-//   D128 causal B4 H16 T4096 2427 / 3757 / 5406 -> 1787 / 2259 / 3295   B1 H32 T2048 326 / 520 / 708 -> 270 / 356 / 415   B8 H32 T300 129 / 229 / 218 -> 93 / 122 / 144
-//       window 100 + 30 B8 H32 T800 478 / 509 / 679 -> 255 / 345 / 459   16 + 16 B8 H8 T3000 285 / 347 / 449 -> 169 / 232 / 309
-//       grouped heads B4 H32/8 T2085 1498 / 2154 / 3093 -> 1018 / 1307 / 1843
-//   D128 of 1024 tiles: causal B1 H16 T2048 202 / 279 / 667 -> 198 / 255 / 361   B1 H4 T8192 672 / 908 / 2536 -> 674 / 875 / 1270   B8 H32 T128 46 / 71 / 56 -> 24 / 33 / 43
-//       full mask B1 H16 T2048 368 / 501 / 703 -> 242 / 313 / 417
+//   D128 causal B4 H16 T4096 2414 / 3761 / 5432 -> 1632 / 2144 / 2810   B1 H32 T2048 321 / 515 / 701 -> 246 / 331 / 352   B8 H32 T300 129 / 229 / 217 -> 87 / 116 / 125
+//       window 100 + 30 B8 H32 T800 475 / 507 / 675 -> 232 / 316 / 363   16 + 16 B8 H8 T3000 284 / 348 / 450 -> 162 / 224 / 261
+//       grouped heads B4 H32/8 T2085 1499 / 2159 / 3103 -> 963 / 1266 / 1543   B4 H32/4 T512 111 / 219 / 1271 -> 85 / 113 / 631
+//   D128 of 1024 tiles: causal B1 H16 T2048 197 / 271 / 652 -> 187 / 246 / 314   B1 H4 T8192 688 / 927 / 2561 -> 631 / 839 / 1089   B8 H32 T128 46 / 72 / 56 -> 22 / 31 / 36
+//       full mask B1 H16 T2048 366 / 495 / 697 -> 227 / 302 / 385
 constexpr long long f32_group_tiles(int D) { return D == 128 ? 4 * kComputeUnits - 1 : 8 * kComputeUnits; }
 constexpr bool f32_takes_group(long long heads, int T, int D) { return heads * (((long long)T + 31) / 32) > f32_group_tiles(D); }
 constexpr bool f32_all_parts(int D, int dtype) { return f32_parts_serve(D, dtype) && D < 32; }
 constexpr bool f32_takes_parts(long long band_keys, long long heads, long long kv_heads, int T, int D, int dtype) {
     if (!f32_parts_serve(D, dtype)) return false;
-    if (f32_all_parts(D, dtype) || f32_takes_group(kv_heads, T, D)) return true;
+    if (f32_all_parts(D, dtype) || f32_takes_group(D == 128 ? heads : kv_heads, T, D)) return true;
     if (D == 128) return band_keys >= 512 && (T >= 1024 || (T >= 512 && heads * ((T + 31) / 32) <= kComputeUnits));
     return band_keys >= 256 && T >= (D == 32 ? 257 : 1024);
 }
