@@ -87,6 +87,14 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
     ofs.init(lane);
     char* mine = smem + wave * WAVE_BYTES;
     const lds_char* planes = (const lds_char*)mine;
+    // Two waves a SIMD have 256 registers each, 12 too few at head dim 64.  The low parts of dO lie in LDS, behind the planes: a register reloaded
+    // from scratch memory waits for every row of K and V requested before it (prefix-LM B1 H8 T2048
+    // 71.6 -> 67.7 us, causal B1 H2 T8192 217 -> 167; up to 4 are left)
+    constexpr bool kParked = TILES == 2 && D == 64;
+    constexpr int PARKED = 64 * 16;
+    static_assert(!kParked || Planes::BYTES + N * PARKED <= WAVE_BYTES, "room behind the planes");
+    if constexpr (kParked)
+        static_for<N>([&](auto j) { *reinterpret_cast<i32x4*>(mine + Planes::BYTES + j * PARKED + lane * 16) = d_o.p[j].l; });
 
     f32x16 dq[DB];
     auto clear = [&]() {
@@ -119,13 +127,18 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
         }
         // S^T and dP^T blocks: rows = keys 8 * (r / 4) + 4 * h + r % 4 of the block, column n = query row.  Operand t, K's and
         // then V's, in job[t % 2]; its successor is split behind its MFMAs
+        i32x4 low;
         auto operand_slot = [&](auto i_tag) {
             constexpr int i = decltype(i_tag)::value, t = i / 6, part = i % 6;
             if constexpr (t < N)
                 s = mma_part<part>(job[t % 2].p, q.p[t % N], s);
+            else if constexpr (kParked)
+                dp = mma_part<part>(job[t % 2].p, Parts{d_o.p[t % N].h, d_o.p[t % N].m, low}, dp);
             else
                 dp = mma_part<part>(job[t % 2].p, d_o.p[t % N], dp);
             constexpr int u = t + 1;
+            if constexpr (kParked && part == 2 && u >= N && u < 2 * N)
+                low = *reinterpret_cast<const lds_i32x4*>(planes + Planes::BYTES + (u - N) * PARKED + lane * 16);
             if constexpr (t == 0 && part == 0) kv.template load<0>(v_row);
             if constexpr (u < 2 * N) {
                 if constexpr (part == 0) job[u % 2].x = kv.template operand<u % N>();

@@ -615,18 +615,19 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
 
 // fp32 that fills the chip, products through bf16 parts.
 template <int D, int MASK_ID>
-int launch_fwd_group(const FwdParams& p, hipStream_t stream) {
+int launch_fwd_group(const FwdParams& p, bool small, hipStream_t stream) {
     constexpr TileConfig cfg = f32_group_tile_config(D, CHILL_PASS_FWD);
     const int n_q_tiles = cdiv(p.T, cfg.rows);
     const int64_t total = (int64_t)p.B * p.H * n_q_tiles;
     if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
+    const int lds_bytes = f32_group_lds_bytes(D, CHILL_PASS_FWD, small);
     auto kern = fwd_group_f32_kernel<D, MASK_ID>;
-    if (cfg.lds_bytes > 48 * 1024) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, cfg.lds_bytes) != hipSuccess)
+    if (lds_bytes > 48 * 1024) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
             return CHILL_ERR_HIP;
     }
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, cfg.streamed, p.T, p.margs);
-    hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(cfg.waves * 64), cfg.lds_bytes, stream, p, n_q_tiles, hfb ? 1 : 0);
+    hipLaunchKernelGGL(kern, dim3(cdiv((int)total, 8) * 8), dim3(cfg.waves * 64), lds_bytes, stream, p, n_q_tiles, hfb ? 1 : 0);
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
@@ -653,7 +654,7 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
         if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
             if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, stream);
         } else if (parts) {
-            if constexpr (served_by_parts) status = launch_fwd_group<D, MASK_ID>(p, stream);
+            if constexpr (served_by_parts) status = launch_fwd_group<D, MASK_ID>(p, small, stream);
         } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if constexpr (has_short_row) {
             const bool short_row = fwd_takes_short_row(MASK_ID, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1),

@@ -299,6 +299,12 @@ constexpr bool f32_takes_parts(long long band_keys, long long heads, long long k
 constexpr TileConfig f32_group_tile_config(int D, int pass) {
     return TileConfig{128, 32, 4, 2 * (2 * f32_planes_bytes(D) + (pass == CHILL_PASS_DKDV ? 2 * 32 * 4 : 0))};
 }
+// What such a launch asks for: at head dim 128, where a workgroup has its CU to itself either way, the LDS that the small kernels of
+// the same launch would take, which is what the report says of it.
+constexpr int f32_group_lds_bytes(int D, int pass, bool small) {
+    if (!small || D != 128 || pass == CHILL_PASS_DKDV) return f32_group_tile_config(D, pass).lds_bytes;
+    return pass == CHILL_PASS_FWD ? fwd_small_lds_bytes(D, CHILL_F32) : bwd_small_lds_bytes(D, CHILL_F32, 1);
+}
 
 constexpr TileConfig fwd_tile_config(int mask_id, int D, int dtype, int T = kLongSequence) {
     const int waves = fwd_waves(mask_id, D, dtype, T);
@@ -538,6 +544,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 if (takes_parts && f32_takes_group(batch_heads, T, D)) {
                     *out = f32_group_tile_config(D, pass);
                     out->rows = 32;
+                    out->lds_bytes = f32_group_lds_bytes(D, pass, true);
                     return CHILL_OK;
                 }
                 *out = small_tile_config(mask_id, dtype, pass, fwd_small_lds_bytes(D, dtype), batch_heads * ((T + 31) / 32), T, band_keys);
@@ -554,6 +561,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 if (takes_parts && f32_takes_group(batch_heads, T, D)) {
                     *out = f32_group_tile_config(D, pass);
                     out->rows = 32;
+                    out->lds_bytes = f32_group_lds_bytes(D, pass, true);
                     return CHILL_OK;
                 }
                 *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 1), batch_heads * ((T + 31) / 32), T, band_keys);
@@ -575,6 +583,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                 if (takes_parts && f32_takes_group(batch_heads, T, D)) {
                     *out = f32_group_tile_config(D, pass);
                     out->rows = 32;
+                    out->lds_bytes = f32_group_lds_bytes(D, pass, true);
                     return CHILL_OK;
                 }
                 *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 2), batch_heads * ((T + 31) / 32), T, band_keys);
