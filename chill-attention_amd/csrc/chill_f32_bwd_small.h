@@ -62,7 +62,8 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
         rows.load_all(F32Rows<D>::at(doptr, p.sdo.t, qb, seq_len, lane));
         if (q_pos < p.T) lse_q = p.lse[b * p.lse_b + hd * p.lse_h + q_pos];
         if (p.delta_out != nullptr) {
-            // delta = rowsum(O * dO); every wave of the workgroup holds the same 32 rows, the first one writes
+            // delta = rowsum(O * dO), 0 for rows past the sequence (the rows here repeat the last one); every wave of the workgroup
+            // holds the same 32 rows, the first one writes
             F32Rows<D> out;
             const float* optr = reinterpret_cast<const float*>(p.o) + b * p.so.b + hd * p.so.h;
             out.load_all(F32Rows<D>::at(optr, p.so.t, qb, seq_len, lane));
@@ -71,6 +72,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
 #pragma unroll
                 for (int e = 0; e < 4; e++) delta_q += out.c[i][e] * rows.c[i][e];
             delta_q += __shfl_xor(delta_q, 32, 64);
+            if (q_pos >= seq_len) delta_q = 0.f;
             if (wave == 0 && h == 0 && q_pos < p.T) p.delta_out[b * p.delta_b + hd * p.delta_h + q_pos] = delta_q;
         } else if (q_pos < p.T) {
             delta_q = p.delta[b * p.delta_b + hd * p.delta_h + q_pos];
@@ -245,7 +247,8 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
         const int hq = hkv * p.group + it / n_blocks;
         return F32Rows<D>::at(reinterpret_cast<const float*>(p.d_o) + b * p.sdo.b + hq * p.sdo.h, p.sdo.t, (wr.start + it % n_blocks) * 32, seq_len, lane);
     };
-    // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the sequence read as zero
+    // LSE2 (lanes 0..31) and delta (lanes 32..63) of the block's rows; rows past the sequence repeat the last one, as those of Q and dO
+    // do (no key sees them)
     auto row_vec = [&](int it) {
         const int hq = hkv * p.group + it / n_blocks, q = (wr.start + it % n_blocks) * 32 + n;
         const float* src = h == 0 ? p.lse + b * p.lse_b + hq * p.lse_h : p.delta + b * p.delta_b + hq * p.delta_h;

@@ -892,6 +892,11 @@ DQ_DELTA_CASES = [
     ("f32-64", torch.float32, 64, 4, 12, 12, 1500, ("ChunkwiseChillMask", (64, 2)), (1500, 65, 1, 777), (128, 4, 32)),
     ("small-launch", torch.bfloat16, 64, 1, 2, 1, 300, ("CausalChillMask", ()), (129,), (32, 4, 32)),
     ("small-launch-f32", torch.float32, 32, 1, 3, 3, 257, ("FullChillMask", ()), None, (32, 4, 32)),
+    # (through bf16 parts: one tile a workgroup, two, the narrowest and the widest head; sequences that end within a tile)
+    ("small-launch-f32-parts", torch.float32, 64, 2, 2, 1, 1100, ("CausalChillMask", ()), (1001, 33), (32, 4, 32)),
+    ("small-launch-f32-parts-pairs", torch.float32, 64, 2, 6, 6, 1100, ("FullChillMask", ()), (1099, 40), (32, 4, 32)),
+    ("small-launch-f32-parts-16", torch.float32, 16, 2, 3, 1, 300, ("CausalChillMask", ()), (1, 290), (32, 4, 32)),
+    ("small-launch-f32-parts-128", torch.float32, 128, 2, 2, 2, 1030, ("CausalChillMask", ()), (1027, 513), (32, 4, 32)),
 ]
 
 
@@ -899,7 +904,7 @@ DQ_DELTA_CASES = [
 def test_dq_computes_delta_on_its_way(case):
     """chill_bwd_dq_delta (what the operator's backward launches before dK/dV) through the C ABI, on one shape per dQ
     kernel (route asserted from the tile table): the delta rows it leaves behind equal the closed form rowsum(O * dO)
-    in fp64 (utils.py:190) on every row below lens[b] and are finite on every other row (the buffer starts as NaN),
+    in fp64 (utils.py:190) on every row below lens[b] and are zero on every other row (the buffer starts as NaN),
     and its dQ equals what chill_bwd_dq computes from chill_bwd_delta's rows, up to the rounding of a sum of D
     products taken in another order."""
     import ctypes
@@ -945,6 +950,7 @@ def test_dq_computes_delta_on_its_way(case):
     for b in range(B):
         n = T if lens is None else lens[b]
         np.testing.assert_allclose(delta2[b, :, :n].cpu().numpy(), closed[b, :, :n], atol=2e-5 * D, rtol=1e-5)
+        assert (delta2[b, :, n:] == 0).all(), "delta behind the sequence"
     assert torch.isfinite(got).all()
     tol = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype]
     torch.testing.assert_close(got.float(), want.float(), atol=tol, rtol=tol)
