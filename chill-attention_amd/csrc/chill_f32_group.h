@@ -4,9 +4,10 @@
 // other axis.  Its four waves share the splits of a block: each takes a quarter of the block's rows from global memory into
 // registers two blocks ahead, splits it between the matrix instructions of the block before, and leaves the parts in LDS
 // (F32Planes), where every wave reads them row by row and transposed.  Two stages, one workgroup barrier a block.  The forward and
-// dQ fit in 256 registers, two workgroups a CU; dK/dV at head dim 64, with the parts of K and V and two accumulators, takes one wave a
-// SIMD, and so does everything at head dim 128, where the two stages are 96 KiB of LDS: 309, 425 and 510 registers in the three
-// kernels.
+// dQ (at head dim 64 with the low parts of dO in LDS) fit in 256 registers, two workgroups a CU; dK/dV at head dim 64, with the parts of
+// K and V and two accumulators, takes one wave a SIMD, and so does everything at head dim 128, where the two stages are 96 KiB of LDS:
+// 309, 425 and 510 registers in the three kernels.  dK/dV at head dim 16 spills 43 to 53 of 256, all but four of them around what it
+// leaves to the fp32 instruction, behind the loop.
 // What bounds it: issue.  At head dim 64 a block is 48, 72 and 96 MFMAs of 32 cycles and 330 to 560 vector instructions to a wave, which
 // hide behind the MFMAs in part: those are 54, 65 and 48 % of the time (causal B4 H16 T4096, 704 / 936 / 1460 us; the fp32
 // instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).  At head dim 128 (the same sizes, 2414 / 3761 / 5432 -> 1632 /
@@ -281,6 +282,11 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     constexpr int TQ = kF32GroupWaves * 32, NT = kF32GroupWaves * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
     constexpr int STAGE = 2 * Planes::BYTES;  // K, V
+    // Two waves a SIMD have 256 registers each, too few at head dim 64: the low parts of the wave's dO lie in LDS, behind the stages
+    // (5 to 7 registers were spilled in the loop
+    // otherwise; causal B8 H32 T300 49.5 -> 45.5 us, B32 H32 T128 52.1 -> 47.6, window 100 + 30 B8 H32 T800 127 -> 119, B4 H16 T4096 equal)
+    constexpr bool kParked = f32_group_parks(D);
+    constexpr int PARKED = 64 * 16;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int bh, qt;
     if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, 2, &bh, &qt)) return;
@@ -350,6 +356,8 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     if (lse_q == -INFINITY) lse_q = 0.f;
     OperandOffsets<bf16_t, D> ofs;
     ofs.init(lane);
+    char* parked = smem + 2 * STAGE + wave * N * PARKED + lane * 16;
+    if constexpr (kParked) static_for<N>([&](auto j) { *reinterpret_cast<i32x4*>(parked + j * PARKED) = d_o.p[j].l; });
 
     f32x16 dq[DB];
     clear_f32_blocks(dq);
@@ -377,11 +385,14 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             Parts x[2];
             x[0] = f32_row_operand<D>(k_planes, ofs, 0, lane);
             auto operand = [&](auto t) { x[t % 2] = f32_row_operand<D>(t < N ? k_planes : v_planes, ofs, t % N, lane); };
+            i32x4 low;
+            auto low_of = [&](auto j) { low = *reinterpret_cast<const lds_i32x4*>((const lds_char*)parked + j * PARKED); };
             slots<6 * N>([&](auto i) {
                 constexpr int t = i / 6, part = i % 6;
                 if constexpr (part == 0) operand(std::integral_constant<int, t + 1>{});
                 s = mma_part<part>(x[t % 2], q.p[t], s);
                 share.template slot<i>(next, load_next);
+                if constexpr (kParked && i == 6 * N - 4) low_of(std::integral_constant<int, 0>{});
             });
             mask(s, blk);
             constexpr int PER = (16 + 6 * N - 1) / (6 * N);  // exponentials a slot
@@ -393,7 +404,11 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
                     else
                         x[(t + 1) % 2] = Planes::transposed(k_planes, ofs, 0, 0, lane);
                 }
-                dp = mma_part<part>(x[t % 2], d_o.p[t - N], dp);
+                if constexpr (kParked)
+                    dp = mma_part<part>(x[t % 2], Parts{d_o.p[t - N].h, d_o.p[t - N].m, low}, dp);
+                else
+                    dp = mma_part<part>(x[t % 2], d_o.p[t - N], dp);
+                if constexpr (kParked && part == 2 && t + 1 < 2 * N) low_of(std::integral_constant<int, t + 1 - N>{});
 #pragma unroll
                 for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse_q);
             });

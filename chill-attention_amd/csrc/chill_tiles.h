@@ -296,8 +296,11 @@ constexpr bool f32_takes_parts(long long band_keys, long long heads, long long k
 // 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
 // 251 -> 199, at 1024 103 -> 116 and 129 -> 166), and at head dim 128 all of at least 1024; the report then says the 32 rows of a tile, as it does of every small launch, and
 // the waves and the LDS of the workgroup, which holds four.
+// (dQ at head dim 64: the low parts of dO, a thread's 16 bytes of each of four operands)
+constexpr bool f32_group_parks(int D) { return D == 64; }
 constexpr TileConfig f32_group_tile_config(int D, int pass) {
-    return TileConfig{128, 32, 4, 2 * (2 * f32_planes_bytes(D) + (pass == CHILL_PASS_DKDV ? 2 * 32 * 4 : 0))};
+    const int stage = 2 * f32_planes_bytes(D) + (pass == CHILL_PASS_DKDV ? 2 * 32 * 4 : 0);
+    return TileConfig{128, 32, 4, 2 * stage + (pass == CHILL_PASS_DQ && f32_group_parks(D) ? 4 * 64 * 16 * (D / 16) : 0)};
 }
 // What such a launch asks for: at head dim 128, where a workgroup has its CU to itself either way, the LDS that the small kernels of
 // the same launch would take, which is what the report says of it.
