@@ -57,6 +57,8 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
     F32Rows<D> kv;  // K of the block that is due, then its V, then the next block's K
     F32Resident<D> q, d_o;
     float lse_q = 0.f, delta_q = 0.f;
+    int lost = 0;  // (of K and V)
+    uint64_t lost_rows;
     {
         F32Rows<D> rows;
         rows.load_all(F32Rows<D>::at(doptr, p.sdo.t, qb, seq_len, lane));
@@ -77,11 +79,13 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
         } else if (q_pos < p.T) {
             delta_q = p.delta[b * p.delta_b + hd * p.delta_h + q_pos];
         }
-        d_o.split(rows);
+        d_o.split_scaled_up(rows);
         rows.load_all(F32Rows<D>::at(qptr, p.sq.t, qb, seq_len, lane));
         const int blk = imax(imin(first, wr.end - 1), 0);  // (a wave without blocks loads one all the same)
         kv.load_all(F32Rows<D>::at(kptr, p.sk.t, blk * 32, seq_len, lane));
-        q.split(rows);
+        int lost_q = 0;
+        q.split(rows, lost_q);
+        lost_rows = lanes_that_lost(lost_q);
     }
     // a row that attends to nothing has LSE2 = -inf and only masked entries (score -inf): P = exp2(-inf - 0)
     if (lse_q == -INFINITY) lse_q = 0.f;
@@ -116,7 +120,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
 
     SplitJob job[2];
     job[0].x = kv.template operand<0>();
-    job[0].all();
+    job[0].all(lost);
     for (int blk = first; blk < wr.end; blk += NW) {
         const int next = blk + NW < wr.end ? blk + NW : blk;
         const float* k_next = F32Rows<D>::at(kptr, p.sk.t, next * 32, seq_len, lane);
@@ -125,9 +129,9 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             s[r] = 0.f;
-            dp[r] = -delta_q;
+            dp[r] = -delta_q * kPartsUp;
         }
-        // S^T and dP^T blocks: rows = keys 8 * (r / 4) + 4 * h + r % 4 of the block, column n = query row.  Operand t, K's and
+        // S^T and, scaled up, dP^T blocks: rows = keys 8 * (r / 4) + 4 * h + r % 4 of the block, column n = query row.  Operand t, K's and
         // then V's, in job[t % 2]; its successor is split behind its MFMAs
         i32x4 low;
         auto operand_slot = [&](auto i_tag) {
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
             if constexpr (t == 0 && part == 0) kv.template load<0>(v_row);
             if constexpr (u < 2 * N) {
                 if constexpr (part == 0) job[u % 2].x = kv.template operand<u % N>();
-                job[u % 2].template share<part>();
+                job[u % 2].template share<part>(lost);
                 if constexpr (part == 5 && u == N) job[u % 2].pin();
                 // (what is due a phase later takes the place of the rows just split)
                 if constexpr (part == 2) kv.template load<u % N>(u < N ? v_row : k_next);
@@ -177,13 +181,15 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
             if constexpr (step == 0) job[1].template share<part>();
             if constexpr (step == DB) {
                 if constexpr (part == 0) job[0].x = kv.template operand<0>();
-                job[0].template share<part>();
+                job[0].template share<part>(lost);
             }
         });
     }
+    scale_f32_blocks(dq, kPartsDown);
     bwd_small_leave<DB>(mine, 0, dq, lane);
     const float bad = nan_if_not_finite(dq);
-    if (__builtin_amdgcn_ballot_w64(bad != bad) != 0) {
+    const bool again = bad != bad || row_that_lost(lost_rows, lane) || lanes_that_lost(lost) != 0;
+    if (__builtin_amdgcn_ballot_w64(again) != 0) {
         clear();
         for (int blk = first; blk < wr.end; blk += NW) {
             const int k0 = blk * 32;
@@ -195,7 +201,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
             for (int r = 0; r < 16; r++) dp[r] = f32_probability(s[r], scale, lse_q) * (dp[r] - delta_q);
             native_transposed<D>(kb, p.sk.t, seq_len - k0, dp, dq, lane);
         }
-        if (bad != bad) bwd_small_leave<DB>(mine, 0, dq, lane);
+        if (again) bwd_small_leave<DB>(mine, 0, dq, lane);
     }
     __syncthreads();
     float* const rows[1] = {dqbase + (int64_t)q_pos * p.sdq.t};
@@ -259,6 +265,8 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
     F32Rows<D> q, d_o;
     F32Resident<D> k, v;
     float vec_next = 0.f;
+    int lost = 0;  // (of Q and dO)
+    uint64_t lost_rows;
     {
         F32Rows<D> kr, vr;
         kr.load_all(F32Rows<D>::at(kptr, p.sk.t, 0, seq_len - kb0, lane));
@@ -268,8 +276,10 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
             d_o.load_all(do_rows(wave));
             vec_next = row_vec(wave);
         }
-        k.split(kr);
-        v.split(vr);
+        int lost_kv = 0;
+        k.split(kr, lost_kv);
+        v.split(vr, lost_kv);
+        lost_rows = lanes_that_lost(lost_kv);
     }
     const int k_pos = kb0 + n;
     const Range vis = visible_range<MASK, false>(k_pos, seq_len, p.margs);
@@ -315,7 +325,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
     SplitJob job[2];
     if (wave < n_iters) {
         job[0].x = q.template operand<0>();
-        job[0].all();
+        job[0].all(lost);
     }
     for (int it = wave; it < n_iters; it += NW) {
         const int blk = wr.start + it % n_blocks;
@@ -342,7 +352,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
                     else
                         job[u % 2].x = d_o.template operand<u % N>();
                 }
-                job[u % 2].template share<part>();
+                job[u % 2].template share<part>(lost);
                 if constexpr (part == 5 && u == N) job[u % 2].pin();
                 // (the rows of the next block take the place of those just split)
                 if constexpr (part == 2 && u < N) q.template load<u % N>(q_next);
@@ -354,21 +364,21 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
         slots<6 * N>([&](auto i) { operand_slot(i); });
         const f32x16 lse = read_vec(0);
         mask(s, blk);
-        // the exponentials of the first half of P in the first half of the dP chain, so that it can be split in the last step
+        // the exponentials (P, and with it dS, scaled up) of the first half of P in the first half of the dP chain, so that it can be split in the last step
         SplitJob pj[2];
         constexpr int PER = (16 + 6 * N - 7) / (6 * N - 6 > 0 ? 6 * N - 6 : 1);
         slots<6 * N>([&](auto i) {
             operand_slot(std::integral_constant<int, 6 * N + i>{});
             if constexpr (N > 1) {
 #pragma unroll
-                for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]);
+                for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]) * kPartsUp;
                 if constexpr (i == 6 * N - 6) pj[0].x = half_of<0>(s);
                 if constexpr (i >= 6 * N - 6) pj[0].template share<i % 6>();
             }
         });
         if constexpr (N == 1) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]);
+            for (int r = 0; r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]) * kPartsUp;
             pj[0].x = half_of<0>(s);
             pj[0].all();
         }
@@ -402,14 +412,17 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
             }
             if constexpr (w == 3 * DB) {
                 if constexpr (part == 0) job[0].x = q.template operand<0>();
-                job[0].template share<part>();
+                job[0].template share<part>(lost);
             }
         });
     }
+    scale_f32_blocks(dk, kPartsDown);
+    scale_f32_blocks(dv, kPartsDown);
     bwd_small_leave<DB>(mine, 0, dk, lane);
     bwd_small_leave<DB>(mine, DB, dv, lane);
     const float bad = nan_if_not_finite(dk, nan_if_not_finite(dv));
-    if (__builtin_amdgcn_ballot_w64(bad != bad) != 0) {
+    const bool again = bad != bad || row_that_lost(lost_rows, lane) || lanes_that_lost(lost) != 0;
+    if (__builtin_amdgcn_ballot_w64(again) != 0) {
         clear();
         for (int it = wave; it < n_iters; it += NW) {
             const int hq = hkv * p.group + it / n_blocks, blk = wr.start + it % n_blocks, q0 = blk * 32;
@@ -428,7 +441,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(Bwd
             native_transposed<D>(dob, p.sdo.t, seq_len - q0, s, dv, lane);
             native_transposed<D>(qb, p.sq.t, seq_len - q0, dp, dk, lane);
         }
-        if (bad != bad) {
+        if (again) {
             bwd_small_leave<DB>(mine, 0, dk, lane);
             bwd_small_leave<DB>(mine, DB, dv, lane);
         }

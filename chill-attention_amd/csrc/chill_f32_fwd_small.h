@@ -14,9 +14,10 @@
 
 namespace chill {
 
-// (TILES and SETS as in fwd_small_kernel)
+// (TILES and SETS as in fwd_small_kernel; at head dim 16 four waves a SIMD, 128 registers: with three, which the compiler would take,
+// causal B4 H8 T1100 is 29 us instead of 24)
 template <int D, int MASK, int TILES, int SETS>
-__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((amdgpu_waves_per_eu(D < 128 ? 2 : 1))) void fwd_small_f32_kernel(FwdParams p, int n_q_tiles, int total_items, int has_full_blocks) {
+__global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((amdgpu_waves_per_eu(D < 32 ? 4 : D < 128 ? 2 : 1))) void fwd_small_f32_kernel(FwdParams p, int n_q_tiles, int total_items, int has_full_blocks) {
     constexpr int NW = kFwdSmallWaves * SETS, NT = NW * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
     constexpr int WAVE_BYTES = fwd_small_wave_bytes(D, CHILL_F32);
@@ -61,13 +62,17 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
     const int first = wr.start + wave;
     F32Rows<D> k, v;
     F32Resident<D> q;
+    int lost = 0;  // (of K and V)
+    uint64_t lost_rows;
     {
         F32Rows<D> rows;
         rows.load_all(F32Rows<D>::at(qptr, p.sq.t, qb, seq_len, lane));
         const int blk = imax(imin(first, wr.end - 1), 0);  // (a wave without blocks loads one all the same)
         k.load_all(F32Rows<D>::at(kptr, p.sk.t, blk * 32, seq_len, lane));
         v.load_all(F32Rows<D>::at(vptr, p.sv.t, blk * 32, seq_len, lane));
-        q.split(rows);
+        int lost_q = 0;
+        q.split(rows, lost_q);
+        lost_rows = lanes_that_lost(lost_q);
     }
     OperandOffsets<bf16_t, D> ofs;
     ofs.init(lane);
@@ -126,7 +131,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
     SplitJob kj[N];  // K of the block that is due
     static_for<N>([&](auto j) {
         kj[j].x = k.template operand<j>();
-        kj[j].all();
+        kj[j].all(lost);
     });
     for (int blk = first; blk < wr.end; blk += NW) {
         const int next = blk + NW < wr.end ? blk + NW : blk;
@@ -142,7 +147,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
             constexpr int j = i / 6, part = i % 6;
             s = mma_part<part>(kj[j].p, q.p[j], s);
             if constexpr (part == 0) vj[j % 2].x = v.template operand<j>();
-            vj[j % 2].template share<part>();
+            vj[j % 2].template share<part>(lost);
             if constexpr (part == 2) v.template load<j>(v_next);
             // (at head dim 128 into the registers of the operand that was due: no register is spilled, where 8 were under a causal mask, and
             // a band of 256 + 256 took three times as long)
@@ -154,11 +159,11 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
         vt[0] = Planes::transposed(planes, ofs, 0, 0, lane);
         softmax(s, blk);
         SplitJob pj[2];
-        pj[0].x = half_of<0>(s);
-        pj[1].x = half_of<1>(s);
+        pj[0].x = half_of<0>(s) * kPartsUp;
+        pj[1].x = half_of<1>(s) * kPartsUp;
         pj[0].all();
         __builtin_amdgcn_sched_barrier(0);
-        // O^T += V^T P^T; the second half of P and the next block's K are split beside it
+        // O^T += V^T P^T, P scaled up; the second half of P and the next block's K are split beside it
         slots<12 * DB>([&](auto i) {
             constexpr int step = i / 6, part = i % 6, half = step / DB, db = step % DB;
             o[db] = mma_part<part>(vt[step % 2], pj[half].p, o[db]);
@@ -169,13 +174,15 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
             constexpr int j = step;
             if constexpr (j < N) {
                 if constexpr (part == 0) kj[j].x = k.template operand<j>();
-                kj[j].template share<part>();
+                kj[j].template share<part>(lost);
             }
         });
     }
+    scale_f32_blocks(o, kPartsDown);
     fwd_small_leave<DB>(mine, WAVE_BYTES, lane, o, m_run, sum_across_halves(l_run));
     const float bad = nan_if_not_finite(o, l_run);
-    if (__builtin_amdgcn_ballot_w64(bad != bad) != 0) {
+    const bool again = bad != bad || row_that_lost(lost_rows, lane) || lanes_that_lost(lost) != 0;
+    if (__builtin_amdgcn_ballot_w64(again) != 0) {
         clear();
         for (int blk = first; blk < wr.end; blk += NW) {
             const int k0 = blk * 32;
@@ -184,7 +191,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES * SETS) __attribute__((
             native_transposed<D>(vptr + (int64_t)k0 * p.sv.t, p.sv.t, seq_len - k0, s, o, lane);
         }
         const float l_row = sum_across_halves(l_run);
-        if (bad != bad) fwd_small_leave<DB>(mine, WAVE_BYTES, lane, o, m_run, l_row);
+        if (again) fwd_small_leave<DB>(mine, WAVE_BYTES, lane, o, m_run, l_row);
     }
     __syncthreads();
     fwd_small_merge<f32_t, D, NW>(p, smem, WAVE_BYTES, wave, lane, obase, lse_base, q_pos, seq_len);

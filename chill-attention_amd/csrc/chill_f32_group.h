@@ -36,6 +36,7 @@ struct F32Share {
     int row, col, dst;  // row of the block, first column, their place in the planes of a tensor
     f32x4 x[JOBS][2];
     SplitJob job[JOBS];
+    int lost = 0;  // as SplitJob's
     __device__ __forceinline__ void init(int tid) {
         static_assert(JOBS * kF32GroupWaves * 64 >= 2 * 32 * CHUNKS && JOBS <= 4, "a share covers a block");
         const int at = JOBS >= 2 ? tid : tid % (2 * 32 * CHUNKS);
@@ -68,7 +69,7 @@ struct F32Share {
         static_for<JOBS>([&](auto i) {
             take<i>();
             load_next(i);
-            job[i].all();
+            job[i].all(lost);
             static_for<3>([&](auto part) { write<i, part>(stage); });
         });
     }
@@ -78,11 +79,34 @@ struct F32Share {
         constexpr int t = I / 6, part = I % 6;
         if constexpr (t < JOBS) {
             if constexpr (part == 0) take<t>();
-            job[t].template share<part>();
+            job[t].template share<part>(lost);
             if constexpr (part == 1) load_next(std::integral_constant<int, t>{});
         }
         if constexpr (t > 0 && t <= JOBS && part < 3) write<t - 1, part>(stage);
         if constexpr (I == 6 * N - 1 && N == JOBS) static_for<3>([&](auto k) { write<JOBS - 1, k>(stage); });
+    }
+};
+
+// Which waves have, among their own blocks, one whose splits lost bits: bit w for wave w, whose 32 rows begin 32 w behind `first`.
+// `lost` is a thread's share of block blk.  (what is in the branch runs for values below 2^-109)
+template <int MASK, bool QROWS>
+struct F32LostBlocks {
+    int waves = 0;
+    __device__ __forceinline__ void note(int& lost, int blk, int first, int seq_len, MaskArgs a) {
+        if (lanes_that_lost(lost) == 0) return;
+        lost = 0;
+#pragma unroll 1
+        for (int w = 0; w < kF32GroupWaves; w++) {
+            const TileRange wr = tile_range<MASK, QROWS>(first + 32 * w, 32, 32, seq_len, false, a);
+            if (blk >= wr.start && blk < wr.end) waves |= 1 << w;
+        }
+    }
+    // whether this wave is one of them, by what the four have seen (words at 1024 of LDS that nobody reads any more)
+    __device__ __forceinline__ bool mine(char* smem, int wave, int lane) const {
+        int* words = reinterpret_cast<int*>(smem + 1024);
+        if (lane == 0) words[wave] = waves;
+        __syncthreads();
+        return ((words[0] | words[1] | words[2] | words[3]) >> wave & 1) != 0;
     }
 };
 
@@ -102,7 +126,7 @@ __device__ __forceinline__ void clear_f32_blocks(f32x16 (&acc)[N]) {
 
 // ------------------------------------------------------------------------------------------ forward
 template <int D, int MASK>
-__global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_per_eu(D < 128 ? 2 : 1))) void fwd_group_f32_kernel(FwdParams p, int n_q_tiles, int has_full_blocks) {
+__global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_per_eu(D < 64 ? 4 : D < 128 ? 2 : 1))) void fwd_group_f32_kernel(FwdParams p, int n_q_tiles, int has_full_blocks) {
     constexpr int TQ = kF32GroupWaves * 32, NT = kF32GroupWaves * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
     constexpr int STAGE = 2 * Planes::BYTES;  // K, V
@@ -144,12 +168,17 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     auto load = [&](auto i, int blk) { share.template load<i>(kptr, p.sk.t, vptr, p.sv.t, imin(blk, last) * 32, seq_len); };
     static_for<F32Share<D>::JOBS>([&](auto i) { load(i, wg.start); });
     F32Resident<D> q;
+    uint64_t lost_rows;
     {
         F32Rows<D> rows;
         rows.load_all(F32Rows<D>::at(qptr, p.sq.t, qw, seq_len, lane));
         share.at_once(smem, [&](auto i) { load(i, wg.start + 1); });
-        q.split(rows);
+        int lost_q = 0;
+        q.split(rows, lost_q);
+        lost_rows = lanes_that_lost(lost_q);
     }
+    F32LostBlocks<MASK, true> lost;
+    lost.note(share.lost, wg.start, qb, seq_len, p.margs);
     OperandOffsets<bf16_t, D> ofs;
     ofs.init(lane);
 
@@ -215,11 +244,11 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             v[0] = Planes::transposed(v_planes, ofs, 0, 0, lane);
             softmax(s, blk);
             SplitJob pj[2];
-            pj[0].x = half_of<0>(s);
-            pj[1].x = half_of<1>(s);
+            pj[0].x = half_of<0>(s) * kPartsUp;
+            pj[1].x = half_of<1>(s) * kPartsUp;
             pj[0].all();
             __builtin_amdgcn_sched_barrier(0);
-            // O^T += V^T P^T; the second half of P is split beside it
+            // O^T += V^T P^T, P scaled up; the second half of P is split beside it
             if constexpr (D == 128) {
                 // (a block's share of O added up by itself, as in dQ: the launches of 1024 tiles and more whose keys were shared by four
                 // waves had sums a quarter as long.  Full mask B1 H4 T8192 against 64 bits, relative: four sums 7.9e-7, one 14.2e-7, this 3.6e-7)
@@ -249,6 +278,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         } else {
             share.at_once(next, load_next);
         }
+        lost.note(share.lost, imin(blk + 1, last), qb, seq_len, p.margs);
         __syncthreads();
     }
 
@@ -260,9 +290,11 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         store_row_transposed<f32_t, D>(obase + (int64_t)q_pos * p.so.t, o, 1.f / l_safe, valid, h);
         if (lse_base != nullptr && h == 0) lse_base[q_pos] = valid ? m_run + __log2f(l_safe) : 0.f;
     };
+    scale_f32_blocks(o, kPartsDown);
     store(true);
     const float bad = nan_if_not_finite(o, l_run);
-    if (__builtin_amdgcn_ballot_w64(bad != bad) != 0) {
+    const bool again = lost.mine(smem, wave, lane) || row_that_lost(lost_rows, lane) || bad != bad;
+    if (__builtin_amdgcn_ballot_w64(again) != 0) {
         clear_f32_blocks(o);
         m_run = -INFINITY;
         l_run = 0.f;
@@ -272,7 +304,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             softmax(s, blk);
             native_transposed<D>(vptr + (int64_t)k0 * p.sv.t, p.sv.t, seq_len - k0, s, o, lane);
         }
-        store(bad != bad);
+        store(again);
     }
 }
 
@@ -328,6 +360,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     const int q_pos = qw + n;
     F32Resident<D> q, d_o;
     float lse_q = 0.f, delta_q = 0.f;
+    uint64_t lost_rows;
     {
         F32Rows<D> rows;
         rows.load_all(F32Rows<D>::at(doptr, p.sdo.t, qw, seq_len, lane));
@@ -347,11 +380,15 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         } else if (q_pos < p.T) {
             delta_q = p.delta[b * p.delta_b + hd * p.delta_h + q_pos];
         }
-        d_o.split(rows);
+        d_o.split_scaled_up(rows);
         rows.load_all(F32Rows<D>::at(qptr, p.sq.t, qw, seq_len, lane));
         share.at_once(smem, [&](auto i) { load(i, wg.start + 1); });
-        q.split(rows);
+        int lost_q = 0;
+        q.split(rows, lost_q);
+        lost_rows = lanes_that_lost(lost_q);
     }
+    F32LostBlocks<MASK, true> lost;
+    lost.note(share.lost, wg.start, qb, seq_len, p.margs);
     // a row that attends to nothing has LSE2 = -inf and only masked entries (score -inf): P = exp2(-inf - 0)
     if (lse_q == -INFINITY) lse_q = 0.f;
     OperandOffsets<bf16_t, D> ofs;
@@ -379,9 +416,9 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 s[r] = 0.f;
-                dp[r] = -delta_q;
+                dp[r] = -delta_q * kPartsUp;
             }
-            // S^T and dP^T blocks: rows = keys 8 * (r / 4) + 4 * h + r % 4 of the block, column n = query row
+            // S^T and, scaled up, dP^T blocks: rows = keys 8 * (r / 4) + 4 * h + r % 4 of the block, column n = query row
             Parts x[2];
             x[0] = f32_row_operand<D>(k_planes, ofs, 0, lane);
             auto operand = [&](auto t) { x[t % 2] = f32_row_operand<D>(t < N ? k_planes : v_planes, ofs, t % N, lane); };
@@ -438,15 +475,18 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         } else {
             share.at_once(next, load_next);
         }
+        lost.note(share.lost, imin(blk + 1, last), qb, seq_len, p.margs);
         __syncthreads();
     }
 
     auto store = [&](bool mine) {
         if (mine && q_pos < p.T) store_row_transposed<f32_t, D>(dqbase + (int64_t)q_pos * p.sdq.t, dq, p.sm_scale, q_pos < seq_len, h);
     };
+    scale_f32_blocks(dq, kPartsDown);
     store(true);
     const float bad = nan_if_not_finite(dq);
-    if (__builtin_amdgcn_ballot_w64(bad != bad) != 0) {
+    const bool again = lost.mine(smem, wave, lane) || row_that_lost(lost_rows, lane) || bad != bad;
+    if (__builtin_amdgcn_ballot_w64(again) != 0) {
         clear_f32_blocks(dq);
         for (int blk = wr.start; blk < wr.end; blk++) {
             const int k0 = blk * 32;
@@ -458,7 +498,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             for (int r = 0; r < 16; r++) dp[r] = f32_probability(s[r], scale, lse_q) * (dp[r] - delta_q);
             native_transposed<D>(kb, p.sk.t, seq_len - k0, dp, dq, lane);
         }
-        store(bad != bad);
+        store(again);
     }
 }
 
@@ -537,6 +577,8 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     };
     F32Resident<D> k, v;
     float vec_next = 0.f;
+    uint64_t lost_rows = 0;
+    F32LostBlocks<MASK, false> lost;
     if (n_iters > 0) {
         static_for<F32Share<D>::JOBS>([&](auto i) { load(i); });
         vec_next = row_vec();
@@ -547,8 +589,11 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         advance();
         vec_next = row_vec();
         share.at_once(smem, [&](auto i) { load(i); });
-        k.split(kr);
-        v.split(vr);
+        int lost_kv = 0;
+        k.split(kr, lost_kv);
+        v.split(vr, lost_kv);
+        lost_rows = lanes_that_lost(lost_kv);
+        lost.note(share.lost, wg.start, kb0, seq_len, p.margs);
     }
     const int k_pos = kw + n;
     const Range vis = visible_range<MASK, false>(k_pos, seq_len, p.margs);
@@ -589,7 +634,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             });
             const f32x16 lse = read_vec(stage, 0);
             mask(s, blk);
-            // the exponentials of the first half of P in the first half of the dP chain, so that it can be split in the last step
+            // the exponentials (P, and with it dS, scaled up) of the first half of P in the first half of the dP chain, so that it can be split in the last step
             SplitJob pj[2];
             constexpr int PER = (16 + 6 * N - 7) / (6 * N - 6 > 0 ? 6 * N - 6 : 1);
             slots<6 * N>([&](auto i) {
@@ -603,14 +648,14 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
                 dp = mma_part<part>(x[t % 2], v.p[t - N], dp);
                 if constexpr (N > 1) {
 #pragma unroll
-                    for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]);
+                    for (int r = PER * i; r < PER * (i + 1) && r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]) * kPartsUp;
                     if constexpr (i == 6 * N - 6) pj[0].x = half_of<0>(s);
                     if constexpr (i >= 6 * N - 6) pj[0].template share<i % 6>();
                 }
             });
             if constexpr (N == 1) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]);
+                for (int r = 0; r < 16; r++) s[r] = f32_probability(s[r], scale, lse[r]) * kPartsUp;
                 pj[0].x = half_of<0>(s);
                 pj[0].all();
             }
@@ -655,6 +700,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
             share.at_once(next, load);
         }
         if (++blk >= wg.end) blk = wg.start;
+        if (it + 1 < n_iters) lost.note(share.lost, blk, kb0, seq_len, p.margs);
         __syncthreads();
     }
 
@@ -663,9 +709,12 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
         store_row_transposed<f32_t, D>(dkbase + (int64_t)k_pos * p.sdk.t, dk, p.sm_scale, k_pos < seq_len, h);
         store_row_transposed<f32_t, D>(dvbase + (int64_t)k_pos * p.sdv.t, dv, 1.f, k_pos < seq_len, h);
     };
+    scale_f32_blocks(dk, kPartsDown);
+    scale_f32_blocks(dv, kPartsDown);
     store(true);
     const float bad = nan_if_not_finite(dk, nan_if_not_finite(dv));
-    if (__builtin_amdgcn_ballot_w64(bad != bad) != 0) {
+    const bool again = lost.mine(smem, wave, lane) || row_that_lost(lost_rows, lane) || bad != bad;
+    if (__builtin_amdgcn_ballot_w64(again) != 0) {
         clear_f32_blocks(dk);
         clear_f32_blocks(dv);
         char* mine = smem + wave * (2 * 32 * 4) - VECS;  // (leave_vec and read_vec add VECS)
@@ -688,7 +737,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
                 native_transposed<D>(qb, p.sq.t, seq_len - row0, dp, dk, lane);
             }
         }
-        store(bad != bad);
+        store(again);
     }
 }
 

@@ -1,9 +1,9 @@
 // fp32 matrix products on the bf16 matrix instructions, without a scale.
 //
 // An fp32 value is the sum of three bf16 values, high = bf16(x), mid = bf16(x - high), low = x - high - mid, each rounded to
-// nearest: 3 x 8 bits hold the 24 of x, and bf16 has the exponent range of fp32, so the sum is exact down to 2^-109 (below it the
-// low part loses what lies under 2^-133, the smallest bf16).  Of the nine products of two such sums the three smallest, together
-// at most 2^-25 of the whole and of either sign, are left out.  v_mfma_f32_32x32x16_bf16 takes 32 cycles for 16 contraction
+// nearest: 3 x 8 bits hold the 24 of x, and bf16 has the exponent range of fp32, so the sum is exact down to 2^-109.  Of the nine
+// products of two such sums the three smallest, mid low, low mid and low low, together less than 2^-24 of the whole (2 x 2^-8 x 2^-17
+// and 2^-34), are left out.  v_mfma_f32_32x32x16_bf16 takes 32 cycles for 16 contraction
 // steps, v_mfma_f32_32x32x2_f32 64 cycles for 2: the six products take 192 cycles where the fp32 instruction takes 512.  The
 // split of an operand's eight values takes 44 vector instructions, which a wave issues between the MFMAs (SplitJob).  Every value
 // has its own exponent: no scale is shared by a slice of rows, so what a row sees decides it and nothing else.
@@ -11,6 +11,13 @@
 // An infinity has the parts inf and NaN, and so has a value that bf16(x) rounds beyond its range: sums that see one are NaN.  A
 // wave that has such sums computes its blocks again with the fp32 instruction (native_rowwise, native_transposed), and the rows that
 // have them take their result from there; the other rows keep theirs.
+//
+// Below 2^-109 the low part loses what lies under 2^-133, the smallest bf16.  P and dS, which come there by themselves, are scaled
+// by 2^16 before their split, which then is exact for every fp32 value, and the sums over them by 2^-16 at the end.  Rows of
+// Q, K, V and dO with bits below 2^-133 are noticed as they are split (SplitJob) and left to the fp32 instruction: by the waves whose
+// blocks have them, or, where the row is a wave's own, for that row alone.  Forward / dQ / dK/dV in us without both -> with them, causal
+// B4 H16 T4096 D64 720 / 940 / 1428 -> 720 / 942 / 1477, D32 389 / 521 / 712 -> 398 / 522 / 722, D128 1524 / 2084 / 2706 -> 1549 /
+// 2014 / 2727, prefix-LM B1 H8 T2048 D64 53.4 / 61.8 / 81.8 -> 53.4 / 59.7 / 84.6.
 #pragma once
 
 #include "chill_device.h"
@@ -23,6 +30,9 @@ namespace chill {
 struct Parts {
     i32x4 h, m, l;
 };
+
+// P and dS are split scaled by this (above)
+constexpr float kPartsUp = 65536.f, kPartsDown = 1.f / 65536.f;
 
 // The split of eight values, in the six shares that go behind the six MFMAs of the operand before: 44 instructions, in the order
 // of the steps and not of the values, so that four others lie between an instruction and the one that needs its result (a wave
@@ -53,6 +63,24 @@ struct SplitJob {
     }
     __device__ __forceinline__ void all() {
         static_for<44>([&](auto i) { step<i>(); });
+    }
+    // The same with a look at what the low parts round (four instructions): bits of `lost` below the 16th say that one of them is no
+    // bf16, which has the high 16.
+    template <int SHARE>
+    __device__ __forceinline__ void share(int& lost) {
+        static_for<8>([&](auto i) { watched_step<8 * SHARE + i>(lost); });
+    }
+    __device__ __forceinline__ void all(int& lost) {
+        static_for<48>([&](auto i) { watched_step<i>(lost); });
+    }
+    template <int K>
+    __device__ __forceinline__ void watched_step(int& lost) {
+        if constexpr (K < 44)
+            step<K>();
+        else
+            lost |= __builtin_bit_cast(int, x[2 * (K - 44)]) | __builtin_bit_cast(int, x[2 * (K - 44) + 1]);
+        // (here and not behind all splits, where what they round would have to be kept: dQ at head dim 128 spilled 73 registers)
+        if constexpr (K == 47) asm volatile("" : "+v"(lost));
     }
     // holds the split where it stands (the compiler moves one that is used behind a branch there)
     __device__ __forceinline__ void pin() { asm volatile("" : "+v"(p.h), "+v"(p.m), "+v"(p.l)); }
@@ -109,15 +137,31 @@ template <int D>
 struct F32Resident {
     static constexpr int N = D / 16;
     Parts p[N];
-    __device__ __forceinline__ void split(const F32Rows<D>& rows) {
+    __device__ __forceinline__ void split(const F32Rows<D>& rows, int& lost) {
         static_for<N>([&](auto j) {
             SplitJob job;
             job.x = rows.template operand<j>();
+            job.all(lost);
+            p[j] = job.p;
+        });
+    }
+    // (exact: see kPartsUp)
+    __device__ __forceinline__ void split_scaled_up(const F32Rows<D>& rows) {
+        static_for<N>([&](auto j) {
+            SplitJob job;
+            job.x = rows.template operand<j>() * kPartsUp;
             job.all();
             p[j] = job.p;
         });
     }
 };
+
+// the lanes whose splits have lost a bit
+__device__ __forceinline__ uint64_t lanes_that_lost(int lost) { return __builtin_amdgcn_ballot_w64((lost & 0xffff) != 0); }
+// whether row n, lanes n and n + 32, is among them
+__device__ __forceinline__ bool row_that_lost(uint64_t lanes, int lane) {
+    return (((uint32_t)lanes | (uint32_t)(lanes >> 32)) >> (lane & 31) & 1) != 0;
+}
 
 // The parts of 32 rows in LDS as three swizzled bf16 tiles, written row by row and read transposed.
 template <int D>
@@ -179,6 +223,14 @@ __device__ __forceinline__ float nan_if_not_finite(const f32x16 (&acc)[N], float
 #pragma unroll
         for (int r = 0; r < 16; r++) t = __builtin_fmaf(acc[i][r], 0.f, t);
     return sum_across_halves(t);
+}
+
+template <int N>
+__device__ __forceinline__ void scale_f32_blocks(f32x16 (&acc)[N], float by) {
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] *= by;
 }
 
 // ---------------------------------------------------------------- the fp32 instruction, operands from global memory
