@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     constexpr int STAGE = 2 * Planes::BYTES;  // K, V
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int bh, qt;
-    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, 2, &bh, &qt)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, f32_group_resident(D, CHILL_PASS_FWD), &bh, &qt)) return;
     qt = n_q_tiles - 1 - qt;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H, hkv = hd / p.group;
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     constexpr int PARKED = 64 * 16;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int bh, qt;
-    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, 2, &bh, &qt)) return;
+    if (!work_item(blockIdx.x, p.B * p.H, n_q_tiles, order_of(p), p.group, f32_group_resident(D, CHILL_PASS_DQ), &bh, &qt)) return;
     qt = n_q_tiles - 1 - qt;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H);
     const int hd = bh % p.H, hkv = hd / p.group;
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(kF32GroupWaves * 64) __attribute__((amdgpu_waves_pe
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // key tiles first-to-last: for causal-like masks the longest run first
     int bh, ktile;
-    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, 1, &bh, &ktile)) return;
+    if (!work_item(blockIdx.x, p.B * p.H_kv, n_k_tiles, order_of(p), 1, f32_group_resident(D, CHILL_PASS_DKDV), &bh, &ktile)) return;
     const int b = batch_by_length(p.lens, p.lens_stride, p.B, p.T, bh / p.H_kv);
     const int hkv = bh % p.H_kv;
     const int tid = threadIdx.x, lane = tid & 63;

@@ -277,7 +277,7 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 //   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 704 / 936 / 1460   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
 //       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1345 / 1792 / 2820   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
 //   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 383 / 512 / 704   D16 511 / 580 / 930 -> 321 / 382 / 597
-//   D128 causal B4 H16 T4096 2414 / 3761 / 5432 -> 1632 / 2144 / 2810   B1 H32 T2048 321 / 515 / 701 -> 246 / 331 / 352   B8 H32 T300 129 / 229 / 217 -> 87 / 116 / 125
+//   D128 causal B4 H16 T4096 2414 / 3761 / 5432 -> 1632 / 2144 / 2810   B1 H32 T2048 321 / 515 / 701 -> 208 / 276 / 358   B8 H32 T300 129 / 229 / 217 -> 87 / 116 / 125
 //       window 100 + 30 B8 H32 T800 475 / 507 / 675 -> 232 / 316 / 363   16 + 16 B8 H8 T3000 284 / 348 / 450 -> 162 / 224 / 261
 //       grouped heads B4 H32/8 T2085 1499 / 2159 / 3103 -> 963 / 1266 / 1543   B4 H32/4 T512 111 / 219 / 1271 -> 85 / 113 / 631
 //   D128 of 1024 tiles: causal B1 H16 T2048 197 / 271 / 652 -> 187 / 246 / 314   B1 H4 T8192 688 / 927 / 2561 -> 631 / 839 / 1089   B8 H32 T128 46 / 72 / 56 -> 22 / 31 / 36
@@ -302,6 +302,20 @@ constexpr TileConfig f32_group_tile_config(int D, int pass) {
     const int stage = 2 * f32_planes_bytes(D) + (pass == CHILL_PASS_DKDV ? 2 * 32 * 4 : 0);
     return TileConfig{128, 32, 4, 2 * stage + (pass == CHILL_PASS_DQ && f32_group_parks(D) ? 4 * 64 * 16 * (D / 16) : 0)};
 }
+// Workgroups that share a CU (work_item's `resident`), by the kernels' registers and LDS.  (Forward and dQ at head dim 128 with 2, by
+// which the second half of a grid of 257 to 512 came shortest first: causal B1 H32 T2048 259 / 331 us where longest first takes 216 / 278,
+// H16 T4096 486 / 627 and 407 / 532; the forward at head dims 32 and 16 with 2: B2 H24 T2048 99 and 87 us, 90 and 78 with 4; dQ at 16 92, 84)
+constexpr int f32_group_resident(int D, int pass) {
+    if (D == 128) return 1;
+    if (pass == CHILL_PASS_DKDV) return D == 64 ? 1 : 2;
+    return D == 64 ? 2 : pass == CHILL_PASS_FWD ? 4 : D == 32 ? 2 : 3;
+}
+constexpr bool f32_group_resident_fits(int D) {
+    return f32_group_resident(D, CHILL_PASS_FWD) * f32_group_tile_config(D, CHILL_PASS_FWD).lds_bytes <= 160 * 1024 &&
+           f32_group_resident(D, CHILL_PASS_DQ) * f32_group_tile_config(D, CHILL_PASS_DQ).lds_bytes <= 160 * 1024 &&
+           f32_group_resident(D, CHILL_PASS_DKDV) * f32_group_tile_config(D, CHILL_PASS_DKDV).lds_bytes <= 160 * 1024;
+}
+static_assert(f32_group_resident_fits(16) && f32_group_resident_fits(32) && f32_group_resident_fits(64) && f32_group_resident_fits(128), "LDS");
 // What such a launch asks for: at head dim 128, where a workgroup has its CU to itself either way, the LDS that the small kernels of
 // the same launch would take, which is what the report says of it.
 constexpr int f32_group_lds_bytes(int D, int pass, bool small) {
