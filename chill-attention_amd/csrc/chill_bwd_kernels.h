@@ -433,8 +433,11 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
     const long long band = mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1);
     const bool two = kDouble && PASS == 1 && small_takes_two_tiles(tiles);
     bool sets = false;
+    int lds_one = kLdsOne;
     void (*kern)(BwdParams, int, int, int) = nullptr;
     if constexpr (f32_parts_serve(D, DT)) {
+        constexpr int kLdsParts = bwd_small_lds_bytes(D, DT, PASS, true);
+        static_assert(PASS == 2 || kLdsParts == kLdsOne, "dQ: two tiles fit either way");
         if (f32_takes_parts(band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
             if constexpr (PASS == 1) {
                 kern = dq_small_f32_kernel<D, MASK_ID, 1>;
@@ -443,6 +446,7 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
             } else {
                 kern = dkdv_small_f32_kernel<D, MASK_ID>;
             }
+            lds_one = kLdsParts;
         }
     }
     if constexpr (!f32_all_parts(D, DT)) {
@@ -465,7 +469,7 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
         }
     }
     const int total = (int)(heads * (two ? (n_tiles + 1) / 2 : n_tiles));
-    const int lds_bytes = two || sets ? 2 * kLdsOne : kLdsOne;
+    const int lds_bytes = two || sets ? 2 * lds_one : lds_one;
     const bool hfb = Mask<MASK_ID>::has_full_blocks(32, 32, p.T, p.margs);
     if (lds_bytes > 48 * 1024) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -12,7 +12,7 @@ template <int D, int MASK, int TILES>
 __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_waves_per_eu(TILES))) void dq_small_f32_kernel(BwdParams p, int n_q_tiles, int total_items, int has_full_blocks) {
     constexpr int NW = kFwdSmallWaves, NT = NW * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
-    constexpr int WAVE_BYTES = bwd_small_wave_bytes(D, CHILL_F32, 1);
+    constexpr int WAVE_BYTES = bwd_small_wave_bytes(D, CHILL_F32, 1, true);
     extern __shared__ __attribute__((aligned(16))) char smem_all[];
     const int item = blockIdx.x;
     if (item >= total_items) return;
@@ -214,7 +214,7 @@ template <int D, int MASK>
 __global__ __launch_bounds__(kFwdSmallWaves * 64) void dkdv_small_f32_kernel(BwdParams p, int n_k_tiles, int total_items, int has_full_blocks) {
     constexpr int NW = kFwdSmallWaves, NT = NW * 64, DB = (D + 31) / 32, N = D / 16;
     typedef F32Planes<D> Planes;
-    constexpr int WAVE_BYTES = bwd_small_wave_bytes(D, CHILL_F32, 2);
+    constexpr int WAVE_BYTES = bwd_small_wave_bytes(D, CHILL_F32, 2, true);
     constexpr int VEC_OFF = WAVE_BYTES - 2 * 32 * 4;  // LSE2 and -delta of a block's query rows
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int item = blockIdx.x;

@@ -223,12 +223,15 @@ constexpr TileConfig small_tile_config(int mask_id, int dtype, int pass, int lds
 #ifndef CHILL_TUNE_BWD_SMALL
 #define CHILL_TUNE_BWD_SMALL 1
 #endif
-constexpr int bwd_small_wave_bytes(int D, int dtype, int outputs) {
-    const int rows = 2 * 32 * D * elem_bytes(dtype), parts = f32_parts_serve(D, dtype) ? outputs * f32_planes_bytes(D) : 0;
-    const int blocks = rows > parts ? rows : parts, partial = outputs * ((D + 31) / 32) * 16 * 64 * 4;
+// (`in_parts`: dK/dV of fp32 through bf16 parts holds three planes of both, half as much again)
+constexpr int bwd_small_wave_bytes(int D, int dtype, int outputs, bool in_parts = false) {
+    const int rows = 2 * 32 * D * elem_bytes(dtype), planes = in_parts ? outputs * f32_planes_bytes(D) : 0;
+    const int blocks = rows > planes ? rows : planes, partial = outputs * ((D + 31) / 32) * 16 * 64 * 4;
     return (blocks > partial ? blocks : partial) + 2 * 32 * 4;
 }
-constexpr int bwd_small_lds_bytes(int D, int dtype, int outputs) { return kFwdSmallWaves * bwd_small_wave_bytes(D, dtype, outputs); }
+constexpr int bwd_small_lds_bytes(int D, int dtype, int outputs, bool in_parts = false) {
+    return kFwdSmallWaves * bwd_small_wave_bytes(D, dtype, outputs, in_parts);
+}
 #ifndef CHILL_TUNE_BWD_SMALL_SCALE
 #define CHILL_TUNE_BWD_SMALL_SCALE 1
 #endif
@@ -603,7 +606,7 @@ inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, in
                     out->lds_bytes = f32_group_lds_bytes(D, pass, true);
                     return CHILL_OK;
                 }
-                *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 2), batch_heads * ((T + 31) / 32), T, band_keys);
+                *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 2, takes_parts), batch_heads * ((T + 31) / 32), T, band_keys);
                 return CHILL_OK;
             }
             if (takes_parts) {

@@ -201,6 +201,11 @@ def test_tile_table():
     assert tile_config(causal, 64, torch.float32, _lib.PASS_DQ, seq_len=1024, batch_heads=8)["lds_bytes"] < 2 * one
     assert tile_config(causal, 64, torch.float32, _lib.PASS_FWD, seq_len=1024, batch_heads=9)["lds_bytes"] == 2 * one
     assert tile_config(causal, 128, torch.float32, _lib.PASS_FWD, seq_len=1024, batch_heads=9)["lds_bytes"] == 4 * (2 * 32 * 512 + 512)
+    # (a wave's area in dK/dV: two blocks of rows, through bf16 parts, from 1024 rows on, three planes of both)
+    for D in (32, 64):
+        for T, row in ((255, 2 * 32 * 4), (1100, 2 * 3 * 32 * 2)):
+            c = tile_config(causal, D, torch.float32, _lib.PASS_DKDV, seq_len=T, batch_heads=8)
+            assert (c["rows"], c["lds_bytes"]) == (32, 4 * (row * D + 256)), (D, T, c)
     # dK/dV at 16-bit head dims <= 64: 64 key rows per workgroup of 4 waves, several workgroups per CU (at head dim 64
     # for short sequences, small grids and banded masks; long sequences: K in registers, below)
     for D, T, rows, waves in ((64, 3499, 64, 4), (32, None, 64, 4), (32, 8192, 64, 4)):

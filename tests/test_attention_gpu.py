@@ -240,7 +240,8 @@ def test_small_launch_with_two_tiles_per_workgroup(case):
             # these sizes takes ordinary kernels)
             assert pass_id != _lib.PASS_FWD and (dtype != torch.float32 or pass_id == _lib.PASS_DKDV), f"pass {pass_id} served by {cfg}"
             continue
-        single = tile_config(mask, D, dtype, pass_id, seq_len=32, batch_heads=1)
+        # (fp32 dK/dV of long rows goes through bf16 parts, which take more LDS: a launch of one such head)
+        single = tile_config(mask, D, dtype, pass_id, seq_len=T if pass_id == _lib.PASS_DKDV and dtype == torch.float32 else 32, batch_heads=1)
         assert (cfg["waves"], cfg["streamed"]) == (4, 32) and single["rows"] == 32
         if 2 * single["lds_bytes"] > 160 * 1024:
             tiles = 1
