@@ -570,9 +570,9 @@ int launch_fwd_split(const FwdParams& p, const FwdSplit& split, hipStream_t stre
     return (hipGetLastError() == hipSuccess) ? CHILL_OK : CHILL_ERR_HIP;
 }
 
-// A launch far too small for the chip: 32 query rows per workgroup, the keys split over its waves.
+// A launch far too small for the chip: 32 query rows per workgroup, the keys split over its waves (fp32: `parts`, through bf16 parts).
 template <typename E, int D, int MASK_ID>
-int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
+int launch_fwd_small(const FwdParams& p, bool parts, hipStream_t stream) {
     constexpr int kLdsOne = fwd_small_lds_bytes(D, Elem<E>::kDType);
     const int n_q_tiles = cdiv(p.T, 32);
     const long long tiles = (long long)p.B * p.H * n_q_tiles;
@@ -583,7 +583,7 @@ int launch_fwd_small(const FwdParams& p, hipStream_t stream) {
     const bool sets = kDouble && small_takes_two_sets(MASK_ID, DT, CHILL_PASS_FWD, tiles, p.T, band);
     void (*kern)(FwdParams, int, int, int) = nullptr;
     if constexpr (f32_parts_serve(D, DT)) {
-        if (f32_takes_parts(band, (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, DT)) {
+        if (parts) {
             kern = fwd_small_f32_kernel<D, MASK_ID, 1, 1>;
             if constexpr (kDouble) {
                 if (two) kern = fwd_small_f32_kernel<D, MASK_ID, 2, 1>;
@@ -652,7 +652,8 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
         constexpr bool served_by_parts = f32_parts_serve(D, Elem<E>::kDType);
         const bool parts = served_by_parts && f32_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), (long long)p.B * p.H, (long long)p.B * p.H_kv, p.T, D, Elem<E>::kDType);
         if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
-            if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, stream);
+            const bool ahead = p.lse != nullptr || f32_forward_alone_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), p.T, D);
+            if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, parts && ahead, stream);
         } else if (parts) {
             if constexpr (served_by_parts) status = launch_fwd_group<D, MASK_ID>(p, small, stream);
         } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {

@@ -294,6 +294,16 @@ constexpr bool f32_takes_parts(long long band_keys, long long heads, long long k
     if (D == 128) return band_keys >= 512 && (T >= 1024 || (T >= 512 && heads * ((T + 31) / 32) <= kComputeUnits));
     return band_keys >= 256 && T >= (D == 32 ? 257 : 1024);
 }
+// A forward without LSE2 has no backward that must see its rounding.  On few tiles at head dims 32 and 64 it takes the parts only where
+// they are ahead by themselves; the two report the same workgroup.  us, fp32 instruction -> parts:
+//   D32 causal B1 H8 T384 7.3 -> 8.4   T512 8.8 -> 9.5   full mask H8 T384 7.4 -> 8.5   window 255 + 1 H16 T2048 19.8 -> 21.9, H40 T1024 25.2 -> 29.3   chunkwise 128, 2
+//       H12 T2048 18.6 -> 21.2;   causal B1 H8 T1000 14.7 -> 13.3   H14 T1100 20.0 -> 16.3   B2 H16 T1024 25.4 -> 27.3   B2 H24 T1024 47.2 -> 40.2   B2 H16
+//       T1500 63.2 -> 50.5   window 1023 + 0 H12 T4096 69.1 -> 62.2
+//   D64 causal B1 H2 T1024 21.6 -> 22.9   window 255 + 1 H2 T2048 11.3 -> 13.9, 511 + 0 H2 T4096 15.8 -> 17.2;   causal B1 H8 T1100 29.1 -> 26.3   H24 T1300
+//       59.2 -> 56.4   H12 T3000 167 -> 152   window 1023 + 0 H12 T4096 122 -> 113
+constexpr bool f32_forward_alone_takes_parts(long long band_keys, int T, int D) {
+    return (D != 32 && D != 64) || (band_keys >= 1024 && T >= (D == 32 ? 1000 : 1025));
+}
 // The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
 // dO with LSE2 and delta.  They take every launch that the small kernels do not, of those launches the dQ and dK/dV of more than
 // 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and

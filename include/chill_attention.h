@@ -95,7 +95,8 @@ typedef enum ChillPass {
  * Every row of `o` (and of `lse`) is written: rows at or beyond lens[b] and rows whose q-tile has
  * no k-tile receive 0 (the reference leaves them at the adapter's zero-fill, chill.py:96 and
  * chill_fwd.py:70-71), so the caller may pass uninitialised memory.
- * `lse` may be NULL (return_lse = False). */
+ * `lse` may be NULL (return_lse = False).  In fp32 the rounding of `o` can depend on that: with `lse` the scores are
+ * rounded as the backward rounds them. */
 int chill_fwd(const ChillTensor4* q, const ChillTensor4* k, const ChillTensor4* v,
               const ChillTensor4* o,
               float* lse, const int64_t lse_stride[3],
