@@ -85,6 +85,7 @@ def load_library(path: str) -> ctypes.CDLL:
         "chill_tile_config": (c_int32, [c_int32, c_int32, c_int32, c_int32, P(c_int32)]),
         "chill_tile_config_for_shape": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int64, c_int32, P(c_int32)]),
         "chill_tile_config_for_launch": (c_int32, [P(ChillMaskDesc), c_int32, c_int32, c_int32, c_int64, c_int32, P(c_int32)]),
+        "chill_tile_config_for_heads": (c_int32, [P(ChillMaskDesc), c_int32, c_int32, c_int32, c_int64, c_int64, c_int32, P(c_int32)]),
         "chill_work_item": (c_int32, [c_int32, c_int32, c_int32]),
         "chill_launch_item": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, P(c_int32)]),
         "chill_launch_block": (c_int32, [MD] + [c_int32] * 8),
@@ -105,7 +106,7 @@ EXPORTED_SYMBOLS = (
     "chill_fwd", "chill_fwd_workspace", "chill_fwd_workspace_bytes", "chill_fwd_split_items", "chill_bwd_delta", "chill_bwd_dq", "chill_bwd_dq_delta", "chill_bwd_dkdv", "chill_bwd_noalloc", "chill_mask_eval_device",
     "chill_tile_ranges_device", "chill_mask_eval", "chill_mask_limits", "chill_tile_ranges",
     "chill_mask_is_full_block", "chill_mask_has_full_blocks", "chill_tile_config", "chill_tile_config_for_shape",
-    "chill_tile_config_for_launch", "chill_work_item", "chill_launch_item", "chill_launch_block",
+    "chill_tile_config_for_launch", "chill_tile_config_for_heads", "chill_work_item", "chill_launch_item", "chill_launch_block",
     "chill_mask_nnz",
     "chill_status_string", "chill_abi_version", "chill_has_user_mask",
 )

@@ -16,9 +16,10 @@ _DTYPES = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _li
 
 
 def tile_config(mask, head_dim: int, dtype: torch.dtype, pass_id: int, seq_len: int | None = None,
-                batch_heads: int = 1 << 20) -> dict:
+                batch_heads: int = 1 << 20, group: int = 1) -> dict:
     """Tile shape the library uses for ``(mask class, head_dim, dtype, pass)``; with ``seq_len`` (and
-    ``batch_heads`` = B * H) for a launch of that shape: the forward and dQ rows of 16-bit inputs at
+    ``batch_heads`` = B * H, for dK/dV B * H_kv, and ``group`` = H / H_kv, on both of which the kernels of
+    fp32 depend) for a launch of that shape: the forward and dQ rows of 16-bit inputs at
     head dim 128 use a smaller workgroup for short sequences and for grids that would not fill the chip.
     Without ``seq_len``: the row of long sequences on a full chip.
 
@@ -34,9 +35,10 @@ def tile_config(mask, head_dim: int, dtype: torch.dtype, pass_id: int, seq_len: 
     else:
         # (with the mask's arguments: the dK/dV row of a chunkwise mask depends on the chunk size)
         desc = mask.descriptor()
+        heads, kv_heads = (batch_heads * group, batch_heads) if pass_id == _lib.PASS_DKDV else (batch_heads, batch_heads // group)
         _lib.check(
-            "chill_tile_config_for_launch",
-            lib.chill_tile_config_for_launch(ctypes.byref(desc), head_dim, _DTYPES[dtype], pass_id, batch_heads, seq_len, out),
+            "chill_tile_config_for_heads",
+            lib.chill_tile_config_for_heads(ctypes.byref(desc), head_dim, _DTYPES[dtype], pass_id, heads, kv_heads, seq_len, out),
         )
     return {"rows": out[0], "streamed": out[1], "waves": out[2], "lds_bytes": out[3]}
 

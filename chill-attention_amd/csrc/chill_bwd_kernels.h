@@ -483,12 +483,12 @@ int launch_bwd_small(const BwdParams& p, hipStream_t stream) {
 
 // fp32 that fills the chip, products through bf16 parts: dQ or dK/dV.
 template <int D, int MASK_ID, int PASS>
-int launch_bwd_group(const BwdParams& p, bool small, hipStream_t stream) {
+int launch_bwd_group(const BwdParams& p, hipStream_t stream) {
     constexpr TileConfig cfg = f32_group_tile_config(D, PASS);
     const int n_tiles = cdiv(p.T, cfg.rows);
     const int64_t total = (int64_t)p.B * (PASS == CHILL_PASS_DQ ? p.H : p.H_kv) * n_tiles;
     if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
-    const int lds_bytes = f32_group_lds_bytes(D, PASS, small);
+    constexpr int lds_bytes = cfg.lds_bytes;
     void (*kern)(BwdParams, int, int);
     if constexpr (PASS == CHILL_PASS_DQ)
         kern = dq_group_f32_kernel<D, MASK_ID>;
@@ -525,7 +525,7 @@ int launch_dq(const BwdParams& args, int mask_id, hipStream_t stream) {
         if (small && !(parts && f32_takes_group((long long)p.B * p.H, p.T, D))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 1>(p, stream);
         } else if (parts) {
-            if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DQ>(p, small, stream);
+            if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DQ>(p, stream);
         } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if (regs2) {
             if constexpr (dq_regs2_is_optional(D, Elem<E>::kDType)) status = launch_dq_regs2<E, D, MASK_ID>(p, stream);
@@ -1491,7 +1491,7 @@ int launch_dkdv(const BwdParams& args, int mask_id, hipStream_t stream) {
         if (small && !(parts && f32_takes_group((long long)p.B * p.H_kv, p.T, D))) {
             if constexpr (served) status = launch_bwd_small<E, D, MASK_ID, 2>(p, stream);
         } else if (parts) {
-            if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DKDV>(p, small, stream);
+            if constexpr (served_by_parts) status = launch_bwd_group<D, MASK_ID, CHILL_PASS_DKDV>(p, stream);
         } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if (regs) {
             if constexpr (dkdv_regs_is_optional(D, Elem<E>::kDType)) status = launch_dkdv_shape<E, D, MASK_ID, false, true>(p, stream);

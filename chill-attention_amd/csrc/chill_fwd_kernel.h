@@ -615,12 +615,12 @@ int launch_fwd_small(const FwdParams& p, bool parts, hipStream_t stream) {
 
 // fp32 that fills the chip, products through bf16 parts.
 template <int D, int MASK_ID>
-int launch_fwd_group(const FwdParams& p, bool small, hipStream_t stream) {
+int launch_fwd_group(const FwdParams& p, hipStream_t stream) {
     constexpr TileConfig cfg = f32_group_tile_config(D, CHILL_PASS_FWD);
     const int n_q_tiles = cdiv(p.T, cfg.rows);
     const int64_t total = (int64_t)p.B * p.H * n_q_tiles;
     if (total > ((int64_t)1 << 30)) return CHILL_ERR_TOO_LARGE;
-    const int lds_bytes = f32_group_lds_bytes(D, CHILL_PASS_FWD, small);
+    constexpr int lds_bytes = cfg.lds_bytes;
     auto kern = fwd_group_f32_kernel<D, MASK_ID>;
     if (lds_bytes > 48 * 1024) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
@@ -655,7 +655,7 @@ int launch_fwd(const FwdParams& args, int mask_id, const FwdSplit* split, hipStr
             const bool ahead = p.lse != nullptr || f32_forward_alone_takes_parts(mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1), p.T, D);
             if constexpr (D * Elem<E>::kBytes <= 512) status = launch_fwd_small<E, D, MASK_ID>(p, parts && ahead, stream);
         } else if (parts) {
-            if constexpr (served_by_parts) status = launch_fwd_group<D, MASK_ID>(p, small, stream);
+            if constexpr (served_by_parts) status = launch_fwd_group<D, MASK_ID>(p, stream);
         } else if constexpr (f32_all_parts(D, Elem<E>::kDType)) {
         } else if constexpr (has_short_row) {
             const bool short_row = fwd_takes_short_row(MASK_ID, mask_band_keys(MASK_ID, p.margs.a0, p.margs.a1),

@@ -307,8 +307,7 @@ constexpr bool f32_forward_alone_takes_parts(long long band_keys, int T, int D) 
 // The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
 // dO with LSE2 and delta.  They take every launch that the small kernels do not, of those launches the dQ and dK/dV of more than
 // 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
-// 251 -> 199, at 1024 103 -> 116 and 129 -> 166), and at head dim 128 all of at least 1024; the report then says the 32 rows of a tile, as it does of every small launch, and
-// the waves and the LDS of the workgroup, which holds four.
+// 251 -> 199, at 1024 103 -> 116 and 129 -> 166), and at head dim 128 all of at least 1024.
 // (dQ at head dim 64: the low parts of dO, a thread's 16 bytes of each of four operands)
 constexpr bool f32_group_parks(int D) { return D == 64; }
 constexpr TileConfig f32_group_tile_config(int D, int pass) {
@@ -329,13 +328,6 @@ constexpr bool f32_group_resident_fits(int D) {
            f32_group_resident(D, CHILL_PASS_DKDV) * f32_group_tile_config(D, CHILL_PASS_DKDV).lds_bytes <= 160 * 1024;
 }
 static_assert(f32_group_resident_fits(16) && f32_group_resident_fits(32) && f32_group_resident_fits(64) && f32_group_resident_fits(128), "LDS");
-// What such a launch asks for: at head dim 128, where a workgroup has its CU to itself either way, the LDS that the small kernels of
-// the same launch would take, which is what the report says of it.
-constexpr int f32_group_lds_bytes(int D, int pass, bool small) {
-    if (!small || D != 128 || pass == CHILL_PASS_DKDV) return f32_group_tile_config(D, pass).lds_bytes;
-    return pass == CHILL_PASS_FWD ? fwd_small_lds_bytes(D, CHILL_F32) : bwd_small_lds_bytes(D, CHILL_F32, 1);
-}
-
 constexpr TileConfig fwd_tile_config(int mask_id, int D, int dtype, int T = kLongSequence) {
     const int waves = fwd_waves(mask_id, D, dtype, T);
     const int streamed = fwd_streamed(mask_id, D, dtype, T);
@@ -558,83 +550,51 @@ constexpr TileConfig dkdv_tile_config(int mask_id, int D, int dtype, bool small_
     return TileConfig{32 * dkdv_split_waves(D) / dkdv_split(D), 32, dkdv_split_waves(D), dkdv_split_lds_bytes(D, dtype)};
 }
 
-// batch_heads = B * H and T = sequence length of the launch (the forward and dQ rows depend on them);
-// T = kLongSequence for the row of long sequences on a full chip.
+// heads = B * H, kv_heads = B * H_kv and T = sequence length of the launch (the rows of a pass depend on the heads its tiles belong
+// to, in fp32 on both); T = kLongSequence for the row of long sequences on a full chip.
 // mask_arg0 = the mask's first argument (the dK/dV row of chunkwise masks depends on the chunk size), band_keys =
 // mask_band_keys of the mask (the forward and dK/dV rows of banded masks depend on the width of the band).
-inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, int D, int dtype, int pass, long long batch_heads,
-                       int T, TileConfig* out) {
+inline int tile_config(int mask_id, long long mask_arg0, long long band_keys, int D, int dtype, int pass, long long heads,
+                       long long kv_heads, int T, TileConfig* out) {
     if (dtype != CHILL_F32 && dtype != CHILL_F16 && dtype != CHILL_BF16) return CHILL_ERR_BAD_DTYPE;
     if (D != 16 && D != 32 && D != 64 && D != 128 && D != 256) return CHILL_ERR_BAD_HEAD_DIM;
-    // (the row of long sequences of fp32 at head dim 128 is that of the fp32 instruction, which the launches of few tiles take)
-    const bool takes_parts = f32_takes_parts(band_keys, batch_heads, batch_heads, T, D, dtype) && !(T == kLongSequence && D == 128);
+    if (pass != CHILL_PASS_FWD && pass != CHILL_PASS_DQ && pass != CHILL_PASS_DKDV) return CHILL_ERR_BAD_ARGUMENT;
+    const long long batch_heads = pass == CHILL_PASS_DKDV ? kv_heads : heads;
+    const bool small = T != kLongSequence && (pass == CHILL_PASS_FWD ? fwd_takes_small(mask_id, batch_heads, T, D, dtype)
+                                                                    : bwd_takes_small(mask_id, batch_heads, T, D, dtype, pass));
+    const bool parts = f32_takes_parts(band_keys, heads, kv_heads, T, D, dtype);
+    if (small && !(parts && f32_takes_group(batch_heads, T, D))) {
+        const int lds = pass == CHILL_PASS_FWD ? fwd_small_lds_bytes(D, dtype) : bwd_small_lds_bytes(D, dtype, pass == CHILL_PASS_DQ ? 1 : 2, parts);
+        *out = small_tile_config(mask_id, dtype, pass, lds, batch_heads * ((T + 31) / 32), T, band_keys);
+        return CHILL_OK;
+    }
+    if (parts) {
+        *out = f32_group_tile_config(D, pass);
+        return CHILL_OK;
+    }
     switch (pass) {
         case CHILL_PASS_FWD:
-            if (T != kLongSequence && fwd_takes_small(mask_id, batch_heads, T, D, dtype)) {
-                if (takes_parts && f32_takes_group(batch_heads, T, D)) {
-                    *out = f32_group_tile_config(D, pass);
-                    out->rows = 32;
-                    out->lds_bytes = f32_group_lds_bytes(D, pass, true);
-                    return CHILL_OK;
-                }
-                *out = small_tile_config(mask_id, dtype, pass, fwd_small_lds_bytes(D, dtype), batch_heads * ((T + 31) / 32), T, band_keys);
-                return CHILL_OK;
-            }
-            if (takes_parts) {
-                *out = f32_group_tile_config(D, pass);
-                return CHILL_OK;
-            }
             *out = fwd_tile_config(mask_id, D, dtype, fwd_takes_short_row(mask_id, band_keys, batch_heads, T) ? 1 : kLongSequence);
             return CHILL_OK;
         case CHILL_PASS_DQ:
-            if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DQ)) {
-                if (takes_parts && f32_takes_group(batch_heads, T, D)) {
-                    *out = f32_group_tile_config(D, pass);
-                    out->rows = 32;
-                    out->lds_bytes = f32_group_lds_bytes(D, pass, true);
-                    return CHILL_OK;
-                }
-                *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 1), batch_heads * ((T + 31) / 32), T, band_keys);
-                return CHILL_OK;
-            }
-            if (takes_parts) {
-                *out = f32_group_tile_config(D, pass);
-                return CHILL_OK;
-            }
             if (dq_regs2_is_optional(D, dtype) && (T == kLongSequence ? !mask_is_banded(mask_id) : dq_takes_regs2(mask_id, batch_heads, T))) {
                 *out = dq_regs2_tile_config(D, dtype);
                 return CHILL_OK;
             }
             *out = dq_tile_config(mask_id, D, dtype, (T != kLongSequence && dq_takes_short_row(batch_heads, T)) ? 1 : kLongSequence);
             return CHILL_OK;
-        case CHILL_PASS_DKDV:
-            // (for this pass batch_heads counts the key / value heads)
-            if (T != kLongSequence && bwd_takes_small(mask_id, batch_heads, T, D, dtype, CHILL_PASS_DKDV)) {
-                if (takes_parts && f32_takes_group(batch_heads, T, D)) {
-                    *out = f32_group_tile_config(D, pass);
-                    out->rows = 32;
-                    out->lds_bytes = f32_group_lds_bytes(D, pass, true);
-                    return CHILL_OK;
-                }
-                *out = small_tile_config(mask_id, dtype, pass, bwd_small_lds_bytes(D, dtype, 2, takes_parts), batch_heads * ((T + 31) / 32), T, band_keys);
-                return CHILL_OK;
-            }
-            if (takes_parts) {
-                *out = f32_group_tile_config(D, pass);
-                return CHILL_OK;
-            }
-            {
-                // (the row of long sequences on a full chip: the generated loop where there is one)
-                const bool is_long = T == kLongSequence;
-                const bool regs = dkdv_regs_is_optional(D, dtype) &&
-                                  (is_long ? (!mask_is_banded(mask_id) || dkdv_regs_serves_band(mask_id, mask_arg0, band_keys, D))
-                                           : dkdv_takes_regs(mask_id, mask_arg0, band_keys, D, batch_heads, T));
-                const bool small_row = !regs && !is_long && dkdv_takes_small_row(mask_id, batch_heads, T);
-                const bool one_stage = !regs && !small_row && dkdv_one_stage_serves(mask_id, D, dtype) &&
-                                       dkdv_takes_one_stage(mask_id, band_keys, batch_heads, is_long ? 1 : T, false);
-                *out = dkdv_tile_config(mask_id, D, dtype, small_row, regs, one_stage);
-                return CHILL_OK;
-            }
+        case CHILL_PASS_DKDV: {
+            // (the row of long sequences on a full chip: the generated loop where there is one)
+            const bool is_long = T == kLongSequence;
+            const bool regs = dkdv_regs_is_optional(D, dtype) &&
+                              (is_long ? (!mask_is_banded(mask_id) || dkdv_regs_serves_band(mask_id, mask_arg0, band_keys, D))
+                                       : dkdv_takes_regs(mask_id, mask_arg0, band_keys, D, batch_heads, T));
+            const bool small_row = !regs && !is_long && dkdv_takes_small_row(mask_id, batch_heads, T);
+            const bool one_stage = !regs && !small_row && dkdv_one_stage_serves(mask_id, D, dtype) &&
+                                   dkdv_takes_one_stage(mask_id, band_keys, batch_heads, is_long ? 1 : T, false);
+            *out = dkdv_tile_config(mask_id, D, dtype, small_row, regs, one_stage);
+            return CHILL_OK;
+        }
         default: return CHILL_ERR_BAD_ARGUMENT;
     }
 }

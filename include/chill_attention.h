@@ -276,9 +276,8 @@ int chill_tile_config(int32_t mask_id, int32_t D, int32_t dtype, int32_t pass, i
  * as {32, 32, 4, lds_bytes}, lds_bytes being the workgroup's, which in the forward and dQ holds two such
  * blocks of eight waves in all when the launch has more blocks than the chip has CUs.  Where it has no more
  * and a row sees many streamed rows, eight waves split them: {32, 32, 8, lds_bytes}.
- * chill_tile_config reports the row of long sequences on a full chip (of fp32 at head dim 128 the row of narrow
- * bands on grids of few blocks; other launches take another).  In fp32 a launch's kernels follow from H and from H_kv, and
- * the report takes batch_heads for both. */
+ * chill_tile_config reports the row of long sequences on a full chip.  In fp32 a launch's kernels follow from H and
+ * from H_kv; the report takes batch_heads for both (chill_tile_config_for_heads takes the two). */
 int chill_tile_config_for_shape(int32_t mask_id, int32_t D, int32_t dtype, int32_t pass, int64_t batch_heads,
                                 int32_t T, int32_t out[4]);
 
@@ -292,6 +291,10 @@ int chill_tile_config_for_shape(int32_t mask_id, int32_t D, int32_t dtype, int32
  * Counterpart of the autotuner's key, which includes the mask's constants (autotune.py:129-240). */
 int chill_tile_config_for_launch(const ChillMaskDesc* mask, int32_t D, int32_t dtype, int32_t pass,
                                  int64_t batch_heads, int32_t T, int32_t out[4]);
+
+/* The same for a launch of shared key / value heads: batch_heads = B * H and batch_kv_heads = B * H_kv in every pass. */
+int chill_tile_config_for_heads(const ChillMaskDesc* mask, int32_t D, int32_t dtype, int32_t pass, int64_t batch_heads,
+                                int64_t batch_kv_heads, int32_t T, int32_t out[4]);
 
 /* Number of unmasked (q, k) pairs with q, k < T, closed form per mask — the numerator of the
  * effective-FLOP metric (benchmark/benchmark.py:271-276 takes it from the dense mask). */

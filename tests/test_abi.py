@@ -133,9 +133,9 @@ def test_tile_table():
                     # one wave per 32 resident rows, or (dK/dV) two or four waves per 32 rows, or one wave per 64
                     assert c["rows"] in (64 * c["waves"], 32 * c["waves"], 16 * c["waves"], 8 * c["waves"]) and c["streamed"] % 32 == 0
                     assert 0 < c["lds_bytes"] <= 160 * 1024
-    # fp32 rows of 512 bytes and more: the waves of a 32-key block split its state
-    assert tile_config(ca.CausalChillMask(), 128, torch.float32, _lib.PASS_DKDV)["waves"] == 8
-    assert tile_config(ca.CausalChillMask(), 128, torch.float32, _lib.PASS_DKDV)["rows"] == 128
+    # fp32 rows of 512 bytes and more: the waves of a 32-key block split its state (at head dim 128 on short rows and few tiles)
+    c = tile_config(ca.CausalChillMask(), 128, torch.float32, _lib.PASS_DKDV, seq_len=500, batch_heads=8)
+    assert c["waves"] == 8 and c["rows"] == 128
     assert tile_config(ca.CausalChillMask(), 256, torch.float32, _lib.PASS_DKDV)["rows"] == 32
     # rows the tile sweep put into the table (mask- and head-dim-specific)
     causal, window = ca.CausalChillMask(), ca.SlidingWindowChillMask(128, 128)
@@ -171,17 +171,17 @@ def test_tile_table():
             (causal, torch.bfloat16, 64, _lib.PASS_FWD, 16, 1024, True), (prefix, torch.float16, 32, _lib.PASS_FWD, 17, 1024, False),
             (causal, torch.bfloat16, 128, _lib.PASS_FWD, 16, 1024, True), (causal, torch.bfloat16, 128, _lib.PASS_FWD, 17, 1024, False),
             (causal, torch.float32, 64, _lib.PASS_FWD, 32, 2048, True), (causal, torch.float32, 64, _lib.PASS_FWD, 33, 2048, False),
-            (prefix, torch.float32, 128, _lib.PASS_FWD, 24, 2048, True), (prefix, torch.float32, 128, _lib.PASS_FWD, 25, 2048, False),
+            (prefix, torch.float32, 128, _lib.PASS_FWD, 15, 2048, True), (prefix, torch.float32, 128, _lib.PASS_FWD, 16, 2048, False),
             (full, torch.float32, 64, _lib.PASS_FWD, 24, 2048, True), (window, torch.float32, 64, _lib.PASS_FWD, 25, 2048, False),
             (causal, torch.float32, 64, _lib.PASS_FWD, 1, 16384, True), (causal, torch.float32, 64, _lib.PASS_FWD, 1, 16385, False),
             (causal, torch.bfloat16, 64, _lib.PASS_FWD, 1, 16384, True), (causal, torch.bfloat16, 64, _lib.PASS_FWD, 1, 16385, False),
             (full, torch.float32, 128, _lib.PASS_DQ, 2, 8192, True), (full, torch.float32, 64, _lib.PASS_DKDV, 2, 8192, True),
-            (causal, torch.float32, 64, _lib.PASS_DQ, 128, 4096, True), (causal, torch.float32, 32, _lib.PASS_DQ, 129, 4096, False),
-            (causal, torch.float32, 128, _lib.PASS_DQ, 64, 4096, True), (causal, torch.float32, 128, _lib.PASS_DQ, 65, 4096, False),
+            (causal, torch.float32, 64, _lib.PASS_DQ, 16, 4096, True), (causal, torch.float32, 32, _lib.PASS_DQ, 17, 4096, False),
+            (causal, torch.float32, 128, _lib.PASS_DQ, 7, 4096, True), (causal, torch.float32, 128, _lib.PASS_DQ, 8, 4096, False),
             (full, torch.float32, 64, _lib.PASS_DQ, 24, 2048, True), (full, torch.float32, 64, _lib.PASS_DQ, 25, 2048, False),
             (causal, torch.float16, 64, _lib.PASS_DQ, 16, 1024, True), (full, torch.float16, 128, _lib.PASS_DQ, 16, 1024, True),
             (causal, torch.float16, 128, _lib.PASS_DQ, 17, 1024, False), (window, torch.float16, 128, _lib.PASS_DQ, 2, 8192, True),
-            (causal, torch.float32, 64, _lib.PASS_DKDV, 64, 2048, True), (causal, torch.float32, 64, _lib.PASS_DKDV, 65, 2048, False),
+            (causal, torch.float32, 64, _lib.PASS_DKDV, 32, 2048, True), (causal, torch.float32, 64, _lib.PASS_DKDV, 33, 2048, False),
             (prefix, torch.float32, 32, _lib.PASS_DKDV, 8, 4096, True), (prefix, torch.float32, 32, _lib.PASS_DKDV, 9, 4096, False),
             (full, torch.float32, 64, _lib.PASS_DKDV, 8, 2048, True), (full, torch.float32, 64, _lib.PASS_DKDV, 9, 2048, False),
             (causal, torch.float32, 128, _lib.PASS_DKDV, 1, 512, False), (causal, torch.bfloat16, 64, _lib.PASS_DKDV, 8, 1024, True),
@@ -201,6 +201,18 @@ def test_tile_table():
     assert tile_config(causal, 64, torch.float32, _lib.PASS_DQ, seq_len=1024, batch_heads=8)["lds_bytes"] < 2 * one
     assert tile_config(causal, 64, torch.float32, _lib.PASS_FWD, seq_len=1024, batch_heads=9)["lds_bytes"] == 2 * one
     assert tile_config(causal, 128, torch.float32, _lib.PASS_FWD, seq_len=1024, batch_heads=9)["lds_bytes"] == 4 * (2 * 32 * 512 + 512)
+    # fp32 that fills the chip: 128 rows a workgroup, two stages of the three planes of two tensors (the low parts of dO, or LSE2 and delta)
+    for mask, D, p, bh, T in ((causal, 64, _lib.PASS_DQ, 128, 4096), (causal, 64, _lib.PASS_DKDV, 64, 2048), (causal, 128, _lib.PASS_FWD, 24, 2048),
+                              (window, 128, _lib.PASS_DKDV, 128, 300), (causal, 32, _lib.PASS_DQ, 65, 1024), (full, 16, _lib.PASS_FWD, 65, 1024)):
+        want = {"rows": 128, "streamed": 32, "waves": 4,
+                "lds_bytes": 2 * 2 * 3 * 32 * 2 * D + {_lib.PASS_FWD: 0, _lib.PASS_DQ: 16384 * (D == 64), _lib.PASS_DKDV: 512}[p]}
+        assert tile_config(mask, D, torch.float32, p, seq_len=T, batch_heads=bh) == want, (mask, D, p, bh, T)
+        assert tile_config(mask, D, torch.float32, p) == want
+    # (which kernels follow from both numbers of heads: 1024 tiles of query heads at head dim 128, of key / value heads 128)
+    assert tile_config(causal, 128, torch.float32, _lib.PASS_DKDV, seq_len=128, batch_heads=32, group=8)["waves"] == 4
+    assert tile_config(causal, 128, torch.float32, _lib.PASS_DKDV, seq_len=128, batch_heads=32)["waves"] == 8
+    assert tile_config(causal, 64, torch.float32, _lib.PASS_FWD, seq_len=300, batch_heads=256)["rows"] == 128
+    assert tile_config(causal, 64, torch.float32, _lib.PASS_FWD, seq_len=300, batch_heads=256, group=4)["lds_bytes"] != 2 * 2 * 3 * 32 * 2 * 64
     # (a wave's area in dK/dV: two blocks of rows, through bf16 parts, from 1024 rows on, three planes of both)
     for D in (32, 64):
         for T, row in ((255, 2 * 32 * 4), (1100, 2 * 3 * 32 * 2)):
