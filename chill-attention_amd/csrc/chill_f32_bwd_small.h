@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kFwdSmallWaves * 64 * TILES) __attribute__((amdgpu_
     const lds_char* planes = (const lds_char*)mine;
     // Two waves a SIMD have 256 registers each, 12 too few at head dim 64.  The low parts of dO lie in LDS, behind the planes: a register reloaded
     // from scratch memory waits for every row of K and V requested before it (prefix-LM B1 H8 T2048
-    // 71.6 -> 67.7 us, causal B1 H2 T8192 217 -> 167; up to 4 are left)
+    // 71.6 -> 67.7 us, causal B1 H2 T8192 217 -> 167; one is left)
     constexpr bool kParked = TILES == 2 && D == 64;
     constexpr int PARKED = 64 * 16;
     static_assert(!kParked || Planes::BYTES + N * PARKED <= WAVE_BYTES, "room behind the planes");

@@ -9,9 +9,9 @@
 // 309, 425 and 510 registers in the three kernels.  dK/dV at head dim 16 spills 43 to 53 of 256, all but four of them around what it
 // leaves to the fp32 instruction, behind the loop.
 // What bounds it: issue.  At head dim 64 a block is 48, 72 and 96 MFMAs of 32 cycles and 330 to 560 vector instructions to a wave, which
-// hide behind the MFMAs in part: those are 54, 65 and 48 % of the time (causal B4 H16 T4096, 704 / 936 / 1460 us; the fp32
-// instruction's own cycles are 86, 90 and 84 % of its 1157 / 1681 / 2212).  At head dim 128 (the same sizes, 2414 / 3761 / 5432 -> 1632 /
-// 2144 / 2810 us) it is 96, 144 and 192 MFMAs, 40, 46 and 47 % of the time at 2.4 GHz: a wave has its SIMD to itself.
+// hide behind the MFMAs in part: those are 53, 65 and 47 % of the time (causal B4 H16 T4096, 720 / 942 / 1477 us; the fp32
+// instruction's own cycles are 89, 89 and 84 % of its 1119 / 1708 / 2209).  At head dim 128 (the same sizes, 2300 / 3605 / 5325 -> 1549 /
+// 2014 / 2727 us) it is 96, 144 and 192 MFMAs, 42, 49 and 48 % of the time at 2.4 GHz: a wave has its SIMD to itself.
 #pragma once
 
 #include "chill_device.h"

@@ -265,26 +265,28 @@ constexpr bool bwd_takes_small(int mask_id, long long batch_heads, int T, int D,
 // together: P comes out of a score and an LSE2 of the same rounding (dQ of scores up to 50, B1 H8 T1024, off by 2.2e-6 with both
 // through the fp32 instruction, 2.0e-6 with both through parts, 4.2e-6 with one of each).
 // Forward / dQ / dK/dV in us, fp32 instruction -> parts, in the kernels of few tiles (chill_f32_fwd_small.h, chill_f32_bwd_small.h):
-//   D64 causal B2 H16 T512 18 / 25 / 35 -> 20 / 24 / 30      B1 H8 T1024 24 / 35 / 44 -> 24 / 24 / 31     B1 H4 T1111 25 / 38 / 47 -> 25 / 24 / 32
-//       B2 H16 T2048 166 / 228 / 347 -> 157 / 197 / 251      full mask B1 H8 T2048 76 / 103 / 154 -> 71 / 87 / 109
-//       window 256 B1 H8 T2048 20 / 27 / 40 -> 20 / 25 / 33  window 100 + 30 B1 H4 T1111 10 / 15 / 17 -> 12 / 11 / 15
+//   D64 causal B1 H8 T1024 22 / 31 / 41 -> 24 / 22 / 30   B1 H4 T1111 24 / 36 / 45 -> 25 / 23 / 32   B2 H16 T2048 166 / 231 / 337 -> 162 / 187 / 262
+//       full mask B1 H8 T2048 78 / 104 / 144 -> 72 / 83 / 114   window 256 B1 H8 T2048 19 / 28 / 39 -> 20 / 23 / 34
 //   D128 (dK/dV in the kernel of launches that fill the chip, which is ahead however few tiles there are: the parts of Q and dO of four
-//        waves do not fit in LDS)   causal B1 H8 T512 26 / 37 / 168 -> 25 / 27 / 80   B1 H8 T1024 47 / 66 / 329 -> 42 / 44 / 148
-//       B1 H24 T1024 92 / 131 / 339 -> 78 / 88 / 144   B1 H8 T2048 98 / 136 / 635 -> 85 / 94 / 276   B1 H2 T8192 368 / 496 / 2546 -> 262 / 303 / 1063
-//       full mask B1 H8 T2048 168 / 231 / 637 -> 155 / 167 / 306   window 256 + 256 B1 H4 T2048 35 / 47 / 212 -> 32 / 35 / 102
-//       outside the rule, the forward: causal B1 H8 T256 15.9 -> 18.3   B4 H8 T512 37.1 -> 38.7   window 100 + 30 B1 H16 T1024 34.2 -> 37.8
-//       chunkwise 128, 2 B1 H8 T4001 85.4 -> 90.4
-//   D32 causal B8 H8 T256 9 / 12 / 13 -> 10 / 11 / 16        B1 H8 T512 9 / 12 / 15 -> 11 / 10 / 12       B1 H16 T1100 30 / 43 / 38 -> 30 / 32 / 35
-//   D16 causal B8 H8 T256 7 / 8 / 10 -> 7 / 7 / 9            B4 H8 T1100 32 / 37 / 47 -> 25 / 29 / 33
+//        waves do not fit in LDS)   causal B1 H8 T512 23 / 35 / 164 -> 24 / 27 / 80   B1 H8 T1024 42 / 61 / 317 -> 41 / 44 / 148
+//       B1 H24 T1024 77 / 115 / 319 -> 82 / 92 / 150   B1 H8 T2048 89 / 128 / 623 -> 89 / 98 / 282   B1 H2 T8192 341 / 474 / 2516 -> 330 / 361 / 1144
+//       full mask B1 H8 T2048 155 / 216 / 628 -> 152 / 168 / 290   window 256 + 256 B1 H4 T2048 30 / 43 / 201 -> 30 / 34 / 98
+//   D32 causal B1 H8 T512 9 / 11 / 14 -> 10 / 9 / 12   B1 H16 T1100 28 / 41 / 34 -> 28 / 31 / 27   D16 B8 H8 T256 6.5 / 7.1 / 9.1 -> 5.8 / 6.1 / 7.8
+//       B4 H8 T1100 32 / 36 / 43 -> 25 / 29 / 32
+//   outside the rule, the forward alone: D64 causal B2 H16 T512 18 -> 20   window 100 + 30 B1 H4 T1111 10 -> 12   D128 causal B1 H8 T256 15.9 -> 18.3
+//       B4 H8 T512 37.1 -> 38.7   window 100 + 30 B1 H16 T1024 34.2 -> 37.8   chunkwise 128, 2 B1 H8 T4001 85.4 -> 90.4
 // and in those that fill the chip (chill_f32_group.h):
-//   D64 causal B4 H16 T4096 1157 / 1681 / 2212 -> 704 / 936 / 1460   B8 H32 T300 63 / 100 / 143 -> 40 / 51 / 77   B32 H32 T128 51 / 114 / 156 -> 37 / 54 / 87
-//       full mask B4 H16 T4096 2231 / 3187 / 4237 -> 1345 / 1792 / 2820   window 100 + 30 B8 H32 T800 205 / 267 / 335 -> 96 / 125 / 212
-//   D32 causal B4 H16 T4096 634 / 934 / 1140 -> 383 / 512 / 704   D16 511 / 580 / 930 -> 321 / 382 / 597
-//   D128 causal B4 H16 T4096 2414 / 3761 / 5432 -> 1632 / 2144 / 2810   B1 H32 T2048 321 / 515 / 701 -> 208 / 276 / 358   B8 H32 T300 129 / 229 / 217 -> 87 / 116 / 125
-//       window 100 + 30 B8 H32 T800 475 / 507 / 675 -> 232 / 316 / 363   16 + 16 B8 H8 T3000 284 / 348 / 450 -> 162 / 224 / 261
-//       grouped heads B4 H32/8 T2085 1499 / 2159 / 3103 -> 963 / 1266 / 1543   B4 H32/4 T512 111 / 219 / 1271 -> 85 / 113 / 631
-//   D128 of 1024 tiles: causal B1 H16 T2048 197 / 271 / 652 -> 187 / 246 / 314   B1 H4 T8192 688 / 927 / 2561 -> 631 / 839 / 1089   B8 H32 T128 46 / 72 / 56 -> 22 / 31 / 36
-//       full mask B1 H16 T2048 366 / 495 / 697 -> 227 / 302 / 385
+//   D64 causal B4 H16 T4096 1119 / 1708 / 2209 -> 745 / 971 / 1531   B8 H32 T300 55 / 96 / 139 -> 38 / 47 / 72   B32 H32 T128 49 / 118 / 163 -> 39 / 50 / 86
+//       full mask B4 H16 T4096 2101 / 3014 / 4227 -> 1428 / 1885 / 2822   window 100 + 30 B8 H32 T800 182 / 207 / 329 -> 94 / 125 / 205
+//   D32 causal B4 H16 T4096 660 / 987 / 1147 -> 409 / 539 / 758   D16 503 / 592 / 920 -> 350 / 403 / 660
+//   D128 causal B4 H16 T4096 2300 / 3605 / 5325 -> 1708 / 2175 / 2865   B1 H32 T2048 301 / 495 / 695 -> 220 / 278 / 372   B8 H32 T300 123 / 219 / 213 -> 90 / 118 / 133
+//       window 100 + 30 B8 H32 T800 440 / 482 / 660 -> 232 / 307 / 368   16 + 16 B8 H8 T3000 258 / 333 / 442 -> 165 / 224 / 275
+//       grouped heads B4 H32/8 T2085 1493 / 2043 / 3044 -> 972 / 1277 / 1666   B4 H32/4 T512 109 / 209 / 1253 -> 83 / 107 / 566
+//   D128 of 1024 tiles: causal B1 H16 T2048 169 / 248 / 628 -> 179 / 218 / 289   B1 H4 T8192 610 / 855 / 2522 -> 688 / 832 / 1119   B8 H32 T128 41 / 69 / 54 -> 23 / 31 / 38
+//       full mask B1 H16 T2048 327 / 441 / 643 -> 198 / 260 / 355
+// (Counting key / value heads at head dims 32 and 64 keeps grouped launches on the fp32 instruction that would be faster through parts in
+// all passes, by the query heads: window 100 + 30 B8 H32/8 T800 D64 181 / 203 / 355 -> 93 / 116 / 197, causal 235 / 374 / 397 -> 147 /
+// 191 / 312, T300 56 / 97 / 84 -> 36 / 45 / 67.  That is not done yet.)
 constexpr long long f32_group_tiles(int D) { return D == 128 ? 4 * kComputeUnits - 1 : 8 * kComputeUnits; }
 constexpr bool f32_takes_group(long long heads, int T, int D) { return heads * (((long long)T + 31) / 32) > f32_group_tiles(D); }
 constexpr bool f32_all_parts(int D, int dtype) { return f32_parts_serve(D, dtype) && D < 32; }
@@ -306,7 +308,7 @@ constexpr bool f32_forward_alone_takes_parts(long long band_keys, int T, int D) 
 }
 // The kernels of launches that fill the chip: 128 rows a workgroup, two stages of the parts of 32 rows of K and V, in dK/dV of Q and
 // dO with LSE2 and delta.  They take every launch that the small kernels do not, of those launches the dQ and dK/dV of more than
-// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 936 us, B4 H16 T2048 394 -> 259; dK/dV 498 -> 421; at 2048 tiles 197 -> 143 and
+// 2048 tiles too (causal D64, dQ B4 H16 T4096 1338 -> 971 us, B4 H16 T2048 394 -> 263; dK/dV 498 -> 415; at 2048 tiles 197 -> 143 and
 // 251 -> 199, at 1024 103 -> 116 and 129 -> 166), and at head dim 128 all of at least 1024.
 // (dQ at head dim 64: the low parts of dO, a thread's 16 bytes of each of four operands)
 constexpr bool f32_group_parks(int D) { return D == 64; }
