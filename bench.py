@@ -39,9 +39,9 @@ PEAK_HBM_GBS = 8000.0
 # sources it was measured on (kernel_sources_digest below); with other sources the line reports null.
 TRAFFIC_SOURCE = "profiles/c3_causal_bf16_fwd_bwd_kernels.md"
 MEASURED_TRAFFIC = {
-    ("C3", "chill_fwd"): (568018 * 2.0 + 352258) * 1024,
-    ("C3", "chill_bwd_dq_delta"): (1131349 * 2.0 + 290816) * 1024,
-    ("C3", "chill_bwd_dkdv"): (1195746 * 2.0 + 573440) * 1024,
+    ("C3", "chill_fwd"): (572901 * 2.0 + 352257) * 1024,
+    ("C3", "chill_bwd_dq_delta"): (1130087 * 2.0 + 290816) * 1024,
+    ("C3", "chill_bwd_dkdv"): (1195244 * 2.0 + 573439) * 1024,
 }
 
 
