@@ -1,7 +1,7 @@
 """Static MI355X tile table (the counterpart of the reference's ``autotune.py`` default tables).
 
-The table itself is compiled into the HIP library (``csrc/chill_tiles.h``) so the kernels and this
-report cannot disagree; these helpers only read it.
+The table and the rules that choose its rows are compiled into the HIP library (``csrc/chill_tiles.h``),
+where the launchers take both from the same functions; these helpers only read them.
 """
 
 from __future__ import annotations
